@@ -46,6 +46,16 @@ def test_int4_gemv_export_equals_the_oracle_and_the_definition(rows, n):
     assert np.max(np.abs(y - want)) <= 1e-5 * max(1.0, np.max(np.abs(want))) + 1e-4
 
 
+@pytest.mark.parametrize("n", [64, 448, 512, 576, 2880])  # under, at and past the eight groups a table of products covers
+@pytest.mark.parametrize("rows", [3, 4, 15, 16, 17, 32, 33, 47, 49])  # blocks of sixteen rows, two at a time, and what is left
+def test_int4_gemv_in_blocks_of_rows_equals_the_oracle(rows, n):
+    tree = S.SeedTree(0xB10C + rows * 4096 + n)
+    w, s, b = S.affine_matrix(tree.key("w"), rows, n, 4, S.META_BF16)
+    x = tree.key("x").normal(n).astype(np.float32)
+    y = HL.int4_affine_gemv(w, s, b, x, rows, n)
+    assert np.array_equal(y.view(np.uint32), O.int4_affine_gemv(w, s, b, x, rows, n, S.META_BF16).view(np.uint32))
+
+
 def test_cpu_expert_ffn_accumulate_equals_the_oracle_bit_for_bit_and_accumulates():
     d, f = 2048, 512
     tree = S.SeedTree(0xA11F)
