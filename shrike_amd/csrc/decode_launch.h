@@ -71,7 +71,7 @@ struct NormArgs {
 
 int launch_router(const RouterArgs &a, uint32_t router_bits, hipStream_t s);
 // the same for `tokens` tokens in one launch; a.counter must have a zeroed word for each
-constexpr uint32_t kRouterLaunchTokens = 16;  // up to here the one-launch router beats the three-launch prefill router
+constexpr uint32_t kRouterLaunchTokens = 16;  // tokens the one-launch router takes at most
 int launch_router_tokens(const RouterArgs &a, uint32_t router_bits, uint32_t tokens, hipStream_t s);
 // router logit rows + the shared expert's gate/up rows in one grid
 // norm: null, or the norm to run in every workgroup's prologue (r.hidden and g.x are then not read)

@@ -9,116 +9,154 @@
 
 namespace shrike {
 
-constexpr uint32_t kRouterTokenBlock = 4;  // tokens a wave runs one expert row against
-
-// prefill.metal:369-439: logits of every (token, expert). A wave holds one expert and walks
-// kRouterTokenBlock tokens, so the row comes from HBM once and from L1 afterwards. The row
-// arithmetic is the decode router's, operand for operand.
+// ---- router logits of a block of tokens (prefill.metal:369-439)
+//
+// x * effective_scale is the same for every expert: a workgroup forms the products (router_row's, moe.metal:357-358) once
+// per token while staging the row in LDS, keeps its experts' rows in registers and walks a block of tokens, TPS of them a
+// step, the next step's rows in flight while one is multiplied. The additions are router_row's, in router_row's order
+// (lane l: chunks l, l + 64, ..., xor butterfly), so the logits are the decode router's bits.
+//
+// A wave keeps ROWS expert rows, MAXC 16-byte chunks a lane and row, as packed fp16: the fp16 rows as they are, the codes
+// of an affine row widened once (every code is exact in fp16). A multiply-add that takes its fp16 factor as it is
+// (v_fma_mix_f32) then widens it for nothing, and a row costs half the registers. An affine row's second operand, the
+// chunk's sum of x, does not depend on the row either: it is formed while staging, in router_row's order.
+//
+// Bound by the vector unit: one multiply-add a code and token (55 us of them for 4,096 tokens of 2,048 against 256 rows).
+// Router launches (logits and select), before and after the affine rows went this way and the butterfly left LDS: 8-bit
+// rows, 1,000 tokens of 2,304 against 256: 195 -> 50 us; 4-bit rows, 512 of 2,048: 176 -> 24; fp16 rows, 1,000 of 2,304:
+// 63 -> 36 (four rows a wave instead of two), 4,096 of 2,048: 94 -> 87.
 template <int RK>
-__global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t query_count, uint32_t stride, float *ws) {
-    warm_kernel_arguments(a);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t e = blockIdx.x * 4u + wave;
-    if (e >= a.sel.num_experts) return;
-#pragma unroll 1
-    for (uint32_t i = 0; i < kRouterTokenBlock; ++i) {
-        const uint32_t t = blockIdx.y * kRouterTokenBlock + i;
-        if (t >= query_count) break;
-        RouterArgs b = a;
-        b.hidden = a.hidden + size_t(t) * stride;
-        b.logits_out = ws + size_t(t) * a.sel.num_experts;
-        router_row<RK>(b, e, lane);
-    }
-}
+constexpr int kRouterChunk = RK == 0 ? 8 : RK == 8 ? 16 : 32;  // elements of a 16-byte chunk of a row
 
-// The fp16 router's fast path. x * effective_scale is the same for every expert: a workgroup forms
-// the products (router_row's, moe.metal:357-358) once per token while staging the row in LDS, keeps its
-// experts' rows in registers and walks a block of tokens, the next step's rows in flight while one is
-// multiplied. The additions are router_row's, in router_row's order, so the logits are the same bits.
-
-// A wave keeps ROWS fp16 router rows in registers (MAXI 16-byte chunks a lane and row); the workgroup
-// walks a block of TOKENS tokens, TPS of them a step: their x rows are staged once in LDS (the next
-// step's in flight while one is multiplied) for the four waves to read, and the TPS * ROWS sums of a step
-// go through the butterfly side by side. Every logit is summed in the decode router's order (lane l:
-// chunks l, l+64, ..., xor butterfly).
 // One stage of the split butterfly over LIVE sums (a power of two above 1) at lane distance 32 >> STAGE: the partner with
 // the distance's bit set keeps the upper half of the sums and sends the lower, the other the reverse; each adds the
-// partner's copy of what it keeps. LIVE / 2 sums are left in v[0 .. LIVE / 2).
+// partner's copy of what it keeps. LIVE / 2 sums are left in v[0 .. LIVE / 2). At distances 32 and 16 the exchange is one
+// swap instruction a pair of sums (after it one register holds what the lane keeps and what its partner sent, the other
+// the rest), at 8 a rotation within the row of sixteen lanes; none goes through LDS as a shuffle would.
 template <uint32_t LIVE, uint32_t STAGE>
 __device__ __forceinline__ void split_stage(float *v, uint32_t lane) {
-    constexpr int kDistance = 32 >> STAGE;
-    const bool upper = (lane & uint32_t(kDistance)) != 0u;
+    static_assert(STAGE <= 2u, "the split stages are those at distances 32, 16 and 8");
 #pragma unroll
     for (uint32_t j = 0; j < LIVE / 2u; ++j) {
-        const float keep = upper ? v[j + LIVE / 2u] : v[j], send = upper ? v[j] : v[j + LIVE / 2u];
-        v[j] = __fadd_rn(keep, __shfl_xor(send, kDistance));
+        const uint32_t a = __float_as_uint(v[j]), b = __float_as_uint(v[j + LIVE / 2u]);
+        if constexpr (STAGE == 0u) {
+            const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+            v[j] = __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        } else if constexpr (STAGE == 1u) {
+            const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+            v[j] = __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        } else {
+            const bool upper = (lane & 8u) != 0u;
+            const float keep = __uint_as_float(upper ? b : a), send = __uint_as_float(upper ? a : b);
+            v[j] = __fadd_rn(keep, dpp_f32<0x128>(send));  // row_ror:8
+        }
     }
 }
-template <uint32_t SUMS, uint32_t STAGES>
-__device__ __forceinline__ void split_stages(float *v, uint32_t lane) {
-    if constexpr (STAGES >= 1u) split_stage<SUMS, 0>(v, lane);
-    if constexpr (STAGES >= 2u) split_stage<SUMS / 2u, 1>(v, lane);
-    if constexpr (STAGES >= 3u) split_stage<SUMS / 4u, 2>(v, lane);
+// A whole stage on one sum: every lane adds the lane at the distance.
+template <uint32_t DISTANCE>
+__device__ __forceinline__ float xor_add(float v) {
+    if constexpr (DISTANCE == 32u) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (DISTANCE == 16u) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (DISTANCE == 8u) {
+        return __fadd_rn(v, dpp_f32<0x128>(v));                // row_ror:8
+    } else if constexpr (DISTANCE == 4u) {
+        return __fadd_rn(v, dpp_f32<0x141>(dpp_f32<0x1B>(v)));  // quad reversed, then the half row mirrored: lane ^ 3 ^ 7
+    } else if constexpr (DISTANCE == 2u) {
+        return __fadd_rn(v, dpp_f32<0x4E>(v));                 // quad_perm [2,3,0,1]
+    } else {
+        return __fadd_rn(v, dpp_f32<0xB1>(v));                 // quad_perm [1,0,3,2]
+    }
 }
 
-template <int MAXI, int ROWS, uint32_t TOKENS, uint32_t TPS>
-__global__ __launch_bounds__(256) void k_prefill_logits_f16(const uint16_t *weights, const uint16_t *hidden, uint32_t stride,
-                                                            const uint16_t *eff, float *logits, uint32_t query_count,
-                                                            uint32_t num_experts, uint32_t d) {
-    // chunk c = lane + 64 i of a row is two float4: half h of it sits at [(2 i + h) * 64 + lane], so that a
-    // wave's read of one half is one contiguous kilobyte
-    __shared__ float4 s_x[2][TPS][MAXI * 2 * 64];
+template <int RK, int MAXC, int ROWS, uint32_t TPS>
+__global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t query_count, uint32_t stride, float *logits,
+                                                        uint32_t tokens_a_group) {
+    warm_kernel_arguments(a);
+    constexpr int E = kRouterChunk<RK>, P = E / 4, W = E / 2;  // a chunk's elements, float4 of x, packed fp16 words
+    // chunk c = lane + 64 i of a row is P float4: piece h sits at [(P i + h) * 64 + lane], so that a wave's read of one
+    // piece is one contiguous kilobyte
+    __shared__ float4 s_x[2][TPS][MAXC * P * 64];
+    __shared__ float s_sum[RK ? 2 : 1][RK ? TPS : 1][RK ? MAXC * 64 : 1];
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
+    const uint32_t num_experts = a.sel.num_experts, d = a.d;
     const uint32_t e0 = (blockIdx.x * 4u + wave) * ROWS;
-    const uint32_t chunks = d / 8u;
-    // the rows stay packed: a multiply-add that takes its fp16 factor as it is (v_fma_mix_f32) widens it
-    // exactly, so the sums are those of converting first, and a row costs half the registers
-    uint4 w[ROWS][MAXI];
+    const uint32_t chunks = d / E;
+    uint32_t w[ROWS][MAXC][W];
+    float sc[ROWS][MAXC], bi[ROWS][MAXC];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
         const uint32_t e = min(e0 + uint32_t(r), num_experts - 1u);  // past the last row: a copy, never stored
 #pragma unroll
-        for (int i = 0; i < MAXI; ++i) {
-            const uint32_t c = lane + 64u * i;
-            w[r][i] = *reinterpret_cast<const uint4 *>(weights + size_t(e) * d + size_t(c < chunks ? c : 0u) * 8u);
+        for (int i = 0; i < MAXC; ++i) {
+            const uint32_t c = lane + 64u * i, cc = c < chunks ? c : 0u;
+            const uint4 v = *reinterpret_cast<const uint4 *>(static_cast<const uint8_t *>(a.weights) + (size_t(e) * chunks + cc) * 16u);
+            const uint32_t vw[4] = {v.x, v.y, v.z, v.w};
+            if (RK == 0) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) w[r][i][j] = vw[j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    constexpr uint32_t mask = RK == 8 ? 0xffu : 0xfu;
+                    const uint32_t pair = vw[j * RK / 16] >> ((2 * RK * j) % 32);
+                    w[r][i][j] = as_u32(h2_t{_Float16(float(pair & mask)), _Float16(float((pair >> RK) & mask))});
+                }
+                sc[r][i] = meta_f32(a.scales[size_t(e) * (d / kGroup) + cc * E / kGroup], a.meta);
+                bi[r][i] = meta_f32(a.biases[size_t(e) * (d / kGroup) + cc * E / kGroup], a.meta);
+            }
         }
     }
-    const uint32_t t0 = blockIdx.y * TOKENS;
-    const uint32_t t1 = min(t0 + TOKENS, query_count);
+    const uint32_t t0 = blockIdx.y * tokens_a_group;
+    const uint32_t t1 = min(t0 + tokens_a_group, query_count);
     if (t0 >= t1) return;
-    // a thread stages kStage 8-element chunks of a token's row: fp16 x times bf16 effective scale, the
-    // exact fp32 product, two float4 a chunk
-    static_assert(MAXI % 4 == 0, "a workgroup of 256 threads stages 64 * MAXI chunks a token");
-    constexpr int kStage = MAXI / 4;
-    uint4 eff_c[kStage];
+    // a thread stages whole chunks of a token's row: fp16 x times bf16 effective scale, the exact fp32 product, P float4 a
+    // chunk, and for an affine row the chunk's sum
+    constexpr int kStage = (MAXC * 64 + 255) / 256, Q = E / 8;
+    uint4 eff_c[kStage][Q];
 #pragma unroll
-    for (int j = 0; j < kStage; ++j) eff_c[j] = reinterpret_cast<const uint4 *>(eff)[min(threadIdx.x + 256u * j, chunks - 1u)];
-    auto stage_load = [&](uint4 (&st)[TPS][kStage], uint32_t t) {
+    for (int j = 0; j < kStage; ++j)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) eff_c[j][q] = reinterpret_cast<const uint4 *>(a.effective_scale)[min(threadIdx.x + 256u * j, chunks - 1u) * Q + q];
+    auto stage_load = [&](uint4 (&st)[TPS][kStage][Q], uint32_t t) {
 #pragma unroll
         for (uint32_t u = 0; u < TPS; ++u) {
-            const uint4 *row = reinterpret_cast<const uint4 *>(hidden + size_t(min(t + u, t1 - 1u)) * stride);
+            const uint4 *row = reinterpret_cast<const uint4 *>(a.hidden + size_t(min(t + u, t1 - 1u)) * stride);
 #pragma unroll
-            for (int j = 0; j < kStage; ++j) st[u][j] = row[min(threadIdx.x + 256u * j, chunks - 1u)];  // past the row: a copy, never stored
+            for (int j = 0; j < kStage; ++j)
+#pragma unroll
+                for (int q = 0; q < Q; ++q) st[u][j][q] = row[min(threadIdx.x + 256u * j, chunks - 1u) * Q + q];  // past the row: a copy, never stored
         }
     };
-    auto stage_store = [&](const uint4 (&st)[TPS][kStage], uint32_t buf) {
+    auto stage_store = [&](const uint4 (&st)[TPS][kStage][Q], uint32_t buf) {
 #pragma unroll
         for (uint32_t u = 0; u < TPS; ++u)
 #pragma unroll
             for (int j = 0; j < kStage; ++j) {
                 const uint32_t c = threadIdx.x + 256u * j;
-                const uint4 xv = st[u][j], ev = eff_c[j];
-                const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w}, ew[4] = {ev.x, ev.y, ev.z, ev.w};
-                float o[8];
+                float sum = 0.0f;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {  // moe.metal:357-358 (exact product)
-                    o[2 * q] = __fmul_rn(f16_to_f32(uint16_t(xw[q])), bf16_to_f32(uint16_t(ew[q])));
-                    o[2 * q + 1] = __fmul_rn(f16_to_f32(uint16_t(xw[q] >> 16)), bf16_to_f32(uint16_t(ew[q] >> 16)));
+                for (int q = 0; q < Q; ++q) {
+                    const uint4 xv = st[u][j][q], ev = eff_c[j][q];
+                    const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w}, ew[4] = {ev.x, ev.y, ev.z, ev.w};
+                    float o[8];
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) {  // moe.metal:357-358 (exact product)
+                        o[2 * p] = __fmul_rn(f16_to_f32(uint16_t(xw[p])), bf16_to_f32(uint16_t(ew[p])));
+                        o[2 * p + 1] = __fmul_rn(f16_to_f32(uint16_t(xw[p] >> 16)), bf16_to_f32(uint16_t(ew[p] >> 16)));
+                    }
+                    if (RK != 0)
+#pragma unroll
+                        for (int p = 0; p < 8; ++p) sum = __fadd_rn(sum, o[p]);
+                    if (c < chunks) {
+                        s_x[buf][u][(P * (c >> 6) + 2u * q) * 64u + (c & 63u)] = make_float4(o[0], o[1], o[2], o[3]);
+                        s_x[buf][u][(P * (c >> 6) + 2u * q + 1u) * 64u + (c & 63u)] = make_float4(o[4], o[5], o[6], o[7]);
+                    }
                 }
-                if (c < chunks) {
-                    s_x[buf][u][(2u * (c >> 6)) * 64u + (c & 63u)] = make_float4(o[0], o[1], o[2], o[3]);
-                    s_x[buf][u][(2u * (c >> 6) + 1u) * 64u + (c & 63u)] = make_float4(o[4], o[5], o[6], o[7]);
-                }
+                if (RK != 0 && c < chunks) s_sum[buf][u][c] = sum;
             }
     };
     auto step = [&](uint32_t buf, uint32_t t) {
@@ -128,25 +166,38 @@ __global__ __launch_bounds__(256) void k_prefill_logits_f16(const uint16_t *weig
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) acc[u][r] = 0.0f;
 #pragma unroll
-        for (int i = 0; i < MAXI; ++i) {
+        for (int i = 0; i < MAXC; ++i) {
             if (lane + 64u * i < chunks) {
-                uint32_t ww[ROWS][4];
+                // the widening belongs to the multiply-add: keep it from being hoisted out of the token loop. The row's own
+                // registers are named as changed (they are not), so that nothing is copied for it.
 #pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    // the widening belongs to the multiply-add: keep it from being hoisted out of the token loop. The row's own
-                    // registers are named as changed (they are not), so that nothing is copied for it.
-                    asm volatile("" : "+v"(w[r][i].x), "+v"(w[r][i].y), "+v"(w[r][i].z), "+v"(w[r][i].w));
-                    ww[r][0] = w[r][i].x; ww[r][1] = w[r][i].y; ww[r][2] = w[r][i].z; ww[r][3] = w[r][i].w;
-                }
+                for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+                    for (int j = 0; j < W; j += 4)
+                        asm volatile("" : "+v"(w[r][i][j]), "+v"(w[r][i][j + 1]), "+v"(w[r][i][j + 2]), "+v"(w[r][i][j + 3]));
 #pragma unroll
                 for (uint32_t u = 0; u < TPS; ++u) {
-                    const float4 x0 = s_x[buf][u][(2 * i) * 64 + lane], x1 = s_x[buf][u][(2 * i + 1) * 64 + lane];
-                    const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+                    float part[ROWS];
 #pragma unroll
-                    for (int r = 0; r < ROWS; ++r)
+                    for (int r = 0; r < ROWS; ++r) part[r] = RK == 0 ? acc[u][r] : 0.0f;
 #pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            acc[u][r] = fmaf(f16_to_f32(uint16_t(ww[r][j / 2] >> (16 * (j % 2)))), xv[j], acc[u][r]);
+                    for (int h = 0; h < P; ++h) {
+                        const float4 x4 = s_x[buf][u][(P * i + h) * 64 + lane];
+                        const float xv[4] = {x4.x, x4.y, x4.z, x4.w};
+#pragma unroll
+                        for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                part[r] = fmaf(f16_to_f32(uint16_t(w[r][i][2 * h + j / 2] >> (16 * (j % 2)))), xv[j], part[r]);
+                    }
+                    if (RK == 0) {
+#pragma unroll
+                        for (int r = 0; r < ROWS; ++r) acc[u][r] = part[r];
+                    } else {
+                        const float sum = s_sum[buf][u][lane + 64u * i];
+#pragma unroll
+                        for (int r = 0; r < ROWS; ++r) acc[u][r] = fmaf(bi[r][i], sum, fmaf(sc[r][i], part[r], acc[u][r]));
+                    }
                 }
             }
         }
@@ -156,26 +207,27 @@ __global__ __launch_bounds__(256) void k_prefill_logits_f16(const uint16_t *weig
         // lane (the same two operands, and addition commutes), so every sum is router_row's bit for bit. Sum j ends in the
         // lanes whose upper bits spell j.
         constexpr uint32_t kSums = TPS * uint32_t(ROWS);
-        static_assert(kSums == 1u || kSums == 2u || kSums == 4u || kSums == 8u, "the split butterfly takes 1, 2, 4 or 8 sums");
+        static_assert(kSums == 4u || kSums == 8u, "the split butterfly takes 4 or 8 sums");
         float v[kSums];
 #pragma unroll
         for (uint32_t u = 0; u < TPS; ++u)
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) v[u * ROWS + r] = acc[u][r];
         // (every index below is a constant: with the number of live sums in a variable the compiler kept v in private memory)
-        constexpr uint32_t kSplitStages = kSums == 8u ? 3u : kSums == 4u ? 2u : kSums == 2u ? 1u : 0u;
-        split_stages<kSums, kSplitStages>(v, lane);
-#pragma unroll
-        for (int o = 32 >> kSplitStages; o >= 1; o >>= 1) v[0] = __fadd_rn(v[0], __shfl_xor(v[0], o));
+        split_stage<kSums, 0>(v, lane);
+        split_stage<kSums / 2u, 1>(v, lane);
+        if constexpr (kSums == 8u) split_stage<2u, 2>(v, lane);
+        else v[0] = xor_add<8>(v[0]);
+        v[0] = xor_add<1>(xor_add<2>(xor_add<4>(v[0])));
         // which sum this lane holds: one bit a split, from the first split (xor 32) down
-        constexpr uint32_t kSplits = kSums == 8u ? 3u : kSums == 4u ? 2u : kSums == 2u ? 1u : 0u;
-        const uint32_t mine = kSplits ? lane >> (6u - kSplits) : 0u;
+        constexpr uint32_t kSplits = kSums == 8u ? 3u : 2u;
+        const uint32_t mine = lane >> (6u - kSplits);
         if ((lane & ((64u >> kSplits) - 1u)) == 0u) {
             const uint32_t u = mine / uint32_t(ROWS), r = mine % uint32_t(ROWS);
             if (t + u < t1 && e0 + r < num_experts) logits[size_t(t + u) * num_experts + e0 + r] = v[0];
         }
     };
-    uint4 staged[TPS][kStage];  // live across a step's arithmetic; handed to the lambdas as a parameter so it stays in registers
+    uint4 staged[TPS][kStage][Q];  // live across a step's arithmetic; handed to the lambdas as a parameter so it stays in registers
     stage_load(staged, t0);
     stage_store(staged, 0);
     __syncthreads();
@@ -189,16 +241,17 @@ __global__ __launch_bounds__(256) void k_prefill_logits_f16(const uint16_t *weig
     }
 }
 
-constexpr uint32_t kLogitTokens = 8;  // tokens a workgroup walks with its rows: small blocks, many workgroups
-constexpr uint32_t kLogitTokensPerStep = 2;
-
-template <int MAXI, int ROWS>
-static void launch_prefill_logits_f16(const uint16_t *weights, const uint16_t *hidden, uint32_t stride, const uint16_t *eff,
-                                      float *logits, uint32_t query_count, uint32_t num_experts, uint32_t d, hipStream_t s) {
-    const uint32_t per_block = 4u * ROWS;
-    hipLaunchKernelGGL((k_prefill_logits_f16<MAXI, ROWS, kLogitTokens, kLogitTokensPerStep>),
-                       dim3((num_experts + per_block - 1u) / per_block, (query_count + kLogitTokens - 1u) / kLogitTokens),
-                       dim3(256), 0, s, weights, hidden, stride, eff, logits, query_count, num_experts, d);
+template <int RK, int MAXC, int ROWS>
+static void launch_prefill_logits(const RouterArgs &a, uint32_t query_count, uint32_t stride, float *logits, hipStream_t s) {
+    constexpr uint32_t kStepTokens = 2;
+    const uint32_t blocks = (a.sel.num_experts + 4u * ROWS - 1u) / (4u * ROWS);
+    // Tokens a workgroup walks with its rows: as few as a step takes while that still leaves the chip short of workgroups
+    // (37 tokens, 256 rows: 9.1 us with 2, 11.7 with 8), more where there are plenty, since a workgroup first fetches its
+    // rows (4,096 tokens: 114 us with 2, 94 with 4, 87 with 8 and 16; past 16 the last wave of workgroups costs more).
+    uint32_t tokens = kStepTokens;
+    while (tokens < 16u && blocks * ((query_count + tokens - 1u) / tokens) > 1280u) tokens *= 2u;
+    hipLaunchKernelGGL((k_prefill_logits<RK, MAXC, ROWS, kStepTokens>), dim3(blocks, (query_count + tokens - 1u) / tokens), dim3(256),
+                       0, s, a, query_count, stride, logits, tokens);
 }
 
 // prefill.metal:441-563: one wave selects for one token.
@@ -587,9 +640,13 @@ static int prefill_router(shrike_hip_moe *moe, void *stream, const void *d_weigh
     a.sel.sigmoid = moe->desc.sigmoid_router_scores;
     a.sel.scaling = moe->desc.routed_scaling_factor;
     hipStream_t s = as_stream(stream);
-    if (query_count <= kRouterLaunchTokens) {
-        // a handful of tokens (decode for several sequences): the decode router's kernel with the tokens
-        // on the grid, one launch for logits and selection instead of three
+    // A few tokens over a few experts: the decode router's kernel with the tokens on the grid, one launch for logits and
+    // selection. Past about 512 rows in all its workgroups (a row a wave, the rows fetched again for every token) cost more
+    // than a second launch (256 rows: 2 tokens 7.3 against 6.9 us, 8 tokens 11.4 against 7.2), and where the group sums are
+    // wanted too it would need a second launch anyway; of affine rows the two launches widen every code first, which one or
+    // two tokens do not pay back (8.8 against 9.7 us).
+    const bool few_rows = uint64_t(query_count) * num_experts <= 512u && query_count <= kRouterLaunchTokens;
+    if (few_rows && (d_group_sums == nullptr || (moe->desc.router_weight_bits != 0 && query_count <= 2u))) {
         a.logits_out = d_logits_workspace;
         a.sel.logits = d_logits_workspace;
         a.lists.out_indices = d_out_indices;
@@ -599,21 +656,21 @@ static int prefill_router(shrike_hip_moe *moe, void *stream, const void *d_weigh
         if (int rc = launch_router_tokens(a, moe->desc.router_weight_bits, query_count, s)) return rc;
         return d_group_sums ? launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, d_group_sums, nullptr, s) : 0;
     }
-    const dim3 grid((num_experts + 3u) / 4u, (query_count + kRouterTokenBlock - 1u) / kRouterTokenBlock);
+    // as many rows a wave as their registers allow: four where a lane's share of a row is up to 48 elements, else two
     switch (moe->desc.router_weight_bits) {
-        case 0: {
-            // four packed rows a wave where a row is four chunks a lane, two where it is up to eight
-            const uint16_t *w16 = static_cast<const uint16_t *>(d_weights);
-            if (d <= 2048u)
-                launch_prefill_logits_f16<4, 4>(w16, a.hidden, hidden_stride_elements, a.effective_scale, d_logits_workspace, query_count,
-                                                num_experts, d, s);
-            else
-                launch_prefill_logits_f16<8, 2>(w16, a.hidden, hidden_stride_elements, a.effective_scale, d_logits_workspace, query_count,
-                                                num_experts, d, s);
+        case 0:
+            if (d <= 2048u) launch_prefill_logits<0, 4, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
+            else if (d <= 3072u) launch_prefill_logits<0, 6, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
+            else launch_prefill_logits<0, 8, 2>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             break;
-        }
-        case 8: hipLaunchKernelGGL(k_prefill_logits<8>, grid, dim3(256), 0, s, a, query_count, hidden_stride_elements, d_logits_workspace); break;
-        default: hipLaunchKernelGGL(k_prefill_logits<4>, grid, dim3(256), 0, s, a, query_count, hidden_stride_elements, d_logits_workspace); break;
+        case 8:
+            if (d <= 2048u) launch_prefill_logits<8, 2, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
+            else if (d <= 3072u) launch_prefill_logits<8, 3, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
+            else launch_prefill_logits<8, 4, 2>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
+            break;
+        default:
+            if (d <= 2048u) launch_prefill_logits<4, 1, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
+            else launch_prefill_logits<4, 2, 2>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
     }
     SHRIKE_HIP(hipGetLastError());
     if (d_group_sums)  // the selection's waves form them on the side

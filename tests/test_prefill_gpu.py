@@ -61,6 +61,24 @@ def test_prefill_router_bit_exact_and_equal_to_decode(gpu, router_bits, ne, d, k
         assert np.array_equal(dl.out_w.download(np.uint16, k), got_w[tok * k:(tok + 1) * k])
 
 
+@pytest.mark.parametrize("router_bits,ne,d,t", [
+    (0, 19, 64, 18), (0, 37, 2048, 61), (0, 20, 2112, 40), (0, 18, 3072, 35), (0, 18, 4096, 33),  # the fp16 instances' edges
+    (8, 21, 64, 19), (8, 36, 2048, 63), (8, 19, 2112, 30), (8, 18, 3072, 37), (8, 17, 4096, 41),   # the 8-bit ones
+    (4, 33, 128, 17), (4, 50, 2048, 65), (4, 19, 2176, 29), (4, 18, 4096, 31),                     # the 4-bit ones
+    (8, 256, 512, 3), (0, 64, 320, 8), (0, 64, 320, 9), (0, 256, 128, 700), (8, 100, 192, 1300)])  # tokens a launch, a workgroup
+def test_prefill_router_instances_bit_exact(gpu, router_bits, ne, d, t):
+    k = 4
+    L = Layer(0x5EED0A00 + router_bits + d, d, 64, ne, k, router_bits=router_bits)
+    L.logit_bias = S.f32_to_bf16_bits(L.tree.key("bias").normal(ne, std=0.01))
+    dl = DeviceLayer(gpu, L, resident=[])
+    x = token_rows(L, t, d)
+    _, idx, _, ws = run_router(gpu, dl, L, gpu.dev(x), t, d)
+    ref_idx, _, ref_logits = O.prefill_router(L.router_dict(), x, t, d, k, stride=d)
+    logits = ws.download(np.float32, t * ne).reshape(t, ne)
+    assert np.array_equal(logits.view(np.uint32), ref_logits.view(np.uint32))
+    assert np.array_equal(idx.download(np.uint32, t * k), ref_idx)
+
+
 @pytest.mark.parametrize("router_bits,ne,d,f,k,t,pad,bits", [
     (0, 64, 2048, 512, 8, 70, 0, 4),     # the fp16 logits kernel with four packed rows a wave forms the sums itself
     (0, 24, 2880, 384, 4, 21, 8, 8),     # the instance for longer rows; an odd token count, padded rows
