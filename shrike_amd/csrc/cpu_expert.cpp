@@ -79,11 +79,14 @@ void gemv_rows_scalar(const uint8_t *weights, const uint16_t *scales, const uint
 // for all rows (each the very product the scalar loop forms), and a row's code picks its product by a permute, which
 // reads the low four bits of its index lane alone: per sixteen rows and byte of codes two shifts, two permutes, two
 // additions and 0.8 of a shuffle. One expert of 2048 x 512 (1.77 MB) on one core of an EPYC with 512-bit pipes:
-// 591 us row by row (3.0 GB/s), 74 us so (24 GB/s); 2880 x 2880: 4,643 and 619 us.
+// 591 us row by row (3.0 GB/s), so 82 us from the caches and 108 us from DRAM (16 GB/s); 2880 x 2880: 4,643 us, and 585
+// and 815 us. (Tables of eight groups, which fit the first-level cache, have every row visited in shorter pieces: 114 and
+// 1,137 us from DRAM; a table over the whole row: 126 and 793.)
 #define SHRIKE_AVX512 __attribute__((target("avx512f,avx512bw,avx512vl")))
 
 constexpr size_t kLanes = 16;
-constexpr size_t kChunkGroups = 8;  // groups whose product tables are in the first-level cache at once (512 * 64 bytes)
+constexpr size_t kChunkGroups = 8;                   // groups whose metadata a block of rows widens at once
+constexpr size_t kStretchGroups = 4 * kChunkGroups;  // groups of one table of products: 128 KB, from the second-level cache
 
 // The 16-bit metadata of up to eight groups of a block's rows as fp32, out[g] = the rows' values of group g.
 SHRIKE_AVX512 inline void widen_metadata(const uint16_t *const (&row)[kLanes], size_t groups_here, __m512 (&out)[kChunkGroups]) {
@@ -155,7 +158,14 @@ SHRIKE_AVX512 void gemv_block(const uint8_t *weights, const uint16_t *scales, co
         widen_metadata(b_row, groups_here, b[k]);
         acc[k] = first ? _mm512_setzero_ps() : _mm512_maskz_loadu_ps(live[k], out + r0);
     }
+    // the next block's codes are asked for ahead, a line (two groups) of each row at a time: thirty-two rows are more
+    // streams than the processor follows by itself (weights from DRAM: 198 us an expert of 2048 x 512 without, 108 with)
+    const bool ahead = row0 + 2 * kLanes * BLOCKS <= rows;
+    const size_t next = kLanes * BLOCKS * groups * kGroupBytes;
     for (size_t g = 0; g < groups_here; ++g) {
+        if (ahead && g % 2 == 0)
+            for (int k = 0; k < BLOCKS; ++k)
+                for (size_t i = 0; i < kLanes; ++i) _mm_prefetch(reinterpret_cast<const char *>(codes[k][i] + next + g * kGroupBytes), _MM_HINT_T0);
         __m512i w[BLOCKS][8];
         __m512 dot[BLOCKS];
         for (int k = 0; k < BLOCKS; ++k) {
@@ -185,16 +195,20 @@ SHRIKE_AVX512 void gemv_block(const uint8_t *weights, const uint16_t *scales, co
 
 SHRIKE_AVX512 void gemv_rows_avx512(const uint8_t *weights, const uint16_t *scales, const uint16_t *biases, const float *x,
                                     const float *xsum, size_t rows, size_t groups, float *out) {
-    alignas(64) float table[kChunkGroups * kGroupElems * kLanes];
+    alignas(64) float table[kStretchGroups * kGroupElems * kLanes];
     const __m512 codes = _mm512_setr_ps(0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-    for (size_t g0 = 0; g0 < groups; g0 += kChunkGroups) {
-        const size_t groups_here = groups - g0 < kChunkGroups ? groups - g0 : kChunkGroups;
-        for (size_t i = 0; i < groups_here * kGroupElems; ++i)
-            _mm512_store_ps(table + i * kLanes, _mm512_mul_ps(codes, _mm512_set1_ps(x[g0 * kGroupElems + i])));
-        size_t r = 0;
-        for (; r + kLanes < rows; r += 2 * kLanes)
-            gemv_block<2>(weights, scales, biases, table, xsum, r, rows, groups, g0, groups_here, g0 == 0, out);
-        if (r < rows) gemv_block<1>(weights, scales, biases, table, xsum, r, rows, groups, g0, groups_here, g0 == 0, out);
+    for (size_t stretch = 0; stretch < groups; stretch += kStretchGroups) {
+        const size_t end = groups - stretch < kStretchGroups ? groups : stretch + kStretchGroups;
+        for (size_t i = stretch * kGroupElems; i < end * kGroupElems; ++i)
+            _mm512_store_ps(table + (i - stretch * kGroupElems) * kLanes, _mm512_mul_ps(codes, _mm512_set1_ps(x[i])));
+        for (size_t r = 0; r < rows; r += 2 * kLanes) {
+            for (size_t g0 = stretch; g0 < end; g0 += kChunkGroups) {
+                const size_t groups_here = end - g0 < kChunkGroups ? end - g0 : kChunkGroups;
+                const float *t = table + (g0 - stretch) * kGroupElems * kLanes;
+                if (rows - r > kLanes) gemv_block<2>(weights, scales, biases, t, xsum, r, rows, groups, g0, groups_here, g0 == 0, out);
+                else gemv_block<1>(weights, scales, biases, t, xsum, r, rows, groups, g0, groups_here, g0 == 0, out);
+            }
+        }
     }
 }
 
