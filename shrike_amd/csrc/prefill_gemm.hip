@@ -10,6 +10,9 @@
 // by s_g * 2^24 on the vector ALU. The bias term is one more short matrix product between
 // the per-row group sums of X (fp32 sums carried as fp16 hi + lo, see k_row_group_sums) and
 // the group biases.
+//
+// Two kernels: k_grouped_ffn gives a workgroup a row tile (or two) and a block of weight rows, k_ffn_split a smaller piece
+// whose k its waves share; routed_shape and dense_shape choose.
 #include "decode_launch.h"
 #include "prefill_common.h"
 
@@ -20,14 +23,36 @@
 namespace shrike {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr uint32_t kChunkK = 256;                 // k staged in LDS per step: four groups
-constexpr uint32_t kGroupsPerChunk = kChunkK / 64;
-constexpr uint32_t kStagePieces = kChunkK / 8;     // 16-byte pieces of one staged row
-constexpr uint32_t kStageRows = 256 / kStagePieces; // rows one pass of the workgroup stages
-constexpr uint32_t kStagePasses = kRowTile / kStageRows;
-constexpr uint32_t kLdsRow = kChunkK + 8;         // halves per staged row; the pad spreads the banks
+// ---- the shape of a workgroup's work and its LDS: places for two groups (of the codes: stages) of the operands, the one in
+// use and the one on its way, that asynchronous loads fill (lane l's piece of a load lands 16 l bytes behind the load's
+// address), and after the last product the rows on their way out.
+enum class FfnShape {
+    kSplit,  // up to 32 rows against 64 weight rows, a quarter of k a wave (k_ffn_split)
+    kTile,   // one row tile, up to 64 rows, against 256 weight rows; three workgroups a compute unit
+    kWide,   // two row tiles of one expert, up to 128 rows, against 256 weight rows; two workgroups a compute unit
+};
+constexpr uint32_t kUnitB = 64u * 64u;  // 64 bytes of codes of a wave's 64 weight rows: two groups at 4 bits, one at 8
+constexpr uint32_t kUnitS = 64u * 16u;  // four groups' scales (biases) of those rows, in a 12-byte window each
+template <bool WIDE>
+struct Lds {
+    static constexpr uint32_t kRows = WIDE ? 128u : 64u;
+    static constexpr uint32_t kUnitA = kRows * 128u;  // one group (64 k) of the rows
+    static constexpr uint32_t kB = 2u * kUnitA, kS = kB + 8u * kUnitB, kBytes = kS + 4u * kUnitS;
+    // a unit (32 groups) of the rows' group sums, two of them, where the second group's rows and the second stage's codes will be
+    static constexpr uint32_t kSums0 = kUnitA, kSums1 = kB + 4u * kUnitB;
+    static_assert(kUnitA <= 4u * kUnitB, "a unit of sums fits");
+    static constexpr uint32_t kRow = 256u + 8u;  // halves per row on the way out; the pad spreads the banks
+    static constexpr uint32_t kResident = WIDE ? 2u : 3u;  // workgroups a compute unit holds
+    static_assert(kRows * kRow * 2u <= kBytes && kBytes * kResident <= 160u * 1024u, "the rows on the way out fit, and the workgroups a compute unit");
+};
+struct SplitLds {  // of a wave: 32 rows' groups, the codes of 64 weight rows, their scales and biases
+    static constexpr uint32_t kUnitA = 32u * 128u;
+    static constexpr uint32_t kB = 2u * kUnitA, kS = kB + 2u * kUnitB, kBias = kS + kUnitS, kWave = kBias + kUnitS, kBytes = 4u * kWave;
+    static_assert(2u * kBytes <= 160u * 1024u && kBytes >= 4u * 32u * 64u * 4u, "two workgroups fit a compute unit, and the partial sums a workgroup");
+};
 static_assert(kRowTile == 64, "a row tile is one or two 32-row MFMA tiles");
 constexpr float kTwo24 = 16777216.0f;
 
@@ -54,8 +79,29 @@ struct FfnArgs {
     uint32_t dense_rows;
     uint32_t round_gate_up;        // gate and up pass through fp16 before the GLU (dequant_int4.metal:206-287)
     const uint16_t *scalar_gate;   // fp16[rows] or null: row m's output * sigmoid(gate[m]) (moe.metal:1195-1207)
-    uint32_t resident_workgroups;  // workgroups of these kernels the device holds at once (two a compute unit)
+    uint32_t resident_workgroups;  // workgroups of the launched k_grouped_ffn the device holds at once
 };
+
+// The sum of a group of 64 fp16 values of which eight neighbouring lanes hold eight each, in every one of them: a lane's
+// values in order, then the lanes pairwise (k_row_group_sums' order).
+__device__ __forceinline__ float eighth_sum(const uint32_t (&w)[4]) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        sum = __fadd_rn(sum, f16_to_f32(uint16_t(w[t])));
+        sum = __fadd_rn(sum, f16_to_f32(uint16_t(w[t] >> 16)));
+    }
+    sum = __fadd_rn(sum, dpp_f32<0xB1>(sum));  // the lane at distance 1, 2, and (its quad being equal) 4
+    sum = __fadd_rn(sum, dpp_f32<0x4E>(sum));
+    return __fadd_rn(sum, dpp_f32<0x141>(sum));
+}
+
+// The two fp16 values of a word, added to c in fp32.
+__device__ __forceinline__ float dot2_ones(uint32_t w, float c) {
+    half2v v, ones = {_Float16(1.0f), _Float16(1.0f)};
+    __builtin_memcpy(&v, &w, sizeof v);
+    return __builtin_amdgcn_fdot2(v, ones, c, false);
+}
 
 union Frag {
     half8 h;
@@ -63,14 +109,15 @@ union Frag {
     uint4 v;
 };
 
-// 4-bit: the eight codes of one word as fp16 subnormals in the order (0,4,1,5,2,6,3,7),
-// which is the order the staged A rows are permuted to.
+// 4-bit: the eight codes of one word as fp16 subnormals, in order: even and odd codes to a byte each, then pairs of bytes
+// spread over the halves of a word.
 __device__ __forceinline__ half8 codes4(uint32_t w) {
+    const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
     Frag f;
-    f.u[0] = w & 0x000f000fu;
-    f.u[1] = (w >> 4) & 0x000f000fu;
-    f.u[2] = (w >> 8) & 0x000f000fu;
-    f.u[3] = (w >> 12) & 0x000f000fu;
+    f.u[0] = __builtin_amdgcn_perm(odd, even, 0x0c040c00u);
+    f.u[1] = __builtin_amdgcn_perm(odd, even, 0x0c050c01u);
+    f.u[2] = __builtin_amdgcn_perm(odd, even, 0x0c060c02u);
+    f.u[3] = __builtin_amdgcn_perm(odd, even, 0x0c070c03u);
     return f.h;
 }
 // 8-bit: eight codes of two words, in order
@@ -83,123 +130,153 @@ __device__ __forceinline__ half8 codes8(uint32_t w0, uint32_t w1) {
     return f.h;
 }
 
-template <int BITS>
-struct BRegs {  // one lane's codes of one weight row for one group: its 32 k
-    uint4 w[BITS / 4];
-    uint16_t scale;
-};
-
-// row_s == nullptr: the codes alone (the caller has the scale already)
-template <int BITS>
-__device__ __forceinline__ void load_b(BRegs<BITS> &r, const uint8_t *row_w, const uint16_t *row_s, uint32_t g, uint32_t kb) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(row_w + size_t(g) * (kGroup * BITS / 8) + kb * (4 * BITS));
-#pragma unroll
-    for (int i = 0; i < BITS / 4; ++i) r.w[i] = p[i];
-    if (row_s) r.scale = row_s[g];
+// Asynchronous loads into LDS. The compiler does not know of them: the waits for them are counted by hand, and nothing
+// between the first and the last of them may make it issue a vector load of its own.
+__device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+__device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
+__device__ __forceinline__ void lds_load12(uint32_t lds, const void *p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx3 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+// All but the wave's last COUNT loads have landed, and its reads of LDS are done.
+template <int COUNT>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(COUNT) : "memory");
+}
+// All but the last COUNT loads have landed for every wave of the workgroup, and no wave still reads the LDS.
+template <int COUNT>
+__device__ __forceinline__ void wait_loads_and_sync() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(COUNT) : "memory");
 }
 
-template <int BITS>
-__device__ __forceinline__ half8 b_step(const BRegs<BITS> &r, int s) {
-    if (BITS == 4) {
-        const uint32_t w[4] = {r.w[0].x, r.w[0].y, r.w[0].z, r.w[0].w};
-        return codes4(w[s]);
-    } else {
-        const uint32_t w[8] = {r.w[0].x, r.w[0].y, r.w[0].z, r.w[0].w, r.w[BITS / 4 - 1].x, r.w[BITS / 4 - 1].y, r.w[BITS / 4 - 1].z, r.w[BITS / 4 - 1].w};
-        return codes8(w[2 * s], w[2 * s + 1]);
-    }
-}
+typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // eight 16-bit values, wherever they start
 
-// MODE 0: gate and up rows n0..n0+31 of one expert against the gathered token rows, GLU,
-// fp16 activations out. MODE 1: down rows n0..n0+63 against the activations, fp16 partials
-// scattered to (token, rank).
-// One row tile against one block of weight rows. MT = the tile's 32-row MFMA tiles, a template
-// parameter so that the main loop is straight-line code: the compiler is then free to put one
-// chain's matrix instructions beside another chain's vector work.
+// One row tile (WIDE: or two of an expert) against one block of weight rows, 64 rows of them a wave. MODE 0: 32 gate and
+// the same 32 up rows against the gathered token rows, GLU, fp16 activations out. MODE 1: 64 down rows against the
+// activations, fp16 partials scattered to (token, rank). MT = the 32-row MFMA tiles, META = the type of the scales and
+// biases (SHRIKE_META_*), both template parameters, so that the main loop is straight-line code.
+//
+// Everything the loop reads comes through LDS by asynchronous loads, a group of 64 k at a time: the rows (shared by the
+// waves), and each wave's own codes and scales. Loaded by the lanes themselves the codes cost the loop most of its time: a
+// lane's sixteen bytes lay a weight row from its neighbour's, 64 lines a load, and the registers that held them left one
+// workgroup a compute unit fewer. What bounds it now: with many rows the power the matrix cores draw (the clock falls to 1.3
+// to 1.75 GHz, and vector work saved in the loop buys nothing), with few of them the weights' bytes, with few workgroups a
+// wave's own chain of some 1,700 cycles a group (1,200 up to 32 rows). 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens: 843
+// -> 576 us (WIDE 541); 256 of 2,048 x 512, 4,096 tokens: 371 -> 337; 384 of 2,304 x 1,024, 8-bit, 4,000 tokens: 926 -> 758.
+//
 // MODE 0 leaves its activations through LDS: whole 16-byte pieces of a row go out together, and the group sums of the
 // tile's rows that the down product's bias term needs are formed here, in k_row_group_sums' order of additions (eight
 // lanes a group, a lane adds its eight values in order, the partial sums fold pairwise), instead of by a launch of
 // their own between the two products. Every wave of the workgroup stays to the end for the barriers.
-// META: the type of the scales and biases (SHRIKE_META_*), known to the instance so that a scale converts one way.
-template <int BITS, int MODE, bool DENSE, uint32_t MT, int META>
+template <int BITS, int MODE, bool DENSE, uint32_t MT, int META, bool WIDE>
 __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile &tile, uint32_t tile_index, uint32_t col_block,
-                                         uint16_t (&s_a)[2][kRowTile][kLdsRow]) {
+                                         uint8_t *lds) {
+    typedef Lds<WIDE> L;
     const uint32_t K = MODE == 0 ? a.d : a.f, N = MODE == 0 ? a.f : a.d;
     const uint32_t G = K / kGroup;
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
     const uint32_t col = lane & 31u, kb = lane >> 5;
     const uint32_t n0 = (col_block * 4u + wave) * (MODE == 0 ? 32u : 64u);
     const bool active = n0 < N;
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds));
+    uint16_t (*s_out)[L::kRow] = reinterpret_cast<uint16_t (*)[L::kRow]>(lds);
 
-    // ---- A staging: thread -> (row = tid / kStagePieces + kStageRows i, 16-byte piece = tid % kStagePieces)
-    const uint32_t piece = threadIdx.x % kStagePieces, row0 = threadIdx.x / kStagePieces;
-    const uint16_t *src_row[kStagePasses];
+    // ---- A: the tile's rows, a group of them (128 bytes a row) at a time. A load brings eight rows, eight lanes a row, its
+    // sixteen-byte pieces xor-ed with the row so that eight rows read at one piece touch every bank once.
+    constexpr uint32_t kLoadsA = MT;  // a wave's loads a group
+    const uint8_t *a_src[kLoadsA];
+    const uint32_t *a_sums[kLoadsA];  // the rows' group sums, for the bias term
 #pragma unroll
-    for (uint32_t i = 0; i < kStagePasses; ++i) {
-        const uint32_t r = min(row0 + kStageRows * i, tile.rows - 1u);  // rows past the tile repeat its last row
+    for (uint32_t j = 0; j < kLoadsA; ++j) {
+        const uint32_t r = min(8u * (wave + 4u * j) + (lane >> 3), tile.rows - 1u);  // rows past the tile repeat its last row
+        const uint16_t *row;
         if (MODE == 0) {
             const uint32_t token = DENSE ? tile.pair_start + r : a.pairs[tile.pair_start + r].token;
-            src_row[i] = a.hidden + size_t(token) * a.hidden_stride;
+            row = a.hidden + size_t(token) * a.hidden_stride;
+            a_sums[j] = a.hidden_sums + size_t(token) * G;
         } else {
-            src_row[i] = a.act + (size_t(tile_index) * kRowTile + r) * a.f;
+            row = a.act + (size_t(tile_index) * kRowTile + r) * a.f;
+            a_sums[j] = a.act_sums + (size_t(tile_index) * kRowTile + r) * G;
         }
+        a_src[j] = reinterpret_cast<const uint8_t *>(row) + (((lane & 7u) ^ (lane >> 3)) * 16u);
     }
-    uint4 stage[kStagePasses];
-    auto fetch = [&](uint32_t chunk) {
-        const uint32_t k = chunk * kChunkK + piece * 8u;
+    auto load_a = [&](uint32_t slot, uint32_t g) {
 #pragma unroll
-        for (uint32_t i = 0; i < kStagePasses; ++i)
-            if (i * kStageRows < MT * 32u && k < K) stage[i] = *reinterpret_cast<const uint4 *>(src_row[i] + k);
-    };
-    auto commit = [&](uint32_t buf) {
-#pragma unroll
-        for (uint32_t i = 0; i < kStagePasses; ++i) {
-            if (i * kStageRows >= MT * 32u) continue;
-            uint4 v = stage[i];
-            if (BITS == 4) {  // (0,1,2,3,4,5,6,7) -> (0,4,1,5,2,6,3,7), to meet codes4
-                uint4 p;
-                p.x = __builtin_amdgcn_perm(v.z, v.x, 0x05040100u);
-                p.y = __builtin_amdgcn_perm(v.z, v.x, 0x07060302u);
-                p.z = __builtin_amdgcn_perm(v.w, v.y, 0x05040100u);
-                p.w = __builtin_amdgcn_perm(v.w, v.y, 0x07060302u);
-                v = p;
-            }
-            *reinterpret_cast<uint4 *>(&s_a[buf][row0 + kStageRows * i][piece * 8u]) = v;
-        }
+        for (uint32_t j = 0; j < kLoadsA; ++j) lds_load16(lds0 + slot * L::kUnitA + (wave + 4u * j) * 1024u, a_src[j] + size_t(g) * 128u);
     };
 
-    // ---- B rows of this lane
-    const uint8_t *base = DENSE ? nullptr : cell_base(a.pool, tile.cell, a.stride);
+    // ---- B: a wave's own 64 weight rows (two tiles of 32), 64 bytes of each at a time
+    const uint8_t *base = DENSE ? nullptr : cell_base_uniform(a.pool, tile.cell, a.stride);
     const uint32_t row_bytes = K * BITS / 8u;
-    const uint8_t *bw[2];
-    const uint16_t *bs[2], *bb[2];
-    {
-        const uint32_t n = active ? n0 + col : 0u;
+    const uint8_t *w_base[2], *s_base[2];
+    const uint16_t *b_base[2];
+    uint32_t n_first[2];  // the tiles' first rows
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+        n_first[nt] = n0 + (MODE == 0 ? 0u : 32u * uint32_t(nt));
         if (DENSE) {
-            const int first = MODE == 0 ? 0 : 2, second = MODE == 0 ? 1 : 2;
-            const uint32_t n1 = MODE == 0 ? n : n + 32u;
-            bw[0] = a.dense_w[first] + size_t(n) * row_bytes;
-            bw[1] = a.dense_w[second] + size_t(n1) * row_bytes;
-            bs[0] = a.dense_s[first] + size_t(n) * G;
-            bs[1] = a.dense_s[second] + size_t(n1) * G;
-            bb[0] = a.dense_b[first] + size_t(n) * G;
-            bb[1] = a.dense_b[second] + size_t(n1) * G;
+            const int p = MODE == 0 ? nt : 2;
+            w_base[nt] = a.dense_w[p];
+            s_base[nt] = reinterpret_cast<const uint8_t *>(a.dense_s[p]);
+            b_base[nt] = a.dense_b[p];
         } else if (MODE == 0) {
-            bw[0] = base + a.off.gate_w_off + size_t(n) * row_bytes;
-            bw[1] = base + a.off.up_w_off + size_t(n) * row_bytes;
-            bs[0] = reinterpret_cast<const uint16_t *>(base + a.off.gate_s_off) + size_t(n) * G;
-            bs[1] = reinterpret_cast<const uint16_t *>(base + a.off.up_s_off) + size_t(n) * G;
-            bb[0] = reinterpret_cast<const uint16_t *>(base + a.off.gate_b_off) + size_t(n) * G;
-            bb[1] = reinterpret_cast<const uint16_t *>(base + a.off.up_b_off) + size_t(n) * G;
+            w_base[nt] = base + (nt ? a.off.up_w_off : a.off.gate_w_off);
+            s_base[nt] = base + (nt ? a.off.up_s_off : a.off.gate_s_off);
+            b_base[nt] = reinterpret_cast<const uint16_t *>(base + (nt ? a.off.up_b_off : a.off.gate_b_off));
         } else {
-            const uint32_t n1 = n + 32u;
-            bw[0] = base + a.off.down_w_off + size_t(n) * row_bytes;
-            bw[1] = base + a.off.down_w_off + size_t(n1) * row_bytes;
-            bs[0] = reinterpret_cast<const uint16_t *>(base + a.off.down_s_off) + size_t(n) * G;
-            bs[1] = reinterpret_cast<const uint16_t *>(base + a.off.down_s_off) + size_t(n1) * G;
-            bb[0] = reinterpret_cast<const uint16_t *>(base + a.off.down_b_off) + size_t(n) * G;
-            bb[1] = reinterpret_cast<const uint16_t *>(base + a.off.down_b_off) + size_t(n1) * G;
+            w_base[nt] = base + a.off.down_w_off;
+            s_base[nt] = base + a.off.down_s_off;
+            b_base[nt] = reinterpret_cast<const uint16_t *>(base + a.off.down_b_off);
         }
     }
+    // (rows past the last, of a block's waves that have none, are the last one's: loaded, never multiplied)
+    uint32_t b_off[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j)
+        b_off[j] = min(n_first[j >> 1] + 16u * (j & 1u) + (lane >> 2), N - 1u) * row_bytes + ((lane & 3u) ^ ((lane >> 3) & 3u)) * 16u;
+    // (at 4 bits a row of an odd number of groups ends halfway through its last stage: the lanes of the missing half take
+    // the other half's pieces, so that nothing past a tensor's last row is read)
+    const uint32_t half_back = (((lane & 3u) ^ ((lane >> 3) & 3u)) & 2u) * 16u;
+    const uint32_t lds_b = lds0 + L::kB + wave * kUnitB;
+    auto load_b = [&](uint32_t slot, uint32_t stage) {
+        const uint32_t back = BITS == 4 && 2u * stage + 1u >= G ? half_back : 0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j) lds_load16(lds_b + slot * (4u * kUnitB) + j * 1024u, w_base[j >> 1] + size_t(stage) * 64u, b_off[j] - back);
+    };
+
+    // ---- scales: of four groups at a time, lane l row l of the wave's 64. A row's run of scales is two-byte aligned; what
+    // is loaded is the window of three words that holds it, never past the word of the tensor's last scale. `s_at` is where a
+    // row's chunk starts, from the word that holds the tensor's start; the run then starts max(s_at & 3, s_at - last window)
+    // bytes into the window.
+    const uint32_t s_row[2] = {min(n_first[0] + col, N - 1u), min(n_first[1] + col, N - 1u)};
+    uint32_t s_at[2], s_last[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+        const uint32_t skew = uint32_t(reinterpret_cast<uintptr_t>(s_base[nt]) & 3u);
+        s_at[nt] = skew + s_row[nt] * G * 2u;
+        s_last[nt] = ((skew + N * G * 2u + 3u) & ~3u) - 12u;
+    }
+    const uint8_t *s_src = kb ? s_base[1] : s_base[0];
+    s_src -= reinterpret_cast<uintptr_t>(s_src) & 3u;
+    const uint32_t s_mine = kb ? s_at[1] : s_at[0], s_mine_last = kb ? s_last[1] : s_last[0];
+    const uint32_t lds_s = lds0 + L::kS + wave * kUnitS;
+    auto load_s = [&](uint32_t c) { lds_load12(lds_s, s_src + min((s_mine & ~3u) + 8u * c, s_mine_last)); };
+    const uint32_t chunks = (G + 3u) / 4u;
+
+    const uint16_t *bias_row[2] = {b_base[0] + size_t(s_row[0]) * G, b_base[1] + size_t(s_row[1]) * G};
+    auto eight_at = [&](const uint16_t *row, uint32_t at) {  // groups min(at, G - 8) ...
+        const u32x4_by2 v = *reinterpret_cast<const u32x4_by2 *>(row + min(at, G - 8u));
+        return make_uint4(v.x, v.y, v.z, v.w);
+    };
+    // what the first group needs is on its way before anything else
+    constexpr uint32_t kGroupsPerB = BITS == 4 ? 2u : 1u;
+    const uint32_t stages = (G + kGroupsPerB - 1u) / kGroupsPerB;
+    load_s(0);
+    load_b(0, 0);
+    load_a(0, 0);
 
     f32x16 total[2][MT];
 #pragma unroll
@@ -209,181 +286,196 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
 #pragma unroll
             for (int i = 0; i < 16; ++i) total[nt][mt][i] = 0.0f;
 
-    // the rows' group sums for the bias term: their addresses hang on the pair records, so they are
-    // worked out here, far ahead of their use
-    const uint32_t *sums = MODE == 0 ? a.hidden_sums : a.act_sums;
-    const uint32_t *sum_row[MT];
+    // ---- bias term: (group sums of the rows) x (group biases), sixteen k' = eight groups an MFMA, four of them a lane.
+    // The sums come through the LDS like the rows, 32 groups (128 bytes a row) a unit, two units at a time, in the places that
+    // the second group's operands will take. A weight row's biases are a lane's own loads, eight groups each; the groups of an
+    // MFMA are dealt so that a lane's eight serve two of them. The last eight start at G - 8 at the latest, and what they
+    // repeat counts as zero.
+    auto bias_f16 = [&](uint16_t bits) { return META == SHRIKE_META_BF16 ? f32_to_f16(bf16_to_f32(bits)) : bits; };
+    if (G >= 8u) {
+        for (uint32_t g0 = 0; g0 < G; g0 += 64u) {
+            if (g0) wait_loads_and_sync<0>();
+            // piece q of a unit: the four groups h of lane half k's eight, load i
 #pragma unroll
-    for (uint32_t mt = 0; mt < MT; ++mt) {
-        const uint32_t r = min(mt * 32u + col, tile.rows - 1u);
-        const uint32_t token = (MODE != 0) ? 0u : DENSE ? tile.pair_start + r : a.pairs[tile.pair_start + r].token;
-        sum_row[mt] = MODE == 0 ? sums + size_t(token) * G : sums + (size_t(tile_index) * kRowTile + r) * G;
-    }
-
-    // A row's scales for the four groups of a staged chunk are one aligned 8-byte run when G is a
-    // multiple of 4: they are then fetched a chunk ahead with one load instead of four two-byte ones
-    // (every such load costs a cache-line look-up per lane, as each lane reads a row of its own).
-    // Decided from the tensors' start (the same for every lane, a row's scales being G * 2 bytes), so
-    // that the choice is uniform over the workgroup and each variant of the loop is straight-line code.
-    static_assert(kGroupsPerChunk == 4, "a chunk's scales are read as four 16-bit values");
-    const uint32_t scale_misalign = uint32_t((reinterpret_cast<uintptr_t>(bs[0]) | reinterpret_cast<uintptr_t>(bs[1])) & 7u);
-    const bool wide_scales = (G & 3u) == 0u && __builtin_amdgcn_readfirstlane(int(scale_misalign)) == 0;
-    uint2 scales_cur[2] = {make_uint2(0u, 0u), make_uint2(0u, 0u)}, scales_nxt[2] = {make_uint2(0u, 0u), make_uint2(0u, 0u)};
-    // the codes of one group (8-bit) or two (4-bit, where the registers allow it) are on their way while a group is multiplied
-    constexpr uint32_t kAhead = BITS == 4 ? 2u : 1u;
-    BRegs<BITS> cur[2], nxt[2], nx2[2];
-    const uint32_t chunks = (K + kChunkK - 1u) / kChunkK;
-
-    // One group of 64 k: the codes of the group kAhead further on are put in flight, this group's are unpacked and
-    // multiplied, and the products are scaled into the totals.
-    auto group_step = [&](uint32_t c, uint32_t buf, uint32_t gi, auto wide_tag) {
-        constexpr bool WIDE = decltype(wide_tag)::value;
-        const uint32_t gn = min(kGroupsPerChunk * c + gi + kAhead, G - 1u);
+            for (uint32_t u = 0; u < 2u; ++u) {
+                if (g0 + 32u * u >= G) break;
+                const uint32_t q = (lane & 7u) ^ (lane >> 3);
+                const uint32_t at = min(g0 + 32u * u + 16u * (q >> 2) + 8u * ((q >> 1) & 1u), G - 8u) + 4u * (q & 1u);
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) load_b<BITS>(kAhead == 2u ? nx2[nt] : nxt[nt], bw[nt], WIDE ? nullptr : bs[nt], gn, kb);
-        half8 af[MT][4];
+                for (uint32_t j = 0; j < kLoadsA; ++j)
+                    lds_load16(lds0 + (u ? L::kSums1 : L::kSums0) + (wave + 4u * j) * 1024u, a_sums[j] + at);
+            }
+            uint4 b8[2][2][2];  // [unit][load][nt]
+            if (active) {
 #pragma unroll
-        for (uint32_t mt = 0; mt < MT; ++mt)
+                for (uint32_t u = 0; u < 2u; ++u)
 #pragma unroll
-            for (int s = 0; s < 4; ++s)
-                af[mt][s] = *reinterpret_cast<const half8 *>(&s_a[buf][mt * 32u + col][gi * 64u + kb * 32u + s * 8u]);
+                    for (uint32_t i = 0; i < 2u; ++i) {
+                        const uint32_t at = g0 + 32u * u + 16u * i;
+                        if (at >= G) break;
+#pragma unroll
+                        for (int nt = 0; nt < 2; ++nt) b8[u][i][nt] = eight_at(bias_row[nt], at + 8u * kb);
+                    }
+            }
+            wait_loads_and_sync<0>();
+            if (!active) continue;
+#pragma unroll
+            for (uint32_t u = 0; u < 2u; ++u)
+#pragma unroll
+                for (uint32_t i = 0; i < 2u; ++i) {
+                    if (g0 + 32u * u + 16u * i >= G) break;
+                    const uint32_t at = g0 + 32u * u + 16u * i + 8u * kb, repeated = at - min(at, G - 8u);
+#pragma unroll
+                    for (uint32_t h = 0; h < 2u; ++h) {
+                        const uint8_t *p = lds + (u ? L::kSums1 : L::kSums0) + col * 128u + (((4u * i + 2u * kb + h) ^ (col & 7u)) * 16u);
+                        half8 sums[MT];
+#pragma unroll
+                        for (uint32_t mt = 0; mt < MT; ++mt) sums[mt] = *reinterpret_cast<const half8 *>(p + mt * 4096u);
+#pragma unroll
+                        for (int nt = 0; nt < 2; ++nt) {
+                            const uint32_t w[4] = {b8[u][i][nt].x, b8[u][i][nt].y, b8[u][i][nt].z, b8[u][i][nt].w};
+                            Frag f;
+#pragma unroll
+                            for (uint32_t jj = 0; jj < 4u; ++jj) {  // as fp16, doubled against (hi, lo)
+                                const uint16_t bits = uint16_t(w[2u * h + jj / 2u] >> (16u * (jj & 1u)));
+                                f.u[jj] = repeated <= 4u * h + jj ? uint32_t(bias_f16(bits)) * 0x00010001u : 0u;
+                            }
+#pragma unroll
+                            for (uint32_t mt = 0; mt < MT; ++mt) total[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums[mt], f.h, total[nt][mt], 0, 0, 0);
+                        }
+                    }
+                }
+        }
+    } else if (active) {  // fewer than eight groups: one MFMA, value by value
+        const uint32_t *sums = MODE == 0 ? a.hidden_sums : a.act_sums;
+        Frag afr[MT];
+#pragma unroll
+        for (uint32_t mt = 0; mt < MT; ++mt) {
+            const uint32_t r = min(mt * 32u + col, tile.rows - 1u);
+            const uint32_t token = (MODE != 0) ? 0u : DENSE ? tile.pair_start + r : a.pairs[tile.pair_start + r].token;
+            const uint32_t *row = MODE == 0 ? sums + size_t(token) * G : sums + (size_t(tile_index) * kRowTile + r) * G;
+#pragma unroll
+            for (uint32_t jj = 0; jj < 4u; ++jj) afr[mt].u[jj] = 4u * kb + jj < G ? row[4u * kb + jj] : 0u;
+        }
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
-            half8 bf[4];
+            Frag f;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) bf[s] = b_step<BITS>(cur[nt], s);
-            const uint32_t pair = gi < 2u ? scales_cur[nt].x : scales_cur[nt].y;
-            const uint16_t scale_bits = WIDE ? uint16_t(pair >> (16u * (gi & 1u))) : cur[nt].scale;
-            const float sc = meta_f32(scale_bits, uint32_t(META)) * kTwo24;
+            for (uint32_t jj = 0; jj < 4u; ++jj)
+                f.u[jj] = 4u * kb + jj < G ? uint32_t(bias_f16(bias_row[nt][4u * kb + jj])) * 0x00010001u : 0u;
 #pragma unroll
-            for (uint32_t mt = 0; mt < MT; ++mt) {
-                f32x16 p = {0};
-#pragma unroll
-                for (int s = 0; s < 4; ++s) p = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt][s], bf[s], p, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 16; ++i) total[nt][mt][i] = fmaf(sc, p[i], total[nt][mt][i]);
-            }
-        }
-        cur[0] = nxt[0];
-        cur[1] = nxt[1];
-        if (kAhead == 2u) {
-            nxt[0] = nx2[0];
-            nxt[1] = nx2[1];
-        }
-    };
-    auto main_loop = [&](auto wide_tag) {
-        constexpr bool WIDE = decltype(wide_tag)::value;
-        if (active) {
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                load_b<BITS>(cur[nt], bw[nt], WIDE ? nullptr : bs[nt], 0, kb);
-                if (kAhead == 2u) load_b<BITS>(nxt[nt], bw[nt], WIDE ? nullptr : bs[nt], min(1u, G - 1u), kb);
-                if (WIDE) scales_cur[nt] = *reinterpret_cast<const uint2 *>(bs[nt]);
-            }
-        }
-        fetch(0);
-        commit(0);
-        __syncthreads();
-        for (uint32_t c = 0; c < chunks; ++c) {
-            const uint32_t buf = c & 1u;
-            if (c + 1u < chunks) fetch(c + 1u);
-            if (active) {
-                if (WIDE) {  // G is a multiple of 4: every chunk is whole and its four groups are one block of code
-                    if (c + 1u < chunks) {
-                        scales_nxt[0] = reinterpret_cast<const uint2 *>(bs[0])[c + 1u];
-                        scales_nxt[1] = reinterpret_cast<const uint2 *>(bs[1])[c + 1u];
-                    }
-#pragma unroll
-                    for (uint32_t gi = 0; gi < kGroupsPerChunk; ++gi) group_step(c, buf, gi, wide_tag);
-                    scales_cur[0] = scales_nxt[0];
-                    scales_cur[1] = scales_nxt[1];
-                } else {
-                    const uint32_t groups_here = min(kGroupsPerChunk, G - kGroupsPerChunk * c);
-                    for (uint32_t gi = 0; gi < groups_here; ++gi) group_step(c, buf, gi, wide_tag);
-                }
-            }
-            if (c + 1u < chunks) commit(buf ^ 1u);
-            __syncthreads();
-        }
-    };
-    if (wide_scales) main_loop(std::true_type{});
-    else main_loop(std::false_type{});
-    // (no wave leaves here: the epilogue's barrier needs them all)
-
-    // ---- bias term: (group sums of the rows) x (group biases), sixteen k' = eight groups an MFMA.
-    // The operands of four steps are fetched together, four values a load where the rows allow it.
-    if (active) {
-        // a lane's four groups are one aligned 8- or 16-byte run when G is a multiple of 4 and the bias rows start aligned
-        const bool wide = (G & 3u) == 0u && ((reinterpret_cast<uintptr_t>(bb[0]) | reinterpret_cast<uintptr_t>(bb[1])) & 7u) == 0u;
-        for (uint32_t gbase = 0; gbase < G; gbase += 32u) {
-            Frag bfr[4][2], afr[4][MT];
-#pragma unroll
-            for (uint32_t step = 0; step < 4; ++step) {
-                const uint32_t gl = gbase + 8u * step + 4u * kb;  // this lane's four groups
-                if (wide) {
-                    const bool on = gl < G;
-#pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) {
-                        const uint2 b4 = on ? *reinterpret_cast<const uint2 *>(bb[nt] + gl) : make_uint2(0u, 0u);
-                        bfr[step][nt].u[0] = b4.x & 0xffffu; bfr[step][nt].u[1] = b4.x >> 16;
-                        bfr[step][nt].u[2] = b4.y & 0xffffu; bfr[step][nt].u[3] = b4.y >> 16;
-                    }
-#pragma unroll
-                    for (uint32_t mt = 0; mt < MT; ++mt)
-                        afr[step][mt].v = on ? *reinterpret_cast<const uint4 *>(sum_row[mt] + gl) : zero4();
-                } else {
-#pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) {
-                        const bool on = gl + jj < G;
-#pragma unroll
-                        for (int nt = 0; nt < 2; ++nt) bfr[step][nt].u[jj] = on ? bb[nt][gl + jj] : 0u;
-#pragma unroll
-                        for (uint32_t mt = 0; mt < MT; ++mt) afr[step][mt].u[jj] = on ? sum_row[mt][gl + jj] : 0u;
-                    }
-                }
-            }
-#pragma unroll
-            for (uint32_t step = 0; step < 4; ++step) {
-                if (gbase + 8u * step >= G) break;
-#pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-#pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) {  // the bias as fp16, doubled against (hi, lo)
-                        uint16_t bits = uint16_t(bfr[step][nt].u[jj]);
-                        if (META == SHRIKE_META_BF16) bits = f32_to_f16(bf16_to_f32(bits));
-                        bfr[step][nt].u[jj] = uint32_t(bits) * 0x00010001u;
-                    }
-#pragma unroll
-                    for (uint32_t mt = 0; mt < MT; ++mt)
-                            total[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[step][mt].h, bfr[step][nt].h, total[nt][mt], 0, 0, 0);
-                }
-            }
+            for (uint32_t mt = 0; mt < MT; ++mt) total[nt][mt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[mt].h, f.h, total[nt][mt], 0, 0, 0);
         }
     }
+
+    // ---- the groups. Step g waits for what its group needs (the first also until nobody reads the sums any more) and asks for
+    // what a later group will, in the place that group g - 1 left.
+    uint32_t run[2][4];  // the scales of a chunk of four groups
+    auto step = [&](uint32_t g, auto par) {
+        constexpr uint32_t P = decltype(par)::value;  // g & 1
+        const uint32_t b_place = BITS == 8 ? P : (g >> 1) & 1u;
+        if (BITS == 4 && P == 1u && g + 1u < G) wait_loads_and_sync<4>();  // (the next stage's codes may still be on their way)
+        else wait_loads_and_sync<0>();
+        if (g + 1u < G) {
+            load_a(P ^ 1u, g + 1u);
+            if (BITS == 8) load_b(b_place ^ 1u, g + 1u);
+        }
+        if (BITS == 4 && P == 0u && g + 2u < G) load_b(b_place ^ 1u, (g >> 1) + 1u);
+        if (active) {
+            if ((g & 3u) == 0u) {
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) {
+                    const int into = max(int(s_at[nt] & 3u), int(s_at[nt] + g * 2u) - int(s_last[nt]));
+                    const uint8_t *p = lds + L::kS + wave * kUnitS + (uint32_t(nt) * 32u + col) * 16u + uint32_t(into);
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i) run[nt][i] = *reinterpret_cast<const uint16_t *>(p + min(i, G - 1u - g) * 2u);
+                }
+            }
+        }
+        if ((g & 3u) == 1u && g + 3u < G) load_s((g >> 2) + 1u);  // (a step's wait is for the reads above, too)
+        if (active) {
+            const uint8_t *a_rows = lds + P * L::kUnitA + col * 128u;
+            uint4 codes[2][BITS / 4];
+            float sc[2];
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                const uint8_t *rows = lds + L::kB + wave * kUnitB + b_place * (4u * kUnitB) + uint32_t(nt) * 2048u + col * 64u;
+#pragma unroll
+                for (uint32_t i = 0; i < BITS / 4; ++i) {
+                    const uint32_t piece = BITS == 4 ? P * 2u + kb : kb * 2u + i;
+                    codes[nt][i] = *reinterpret_cast<const uint4 *>(rows + ((piece ^ ((col >> 1) & 3u)) * 16u));
+                }
+                sc[nt] = meta_f32(uint16_t(run[nt][0]), uint32_t(META));
+                run[nt][0] = run[nt][1]; run[nt][1] = run[nt][2]; run[nt][2] = run[nt][3];
+            }
+            auto a_frag = [&](uint32_t mt, uint32_t s) { return *reinterpret_cast<const half8 *>(a_rows + mt * 4096u + (((kb * 4u + s) ^ (col & 7u)) * 16u)); };
+            {
+                half8 bf[2][4];
+#pragma unroll
+                for (int nt = 0; nt < 2; ++nt) {
+                    if (BITS == 4) {
+                        const uint4 c = codes[nt][0];
+                        bf[nt][0] = codes4(c.x); bf[nt][1] = codes4(c.y); bf[nt][2] = codes4(c.z); bf[nt][3] = codes4(c.w);
+                    } else {
+                        const uint4 lo = codes[nt][0], hi = codes[nt][BITS / 4 - 1];
+                        bf[nt][0] = codes8(lo.x, lo.y); bf[nt][1] = codes8(lo.z, lo.w);
+                        bf[nt][2] = codes8(hi.x, hi.y); bf[nt][3] = codes8(hi.z, hi.w);
+                    }
+                    sc[nt] *= kTwo24;
+                }
+#pragma unroll
+                for (uint32_t mt = 0; mt < MT; ++mt) {
+                    half8 af[4];
+#pragma unroll
+                    for (uint32_t s = 0; s < 4; ++s) af[s] = a_frag(mt, s);
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt) {
+                        f32x16 p = {0};
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) p = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[s], bf[nt][s], p, 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) total[nt][mt][i] = fmaf(sc[nt], p[i], total[nt][mt][i]);
+                    }
+                }
+            }
+        }
+    };
+    for (uint32_t g = 0; g + 1u < G; g += 2u) {
+        step(g, std::integral_constant<uint32_t, 0>{});
+        step(g + 1u, std::integral_constant<uint32_t, 1>{});
+    }
+    if (G & 1u) step(G - 1u, std::integral_constant<uint32_t, 0>{});
+    // nobody reads the rings any more: the LDS takes the rows on their way out
+    wait_loads_and_sync<0>();
+
     // ---- epilogue: lane holds (m = 32 mt + 8 (i / 4) + 4 kb + i % 4, n = n0 + col)
     const uint32_t n = n0 + col;
     if (MODE == 0) {
-        // the main loop ended on a barrier: nobody reads the staged rows any more, and the first buffer takes the
-        // tile's fp16 activations, [row][column of this block of 128]
+        // the tile's fp16 activations, [row][column of this block of 128]
         if (active) {
             float gab = 0.0f, uab = 0.0f;
             if (!DENSE && a.ebias) {  // moe.metal:261-269
                 gab = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.gate_ab_off)[n]);
                 uab = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.up_ab_off)[n]);
             }
+            auto activate = [&](auto act) {  // (the choice of the activation is outside the loop)
 #pragma unroll
-            for (uint32_t mt = 0; mt < MT; ++mt) {
+                for (uint32_t mt = 0; mt < MT; ++mt) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint32_t m = mt * 32u + 8u * (i / 4) + 4u * kb + (i % 4);
-                    float g = total[0][mt][i] + gab, u = total[1][mt][i] + uab;
-                    if (DENSE && a.round_gate_up) {
-                        g = f16_to_f32(f32_to_f16(g));
-                        u = f16_to_f32(f32_to_f16(u));
+                    for (int i = 0; i < 16; ++i) {
+                        const uint32_t m = mt * 32u + 8u * (i / 4) + 4u * kb + (i % 4);
+                        float g = total[0][mt][i] + gab, u = total[1][mt][i] + uab;
+                        if (DENSE && a.round_gate_up) {
+                            g = f16_to_f32(f32_to_f16(g));
+                            u = f16_to_f32(f32_to_f16(u));
+                        }
+                        s_out[m][wave * 32u + col] = f32_to_f16(glu_fast<decltype(act)::value>(g, u));
                     }
-                    s_a[0][m][wave * 32u + col] = f32_to_f16(glu_rt_fast(g, u, a.act_kind));
                 }
-            }
+            };
+            if (a.act_kind == SHRIKE_ACT_SILU) activate(std::integral_constant<int, 1>{});
+            else if (a.act_kind == SHRIKE_ACT_CLAMPED_SWIGLU) activate(std::integral_constant<int, 2>{});
+            else activate(std::integral_constant<int, 0>{});
         }
         __syncthreads();
         const uint32_t c0 = col_block * 128u, columns = min(128u, N - c0);  // N is a multiple of 64
@@ -391,27 +483,19 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             const uint32_t m = idx >> 4, pc = idx & 15u;
             if (pc * 8u < columns)
                 *reinterpret_cast<uint4 *>(a.act + (size_t(tile_index) * kRowTile + m) * a.f + c0 + pc * 8u) =
-                    *reinterpret_cast<const uint4 *>(&s_a[0][m][pc * 8u]);
+                    *reinterpret_cast<const uint4 *>(&s_out[m][pc * 8u]);
         }
         uint32_t *sums_out = const_cast<uint32_t *>(a.act_sums);
-        for (uint32_t slot = threadIdx.x; slot < kRowTile * 16u; slot += 256u) {  // (row, group of the block, eighth)
+        for (uint32_t slot = threadIdx.x; slot < L::kRows * 16u; slot += 256u) {  // (row, group of the block, eighth)
             const uint32_t m = slot >> 4, gl = (slot >> 3) & 1u, eighth = slot & 7u;
-            const uint4 v = *reinterpret_cast<const uint4 *>(&s_a[0][m][gl * 64u + eighth * 8u]);
+            const uint4 v = *reinterpret_cast<const uint4 *>(&s_out[m][gl * 64u + eighth * 8u]);
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-            float sum = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                sum = __fadd_rn(sum, f16_to_f32(uint16_t(w[t])));
-                sum = __fadd_rn(sum, f16_to_f32(uint16_t(w[t] >> 16)));
-            }
-            sum = __fadd_rn(sum, __shfl_xor(sum, 1));
-            sum = __fadd_rn(sum, __shfl_xor(sum, 2));
-            sum = __fadd_rn(sum, __shfl_xor(sum, 4));
+            const float sum = eighth_sum(w);
             if (eighth == 0u && m < tile.rows && gl * 64u < columns)
                 sums_out[(size_t(tile_index) * kRowTile + m) * (a.f / kGroup) + c0 / kGroup + gl] = split_hi_lo(sum);
         }
     } else {
-        // the down product's rows leave through the first staging buffer too, [row][column of this block of 256], and go
+        // the down product's rows leave through the LDS too, [row][column of this block of 256], and go
         // to their (token, rank) rows as whole 16-byte pieces; a call over a range of the sorted pairs writes the rows of
         // its pairs only
         const uint32_t row_lo = DENSE ? 0u : max(a.pair_lo, tile.pair_start) - tile.pair_start;
@@ -433,40 +517,42 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
                         y0 = f32_to_f16(f16_to_f32(y0) / gate_mul);
                         y1 = f32_to_f16(f16_to_f32(y1) / gate_mul);
                     }
-                    s_a[0][m][wave * 64u + col] = y0;
-                    s_a[0][m][wave * 64u + col + 32u] = y1;
+                    s_out[m][wave * 64u + col] = y0;
+                    s_out[m][wave * 64u + col + 32u] = y1;
                 }
             }
         }
         __syncthreads();
         const uint32_t c0 = col_block * 256u, columns = min(256u, N - c0);  // N is a multiple of 64
-        constexpr uint32_t kPasses = MT * 32u * 32u / 256u;  // 32 pieces a row, 256 threads
-        const uint16_t *dst_row[kPasses];
+        // 32 pieces a row, eight rows a pass; the pair records of eight passes are fetched together
         const uint32_t pc = threadIdx.x & 31u;
+        constexpr uint32_t kPasses = MT * 32u / 8u, kBatch = kPasses < 8u ? kPasses : 8u;
+        for (uint32_t pass0 = 0; pass0 < kPasses; pass0 += kBatch) {
+            const uint16_t *dst_row[kBatch];
 #pragma unroll
-        for (uint32_t pass = 0; pass < kPasses; ++pass) {
-            const uint32_t m = pass * 8u + (threadIdx.x >> 5);
-            const uint32_t mm = min(m, tile.rows - 1u);
-            if (DENSE) {
-                dst_row[pass] = a.partials + size_t(tile.pair_start + mm) * a.d;
-            } else {
-                const shrike_token_expert_pair p = a.pairs[tile.pair_start + mm];
-                dst_row[pass] = a.partials + (size_t(p.token) * a.top_k + p.rank) * a.d;
+            for (uint32_t i = 0; i < kBatch; ++i) {
+                const uint32_t mm = min((pass0 + i) * 8u + (threadIdx.x >> 5), tile.rows - 1u);
+                if (DENSE) {
+                    dst_row[i] = a.partials + size_t(tile.pair_start + mm) * a.d;
+                } else {
+                    const shrike_token_expert_pair p = a.pairs[tile.pair_start + mm];
+                    dst_row[i] = a.partials + (size_t(p.token) * a.top_k + p.rank) * a.d;
+                }
             }
-        }
 #pragma unroll
-        for (uint32_t pass = 0; pass < kPasses; ++pass) {
-            const uint32_t m = pass * 8u + (threadIdx.x >> 5);
-            if (m >= row_lo && m < row_hi && pc * 8u < columns)
-                *reinterpret_cast<uint4 *>(const_cast<uint16_t *>(dst_row[pass]) + c0 + pc * 8u) = *reinterpret_cast<const uint4 *>(&s_a[0][m][pc * 8u]);
+            for (uint32_t i = 0; i < kBatch; ++i) {
+                const uint32_t m = (pass0 + i) * 8u + (threadIdx.x >> 5);
+                if (m >= row_lo && m < row_hi && pc * 8u < columns)
+                    *reinterpret_cast<uint4 *>(const_cast<uint16_t *>(dst_row[i]) + c0 + pc * 8u) = *reinterpret_cast<const uint4 *>(&s_out[m][pc * 8u]);
+            }
         }
     }
 }
 
-template <int BITS, int MODE, bool DENSE, int META>
-__global__ __launch_bounds__(256, 2) void k_grouped_ffn(FfnArgs a) {
+template <int BITS, int MODE, bool DENSE, int META, bool WIDE>
+__global__ __launch_bounds__(256, (Lds<WIDE>::kResident)) void k_grouped_ffn(FfnArgs a) {
     warm_kernel_arguments(a);
-    __shared__ __align__(16) uint16_t s_a[2][kRowTile][kLdsRow];
+    __shared__ __align__(16) uint8_t lds[Lds<WIDE>::kBytes];
     // Which (row tile, column block) this workgroup takes. Workgroups go to the chip's eight XCDs (each
     // with an L2 of its own) round robin in launch order, so workgroup w runs on XCD w % 8 as that XCD's
     // item w / 8. An expert's row tiles are neighbours in the tile table: an XCD takes a contiguous run
@@ -490,10 +576,10 @@ __global__ __launch_bounds__(256, 2) void k_grouped_ffn(FfnArgs a) {
         tile.expert = 0;
     } else {
         if (tile_index >= tile_total) return;
-        // Which tile of the table the workgroup takes. A compute unit holds two of these workgroups, whose waves share its
+        // Which tile of the table the workgroup takes. A compute unit holds several of these workgroups, whose waves share its
         // SIMDs' issue, and an XCD's workgroups reach its compute units in launch order, one each before any gets a second
         // (read from the hardware: item i and item i + 32 of an XCD share a unit). A tile of more than 32 rows is twice a
-        // smaller one's matrix work, and the launch ends with the units that hold two of those.
+        // smaller one's matrix work, and the launch ends with the units that hold more than one of those.
         //  - Where the gate/up launch fits the chip at once: every XCD takes the same number of the larger tiles (a block of
         //    them in table order, so an expert's stay together) and fills its eighth with a block of the smaller ones; the
         //    larger go first, so each gets a smaller neighbour.
@@ -503,7 +589,7 @@ __global__ __launch_bounds__(256, 2) void k_grouped_ffn(FfnArgs a) {
         const uint32_t lane = threadIdx.x & 63u;
         const uint32_t gate_up_blocks = (a.f + 127u) / 128u;
         bool chosen = false;
-        if (tile_total <= 256u && tile_total * gate_up_blocks <= a.resident_workgroups) {
+        if (!WIDE && tile_total <= 256u && tile_total * gate_up_blocks <= a.resident_workgroups) {
             // (four named records, not an array: the compiler kept an array of them in private memory)
             const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
             const uint4 rec0 = lane < tile_total ? table[lane] : zero4();
@@ -550,7 +636,23 @@ __global__ __launch_bounds__(256, 2) void k_grouped_ffn(FfnArgs a) {
             }
         }
         const uint32_t count = run;
-        if (chosen) {
+        if (WIDE) {
+            // Two neighbouring tiles of an expert are one workgroup's work: the first of them takes both. A tile is a first
+            // one where an even number of its expert's tiles are ahead of it.
+            tile = a.tiles[tile_index];
+            uint32_t ahead = 0;
+            for (uint32_t at = tile_index;; at -= 64u) {
+                const bool same = lane < at && a.tiles[at - 1u - lane].expert == tile.expert;
+                const uint64_t others = ~__ballot(same);
+                ahead += others ? uint32_t(__ffsll((long long)others)) - 1u : 64u;
+                if (others) break;
+            }
+            if (ahead & 1u) return;
+            if (tile_index + 1u < tile_total) {
+                const shrike_row_tile second = a.tiles[tile_index + 1u];
+                if (second.expert == tile.expert) tile.rows += second.rows;
+            }
+        } else if (chosen) {
         } else if (count <= 64u) {
             const uint4 rec = lane < count ? reinterpret_cast<const uint4 *>(a.tiles)[first + lane] : zero4();
             const uint64_t heavy = __ballot(lane < count && rec.z > 32u), light = __ballot(lane < count && rec.z <= 32u);
@@ -575,36 +677,345 @@ __global__ __launch_bounds__(256, 2) void k_grouped_ffn(FfnArgs a) {
         if (tile.pair_start + tile.rows <= a.pair_lo || tile.pair_start >= a.pair_hi) return;
     }
 
-    if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META>(a, tile, tile_index, col_block, s_a);
-    else ffn_tile<BITS, MODE, DENSE, 1, META>(a, tile, tile_index, col_block, s_a);
+    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, WIDE>(a, tile, tile_index, col_block, lds);
+    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, WIDE>(a, tile, tile_index, col_block, lds);
+    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, WIDE>(a, tile, tile_index, col_block, lds);
+    else ffn_tile<BITS, MODE, DENSE, 1, META, WIDE>(a, tile, tile_index, col_block, lds);
+}
+
+// ---- few rows: the same products with k split over the waves.
+//
+// Where k_grouped_ffn would leave most of the chip idle (a short chunk, or the shared expert: 512 tokens of one expert are
+// eight row tiles of four column blocks), a workgroup's walk over k is a chain of a microsecond for three groups, whatever
+// its rows. Here a workgroup takes up to 32 rows against 64 weight rows (32 of the gate and 32 of the up product), a quarter
+// of k a wave, and the four partial sums meet in LDS in the order of k at the end: an eighth of the columns and a quarter of
+// the walk. The operands come through LDS as in ffn_tile, each wave's its own, so the loop has no barrier. The bias term
+// needs no sums from elsewhere: a wave adds up its rows while it multiplies them, and four groups of them meet their biases in
+// one MFMA (the lanes' two halves of a group are two of its k). Two workgroups a compute unit, two groups of operands in
+// flight; deeper rings at one workgroup a compute unit were slower (20 against 16 us below): what bounds it is the start and
+// the end of a piece, some 4 us, which a neighbour hides, not the loads between them.
+// The shared expert of 2,048 x 512, 4-bit: 45 -> 13 us for 37 rows, 49 -> 16 for 512.
+template <int BITS, int MODE, bool DENSE, int META>
+__global__ __launch_bounds__(256, 2) void k_ffn_split(FfnArgs a) {
+    warm_kernel_arguments(a);
+    extern __shared__ __align__(16) uint8_t lds[];
+    typedef SplitLds L;
+    const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
+    const uint32_t col = lane & 31u, kb = lane >> 5;
+    const uint32_t K = MODE == 0 ? a.d : a.f, N = MODE == 0 ? a.f : a.d, G = K / kGroup;
+    constexpr uint32_t kColumns = MODE == 0 ? 32u : 64u;  // of the output
+    constexpr uint32_t kGroupsPerB = BITS == 4 ? 2u : 1u;
+    const uint32_t stages = (G + kGroupsPerB - 1u) / kGroupsPerB, row_bytes = K * BITS / 8u;
+    // the wave's quarter of the stages
+    const uint32_t st_lo = stages * wave / 4u, st_hi = stages * (wave + 1u) / 4u;
+    const uint32_t g_lo = st_lo * kGroupsPerB, g_hi = min(st_hi * kGroupsPerB, G), groups = g_hi - g_lo, my_stages = st_hi - st_lo;
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds)) + wave * L::kWave;
+    const uint8_t *my_lds = lds + wave * L::kWave;
+    // An XCD takes a contiguous eighth of the (tile, column block) pairs, its workgroups one after the other: tiles of an
+    // expert share its codes there, the column blocks of a tile its rows.
+    const uint32_t column_blocks = N / kColumns;
+    const uint32_t total_items = (DENSE ? (a.dense_rows + 31u) / 32u : *a.tile_count) * column_blocks;
+    const uint32_t xcd = blockIdx.x & 7u, run = total_items / 8u + (xcd < total_items % 8u ? 1u : 0u);
+    const uint32_t run_first = xcd * (total_items / 8u) + min(xcd, total_items % 8u);
+    for (uint32_t place = blockIdx.x >> 3; place < run; place += gridDim.x >> 3) {
+        const uint32_t item = run_first + place;
+        uint32_t tile_index, col_block;
+        shrike_row_tile tile;
+        if (DENSE) {  // the rows of a column block are neighbours
+            const uint32_t row_tiles = total_items / column_blocks;
+            col_block = item / row_tiles;
+            tile_index = item % row_tiles;
+            tile.cell = 0;
+            tile.pair_start = tile_index * 32u;
+            tile.rows = min(32u, a.dense_rows - tile.pair_start);
+        } else {
+            tile_index = item / column_blocks;
+            col_block = item % column_blocks;
+            tile = a.tiles[tile_index];
+            if (a.residency) {  // moe.metal:136-146: a hit names its cell, anything else is the sentinel
+                const uint64_t word = a.residency[tile.expert];
+                tile.cell = uint32_t(word >> 32) == SHRIKE_RESIDENCY_RESIDENT ? uint32_t(word) : kSentinel;
+            }
+            if (tile.cell == kSentinel) continue;
+            if (tile.pair_start + tile.rows <= a.pair_lo || tile.pair_start >= a.pair_hi) continue;
+        }
+        const uint32_t n0 = col_block * kColumns;
+        const uint8_t *base = DENSE ? nullptr : cell_base_uniform(a.pool, tile.cell, a.stride);
+        const uint8_t *w_base[2];
+        const uint16_t *s_base[2], *b_base[2];
+        uint32_t n_first[2];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            n_first[nt] = n0 + (MODE == 0 ? 0u : 32u * uint32_t(nt));
+            if (DENSE) {
+                const int p = MODE == 0 ? nt : 2;
+                w_base[nt] = a.dense_w[p]; s_base[nt] = a.dense_s[p]; b_base[nt] = a.dense_b[p];
+            } else {
+                w_base[nt] = base + (MODE != 0 ? a.off.down_w_off : nt ? a.off.up_w_off : a.off.gate_w_off);
+                s_base[nt] = reinterpret_cast<const uint16_t *>(base + (MODE != 0 ? a.off.down_s_off : nt ? a.off.up_s_off : a.off.gate_s_off));
+                b_base[nt] = reinterpret_cast<const uint16_t *>(base + (MODE != 0 ? a.off.down_b_off : nt ? a.off.up_b_off : a.off.gate_b_off));
+            }
+        }
+        uint32_t b_off[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j)
+            b_off[j] = (n_first[j >> 1] + 16u * (j & 1u) + (lane >> 2)) * row_bytes + ((lane & 3u) ^ ((lane >> 3) & 3u)) * 16u;
+        const uint32_t half_back = (((lane & 3u) ^ ((lane >> 3) & 3u)) & 2u) * 16u;
+        auto load_b = [&](uint32_t slot, uint32_t stage) {
+            const uint32_t back = BITS == 4 && 2u * stage + 1u >= G ? half_back : 0u;
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) lds_load16(lds0 + L::kB + slot * kUnitB + j * 1024u, w_base[j >> 1] + size_t(stage) * 64u, b_off[j] - back);
+        };
+        // scales and biases: a window of three words a row, as in ffn_tile
+        struct Run { const uint8_t *src; uint32_t mine, mine_last, at[2], last[2]; };
+        auto make_run = [&](const uint16_t *const (&b)[2]) {
+            Run r;
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                const uint32_t skew = uint32_t(reinterpret_cast<uintptr_t>(b[nt]) & 3u);
+                r.at[nt] = skew + ((n_first[nt] + col) * G + g_lo) * 2u;
+                r.last[nt] = ((skew + N * G * 2u + 3u) & ~3u) - 12u;
+            }
+            const uint8_t *p = reinterpret_cast<const uint8_t *>(kb ? b[1] : b[0]);
+            r.src = p - (reinterpret_cast<uintptr_t>(p) & 3u);
+            r.mine = kb ? r.at[1] : r.at[0];
+            r.mine_last = kb ? r.last[1] : r.last[0];
+            return r;
+        };
+        const Run rs = make_run(s_base), rb = make_run(b_base);
+        auto load_s = [&](uint32_t c) {
+            lds_load12(lds0 + L::kS, rs.src + min((rs.mine & ~3u) + 8u * c, rs.mine_last));
+            lds_load12(lds0 + L::kBias, rb.src + min((rb.mine & ~3u) + 8u * c, rb.mine_last));
+        };
+        auto read_run = [&](const Run &r, uint32_t area, uint32_t i0, uint32_t (&v)[2][4]) {
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt) {
+                const int into = max(int(r.at[nt] & 3u), int(r.at[nt] + i0 * 2u) - int(r.last[nt]));
+                const uint8_t *p = my_lds + area + (uint32_t(nt) * 32u + col) * 16u + uint32_t(into);
+#pragma unroll
+                for (uint32_t i = 0; i < 4u; ++i) v[nt][i] = *reinterpret_cast<const uint16_t *>(p + min(i, groups - 1u - i0) * 2u);
+            }
+        };
+        const uint32_t chunks = (groups + 3u) / 4u;
+
+        for (uint32_t skip = 0; skip < tile.rows; skip += 32u) {  // (dense: once)
+            const uint32_t rows = min(32u, tile.rows - skip), first = tile.pair_start + skip;
+            const uint32_t act_row = DENSE ? first : tile_index * kRowTile + skip;
+            f32x16 total[2];
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) total[nt][i] = 0.0f;
+            // (rows past the last eight that hold one are not loaded: what the LDS holds there is multiplied into rows that
+            // nobody reads)
+            auto walk = [&](auto loads_a) {
+                constexpr uint32_t kLoadsA = decltype(loads_a)::value;
+                const uint8_t *a_src[kLoadsA];
+#pragma unroll
+                for (uint32_t j = 0; j < kLoadsA; ++j) {
+                    const uint32_t r = min(8u * j + (lane >> 3), rows - 1u);
+                    const uint16_t *row = MODE != 0 ? a.act + size_t(act_row + r) * a.f
+                                                    : a.hidden + size_t(DENSE ? first + r : a.pairs[first + r].token) * a.hidden_stride;
+                    a_src[j] = reinterpret_cast<const uint8_t *>(row + g_lo * kGroup) + (((lane & 7u) ^ (lane >> 3)) * 16u);
+                }
+                auto load_a = [&](uint32_t slot, uint32_t i) {
+#pragma unroll
+                    for (uint32_t j = 0; j < kLoadsA; ++j) lds_load16(lds0 + slot * L::kUnitA + j * 1024u, a_src[j] + size_t(i) * 128u);
+                };
+                if (groups != 0u) {
+                    load_s(0);
+                    load_b(0, st_lo);
+                    load_a(0, 0);
+                }
+                uint32_t run_s[2][4], run_b[2][4];
+                Frag sums;  // of the chunk's groups: the lane's row over its half of each group's k, hi and lo
+                auto step = [&](uint32_t i, auto par) {
+                    constexpr uint32_t P = decltype(par)::value;
+                    const uint32_t b_place = BITS == 8 ? P : (i >> 1) & 1u;
+                    if (BITS == 4 && P == 1u && i + 1u < groups) wait_loads<4>();  // (the next stage's codes may still be on their way)
+                    else wait_loads<0>();
+                    if (i + 1u < groups) {
+                        load_a(P ^ 1u, i + 1u);
+                        if (BITS == 8) load_b(b_place ^ 1u, st_lo + i + 1u);
+                    }
+                    if (BITS == 4 && P == 0u && i + 2u < groups) load_b(b_place ^ 1u, st_lo + (i >> 1) + 1u);
+                    const uint32_t in_chunk = i & 3u;
+                    if (in_chunk == 0u) {
+                        read_run(rs, L::kS, i, run_s);
+                        read_run(rb, L::kBias, i, run_b);
+                        sums.v = zero4();
+                    }
+                    if (in_chunk == 1u && i + 3u < groups) load_s((i >> 2) + 1u);
+                    const uint8_t *a_rows = my_lds + P * L::kUnitA + col * 128u;
+                    Frag af[4];
+#pragma unroll
+                    for (uint32_t s = 0; s < 4u; ++s) af[s].v = *reinterpret_cast<const uint4 *>(a_rows + (((kb * 4u + s) ^ (col & 7u)) * 16u));
+                    float sum = 0.0f;
+#pragma unroll
+                    for (int nt = 0; nt < 2; ++nt) {
+                        const uint8_t *b_rows = my_lds + L::kB + b_place * kUnitB + uint32_t(nt) * 2048u + col * 64u;
+                        uint4 codes[BITS / 4];
+#pragma unroll
+                        for (uint32_t j = 0; j < BITS / 4; ++j)
+                            codes[j] = *reinterpret_cast<const uint4 *>(b_rows + (((BITS == 4 ? P * 2u + kb : kb * 2u + j) ^ ((col >> 1) & 3u)) * 16u));
+                        half8 bf[4];
+                        if (BITS == 4) {
+                            bf[0] = codes4(codes[0].x); bf[1] = codes4(codes[0].y); bf[2] = codes4(codes[0].z); bf[3] = codes4(codes[0].w);
+                        } else {
+                            const uint4 lo = codes[0], hi = codes[BITS / 4 - 1];
+                            bf[0] = codes8(lo.x, lo.y); bf[1] = codes8(lo.z, lo.w); bf[2] = codes8(hi.x, hi.y); bf[3] = codes8(hi.z, hi.w);
+                        }
+                        f32x16 p = {0};
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) p = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[s].h, bf[s], p, 0, 0, 0);
+                        if (nt == 0) {
+#pragma unroll
+                            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                                for (int w = 0; w < 4; ++w) sum = dot2_ones(af[s].u[w], sum);
+                        }
+                        const float scale = meta_f32(uint16_t(run_s[nt][0]), uint32_t(META)) * kTwo24;
+                        run_s[nt][0] = run_s[nt][1]; run_s[nt][1] = run_s[nt][2]; run_s[nt][2] = run_s[nt][3];
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) total[nt][j] = fmaf(scale, p[j], total[nt][j]);
+                    }
+                    const uint32_t hi_lo = split_hi_lo(sum);
+                    if (in_chunk == 0u) sums.u[0] = hi_lo;
+                    else if (in_chunk == 1u) sums.u[1] = hi_lo;
+                    else if (in_chunk == 2u) sums.u[2] = hi_lo;
+                    else sums.u[3] = hi_lo;
+                    if (in_chunk == 3u || i + 1u == groups) {  // the bias term of a chunk: one MFMA
+#pragma unroll
+                        for (int nt = 0; nt < 2; ++nt) {
+                            Frag f;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) {
+                                const uint16_t bits = META == SHRIKE_META_BF16 ? f32_to_f16(bf16_to_f32(uint16_t(run_b[nt][j]))) : uint16_t(run_b[nt][j]);
+                                f.u[j] = uint32_t(bits) * 0x00010001u;
+                            }
+                            total[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums.h, f.h, total[nt], 0, 0, 0);
+                        }
+                    }
+                };
+                for (uint32_t i = 0; i + 1u < groups; i += 2u) {
+                    step(i, std::integral_constant<uint32_t, 0>{});
+                    step(i + 1u, std::integral_constant<uint32_t, 1>{});
+                }
+                if (groups & 1u) step(groups - 1u, std::integral_constant<uint32_t, 0>{});
+            };
+            if (rows <= 8u) walk(std::integral_constant<uint32_t, 1>{});
+            else if (rows <= 16u) walk(std::integral_constant<uint32_t, 2>{});
+            else walk(std::integral_constant<uint32_t, 4>{});
+            // ---- the quarters meet: eight threads a row
+            __syncthreads();
+            float (*s_part)[32][64] = reinterpret_cast<float (*)[32][64]>(lds);
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s_part[wave][8u * (i / 4) + 4u * kb + (i % 4)][32u * nt + col] = total[nt][i];
+            __syncthreads();
+            const uint32_t r = threadIdx.x >> 3, e = threadIdx.x & 7u;
+            float v[8];  // MODE 0: four columns of the gate, then of the up product; MODE 1: eight columns
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t c = MODE == 0 ? 32u * h + 4u * e : 8u * e + 4u * h;
+                float4 t = *reinterpret_cast<const float4 *>(&s_part[0][r][c]);
+#pragma unroll
+                for (int q = 1; q < 4; ++q) {
+                    const float4 u = *reinterpret_cast<const float4 *>(&s_part[q][r][c]);
+                    t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
+                }
+                v[4 * h] = t.x; v[4 * h + 1] = t.y; v[4 * h + 2] = t.z; v[4 * h + 3] = t.w;
+            }
+            if (r < rows) {
+                if (MODE == 0) {
+                    const uint32_t n = n0 + 4u * e;
+                    uint32_t y[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float g = v[j], u = v[4 + j];
+                        if (!DENSE && a.ebias) {  // moe.metal:261-269
+                            g += bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.gate_ab_off)[n + j]);
+                            u += bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.up_ab_off)[n + j]);
+                        }
+                        if (DENSE && a.round_gate_up) {
+                            g = f16_to_f32(f32_to_f16(g));
+                            u = f16_to_f32(f32_to_f16(u));
+                        }
+                        y[j] = f32_to_f16(glu_rt_fast(g, u, a.act_kind));
+                    }
+                    *reinterpret_cast<uint2 *>(a.act + size_t(act_row + r) * a.f + n) = make_uint2(y[0] | y[1] << 16, y[2] | y[3] << 16);
+                } else if (DENSE || (first + r >= a.pair_lo && first + r < a.pair_hi)) {
+                    const uint32_t n = n0 + 8u * e;
+                    float gate_mul = 1.0f;
+                    if (DENSE && a.scalar_gate) gate_mul = 1.0f + expf(-f16_to_f32(a.scalar_gate[first + r]));  // one gate a token row (moe.metal:1195-1207)
+                    uint16_t *to;
+                    if (DENSE) {
+                        to = a.partials + size_t(first + r) * a.d;
+                    } else {
+                        const shrike_token_expert_pair p = a.pairs[first + r];
+                        to = a.partials + (size_t(p.token) * a.top_k + p.rank) * a.d;
+                    }
+                    uint32_t y[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        float o = v[j];
+                        if (!DENSE && a.ebias) o += bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off)[n + j]);
+                        y[j] = f32_to_f16(o);
+                        if (DENSE && a.scalar_gate) y[j] = f32_to_f16(f16_to_f32(uint16_t(y[j])) / gate_mul);
+                    }
+                    *reinterpret_cast<uint4 *>(to + n) = make_uint4(y[0] | y[1] << 16, y[2] | y[3] << 16, y[4] | y[5] << 16, y[6] | y[7] << 16);
+                }
+            }
+            __syncthreads();  // the partial sums have been read: the next rows' operands may land
+        }
+    }
 }
 
 int launch_row_group_sums(const uint16_t *src, size_t stride, uint32_t rows, uint32_t n, uint32_t *out,
                           const uint32_t *row_limit_tiles, hipStream_t s);
 
-template <int BITS, bool DENSE, int META>
-static int launch_ffn_meta(const FfnArgs &a, uint32_t max_tiles, hipStream_t s) {
-    const dim3 block(256);
-    const uint32_t grid_tiles = (max_tiles + 7u) & ~7u;  // whole runs for the kernel's XCD mapping
-    hipLaunchKernelGGL((k_grouped_ffn<BITS, 0, DENSE, META>), dim3(grid_tiles, (a.f + 127u) / 128u), block, 0, s, a);
-    SHRIKE_HIP(hipGetLastError());
-    // (the activations' group sums were written by the gate/up launch itself)
-    hipLaunchKernelGGL((k_grouped_ffn<BITS, 1, DENSE, META>), dim3(grid_tiles, (a.d + 255u) / 256u), block, 0, s, a);
-    SHRIKE_HIP(hipGetLastError());
-    return 0;
-}
-template <int BITS, bool DENSE>
-static int launch_ffn(const FfnArgs &a, uint32_t max_tiles, hipStream_t s) {
-    return a.meta == SHRIKE_META_F16 ? launch_ffn_meta<BITS, DENSE, SHRIKE_META_F16>(a, max_tiles, s)
-                                     : launch_ffn_meta<BITS, DENSE, SHRIKE_META_BF16>(a, max_tiles, s);
-}
-
-// Two workgroups of the FFN kernels a compute unit (their registers and LDS allow no more).
-static uint32_t resident_ffn_workgroups() {
+static uint32_t compute_units() {
     int device = 0, units = 0;
     if (hipGetDevice(&device) != hipSuccess || hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return 0;
-    return 2u * uint32_t(units);
+    return uint32_t(units);
+}
+
+template <int BITS, bool DENSE, int META, bool WIDE>
+static int launch_ffn_shape(FfnArgs a, uint32_t max_tiles, hipStream_t s) {
+    a.resident_workgroups = Lds<WIDE>::kResident * compute_units();
+    const dim3 block(256);
+    const uint32_t grid_tiles = (max_tiles + 7u) & ~7u;  // whole runs for the kernel's XCD mapping
+    hipLaunchKernelGGL((k_grouped_ffn<BITS, 0, DENSE, META, WIDE>), dim3(grid_tiles, (a.f + 127u) / 128u), block, 0, s, a);
+    SHRIKE_HIP(hipGetLastError());
+    // (the activations' group sums were written by the gate/up launch itself)
+    hipLaunchKernelGGL((k_grouped_ffn<BITS, 1, DENSE, META, WIDE>), dim3(grid_tiles, (a.d + 255u) / 256u), block, 0, s, a);
+    SHRIKE_HIP(hipGetLastError());
+    return 0;
+}
+template <int BITS, bool DENSE, int META>
+static int launch_ffn_split(const FfnArgs &a, uint32_t max_tiles, hipStream_t s) {
+    const uint32_t tiles = DENSE ? (a.dense_rows + 31u) / 32u : max_tiles;
+    auto grid = [&](uint32_t column_blocks) { return dim3((uint32_t(min(uint64_t(tiles) * column_blocks, uint64_t(2u * compute_units()))) + 7u) & ~7u); };
+    hipLaunchKernelGGL((k_ffn_split<BITS, 0, DENSE, META>), grid(a.f / 32u), dim3(256), SplitLds::kBytes, s, a);
+    SHRIKE_HIP(hipGetLastError());
+    hipLaunchKernelGGL((k_ffn_split<BITS, 1, DENSE, META>), grid(a.d / 64u), dim3(256), SplitLds::kBytes, s, a);
+    SHRIKE_HIP(hipGetLastError());
+    return 0;
+}
+
+template <int BITS, bool DENSE, int META>
+static int launch_ffn_meta(const FfnArgs &a, uint32_t max_tiles, FfnShape shape, hipStream_t s) {
+    if (shape == FfnShape::kSplit) return launch_ffn_split<BITS, DENSE, META>(a, max_tiles, s);
+    if constexpr (!DENSE)
+        if (shape == FfnShape::kWide) return launch_ffn_shape<BITS, DENSE, META, true>(a, max_tiles, s);
+    return launch_ffn_shape<BITS, DENSE, META, false>(a, max_tiles, s);
+}
+template <int BITS, bool DENSE>
+static int launch_ffn(const FfnArgs &a, uint32_t max_tiles, FfnShape shape, hipStream_t s) {
+    return a.meta == SHRIKE_META_F16 ? launch_ffn_meta<BITS, DENSE, SHRIKE_META_F16>(a, max_tiles, shape, s)
+                                     : launch_ffn_meta<BITS, DENSE, SHRIKE_META_BF16>(a, max_tiles, shape, s);
 }
 
 struct Workspace {
@@ -627,6 +1038,30 @@ using namespace shrike;
 extern "C" {
 size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max_row_tiles, uint32_t d, uint32_t f) {
     return workspace_layout(query_count, max_row_tiles, d, f).total;
+}
+
+// The shape of the routed products, from what the host knows (and what a call over a range of the pairs shares with the call
+// over all of them: their outputs are the same bytes).
+//  - kSplit up to 1,024 pieces of its gate/up launch, two for each of the 512 workgroups it keeps: with 16 experts of
+//    1,536 x 1,024 it takes 21 us for 16 tokens where kTile takes 30, and 24.6 against 37.9 for 100 (8-bit codes). Past that it
+//    loses: its pieces are short and none of them overlaps the next in its workgroup (256 experts of 2,048 x 512, 128 tokens:
+//    150 against 126 us).
+//  - kWide where the experts' rows fill its tiles: from 48 pairs an expert at 8 bits (384 experts, 2,000 tokens: 528 against
+//    645 us), from 64 at 4 bits, there only where the launch still has several workgroups for every compute unit (32 experts
+//    of 2,880 x 2,880, 2,048 tokens: 541 against 576 us; 256 experts of 2,048 x 512: 337 against 339 at 4,096 tokens, but 193
+//    against 169 at 2,000 unevenly spread ones).
+static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t f, uint32_t bits) {
+    const uint64_t most_tiles = min(pairs, uint64_t(experts)) + pairs / kRowTile;
+    if (most_tiles * (f / 32u) <= 1024u) return FfnShape::kSplit;
+    if (bits == 8 ? pairs >= 48u * uint64_t(experts) : pairs >= 64u * uint64_t(experts) && pairs / kRowTile * ((f + 127u) / 128u) >= 1400u)
+        return FfnShape::kWide;
+    return FfnShape::kTile;
+}
+// ... and of a dense expert's, whose rows are its tiles: kSplit up to two pieces a workgroup (2,048 x 512, 4-bit: 13 against
+// 45 us for 37 rows, 16 against 48 for 512, 32 against 47 for 1,500; 2,304 x 1,024, 8-bit: 44 against 54 for 1,000), kTile
+// past that (60 against 79 us for 4,096 rows).
+static FfnShape dense_shape(uint64_t rows, uint32_t f) {
+    return (rows + 31u) / 32u * (f / 32u) <= 1024u ? FfnShape::kSplit : FfnShape::kTile;
 }
 
 static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_bases *pool, uint64_t pool_slot_stride,
@@ -668,11 +1103,11 @@ static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_base
     a.meta = moe->desc.meta_dtype;
     a.act_kind = moe->desc.activation;
     a.ebias = moe->desc.expert_additive_biases;
-    a.resident_workgroups = resident_ffn_workgroups();
     hipStream_t s = as_stream(stream);
     if (!presummed)
         if (int rc = launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, const_cast<uint32_t *>(a.hidden_sums), nullptr, s)) return rc;
-    return moe->desc.routed_weight_bits == 8 ? launch_ffn<8, false>(a, max_row_tiles, s) : launch_ffn<4, false>(a, max_row_tiles, s);
+    const FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, f, moe->desc.routed_weight_bits);
+    return moe->desc.routed_weight_bits == 8 ? launch_ffn<8, false>(a, max_row_tiles, shape, s) : launch_ffn<4, false>(a, max_row_tiles, shape, s);
 }
 
 int shrike_hip_prefill_grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_bases *pool,
@@ -754,8 +1189,10 @@ int shrike_hip_prefill_shared_expert(shrike_hip_moe *moe, void *stream, const sh
     a.round_gate_up = 1;
     a.scalar_gate = static_cast<const uint16_t *>(d_scalar_gate);
     hipStream_t s = as_stream(stream);
-    if (int rc = launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, const_cast<uint32_t *>(a.hidden_sums), nullptr, s)) return rc;
-    return bits == 8 ? launch_ffn<8, true>(a, tiles, s) : launch_ffn<4, true>(a, tiles, s);
+    const FfnShape shape = dense_shape(query_count, f_shared);
+    if (shape != FfnShape::kSplit)
+        if (int rc = launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, const_cast<uint32_t *>(a.hidden_sums), nullptr, s)) return rc;
+    return bits == 8 ? launch_ffn<8, true>(a, tiles, shape, s) : launch_ffn<4, true>(a, tiles, shape, s);
 }
 
 }  // extern "C"

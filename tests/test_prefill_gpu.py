@@ -298,6 +298,26 @@ def test_grouped_ffn_shape_sweep(gpu, case):
     assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
 
 
+@pytest.mark.parametrize("d,f,ne,k,t,bits,meta", [
+    # k over the waves: one group and one stage in all, a quarter without any, 9 to 16 rows and two pieces of a row tile,
+    # groups that no quarter shares evenly
+    (64, 64, 3, 2, 20, 4, S.META_BF16), (128, 192, 2, 1, 45, 8, S.META_F16), (2880, 64, 4, 2, 50, 4, S.META_F16),
+    # one row tile a workgroup: fewer than eight groups and more than sixty-four, both odd
+    (192, 4160, 6, 2, 70, 4, S.META_BF16), (4032, 1088, 40, 3, 33, 8, S.META_F16),
+    # two row tiles of an expert a workgroup: 128 rows and what is left over, odd groups, column blocks that end inside it
+    (128, 8192, 6, 4, 360, 4, S.META_BF16), (576, 3008, 8, 4, 960, 4, S.META_F16), (960, 832, 24, 4, 300, 8, S.META_BF16)])
+def test_grouped_ffn_shapes_of_a_workgroup(gpu, d, f, ne, k, t, bits, meta):
+    L = Layer(0x5EED0400 + d + f, d, f, ne, k, bits=bits, meta=meta)
+    pc = PrefillCase(gpu, L, t, stride_pad=8, resident=[e for e in range(ne) if e != 1])
+    got = pc.run()
+    here = pc.idx.reshape(t, k) != 1
+    assert np.all(got[~here] == 0xD4D0), "an absent expert's row was written"
+    assert not np.any(np.all(got[here] == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
+    order = np.argwhere(here)
+    for tok, rank in order[np.random.default_rng(6).choice(len(order), min(len(order), 40), replace=False)]:
+        pc.check_pair(got, int(tok), int(rank), f"token {tok} rank {rank}")
+
+
 def test_grouped_ffn_gpt_oss_epilogues(gpu):
     # additive biases + clamped SwiGLU at the gpt-oss shape (moe.metal:257-288), 45 groups per row
     d = f = 2880
@@ -543,6 +563,12 @@ def test_shared_expert_for_a_token_block(gpu, d, fs, bits, t, gated):
         assert np.array_equal(plain.download(np.uint16, t * d).reshape(t, d), got), "fused and two-launch gating differ"
         # the elementwise kernel against the oracle: the device's exp may differ from libm's in the last bit
         assert_ffn_close(plain.download(np.uint16, t * d), O.sigmoid_scalar_mul_rows(ungated.copy(), gates, d, t), "sigmoid rows")
+
+
+@pytest.mark.parametrize("d,fs,bits,t,gated", [(128, 4032, 4, 290, True), (192, 4096, 8, 265, False)])
+def test_shared_expert_for_many_rows(gpu, d, fs, bits, t, gated):
+    # a row tile a workgroup: more than two pieces of k_ffn_split's for each of its workgroups
+    test_shared_expert_for_a_token_block(gpu, d, fs, bits, t, gated)
 
 
 @pytest.mark.parametrize("d,f,ne,k,t,bits,slots,slru", [
