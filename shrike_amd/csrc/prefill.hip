@@ -3,6 +3,7 @@
 // sums the grouped FFN folds the affine biases with, the token-major reduce and the
 // residual add.
 #include "prefill_common.h"
+#include <type_traits>
 #include "router_row.h"
 
 #include "../../include/shrike_host.h"
@@ -239,6 +240,163 @@ __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t q
         if (more) stage_store(staged, buf ^ 1u);
         __syncthreads();
     }
+}
+
+// ---- the same logits on the matrix cores, for many tokens
+//
+// v_mfma_f32_16x16x1_4b_f32 is, in each of its four blocks, one IEEE multiply-add an output (checked against fmaf over
+// subnormal products, cancellations and all exponents: the same bits), so a chain of them adds what a lane of router_row adds,
+// in its order. A block's chain is one of router_row's 64 lanes: an output's lane sums l = p + 16 b, b = 0 .. 3, are the four
+// blocks of one accumulator over chunks l, l + 64, ...; the first two stages of the butterfly (xor 32, 16) add the blocks, the
+// next two (8, 4) the accumulators of p = 4 j + w, j = 0 .. 3, that wave w goes through, and the last two (2, 1) meet the four
+// waves in LDS. An affine row's chunk sums its codes' products from zero, in 8 or 16 chains of their own, and takes scale
+// (a multiply-add an output) and bias (one more MFMA) as router_row does.
+//
+// A workgroup takes 16 tokens and 16 experts and brings both sides' chunks of a j in through LDS, four workgroups a compute
+// unit so that one's loads run beside the others' products (two with the next j's loads beside its own were slower: 82
+// against 69 us in all). The matrix cores do twice the plain vector unit's fp32 multiply-adds, and the vector unit keeps the
+// widening only: 31 us of them for 4,096 tokens of 2,048 against 256 rows, where the vector kernel below has 55. With the
+// selection's 11: 91 -> 67 us; 1,000 tokens of 2,304, 8-bit rows, 51 -> 36; 4-bit rows, 512 of 2,048, 25 -> 18.
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+template <int RK>
+__global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, uint32_t query_count, uint32_t stride, float *logits) {
+    warm_kernel_arguments(a);
+    constexpr uint32_t E = kRouterChunk<RK>, Q = E / 8;  // a chunk's elements, 16-byte pieces of x
+    extern __shared__ __align__(16) uint8_t lds[];
+    const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
+    const uint32_t num_experts = a.sel.num_experts, d = a.d, chunks = d / E, walks = (chunks + 63u) / 64u, groups = d / kGroup;
+    // an XCD takes token tiles with all their expert tiles: the rows of `hidden` come to one L2, the experts' to every one
+    const uint32_t expert_tiles = (num_experts + 15u) / 16u;
+    const uint32_t t0 = ((blockIdx.x >> 3) / expert_tiles * 8u + (blockIdx.x & 7u)) * 16u, e0 = (blockIdx.x >> 3) % expert_tiles * 16u;
+    if (t0 >= query_count) return;
+    const uint32_t w_at = 4u * walks * Q * 1024u;  // behind x
+    float *l_eff = reinterpret_cast<float *>(lds + 4u * walks * (Q + 1u) * 1024u);
+    uint16_t *l_scale = reinterpret_cast<uint16_t *>(l_eff + d), *l_bias = l_scale + 16u * groups;
+    const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds));
+    // A load brings a 16-byte piece of four chunks of sixteen rows, the chunks xor-ed with the row so that sixteen rows read
+    // at one chunk touch every bank once. Wave w brings block w's.
+    const uint32_t l_row = lane >> 2, l_chunk = ((lane & 3u) ^ ((l_row >> 2) & 3u)) + 16u * wave;
+    const uint8_t *w_row = static_cast<const uint8_t *>(a.weights) + size_t(min(e0 + l_row, num_experts - 1u)) * chunks * 16u;
+    const uint16_t *x_row = a.hidden + size_t(min(t0 + l_row, query_count - 1u)) * stride;
+    auto load = [&](uint32_t j) {
+        for (uint32_t i = 0; i < walks; ++i) {
+            const uint32_t c = min(4u * j + l_chunk + 64u * i, chunks - 1u);  // past the row: a copy, taken as zero
+#pragma unroll
+            for (uint32_t q = 0; q < Q; ++q) lds_load16(lds0 + ((wave * walks + i) * Q + q) * 1024u, x_row + c * E + q * 8u);
+            lds_load16(lds0 + w_at + (wave * walks + i) * 1024u, w_row + c * 16u);
+        }
+    };
+    load(0);
+    for (uint32_t i = threadIdx.x; i < d / 2u; i += 256u) {
+        const uint32_t pair = reinterpret_cast<const uint32_t *>(a.effective_scale)[i];
+        reinterpret_cast<float2 *>(l_eff)[i] = make_float2(bf16_to_f32(uint16_t(pair)), bf16_to_f32(uint16_t(pair >> 16)));
+    }
+    if (RK != 0) {
+        for (uint32_t i = threadIdx.x; i < 16u * groups; i += 256u) {
+            const uint32_t e = min(e0 + i / groups, num_experts - 1u);
+            l_scale[i] = a.scales[size_t(e) * groups + i % groups];
+            l_bias[i] = a.biases[size_t(e) * groups + i % groups];
+        }
+    }
+    const uint32_t m = lane & 15u, block = lane >> 4;
+    const uint32_t read_at = m * 64u + ((wave ^ ((m >> 2) & 3u)) * 16u);
+    f32x16_t acc;
+    // chunk 64 i + 4 j + wave of each block; CHECK: it may lie past the row
+    auto chunk = [&](uint32_t j, uint32_t i, auto check) {
+        constexpr bool CHECK = decltype(check)::value;
+        const uint32_t c0 = 4u * j + wave + 64u * i, c = c0 + 16u * block;
+        const bool inside = !CHECK || c < chunks;
+        const uint32_t cc = inside ? c : 0u;
+        const uint4 wv = *reinterpret_cast<const uint4 *>(lds + w_at + (block * walks + i) * 1024u + read_at);
+        uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
+        if (CHECK) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) ww[n] = inside ? ww[n] : 0u;
+        }
+        f32x16_t part = {0};
+        float sum = 0.0f;
+#pragma unroll
+        for (uint32_t q = 0; q < Q; ++q) {
+            const uint4 xv = *reinterpret_cast<const uint4 *>(lds + ((block * walks + i) * Q + q) * 1024u + read_at);
+            uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
+            if (CHECK) {
+#pragma unroll
+                for (int n = 0; n < 4; ++n) xw[n] = inside ? xw[n] : 0u;
+            }
+            const float4 e0v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u), e1v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u + 4u);
+            const float ew[8] = {e0v.x, e0v.y, e0v.z, e0v.w, e1v.x, e1v.y, e1v.z, e1v.w};
+#pragma unroll
+            for (uint32_t k = 0; k < 8u; ++k) {
+                // moe.metal:357-358 (the exact product; + 0 makes it one instruction, and a zero's sign is nothing to a sum
+                // that starts at +0)
+                const float x = fmaf(f16_to_f32(uint16_t(xw[k / 2u] >> (16u * (k & 1u)))), ew[k], 0.0f);
+                if (RK == 0) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x1f32(x, f16_to_f32(uint16_t(ww[k / 2u] >> (16u * (k & 1u)))), acc, 0, 0, 0);
+                } else {
+                    constexpr uint32_t kBits = RK == 0 ? 8u : uint32_t(RK), kPer = 32u / kBits;
+                    const uint32_t n = q * 8u + k;
+                    const float code = float((ww[n / kPer] >> (kBits * (n % kPer))) & ((1u << kBits) - 1u));
+                    part = __builtin_amdgcn_mfma_f32_16x16x1f32(x, code, part, 0, 0, 0);
+                    sum = __fadd_rn(sum, x);
+                }
+            }
+        }
+        if (RK != 0) {
+#pragma unroll
+            for (uint32_t b = 0; b < 4u; ++b) {
+                const uint32_t cb = c0 + 16u * b;
+                const float sc = !CHECK || cb < chunks ? meta_f32(l_scale[m * groups + cb * E / kGroup], a.meta) : 0.0f;
+#pragma unroll
+                for (uint32_t r = 0; r < 4u; ++r) acc[4u * b + r] = fmaf(sc, part[4u * b + r], acc[4u * b + r]);
+            }
+            acc = __builtin_amdgcn_mfma_f32_16x16x1f32(sum, inside ? meta_f32(l_bias[m * groups + cc * E / kGroup], a.meta) : 0.0f, acc, 0, 0, 0);
+        }
+    };
+    float even[4], odd[4];
+#pragma unroll
+    for (uint32_t step = 0; step < 4u; ++step) {
+        constexpr uint32_t kOrder[4] = {0, 2, 1, 3};  // of j: the butterfly's
+        wait_loads_and_sync<0>();
+        acc = f32x16_t{0};
+        for (uint32_t i = 0; i + 1u < walks; ++i) chunk(kOrder[step], i, std::false_type{});
+        if (64u * walks == chunks) chunk(kOrder[step], walks - 1u, std::false_type{});
+        else chunk(kOrder[step], walks - 1u, std::true_type{});
+        __syncthreads();
+        if (step < 3u) load(kOrder[(step + 1u) & 3u]);
+#pragma unroll
+        for (uint32_t r = 0; r < 4u; ++r) {
+            const float v = __fadd_rn(__fadd_rn(acc[r], acc[8u + r]), __fadd_rn(acc[4u + r], acc[12u + r]));
+            if (step == 0u) even[r] = v;
+            else if (step == 1u) even[r] = __fadd_rn(even[r], v);
+            else if (step == 2u) odd[r] = v;
+            else even[r] = __fadd_rn(even[r], __fadd_rn(odd[r], v));
+        }
+    }
+    // (the loop's last barrier: nobody reads the operands any more)
+    float (*meet)[16][17] = reinterpret_cast<float (*)[16][17]>(lds);
+    static_assert(sizeof(float[4][16][17]) <= 4u * 2u * 1024u, "the waves' sums fit where one walk's chunks were");
+#pragma unroll
+    for (uint32_t r = 0; r < 4u; ++r) meet[wave][4u * block + r][m] = even[r];
+    __syncthreads();
+    const uint32_t row = threadIdx.x >> 4, col = threadIdx.x & 15u;
+    const float v = __fadd_rn(__fadd_rn(meet[0][row][col], meet[2][row][col]), __fadd_rn(meet[1][row][col], meet[3][row][col]));
+    if (t0 + row < query_count && e0 + col < num_experts) logits[size_t(t0 + row) * num_experts + e0 + col] = v;
+}
+
+// True if it launched: where 16 tokens by 16 experts make more than one workgroup for most compute units. With fewer the four
+// waits of a workgroup are what it takes, some 8 us, and the vector kernel's many small workgroups are done before (fp16 rows,
+// 256 of 2,048: 300 tokens 16.3 against 15.4 us with the selection, 512 17.3 against 20.2; 8-bit, 2,304: 100 tokens 17.1
+// against 16.2, 300 22.3 against 24.2).
+template <int RK>
+static bool launch_prefill_logits_mfma(const RouterArgs &a, uint32_t query_count, uint32_t stride, float *logits, hipStream_t s) {
+    constexpr uint32_t E = kRouterChunk<RK>, Q = E / 8;
+    const uint32_t expert_tiles = (a.sel.num_experts + 15u) / 16u, token_tiles = (query_count + 15u) / 16u;
+    if (uint64_t(expert_tiles) * token_tiles <= (RK == 0 ? 384u : 256u)) return false;
+    const uint32_t walks = (a.d / E + 63u) / 64u;
+    const uint32_t bytes = 4u * walks * (Q + 1u) * 1024u + a.d * 4u + (RK ? 2u * 16u * (a.d / kGroup) * 2u : 0u);
+    hipLaunchKernelGGL(k_prefill_logits_mfma<RK>, dim3(((token_tiles + 7u) & ~7u) * expert_tiles), dim3(256), bytes, s, a, query_count, stride, logits);
+    return true;
 }
 
 template <int RK, int MAXC, int ROWS>
@@ -656,19 +814,23 @@ static int prefill_router(shrike_hip_moe *moe, void *stream, const void *d_weigh
         if (int rc = launch_router_tokens(a, moe->desc.router_weight_bits, query_count, s)) return rc;
         return d_group_sums ? launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, d_group_sums, nullptr, s) : 0;
     }
-    // as many rows a wave as their registers allow: four where a lane's share of a row is up to 48 elements, else two
+    // the vector kernel with as many rows a wave as their registers allow: four where a lane's share of a row is up to 48
+    // elements, else two
     switch (moe->desc.router_weight_bits) {
         case 0:
+            if (launch_prefill_logits_mfma<0>(a, query_count, hidden_stride_elements, d_logits_workspace, s)) break;
             if (d <= 2048u) launch_prefill_logits<0, 4, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             else if (d <= 3072u) launch_prefill_logits<0, 6, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             else launch_prefill_logits<0, 8, 2>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             break;
         case 8:
+            if (launch_prefill_logits_mfma<8>(a, query_count, hidden_stride_elements, d_logits_workspace, s)) break;
             if (d <= 2048u) launch_prefill_logits<8, 2, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             else if (d <= 3072u) launch_prefill_logits<8, 3, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             else launch_prefill_logits<8, 4, 2>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             break;
         default:
+            if (launch_prefill_logits_mfma<4>(a, query_count, hidden_stride_elements, d_logits_workspace, s)) break;
             if (d <= 2048u) launch_prefill_logits<4, 1, 4>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
             else launch_prefill_logits<4, 2, 2>(a, query_count, hidden_stride_elements, d_logits_workspace, s);
     }

@@ -37,4 +37,23 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_u32(uint32_t v, uint32_t
     return v;
 }
 
+// Asynchronous loads into LDS. The compiler does not know of them: the waits for them are counted by hand, and nothing
+// between the first and the last of them may make it issue a vector load of its own.
+__device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+}
+__device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+}
+// All but the wave's last COUNT loads have landed, and its reads of LDS are done.
+template <int COUNT>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(COUNT) : "memory");
+}
+// All but the last COUNT loads have landed for every wave of the workgroup, and no wave still reads the LDS.
+template <int COUNT>
+__device__ __forceinline__ void wait_loads_and_sync() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(COUNT) : "memory");
+}
+
 }  // namespace shrike

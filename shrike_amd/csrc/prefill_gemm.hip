@@ -130,28 +130,9 @@ __device__ __forceinline__ half8 codes8(uint32_t w0, uint32_t w1) {
     return f.h;
 }
 
-// Asynchronous loads into LDS. The compiler does not know of them: the waits for them are counted by hand, and nothing
-// between the first and the last of them may make it issue a vector load of its own.
-__device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
-}
-__device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
-}
 __device__ __forceinline__ void lds_load12(uint32_t lds, const void *p) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx3 %1, off" ::"s"(lds), "v"(p) : "memory");
 }
-// All but the wave's last COUNT loads have landed, and its reads of LDS are done.
-template <int COUNT>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(COUNT) : "memory");
-}
-// All but the last COUNT loads have landed for every wave of the workgroup, and no wave still reads the LDS.
-template <int COUNT>
-__device__ __forceinline__ void wait_loads_and_sync() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(COUNT) : "memory");
-}
-
 typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // eight 16-bit values, wherever they start
 
 // One row tile (WIDE: or two of an expert) against one block of weight rows, 64 rows of them a wave. MODE 0: 32 gate and

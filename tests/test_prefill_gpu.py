@@ -65,7 +65,10 @@ def test_prefill_router_bit_exact_and_equal_to_decode(gpu, router_bits, ne, d, k
     (0, 19, 64, 18), (0, 37, 2048, 61), (0, 20, 2112, 40), (0, 18, 3072, 35), (0, 18, 4096, 33),  # the fp16 instances' edges
     (8, 21, 64, 19), (8, 36, 2048, 63), (8, 19, 2112, 30), (8, 18, 3072, 37), (8, 17, 4096, 41),   # the 8-bit ones
     (4, 33, 128, 17), (4, 50, 2048, 65), (4, 19, 2176, 29), (4, 18, 4096, 31),                     # the 4-bit ones
-    (8, 256, 512, 3), (0, 64, 320, 8), (0, 64, 320, 9), (0, 256, 128, 700), (8, 100, 192, 1300)])  # tokens a launch, a workgroup
+    (8, 256, 512, 3), (0, 64, 320, 8), (0, 64, 320, 9), (0, 256, 128, 700), (8, 100, 192, 1300),   # tokens a launch, a workgroup
+    # on the matrix cores: part of a lane's chunks, whole ones only, ragged tokens and experts
+    (0, 200, 64, 481), (0, 250, 512, 400), (0, 241, 2112, 390), (0, 250, 4096, 391), (8, 250, 64, 300), (8, 241, 1024, 273),
+    (8, 256, 2304, 258), (8, 241, 4096, 272), (4, 249, 128, 270), (4, 256, 2048, 257), (4, 241, 2176, 273), (4, 241, 4096, 258)])
 def test_prefill_router_instances_bit_exact(gpu, router_bits, ne, d, t):
     k = 4
     L = Layer(0x5EED0A00 + router_bits + d, d, 64, ne, k, router_bits=router_bits)
