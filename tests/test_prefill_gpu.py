@@ -177,6 +177,12 @@ def test_device_grouping_equals_host_grouping(gpu, t, k, ne, mode):
     assert got["row_tile_count"] <= routes.max_row_tiles
 
 
+@pytest.mark.parametrize("t,k,ne,mode", [(683, 3, 256, "plain"), (685, 3, 250, "residency"),  # the most pairs of one run, and four uneven ones
+                                         (7001, 8, 64, "plain"), (18001, 8, 64, "keys")])     # ids without weights in LDS, and neither
+def test_device_grouping_of_many_pairs(gpu, t, k, ne, mode):
+    test_device_grouping_equals_host_grouping(gpu, t, k, ne, mode)
+
+
 def check_pair_stagewise(L: Layer, blob, x_row, dev_act, got_row, what, act=O.ACT_SILU):
     """Stage by stage, so that each comparison holds one rounding: the activations against the
     oracle's, the partial row against the oracle's down projection of the device's own
