@@ -9,9 +9,10 @@
 namespace shrike {
 
 constexpr int kPhase1RowPairs = 4;  // (gate, up) row pairs per wave
-// ... and in a launch that does not route, for one token or for rows of three or more 16-byte chunks a lane: twice the
+// ... and for rows of three or more 16-byte chunks a lane, or for one token in a launch that does not route: twice the
 // waves with half the rows in flight each measured faster there (one token 5.06 -> 4.68 us at hidden 2048, a batch of
-// four tokens at hidden 2880 with 8-bit codes 84 -> 79 us a layer; the same batch with 4-bit codes is slower with them)
+// four tokens at hidden 2880 with 8-bit codes 84 -> 79 us a layer; one token with 8-bit codes in the routing launch 17.2 ->
+// 16.4 us at 2880, 16.7 -> 15.3 at 4096; the shorter rows of 4-bit codes are slower with them there, 11.0 -> 13.1 at 2880)
 constexpr int kPhase1RowPairsNarrow = 2;
 
 // A wave owns RP consecutive f of one routed position: RP gate rows and RP up rows, each a
@@ -132,12 +133,12 @@ uint32_t phase1_blocks(uint32_t top_k, uint32_t f) { return phase1_blocks_of(top
 
 // (a row that ends in half chunks counts the steps it would take without them: the choice stays what it was measured as)
 static bool phase1_narrow(bool routing, bool one_token, uint32_t d, uint32_t bits) {
-    return one_token ? !routing : nch_for(d, bits) >= 3;
+    return (one_token && !routing) || nch_for(d, bits) >= 3;
 }
 
 template <int BITS, bool ROUTE, int SBITS, bool STREAM, int META>
 static void launch_phase1_meta(const Phase1Args &a, dim3 grid, hipStream_t s) {
-    // (the one-token routing launch keeps four pairs; a batch takes the narrow form for long rows whether it routes or not)
+    // (shorter rows: the one-token routing launch keeps four pairs)
     constexpr int RP = kPhase1RowPairs, RN = (ROUTE && STREAM) ? kPhase1RowPairs : kPhase1RowPairsNarrow;
     const dim3 block(256);
     if (BITS == 4 && half_chunk_tail(a.d * BITS / 128u, BITS)) {
@@ -148,8 +149,8 @@ static void launch_phase1_meta(const Phase1Args &a, dim3 grid, hipStream_t s) {
     switch (nch_for(a.d, BITS)) {
         case 1: hipLaunchKernelGGL((k_phase1<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
         case 2: hipLaunchKernelGGL((k_phase1<BITS, 2, STREAM ? RN : RP, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
-        case 3: hipLaunchKernelGGL((k_phase1<BITS, 3, RN, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_phase1<BITS, 4, RN, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
+        case 3: hipLaunchKernelGGL((k_phase1<BITS, 3, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((k_phase1<BITS, 4, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
     }
 }
 

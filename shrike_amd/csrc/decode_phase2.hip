@@ -7,8 +7,7 @@
 
 namespace shrike {
 
-constexpr uint32_t kPhase2Rows = 8;       // output rows per workgroup
-constexpr uint32_t kPhase2RowsBatch = 16;  // the same for a batch of tokens over rows of more than one wave load
+constexpr uint32_t kPhase2Rows = 8;  // output rows per workgroup; 4 to 16 where a row is a whole wave load or more
 
 // moe.metal:889-893
 __device__ __forceinline__ void phase2_finish(uint16_t *y, uint16_t *hidden, uint32_t d, uint16_t value,
@@ -21,8 +20,10 @@ __device__ __forceinline__ void phase2_finish(uint16_t *y, uint16_t *hidden, uin
 // rows. When a down row is shorter than a wave's 1 KiB load, the wave covers 64/cpr rows per
 // load and reduces over lane segments. BATCH row groups are in flight per wave.
 // STREAM: one token, every down row is read once: non-temporal row loads (see k_phase1).
-// ROWS: output rows a workgroup owns. One token takes 8 (at d = 2048 that is one workgroup a compute unit); a batch of
-// tokens over long rows takes 16, so that a wave's slice of the activations, fetched once, serves twice the rows.
+// ROWS: output rows a workgroup owns. Packed rows take 8. Rows of a wave load or more take as many as still leave the launch
+// 640 workgroups, two and a half a compute unit (more rows serve a wave's slice of the activations, fetched once, more often;
+// with fewer workgroups too few loads are in flight): one token at hidden 2,880, 4 rows for 8: 10.5 -> 7.9 us with 4-bit
+// codes, 12.9 -> 9.8 with 8-bit ones; two tokens, 8 for 16: 13.4 -> 10.8; four tokens keep 16 (17.6 against 18.7 with 8).
 // TAIL: the rows end in a step of half chunks (load_slice_regs); NCH then counts the whole steps ahead of it.
 // META: the type of the scales and biases (SHRIKE_META_*), known to the instance so that a row converts them one way.
 template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META>
@@ -153,11 +154,14 @@ static void launch_phase2_rows(const Phase2Args &a, dim3 block, hipStream_t s) {
     else launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_BF16>(a, block, s);
 }
 
-// (rows of more than one step a lane, whole or half)
 template <int BITS, int NCH, bool TAIL>
 static void launch_phase2_batch(const Phase2Args &a, dim3 block, hipStream_t s) {
-    if ((NCH >= 2 || TAIL) && a.tokens > 1u) launch_phase2_rows<BITS, NCH, kPhase2RowsBatch, TAIL>(a, block, s);
-    else launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL>(a, block, s);
+    constexpr bool kLong = NCH >= 2 || TAIL;  // rows of more than one step a lane, whole or half
+    const uint32_t tokens = a.tokens ? a.tokens : 1u, cpr = a.f * BITS / 128u;
+    auto enough = [&](uint32_t rows) { return uint64_t(tokens) * ((a.d + rows - 1u) / rows) >= 640u; };
+    if (kLong && enough(16u)) launch_phase2_rows<BITS, NCH, 16u, TAIL>(a, block, s);
+    else if (enough(8u) || (cpr < 64u && 64u % cpr == 0u)) launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL>(a, block, s);
+    else launch_phase2_rows<BITS, NCH, 4u, TAIL>(a, block, s);
 }
 
 template <int BITS>
