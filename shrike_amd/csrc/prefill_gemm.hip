@@ -27,25 +27,28 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // ---- the shape of a workgroup's work and its LDS: places for two groups (of the codes: stages) of the operands, the one in
-// use and the one on its way, that asynchronous loads fill (lane l's piece of a load lands 16 l bytes behind the load's
+// use and the one on its way (kAhead: for three), that asynchronous loads fill (lane l's piece of a load lands 16 l bytes behind the load's
 // address), and after the last product the rows on their way out.
 enum class FfnShape {
     kSplit,  // up to 32 rows against 64 weight rows, a quarter of k a wave (k_ffn_split)
     kTile,   // one row tile, up to 64 rows, against 256 weight rows; three workgroups a compute unit
     kWide,   // two row tiles of one expert, up to 128 rows, against 256 weight rows; two workgroups a compute unit
+    kAhead,  // as kTile, 8-bit codes, with the operands of two groups on their way; two workgroups a compute unit
 };
 constexpr uint32_t kUnitB = 64u * 64u;  // 64 bytes of codes of a wave's 64 weight rows: two groups at 4 bits, one at 8
 constexpr uint32_t kUnitS = 64u * 16u;  // four groups' scales (biases) of those rows, in a 12-byte window each
-template <bool WIDE>
+template <FfnShape S>
 struct Lds {
-    static constexpr uint32_t kRows = WIDE ? 128u : 64u;
+    static constexpr bool kIsWide = S == FfnShape::kWide;
+    static constexpr uint32_t kPlaces = S == FfnShape::kAhead ? 3u : 2u;
+    static constexpr uint32_t kRows = kIsWide ? 128u : 64u;
     static constexpr uint32_t kUnitA = kRows * 128u;  // one group (64 k) of the rows
-    static constexpr uint32_t kB = 2u * kUnitA, kS = kB + 8u * kUnitB, kBytes = kS + 4u * kUnitS;
-    // a unit (32 groups) of the rows' group sums, two of them, where the second group's rows and the second stage's codes will be
-    static constexpr uint32_t kSums0 = kUnitA, kSums1 = kB + 4u * kUnitB;
+    static constexpr uint32_t kB = kPlaces * kUnitA, kS = kB + kPlaces * 4u * kUnitB, kBytes = kS + 4u * kUnitS;
+    // a unit (32 groups) of the rows' group sums, two of them, where the rows and the codes of the last place will be
+    static constexpr uint32_t kSums0 = kB - kUnitA, kSums1 = kS - 4u * kUnitB;
     static_assert(kUnitA <= 4u * kUnitB, "a unit of sums fits");
     static constexpr uint32_t kRow = 256u + 8u;  // halves per row on the way out; the pad spreads the banks
-    static constexpr uint32_t kResident = WIDE ? 2u : 3u;  // workgroups a compute unit holds
+    static constexpr uint32_t kResident = S == FfnShape::kTile ? 3u : 2u;  // workgroups a compute unit holds
     static_assert(kRows * kRow * 2u <= kBytes && kBytes * kResident <= 160u * 1024u, "the rows on the way out fit, and the workgroups a compute unit");
 };
 struct SplitLds {  // of a wave: 32 rows' groups, the codes of 64 weight rows, their scales and biases
@@ -146,16 +149,16 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // workgroup a compute unit fewer. What bounds it now: with many rows the power the matrix cores draw (the clock falls to 1.3
 // to 1.75 GHz, and vector work saved in the loop buys nothing), with few of them the weights' bytes, with few workgroups a
 // wave's own chain of some 1,700 cycles a group (1,200 up to 32 rows). 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens: 843
-// -> 576 us (WIDE 541); 256 of 2,048 x 512, 4,096 tokens: 371 -> 337; 384 of 2,304 x 1,024, 8-bit, 4,000 tokens: 926 -> 758.
+// -> 576 us (WIDE 541); 256 of 2,048 x 512, 4,096 tokens: 371 -> 337; 256 of 2,304 x 1,024, 8-bit, 4,000 tokens: 926 -> 758.
 //
 // MODE 0 leaves its activations through LDS: whole 16-byte pieces of a row go out together, and the group sums of the
 // tile's rows that the down product's bias term needs are formed here, in k_row_group_sums' order of additions (eight
 // lanes a group, a lane adds its eight values in order, the partial sums fold pairwise), instead of by a launch of
 // their own between the two products. Every wave of the workgroup stays to the end for the barriers.
-template <int BITS, int MODE, bool DENSE, uint32_t MT, int META, bool WIDE>
+template <int BITS, int MODE, bool DENSE, uint32_t MT, int META, FfnShape S>
 __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile &tile, uint32_t tile_index, uint32_t col_block,
                                          uint8_t *lds) {
-    typedef Lds<WIDE> L;
+    typedef Lds<S> L;
     const uint32_t K = MODE == 0 ? a.d : a.f, N = MODE == 0 ? a.f : a.d;
     const uint32_t G = K / kGroup;
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
@@ -258,6 +261,12 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     load_s(0);
     load_b(0, 0);
     load_a(0, 0);
+    if constexpr (S == FfnShape::kAhead) {
+        if (G > 1u) {
+            load_b(1, 1);
+            load_a(1, 1);
+        }
+    }
 
     f32x16 total[2][MT];
 #pragma unroll
@@ -352,16 +361,30 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     // ---- the groups. Step g waits for what its group needs (the first also until nobody reads the sums any more) and asks for
     // what a later group will, in the place that group g - 1 left.
     uint32_t run[2][4];  // the scales of a chunk of four groups
+    uint32_t place = 0;  // kAhead: g % 3
+    if constexpr (S == FfnShape::kAhead) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) in the compiler's own count: else it waits for the biases in the loop
     auto step = [&](uint32_t g, auto par) {
         constexpr uint32_t P = decltype(par)::value;  // g & 1
-        const uint32_t b_place = BITS == 8 ? P : (g >> 1) & 1u;
-        if (BITS == 4 && P == 1u && g + 1u < G) wait_loads_and_sync<4>();  // (the next stage's codes may still be on their way)
-        else wait_loads_and_sync<0>();
-        if (g + 1u < G) {
-            load_a(P ^ 1u, g + 1u);
-            if (BITS == 8) load_b(b_place ^ 1u, g + 1u);
+        const uint32_t a_place = S == FfnShape::kAhead ? place : P;
+        const uint32_t b_place = S == FfnShape::kAhead ? place : BITS == 8 ? P : (g >> 1) & 1u;
+        if constexpr (S == FfnShape::kAhead) {
+            if (g + 1u < G) wait_loads_and_sync<kLoadsA + 4>();  // (the next group's may still be on their way)
+            else wait_loads_and_sync<0>();
+            const uint32_t left = place == 0u ? 2u : place - 1u;
+            if (g + 2u < G) {
+                load_b(left, g + 2u);
+                load_a(left, g + 2u);
+            }
+            place = place == 2u ? 0u : place + 1u;
+        } else {
+            if (BITS == 4 && P == 1u && g + 1u < G) wait_loads_and_sync<4>();  // (the next stage's codes may still be on their way)
+            else wait_loads_and_sync<0>();
+            if (g + 1u < G) {
+                load_a(P ^ 1u, g + 1u);
+                if (BITS == 8) load_b(b_place ^ 1u, g + 1u);
+            }
+            if (BITS == 4 && P == 0u && g + 2u < G) load_b(b_place ^ 1u, (g >> 1) + 1u);
         }
-        if (BITS == 4 && P == 0u && g + 2u < G) load_b(b_place ^ 1u, (g >> 1) + 1u);
         if (active) {
             if ((g & 3u) == 0u) {
 #pragma unroll
@@ -375,7 +398,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         }
         if ((g & 3u) == 1u && g + 3u < G) load_s((g >> 2) + 1u);  // (a step's wait is for the reads above, too)
         if (active) {
-            const uint8_t *a_rows = lds + P * L::kUnitA + col * 128u;
+            const uint8_t *a_rows = lds + a_place * L::kUnitA + col * 128u;
             uint4 codes[2][BITS / 4];
             float sc[2];
 #pragma unroll
@@ -530,10 +553,11 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     }
 }
 
-template <int BITS, int MODE, bool DENSE, int META, bool WIDE>
-__global__ __launch_bounds__(256, (Lds<WIDE>::kResident)) void k_grouped_ffn(FfnArgs a) {
+template <int BITS, int MODE, bool DENSE, int META, FfnShape S>
+__global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArgs a) {
     warm_kernel_arguments(a);
-    __shared__ __align__(16) uint8_t lds[Lds<WIDE>::kBytes];
+    __shared__ __align__(16) uint8_t lds[Lds<S>::kBytes];
+    constexpr bool WIDE = S == FfnShape::kWide;
     // Which (row tile, column block) this workgroup takes. Workgroups go to the chip's eight XCDs (each
     // with an L2 of its own) round robin in launch order, so workgroup w runs on XCD w % 8 as that XCD's
     // item w / 8. An expert's row tiles are neighbours in the tile table: an XCD takes a contiguous run
@@ -658,10 +682,10 @@ __global__ __launch_bounds__(256, (Lds<WIDE>::kResident)) void k_grouped_ffn(Ffn
         if (tile.pair_start + tile.rows <= a.pair_lo || tile.pair_start >= a.pair_hi) return;
     }
 
-    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, WIDE>(a, tile, tile_index, col_block, lds);
-    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, WIDE>(a, tile, tile_index, col_block, lds);
-    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, WIDE>(a, tile, tile_index, col_block, lds);
-    else ffn_tile<BITS, MODE, DENSE, 1, META, WIDE>(a, tile, tile_index, col_block, lds);
+    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, S>(a, tile, tile_index, col_block, lds);
+    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, S>(a, tile, tile_index, col_block, lds);
+    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, S>(a, tile, tile_index, col_block, lds);
+    else ffn_tile<BITS, MODE, DENSE, 1, META, S>(a, tile, tile_index, col_block, lds);
 }
 
 // ---- few rows: the same products with k split over the waves.
@@ -963,15 +987,15 @@ static uint32_t compute_units() {
     return uint32_t(units);
 }
 
-template <int BITS, bool DENSE, int META, bool WIDE>
+template <int BITS, bool DENSE, int META, FfnShape S>
 static int launch_ffn_shape(FfnArgs a, uint32_t max_tiles, hipStream_t s) {
-    a.resident_workgroups = Lds<WIDE>::kResident * compute_units();
+    a.resident_workgroups = Lds<S>::kResident * compute_units();
     const dim3 block(256);
     const uint32_t grid_tiles = (max_tiles + 7u) & ~7u;  // whole runs for the kernel's XCD mapping
-    hipLaunchKernelGGL((k_grouped_ffn<BITS, 0, DENSE, META, WIDE>), dim3(grid_tiles, (a.f + 127u) / 128u), block, 0, s, a);
+    hipLaunchKernelGGL((k_grouped_ffn<BITS, 0, DENSE, META, S>), dim3(grid_tiles, (a.f + 127u) / 128u), block, 0, s, a);
     SHRIKE_HIP(hipGetLastError());
     // (the activations' group sums were written by the gate/up launch itself)
-    hipLaunchKernelGGL((k_grouped_ffn<BITS, 1, DENSE, META, WIDE>), dim3(grid_tiles, (a.d + 255u) / 256u), block, 0, s, a);
+    hipLaunchKernelGGL((k_grouped_ffn<BITS, 1, DENSE, META, S>), dim3(grid_tiles, (a.d + 255u) / 256u), block, 0, s, a);
     SHRIKE_HIP(hipGetLastError());
     return 0;
 }
@@ -990,8 +1014,10 @@ template <int BITS, bool DENSE, int META>
 static int launch_ffn_meta(const FfnArgs &a, uint32_t max_tiles, FfnShape shape, hipStream_t s) {
     if (shape == FfnShape::kSplit) return launch_ffn_split<BITS, DENSE, META>(a, max_tiles, s);
     if constexpr (!DENSE)
-        if (shape == FfnShape::kWide) return launch_ffn_shape<BITS, DENSE, META, true>(a, max_tiles, s);
-    return launch_ffn_shape<BITS, DENSE, META, false>(a, max_tiles, s);
+        if (shape == FfnShape::kWide) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kWide>(a, max_tiles, s);
+    if constexpr (!DENSE && BITS == 8)
+        if (shape == FfnShape::kAhead) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kAhead>(a, max_tiles, s);
+    return launch_ffn_shape<BITS, DENSE, META, FfnShape::kTile>(a, max_tiles, s);
 }
 template <int BITS, bool DENSE>
 static int launch_ffn(const FfnArgs &a, uint32_t max_tiles, FfnShape shape, hipStream_t s) {
@@ -1027,16 +1053,20 @@ size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max
 //    1,536 x 1,024 it takes 21 us for 16 tokens where kTile takes 30, and 24.6 against 37.9 for 100 (8-bit codes). Past that it
 //    loses: its pieces are short and none of them overlaps the next in its workgroup (256 experts of 2,048 x 512, 128 tokens:
 //    150 against 126 us).
-//  - kWide where the experts' rows fill its tiles: from 48 pairs an expert at 8 bits (384 experts, 2,000 tokens: 528 against
+//  - kWide where the experts' rows fill its tiles: from 48 pairs an expert at 8 bits (256 experts of 2,304 x 1,024, 2,000 tokens: 528 against
 //    645 us), from 64 at 4 bits, there only where the launch still has several workgroups for every compute unit (32 experts
 //    of 2,880 x 2,880, 2,048 tokens: 541 against 576 us; 256 experts of 2,048 x 512: 337 against 339 at 4,096 tokens, but 193
 //    against 169 at 2,000 unevenly spread ones).
+//  - kAhead for 8-bit codes up to 16 pairs an expert: the launch is then the weights coming in, and two groups on their way in
+//    two workgroups draw more of them than one group in three (256 experts of 2,304 x 1,024: 16 tokens 182 -> 156 us, 64 346
+//    -> 316, 200 404 -> 376, that is 4.8 TB/s). With more rows the third workgroup's products count (256 experts of 2,048 x
+//    512, 1,000 uneven tokens: 125 against 136 us), and with 4-bit codes they count from the start.
 static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t f, uint32_t bits) {
     const uint64_t most_tiles = min(pairs, uint64_t(experts)) + pairs / kRowTile;
     if (most_tiles * (f / 32u) <= 1024u) return FfnShape::kSplit;
     if (bits == 8 ? pairs >= 48u * uint64_t(experts) : pairs >= 64u * uint64_t(experts) && pairs / kRowTile * ((f + 127u) / 128u) >= 1400u)
         return FfnShape::kWide;
-    return FfnShape::kTile;
+    return bits == 8 && pairs <= 16u * uint64_t(experts) ? FfnShape::kAhead : FfnShape::kTile;
 }
 // ... and of a dense expert's, whose rows are its tiles: kSplit up to two pieces a workgroup (2,048 x 512, 4-bit: 13 against
 // 45 us for 37 rows, 16 against 48 for 512, 32 against 47 for 1,500; 2,304 x 1,024, 8-bit: 44 against 54 for 1,000), kTile

@@ -312,7 +312,9 @@ def test_grouped_ffn_shape_sweep(gpu, case):
     # groups that no quarter shares evenly
     (64, 64, 3, 2, 20, 4, S.META_BF16), (128, 192, 2, 1, 45, 8, S.META_F16), (2880, 64, 4, 2, 50, 4, S.META_F16),
     # one row tile a workgroup: fewer than eight groups and more than sixty-four, both odd
-    (192, 4160, 6, 2, 70, 4, S.META_BF16), (4032, 1088, 40, 3, 33, 8, S.META_F16),
+    (192, 4160, 6, 2, 70, 4, S.META_BF16), (192, 1088, 24, 4, 120, 8, S.META_F16),
+    # the same two groups ahead: one group, two, and odd many
+    (64, 4096, 9, 2, 12, 8, S.META_BF16), (128, 4096, 9, 2, 70, 8, S.META_F16), (4032, 1088, 40, 3, 33, 8, S.META_F16),
     # two row tiles of an expert a workgroup: 128 rows and what is left over, odd groups, column blocks that end inside it
     (128, 8192, 6, 4, 360, 4, S.META_BF16), (576, 3008, 8, 4, 960, 4, S.META_F16), (960, 832, 24, 4, 300, 8, S.META_BF16)])
 def test_grouped_ffn_shapes_of_a_workgroup(gpu, d, f, ne, k, t, bits, meta):
