@@ -156,7 +156,7 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // lanes a group, a lane adds its eight values in order, the partial sums fold pairwise), instead of by a launch of
 // their own between the two products. Every wave of the workgroup stays to the end for the barriers.
 template <int BITS, int MODE, bool DENSE, uint32_t MT, int META, FfnShape S>
-__device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile &tile, uint32_t tile_index, uint32_t col_block,
+__device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile &tile, uint32_t act_row, uint32_t col_block,
                                          uint8_t *lds) {
     typedef Lds<S> L;
     const uint32_t K = MODE == 0 ? a.d : a.f, N = MODE == 0 ? a.f : a.d;
@@ -182,8 +182,8 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             row = a.hidden + size_t(token) * a.hidden_stride;
             a_sums[j] = a.hidden_sums + size_t(token) * G;
         } else {
-            row = a.act + (size_t(tile_index) * kRowTile + r) * a.f;
-            a_sums[j] = a.act_sums + (size_t(tile_index) * kRowTile + r) * G;
+            row = a.act + (size_t(act_row) + r) * a.f;
+            a_sums[j] = a.act_sums + (size_t(act_row) + r) * G;
         }
         a_src[j] = reinterpret_cast<const uint8_t *>(row) + (((lane & 7u) ^ (lane >> 3)) * 16u);
     }
@@ -343,7 +343,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         for (uint32_t mt = 0; mt < MT; ++mt) {
             const uint32_t r = min(mt * 32u + col, tile.rows - 1u);
             const uint32_t token = (MODE != 0) ? 0u : DENSE ? tile.pair_start + r : a.pairs[tile.pair_start + r].token;
-            const uint32_t *row = MODE == 0 ? sums + size_t(token) * G : sums + (size_t(tile_index) * kRowTile + r) * G;
+            const uint32_t *row = MODE == 0 ? sums + size_t(token) * G : sums + (size_t(act_row) + r) * G;
 #pragma unroll
             for (uint32_t jj = 0; jj < 4u; ++jj) afr[mt].u[jj] = 4u * kb + jj < G ? row[4u * kb + jj] : 0u;
         }
@@ -486,7 +486,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         for (uint32_t idx = threadIdx.x; idx < tile.rows * 16u; idx += 256u) {
             const uint32_t m = idx >> 4, pc = idx & 15u;
             if (pc * 8u < columns)
-                *reinterpret_cast<uint4 *>(a.act + (size_t(tile_index) * kRowTile + m) * a.f + c0 + pc * 8u) =
+                *reinterpret_cast<uint4 *>(a.act + (size_t(act_row) + m) * a.f + c0 + pc * 8u) =
                     *reinterpret_cast<const uint4 *>(&s_out[m][pc * 8u]);
         }
         uint32_t *sums_out = const_cast<uint32_t *>(a.act_sums);
@@ -496,7 +496,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
             const float sum = eighth_sum(w);
             if (eighth == 0u && m < tile.rows && gl * 64u < columns)
-                sums_out[(size_t(tile_index) * kRowTile + m) * (a.f / kGroup) + c0 / kGroup + gl] = split_hi_lo(sum);
+                sums_out[(size_t(act_row) + m) * (a.f / kGroup) + c0 / kGroup + gl] = split_hi_lo(sum);
         }
     } else {
         // the down product's rows leave through the LDS too, [row][column of this block of 256], and go
@@ -567,11 +567,29 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
     const uint32_t tile_total = DENSE ? (a.dense_rows + kRowTile - 1u) / kRowTile : *a.tile_count;
     const uint32_t w = blockIdx.y * gridDim.x + blockIdx.x;
     const uint32_t xcd = w & 7u, item = w >> 3;
+    // Where the table is short (64 tiles: one record a lane) and the chip holds the whole launch at once even so, what a tile
+    // has past 32 rows is a workgroup's of its own, behind the others. Such a launch is as long as its longest workgroup, and
+    // one of more than 32 rows has twice the matrix work a group of k. Measured, both products: 37 tokens of the 35B shape, 38
+    // tiles, 45.9 -> 34.8 us; 64 tokens, 49 tiles, 48.3 -> 37.2. Where not every part finds a place at once the codes would be
+    // read and converted twice for nothing, so the tiles stay whole. A row's result does not depend on its place in a tile.
+    uint32_t parts = tile_total;
+    uint64_t larger = 0;
+    uint4 short_table = zero4();
+    if (!WIDE && !DENSE && tile_total <= 64u) {
+        const uint32_t lane = threadIdx.x & 63u;
+        if (lane < tile_total) short_table = reinterpret_cast<const uint4 *>(a.tiles)[lane];
+        larger = __ballot(short_table.z > 32u);
+        parts += uint32_t(__popcll(larger));
+        if (parts * column_blocks > a.resident_workgroups || parts + 7u > gridDim.x) {
+            parts = tile_total;
+            larger = 0;
+        }
+    }
     // tiles an XCD takes: an eighth of them, the first (total mod 8) XCDs one more
-    const uint32_t run = tile_total / 8u + (xcd < tile_total % 8u ? 1u : 0u), first = xcd * (tile_total / 8u) + min(xcd, tile_total % 8u);
+    const uint32_t run = parts / 8u + (xcd < parts % 8u ? 1u : 0u), first = xcd * (parts / 8u) + min(xcd, parts % 8u);
     const uint32_t place = item / column_blocks, col_block = item % column_blocks;  // the workgroup's place in its XCD's run
     if (place >= run) return;
-    uint32_t tile_index = first + place;
+    uint32_t tile_index = first + place, skip = 0;
     shrike_row_tile tile;
     if (DENSE) {
         if (tile_index >= tile_total) return;
@@ -580,7 +598,7 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
         tile.rows = min(kRowTile, a.dense_rows - tile.pair_start);
         tile.expert = 0;
     } else {
-        if (tile_index >= tile_total) return;
+        if (tile_index >= parts) return;
         // Which tile of the table the workgroup takes. A compute unit holds several of these workgroups, whose waves share its
         // SIMDs' issue, and an XCD's workgroups reach its compute units in launch order, one each before any gets a second
         // (read from the hardware: item i and item i + 32 of an XCD share a unit). A tile of more than 32 rows is twice a
@@ -593,8 +611,20 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
         // A lane reads one record; the chosen one is read across (no second load).
         const uint32_t lane = threadIdx.x & 63u;
         const uint32_t gate_up_blocks = (a.f + 127u) / 128u;
-        bool chosen = false;
-        if (!WIDE && tile_total <= 256u && tile_total * gate_up_blocks <= a.resident_workgroups) {
+        bool chosen = larger != 0u;
+        if (chosen) {
+            if (tile_index >= tile_total) {
+                uint64_t rest = larger;
+                for (uint32_t n = tile_index - tile_total; n != 0u; --n) rest &= rest - 1u;
+                tile_index = uint32_t(__ffsll((long long)rest)) - 1u;
+                skip = 32u;
+            }
+            tile.cell = uint32_t(__builtin_amdgcn_readlane(int(short_table.x), int(tile_index)));
+            tile.pair_start = uint32_t(__builtin_amdgcn_readlane(int(short_table.y), int(tile_index))) + skip;
+            const uint32_t rows = uint32_t(__builtin_amdgcn_readlane(int(short_table.z), int(tile_index)));
+            tile.rows = skip ? rows - 32u : min(rows, 32u);
+            tile.expert = uint32_t(__builtin_amdgcn_readlane(int(short_table.w), int(tile_index)));
+        } else if (!WIDE && tile_total <= 256u && tile_total * gate_up_blocks <= a.resident_workgroups) {
             // (four named records, not an array: the compiler kept an array of them in private memory)
             const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
             const uint4 rec0 = lane < tile_total ? table[lane] : zero4();
@@ -682,10 +712,11 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
         if (tile.pair_start + tile.rows <= a.pair_lo || tile.pair_start >= a.pair_hi) return;
     }
 
-    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, S>(a, tile, tile_index, col_block, lds);
-    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, S>(a, tile, tile_index, col_block, lds);
-    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, S>(a, tile, tile_index, col_block, lds);
-    else ffn_tile<BITS, MODE, DENSE, 1, META, S>(a, tile, tile_index, col_block, lds);
+    const uint32_t act_row = tile_index * kRowTile + skip;
+    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, S>(a, tile, act_row, col_block, lds);
+    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, S>(a, tile, act_row, col_block, lds);
+    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, S>(a, tile, act_row, col_block, lds);
+    else ffn_tile<BITS, MODE, DENSE, 1, META, S>(a, tile, act_row, col_block, lds);
 }
 
 // ---- few rows: the same products with k split over the waves.

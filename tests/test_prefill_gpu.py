@@ -329,6 +329,20 @@ def test_grouped_ffn_shapes_of_a_workgroup(gpu, d, f, ne, k, t, bits, meta):
         pc.check_pair(got, int(tok), int(rank), f"token {tok} rank {rank}")
 
 
+@pytest.mark.parametrize("d,f,bits,meta", [(320, 640, 4, S.META_BF16), (1088, 704, 8, S.META_F16)])
+def test_grouped_ffn_of_few_larger_tiles(gpu, d, f, bits, meta):
+    """Experts of 0, 1, 32, 33, 64 and more rows, few enough for a tile's rows past 32 to be a workgroup's of their own."""
+    counts = [33, 64, 65, 96, 97, 32, 1, 0] + [20] * 32
+    idx = np.random.default_rng(8).permutation(np.repeat(np.arange(40), counts)).astype(np.uint32)
+    pc = PrefillCase(gpu, Layer(0x5EED0500 + d, d, f, 40, 1, bits=bits, meta=meta), len(idx), idx=idx)
+    got = pc.run()
+    assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
+    for e in range(6):  # an expert's pairs lie in token order: the first and last row of each part of a tile
+        tokens = np.flatnonzero(idx == e)
+        for r in sorted({r for r in (0, 31, 32, 63, 64, 95, 96, len(tokens) - 1) if r < len(tokens)}):
+            pc.check_pair(got, int(tokens[r]), 0, f"expert {e} row {r}")
+
+
 def test_grouped_ffn_gpt_oss_epilogues(gpu):
     # additive biases + clamped SwiGLU at the gpt-oss shape (moe.metal:257-288), 45 groups per row
     d = f = 2880
