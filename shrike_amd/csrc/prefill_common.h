@@ -38,12 +38,14 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_u32(uint32_t v, uint32_t
 }
 
 // Asynchronous loads into LDS. The compiler does not know of them: the waits for them are counted by hand, and nothing
-// between the first and the last of them may make it issue a vector load of its own.
+// between the first and the last of them may make it issue a vector load of its own. The LDS address goes in m0, which the
+// compiler sets as the operand it is there: a write of m0 inside the assembly would be one that it does not know of either,
+// and its own uses of m0 on both sides would take each other's value for still there.
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
 // All but the wave's last COUNT loads have landed, and its reads of LDS are done.
 template <int COUNT>

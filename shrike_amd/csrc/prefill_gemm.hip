@@ -134,7 +134,7 @@ __device__ __forceinline__ half8 codes8(uint32_t w0, uint32_t w1) {
 }
 
 __device__ __forceinline__ void lds_load12(uint32_t lds, const void *p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx3 %1, off" ::"s"(lds), "v"(p) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx3 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
 typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // eight 16-bit values, wherever they start
 

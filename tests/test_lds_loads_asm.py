@@ -1,0 +1,44 @@
+"""The hand-written loads into LDS beside the compiler's own: both take their LDS address from m0, so each must know of the
+other's. Read from the AMD assembly that the library's own header compiles to; no GPU."""
+import re
+import subprocess
+
+import pytest
+
+from tests.conftest import ROOT
+
+FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         "--cuda-device-only", "-S", "-w"]
+KERNEL = """
+#include "prefill_common.h"
+using namespace shrike;
+__global__ void k(const uint32_t *p, uint32_t *out) {
+    __shared__ uint32_t a[64], b[256];
+    auto into_a = [&](const uint32_t *q) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(q + threadIdx.x),
+                                         (__attribute__((address_space(3))) void *)a, 4, 0, 0);
+    };
+    into_a(p);
+    LOAD;
+    into_a(p + 512);
+    wait_loads_and_sync<0>();
+    out[threadIdx.x] = a[threadIdx.x] + b[threadIdx.x];
+}
+"""
+LDS_B = "uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)b))"
+
+
+@pytest.mark.parametrize("load", [f"lds_load16({LDS_B}, p + 64 + 4 * threadIdx.x)", f"lds_load16({LDS_B}, p, 256 + 16 * threadIdx.x)"])
+def test_the_compiler_knows_what_m0_holds_after_a_hand_written_load(tmp_path, load):
+    source = tmp_path / "k.hip"
+    source.write_text(KERNEL.replace("LOAD", load))
+    subprocess.run(["/opt/rocm/bin/hipcc", *FLAGS, f"-I{ROOT}/shrike_amd/csrc", str(source), "-o", str(tmp_path / "k.s")], check=True)
+    m0 = None
+    addresses = []  # of the loads, in program order
+    for line in (tmp_path / "k.s").read_text().splitlines():
+        if written := re.search(r"s_mov\w* m0, (.+)", line):
+            m0 = written.group(1)
+        elif "global_load_lds" in line:
+            addresses.append(m0)
+    assert len(addresses) == 3
+    assert addresses[0] == addresses[2] != addresses[1], f"the loads' LDS addresses: {addresses}"
