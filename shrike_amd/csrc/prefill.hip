@@ -319,18 +319,15 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
 #pragma unroll
         for (uint32_t q = 0; q < Q; ++q) {
             const uint4 xv = *reinterpret_cast<const uint4 *>(lds + ((block * walks + i) * Q + q) * 1024u + read_at);
-            uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
-            if (CHECK) {
-#pragma unroll
-                for (int n = 0; n < 4; ++n) xw[n] = inside ? xw[n] : 0u;
-            }
+            const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
             const float4 e0v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u), e1v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u + 4u);
             const float ew[8] = {e0v.x, e0v.y, e0v.z, e0v.w, e1v.x, e1v.y, e1v.z, e1v.w};
 #pragma unroll
             for (uint32_t k = 0; k < 8u; ++k) {
                 // moe.metal:357-358 (the exact product; + 0 makes it one instruction, and a zero's sign is nothing to a sum
                 // that starts at +0)
-                const float x = fmaf(f16_to_f32(uint16_t(xw[k / 2u] >> (16u * (k & 1u)))), ew[k], 0.0f);
+                // (past the row the product is the zero, not its factor: chunk 0's effective scale may be infinite)
+                const float product = fmaf(f16_to_f32(uint16_t(xw[k / 2u] >> (16u * (k & 1u)))), ew[k], 0.0f), x = inside ? product : 0.0f;
                 if (RK == 0) {
                     acc = __builtin_amdgcn_mfma_f32_16x16x1f32(x, f16_to_f32(uint16_t(ww[k / 2u] >> (16u * (k & 1u)))), acc, 0, 0, 0);
                 } else {

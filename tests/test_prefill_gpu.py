@@ -82,6 +82,44 @@ def test_prefill_router_instances_bit_exact(gpu, router_bits, ne, d, t):
     assert np.array_equal(idx.download(np.uint32, t * k), ref_idx)
 
 
+@pytest.mark.parametrize("values", ["infinite", "subnormal", "cancelling"])
+@pytest.mark.parametrize("router_bits,ne,d,t", [(0, 241, 2112, 390), (8, 241, 1088, 273), (4, 241, 2176, 273)])
+def test_prefill_router_on_the_matrix_cores_takes_any_values(gpu, router_bits, ne, d, t, values):
+    """Rows that end inside a walk of chunks, on the matrix cores: an infinite effective scale, products and sums down to
+    fp32's smallest subnormals, neighbours that cancel to their last bit."""
+    L = Layer(0x5EED0B00 + router_bits, d, 64, ne, 4, router_bits=router_bits)
+    rows = f16(token_rows(L, t, d)).reshape(t, d)
+    rng = np.random.default_rng(9)
+    eff = np.ones(d, np.float32)
+    if values == "infinite":
+        eff[0] = np.inf
+        if router_bits:  # biases of the scales' sign: an infinite product keeps its sign through scale and bias
+            L.router_b = L.router_b & np.uint16(0x7FFF)
+    elif values == "subnormal":
+        eff = np.exp2(rng.integers(-126, -99, d)).astype(np.float32)
+        rows = rows * np.exp2(-(np.arange(t) % 24.0))[:, None]
+    else:
+        eff = np.repeat(np.exp2(rng.integers(-8, 9, d // 2)), 2).astype(np.float32)
+        rows[:, 1::2] = -rows[:, ::2]
+        if router_bits == 4:
+            low = L.router_w & 0x0F
+            L.router_w = low | (low ^ rng.integers(0, 2, low.shape).astype(np.uint8)) << 4
+        else:
+            L.router_w[:, 1::2] = L.router_w[:, ::2] ^ rng.integers(0, 2, L.router_w[:, ::2].shape).astype(L.router_w.dtype)
+    L.eff_scale = S.f32_to_bf16_bits(eff)
+    x = S.f32_to_f16_bits(rows.astype(np.float32)).reshape(-1)
+    dl = DeviceLayer(gpu, L, resident=[])
+    _, _, _, ws = run_router(gpu, dl, L, gpu.dev(x), t, d)
+    logits = ws.download(np.float32, t * ne).reshape(t, ne)
+    want = np.stack([O.router_logits(L.router_w, L.router_s, L.router_b, router_bits, x[i * d:(i + 1) * d], L.eff_scale, ne, d, meta=L.meta)
+                     for i in range(t)])
+    ordinary = ~np.isnan(want)
+    assert np.array_equal(np.isnan(logits), ~ordinary)
+    assert np.array_equal(logits[ordinary].view(np.uint32), want[ordinary].view(np.uint32))
+    smallest = np.finfo(np.float32).smallest_normal
+    assert {"infinite": np.isinf(want).any(), "subnormal": ((want != 0) & (np.abs(want) < smallest)).any(), "cancelling": True}[values]
+
+
 @pytest.mark.parametrize("router_bits,ne,d,f,k,t,pad,bits", [
     (0, 64, 2048, 512, 8, 70, 0, 4),     # the fp16 logits kernel with four packed rows a wave forms the sums itself
     (0, 24, 2880, 384, 4, 21, 8, 8),     # the instance for longer rows; an odd token count, padded rows
