@@ -5,6 +5,8 @@ the cases of ExpertLoadOperationTests.swift."""
 import ctypes as C
 import json
 import os
+import subprocess
+import sys
 import zlib
 
 import numpy as np
@@ -16,6 +18,7 @@ from shrike_amd import host as HL
 from shrike_amd import synth as S
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
 
 
 def test_int4_gemv_export_gives_the_reference_c_bits():
@@ -54,6 +57,28 @@ def test_int4_gemv_in_blocks_of_rows_equals_the_oracle(rows, n):
     x = tree.key("x").normal(n).astype(np.float32)
     y = HL.int4_affine_gemv(w, s, b, x, rows, n)
     assert np.array_equal(y.view(np.uint32), O.int4_affine_gemv(w, s, b, x, rows, n, S.META_BF16).view(np.uint32))
+
+
+@pytest.mark.parametrize("d,f", [(2048, 512), (2880, 2880)])
+def test_cpu_expert_runs_on_a_thread_of_a_small_stack(d, f):
+    """128 KB of stack, in a process of its own: the call itself may take no more than a small part of it."""
+    program = f"""
+import threading
+import numpy as np
+from shrike_amd import host, synth as S
+from shrike_amd import runtime as rt
+d, f = {d}, {f}
+blob = S.expert_blob(S.SeedTree(3), "e", d, f)
+args = [blob, rt.expert_offsets(d, f, 4)[0], np.ones(d, np.float32), d, f, 0.5, np.zeros(d, np.float32), np.empty(2 * f + d, np.float32)]
+host.cpu_expert_ffn_accumulate(*args)
+want, args[6] = args[6], np.zeros(d, np.float32)
+threading.stack_size(128 * 1024)
+thread = threading.Thread(target=host.cpu_expert_ffn_accumulate, args=args)
+thread.start()
+thread.join()
+assert np.array_equal(args[6], want) and np.any(want)
+"""
+    subprocess.run([sys.executable, "-c", program], check=True, cwd=ROOT)
 
 
 def test_cpu_expert_ffn_accumulate_equals_the_oracle_bit_for_bit_and_accumulates():
