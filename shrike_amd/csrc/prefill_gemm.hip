@@ -672,21 +672,30 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
         }
         const uint32_t count = run;
         if (WIDE) {
-            // Two neighbouring tiles of an expert are one workgroup's work: the first of them takes both. A tile is a first
-            // one where an even number of its expert's tiles are ahead of it.
-            tile = a.tiles[tile_index];
-            uint32_t ahead = 0;
-            for (uint32_t at = tile_index;; at -= 64u) {
-                const bool same = lane < at && a.tiles[at - 1u - lane].expert == tile.expert;
-                const uint64_t others = ~__ballot(same);
-                ahead += others ? uint32_t(__ffsll((long long)others)) - 1u : 64u;
-                if (others) break;
+            // Two neighbouring tiles of an expert are one workgroup's work where the second continues the first's pairs (as
+            // grouping leaves them; a caller's table may leave tiles out): the first of them takes both. A tile is a first one
+            // where an even number of tiles ahead of it, each continuing the one before, run into it. Lane l reads record
+            // at - l; the one before it is lane l + 1's.
+            const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
+            uint32_t ahead = 0, second_rows = 0;
+            for (uint32_t at = tile_index + 1u, skip_links = 1u;; at -= 63u, skip_links = 0u) {
+                const uint4 rec = lane <= at && at - lane < tile_total ? table[at - lane] : zero4();
+                const uint4 before = make_uint4(__shfl_down(rec.x, 1), __shfl_down(rec.y, 1), __shfl_down(rec.z, 1), __shfl_down(rec.w, 1));
+                const bool follows = lane < min(at, 63u) && rec.w == before.w && rec.x == before.x && before.z == kRowTile && rec.y == before.y + kRowTile;
+                const uint64_t links = __ballot(follows);
+                if (skip_links) {
+                    tile.cell = uint32_t(__builtin_amdgcn_readlane(int(rec.x), 1));
+                    tile.pair_start = uint32_t(__builtin_amdgcn_readlane(int(rec.y), 1));
+                    tile.rows = uint32_t(__builtin_amdgcn_readlane(int(rec.z), 1));
+                    tile.expert = uint32_t(__builtin_amdgcn_readlane(int(rec.w), 1));
+                    if (links & 1u) second_rows = uint32_t(__builtin_amdgcn_readlane(int(rec.z), 0));
+                }
+                const uint32_t run_in = uint32_t(__ffsll((long long)~(links >> skip_links))) - 1u;
+                ahead += run_in;
+                if (run_in < 63u - skip_links) break;
             }
             if (ahead & 1u) return;
-            if (tile_index + 1u < tile_total) {
-                const shrike_row_tile second = a.tiles[tile_index + 1u];
-                if (second.expert == tile.expert) tile.rows += second.rows;
-            }
+            tile.rows += second_rows;
         } else if (chosen) {
         } else if (count <= 64u) {
             const uint4 rec = lane < count ? reinterpret_cast<const uint4 *>(a.tiles)[first + lane] : zero4();

@@ -381,6 +381,28 @@ def test_grouped_ffn_of_few_larger_tiles(gpu, d, f, bits, meta):
             pc.check_pair(got, int(tokens[r]), 0, f"expert {e} row {r}")
 
 
+@pytest.mark.parametrize("counts,out", [([200, 330] + [30] * 22, [1, 6]), ([4200, 200, 300, 100], [68])])
+def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out):
+    """Two row tiles a workgroup are two that continue each other, not any two neighbours of the table: tiles inside an expert's
+    left out; an expert of more tiles than a wave reads at once."""
+    ne = len(counts)
+    idx = np.random.default_rng(10).permutation(np.repeat(np.arange(ne), counts)).astype(np.uint32)
+    pc = PrefillCase(gpu, Layer(0x5EED0600, 192, 896, ne, 1, bits=8, meta=S.META_BF16), len(idx), idx=idx)
+    table = pc.routes.download()["row_tiles"]
+    kept = np.delete(table, out, axis=0)
+    pc.routes.row_tiles.upload(np.ascontiguousarray(kept))
+    pc.routes.row_tile_count.upload(np.array([len(kept)], np.uint32))
+    got = pc.run()[:, 0]
+    pair_tokens = pc.routes.download()["sorted_pairs"][:, 0]
+    for i, (_, start, rows, expert) in enumerate(table):
+        tokens = pair_tokens[start:start + rows]
+        written = ~np.all(got[tokens] == 0xD4D0, axis=-1)
+        assert np.all(written == (i not in out)), f"tile {i} of expert {expert}: {written.sum()} of {rows} rows written"
+        if i not in out and (i < 10 or 60 < i < 70):
+            for tok in tokens[[0, -1]]:
+                pc.check_pair(got[:, None], int(tok), 0, f"tile {i} token {tok}")
+
+
 def test_grouped_ffn_gpt_oss_epilogues(gpu):
     # additive biases + clamped SwiGLU at the gpt-oss shape (moe.metal:257-288), 45 groups per row
     d = f = 2880
