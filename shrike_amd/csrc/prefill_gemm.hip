@@ -936,7 +936,7 @@ __global__ __launch_bounds__(256, 2) void k_ffn_split(FfnArgs a) {
 #pragma unroll
                             for (int j = 0; j < 4; ++j) {
                                 const uint16_t bits = META == SHRIKE_META_BF16 ? f32_to_f16(bf16_to_f32(uint16_t(run_b[nt][j]))) : uint16_t(run_b[nt][j]);
-                                f.u[j] = uint32_t(bits) * 0x00010001u;
+                                f.u[j] = uint32_t(bits) * (uint32_t(j) <= in_chunk ? 0x00010001u : 0u);  // (past the last group a copy: zero times it may be no zero)
                             }
                             total[nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(sums.h, f.h, total[nt], 0, 0, 0);
                         }

@@ -403,6 +403,28 @@ def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out):
                 pc.check_pair(got[:, None], int(tok), 0, f"tile {i} token {tok}")
 
 
+@pytest.mark.parametrize("d,last", [(384, 1), (768, 7)])  # the last group of a wave's share of k, which ends inside a chunk of four
+def test_grouped_ffn_with_an_infinite_bias(gpu, d, last):
+    """An infinite bias against a sum that is not zero is an infinite gate, whatever the group's place in a wave's share of k."""
+    L = Layer(0x5EED0700 + d, d, 64, 2, 1, bits=4, meta=S.META_F16)
+    for blob in L.blobs:
+        at = L.off["gate_b"] + 2 * last
+        blob[at:at + 2].view(np.uint16)[0] = 0x7C00
+    t = 20
+    pc = PrefillCase(gpu, L, t)
+    x = pc.x.reshape(t, d)
+    x[:, 64 * last:64 * last + 64] = 0
+    for half in (0, 32):  # each half's sum needs both of its fp16 parts, of one sign
+        x[:, 64 * last + half], x[:, 64 * last + half + 1] = 0x3C00, 0x0800  # 1 and 2^-13
+    pc.hidden = gpu.dev(pc.x)
+    pc.run()
+    for tok in range(t):
+        act = pc.device_act(tok, 0)
+        want = O.moe_phase1([L.blobs[int(pc.idx[tok])]], L.oracle_offsets(), np.ascontiguousarray(x[tok]), d, 64, 4, S.META_F16, O.ACT_SILU, False)
+        assert np.isinf(f16(want[:1]))[0] and act[0] == want.reshape(-1)[0], f"token {tok}: {f16(act[:1])} vs {f16(want.reshape(-1)[:1])}"
+        assert_ffn_close(act[1:], want.reshape(-1)[1:], f"token {tok}")
+
+
 def test_grouped_ffn_gpt_oss_epilogues(gpu):
     # additive biases + clamped SwiGLU at the gpt-oss shape (moe.metal:257-288), 45 groups per row
     d = f = 2880
