@@ -444,7 +444,12 @@ int shrike_hip_group_pairs(void *stream, const uint32_t *d_indices, const void *
  * fp16(down . fp16(glu(gate . x, up . x))) for every pair of a resident expert.
  * hidden: fp16[query_count, hidden_stride_elements]. d_workspace: caller-owned, at least
  * shrike_hip_prefill_ffn_workspace_bytes(). Tiles of absent experts are skipped (their
- * partial rows are left untouched). */
+ * partial rows are left untouched).
+ * Which bits: a pair's row depends on its token, its expert and on the kernel that query_count * top_k, the handle's
+ * experts and widths and f choose, not on the rows beside it, and a call over a range of the pairs
+ * (shrike_hip_prefill_streamed_batched) gives the bytes of the call over all of them. Calls of different query_count may
+ * differ by the rounding of their fp32 sums: in a short chunk over few experts four waves each sum a quarter of k, in any
+ * other one wave sums all of it. So a prompt cut into other chunks may give other last places; the accuracy is the same. */
 size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max_row_tiles,
                                               uint32_t d, uint32_t f);
 int shrike_hip_prefill_grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_bases *pool,
@@ -488,7 +493,8 @@ int shrike_hip_prefill_streamed_batched(shrike_hip_moe *moe, void *stream, const
  * grouped kernel: h1[t, :] = half(down . half(glu(half(gate . x_t), half(up . x_t)))) and, when
  * d_scalar_gate is given, h1[t, :] = half(h1[t, :] * sigmoid(scalar_gate[t])) — ONE GATE A TOKEN,
  * fp16[query_count], as shrike_hip_shared_scalar_gate_rows writes them. The roundings are those of
- * shrike_hip_shared_expert, token by token. h1: fp16[query_count, d]. */
+ * shrike_hip_shared_expert, token by token. h1: fp16[query_count, d]. As with the grouped FFN, calls of different
+ * query_count may differ by the rounding of their fp32 sums (query_count and f_shared choose the kernel). */
 size_t shrike_hip_prefill_shared_expert_workspace_bytes(uint32_t query_count, uint32_t d,
                                                         uint32_t f_shared);
 int shrike_hip_prefill_shared_expert(shrike_hip_moe *moe, void *stream, const shrike_projection *gate,

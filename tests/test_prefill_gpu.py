@@ -403,6 +403,30 @@ def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out):
                 pc.check_pair(got[:, None], int(tok), 0, f"tile {i} token {tok}")
 
 
+@pytest.mark.parametrize("d,f,ne,bits,chunks,split", [
+    (512, 4096, 12, 4, (90, 400, 2900), ()),     # one and two row tiles a workgroup
+    (512, 1024, 40, 8, (150, 1000, 2000), ()),   # 8-bit codes: two groups ahead, one, two row tiles
+    (512, 512, 12, 4, (13, 40), (13, 40)),       # k over the waves
+    (512, 2048, 12, 4, (40, 400), (40,))])       # ... in the shorter chunk
+def test_a_row_of_the_ffn_over_chunks_of_different_lengths(gpu, d, f, ne, bits, chunks, split):
+    """The same bytes where in both chunks one wave sums all of k, or four waves a quarter each; else the end-to-end bound (the
+    sums' rounding moves fp16 activations by their last place)."""
+    first = min(chunks)
+    L = Layer(0x5EED0800, d, f, ne, 1, bits=bits, meta=S.META_BF16)
+    x = token_rows(L, max(chunks), d)
+    idx = np.random.default_rng(11).integers(0, ne, max(chunks)).astype(np.uint32)
+    rows = {}
+    for t in chunks:
+        pc = PrefillCase(gpu, L, t, idx=idx[:t])
+        pc.hidden = gpu.dev(x[:t * d])
+        rows[t] = pc.run()[:first, 0]
+    for t in chunks:
+        if (t in split) == (first in split):
+            assert np.array_equal(rows[t], rows[first]), f"{t} tokens against {first}"
+        else:
+            assert_rel_close(rows[t].reshape(-1), rows[first].reshape(-1), f"{t} tokens against {first}")
+
+
 @pytest.mark.parametrize("d,last", [(384, 1), (768, 7)])  # the last group of a wave's share of k, which ends inside a chunk of four
 def test_grouped_ffn_with_an_infinite_bias(gpu, d, last):
     """An infinite bias against a sum that is not zero is an infinite gate, whatever the group's place in a wave's share of k."""
