@@ -552,7 +552,8 @@ int shrike_prefetch_ring_leased_count(shrike_prefetch_ring *ring);
  * out[r] = sum_i (q[r][i] * scale[r][g(i)] + bias[r][g(i)]) * x[i] over a rows-by-n matrix of 4-bit codes, low nibble
  * first, one bf16 scale and one bf16 bias per group of 64; n a multiple of 64; out is written, not accumulated. The sum
  * is factored per group as scale * sum(q x) + bias * sum(x) and its additions run in the order of the reference's
- * portable branch (:114-134), whose bits the results are. Host memory only; thread-safe. */
+ * portable branch (:114-134), whose bits the results are. Host memory only; thread-safe. A thread that calls this or the
+ * next function keeps up to 128 KB of the library's working memory until it ends (it needs little of its stack). */
 void shrike_int4_affine_gemv(const uint8_t *weights, const uint16_t *scales, const uint16_t *biases, const float *x,
                              size_t rows, size_t n, float *out);
 /* CPUExpertFFN.accumulate, sources/Shrike/Kernels/CPU/CPUExpertFFN.swift:102-140 (called at :82-90 by the CPU expert

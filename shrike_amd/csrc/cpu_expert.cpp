@@ -22,7 +22,6 @@
 namespace {
 
 constexpr size_t kGroupElems = SHRIKE_GROUP_SIZE, kGroupBytes = kGroupElems / 2;
-constexpr size_t kFewRows = 4;  // fewer go one by one: a block costs what sixteen rows cost
 
 struct NibblePair {
     float lo, hi;
@@ -195,7 +194,6 @@ SHRIKE_AVX512 void gemv_block(const uint8_t *weights, const uint16_t *scales, co
     for (int k = 0; k < BLOCKS; ++k) _mm512_mask_storeu_ps(out + row0 + kLanes * size_t(k), live[k], acc[k]);
 }
 
-// `table`: room for the products of min(groups, kStretchGroups) groups
 SHRIKE_AVX512 void gemv_rows_avx512(const uint8_t *weights, const uint16_t *scales, const uint16_t *biases, const float *x,
                                     const float *xsum, size_t rows, size_t groups, float *table, float *out) {
     const __m512 codes = _mm512_setr_ps(0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
@@ -214,42 +212,38 @@ SHRIKE_AVX512 void gemv_rows_avx512(const uint8_t *weights, const uint16_t *scal
     }
 }
 
-// The table of products, allocated once a call of an entry point: 128 KB are more than a small stack of a caller's thread may
-// hold. None where a call has no rows for it, the processor no AVX-512 or the system no memory: the rows then go one by one.
-class ProductTable {
-public:
-    ProductTable(size_t rows, size_t groups) {
-        if (rows < kFewRows || groups == 0 || !has_avx512()) return;
-        floats_ = static_cast<float *>(std::aligned_alloc(64, (groups < kStretchGroups ? groups : kStretchGroups) * kGroupElems * kLanes * sizeof(float)));
-    }
-    ~ProductTable() { std::free(floats_); }
-    ProductTable(const ProductTable &) = delete;
-    ProductTable &operator=(const ProductTable &) = delete;
-    float *floats() const { return floats_; }
+bool has_avx512() {
+    static const bool has = __builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512bw") && __builtin_cpu_supports("avx512vl");
+    return has;
+}
 
-private:
-    static bool has_avx512() {
-        static const bool has = __builtin_cpu_supports("avx512f") && __builtin_cpu_supports("avx512bw") && __builtin_cpu_supports("avx512vl");
-        return has;
-    }
-    float *floats_ = nullptr;
-};
+// The calling thread's table of products, from its first call to its end: 128 KB are more than a small stack of a caller's
+// thread may hold, and allocated anew for every expert they may come as new pages each time. On a page boundary: eight experts
+// from memory took 846 us, from the stack 861, from a table 64 bytes off one 879. Null where the processor has no AVX-512 or the
+// system no memory: the rows then go one by one, to the same bits.
+float *product_table() {
+    struct Table {
+        float *floats = nullptr;
+        ~Table() { std::free(floats); }
+    };
+    thread_local Table table;
+    if (!table.floats && has_avx512())
+        table.floats = static_cast<float *>(std::aligned_alloc(4096, kStretchGroups * kGroupElems * kLanes * sizeof(float)));
+    return table.floats;
+}
 
 #else
 
-class ProductTable {
-public:
-    ProductTable(size_t, size_t) {}
-    float *floats() const { return nullptr; }
-};
+float *product_table() { return nullptr; }
 void gemv_rows_avx512(const uint8_t *, const uint16_t *, const uint16_t *, const float *, const float *, size_t, size_t, float *, float *) {}
 
 #endif
 
-// `table`: null, or one that holds min(groups, kStretchGroups) groups
 void gemv_rows(const uint8_t *weights, const uint16_t *scales, const uint16_t *biases, const float *x, const float *xsum,
-               size_t rows, size_t groups, float *table, float *out) {
-    if (rows >= kFewRows && groups > 0 && table) gemv_rows_avx512(weights, scales, biases, x, xsum, rows, groups, table, out);
+               size_t rows, size_t groups, float *out) {
+    // (a block costs what sixteen rows cost: a handful of rows is better off alone)
+    float *table = rows >= 4 && groups > 0 ? product_table() : nullptr;
+    if (table) gemv_rows_avx512(weights, scales, biases, x, xsum, rows, groups, table, out);
     else gemv_rows_scalar(weights, scales, biases, x, xsum, rows, groups, out);
 }
 
@@ -270,8 +264,7 @@ void shrike_int4_affine_gemv(const uint8_t *weights, const uint16_t *scales, con
         xsum = heap_sums.data();
     }
     group_sums_of(x, groups, xsum);
-    const ProductTable table(rows, groups);
-    gemv_rows(weights, scales, biases, x, xsum, rows, groups, table.floats(), out);
+    gemv_rows(weights, scales, biases, x, xsum, rows, groups, out);
 }
 
 size_t shrike_cpu_expert_ffn_scratch_floats(uint32_t d, uint32_t f) { return 2 * size_t(f) + size_t(d); }
@@ -287,13 +280,12 @@ int shrike_cpu_expert_ffn_accumulate(const void *expert, const shrike_expert_off
     // gate and up share x, and with it x's group sums (kept in the down rows' place until they are needed)
     float *xsum = down;
     group_sums_of(x, d / kGroupElems, xsum);
-    const ProductTable table(d > f ? d : f, (d > f ? d : f) / kGroupElems);
-    gemv_rows(base + offsets->gate_w_off, meta(offsets->gate_s_off), meta(offsets->gate_b_off), x, xsum, f, d / kGroupElems, table.floats(), gate);
-    gemv_rows(base + offsets->up_w_off, meta(offsets->up_s_off), meta(offsets->up_b_off), x, xsum, f, d / kGroupElems, table.floats(), up);
+    gemv_rows(base + offsets->gate_w_off, meta(offsets->gate_s_off), meta(offsets->gate_b_off), x, xsum, f, d / kGroupElems, gate);
+    gemv_rows(base + offsets->up_w_off, meta(offsets->up_s_off), meta(offsets->up_b_off), x, xsum, f, d / kGroupElems, up);
     for (uint32_t i = 0; i < f; ++i) gate[i] = silu(gate[i]) * up[i];
     // the activations' group sums go where `up` was
     group_sums_of(gate, f / kGroupElems, up);
-    gemv_rows(base + offsets->down_w_off, meta(offsets->down_s_off), meta(offsets->down_b_off), gate, up, d, f / kGroupElems, table.floats(), down);
+    gemv_rows(base + offsets->down_w_off, meta(offsets->down_s_off), meta(offsets->down_b_off), gate, up, d, f / kGroupElems, down);
     for (uint32_t r = 0; r < d; ++r) out[r] += route_weight * down[r];
     return 0;
 }
