@@ -146,10 +146,12 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // Everything the loop reads comes through LDS by asynchronous loads, a group of 64 k at a time: the rows (shared by the
 // waves), and each wave's own codes and scales. Loaded by the lanes themselves the codes cost the loop most of its time: a
 // lane's sixteen bytes lay a weight row from its neighbour's, 64 lines a load, and the registers that held them left one
-// workgroup a compute unit fewer. What bounds it now: with many rows the power the matrix cores draw (the clock falls to 1.3
-// to 1.75 GHz, and vector work saved in the loop buys nothing), with few of them the weights' bytes, with few workgroups a
-// wave's own chain of some 1,700 cycles a group (1,200 up to 32 rows). 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens: 843
-// -> 576 us (WIDE 541); 256 of 2,048 x 512, 4,096 tokens: 371 -> 337; 256 of 2,304 x 1,024, 8-bit, 4,000 tokens: 926 -> 758.
+// workgroup a compute unit fewer. What bounds it now: with many rows the two waves of a SIMD, whose matrix and vector work
+// overlap little (the WIDE gate/up launch over 2,048 gpt-oss tokens keeps the matrix pipe busy 38 % of the cycles and vector
+// issue, without the matrix instructions' own, another 37 %, at a clock of 2.1 to 2.2 GHz of 2.4); with few rows the weights'
+// bytes; with few workgroups a wave's own chain of some 1,700 cycles a group (1,200 up to 32 rows). 32 experts of 2,880 x
+// 2,880, 4-bit, 2,048 tokens: 843 -> 576 us (WIDE 541); 256 of 2,048 x 512, 4,096 tokens: 371 -> 337; 256 of 2,304 x 1,024,
+// 8-bit, 4,000 tokens: 926 -> 758.
 //
 // MODE 0 leaves its activations through LDS: whole 16-byte pieces of a row go out together, and the group sums of the
 // tile's rows that the down product's bias term needs are formed here, in k_row_group_sums' order of additions (eight
@@ -248,7 +250,6 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     const uint32_t s_mine = kb ? s_at[1] : s_at[0], s_mine_last = kb ? s_last[1] : s_last[0];
     const uint32_t lds_s = lds0 + L::kS + wave * kUnitS;
     auto load_s = [&](uint32_t c) { lds_load12(lds_s, s_src + min((s_mine & ~3u) + 8u * c, s_mine_last)); };
-    const uint32_t chunks = (G + 3u) / 4u;
 
     const uint16_t *bias_row[2] = {b_base[0] + size_t(s_row[0]) * G, b_base[1] + size_t(s_row[1]) * G};
     auto eight_at = [&](const uint16_t *row, uint32_t at) {  // groups min(at, G - 8) ...
@@ -256,8 +257,6 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         return make_uint4(v.x, v.y, v.z, v.w);
     };
     // what the first group needs is on its way before anything else
-    constexpr uint32_t kGroupsPerB = BITS == 4 ? 2u : 1u;
-    const uint32_t stages = (G + kGroupsPerB - 1u) / kGroupsPerB;
     load_s(0);
     load_b(0, 0);
     load_a(0, 0);
@@ -753,7 +752,7 @@ __global__ __launch_bounds__(256, 2) void k_ffn_split(FfnArgs a) {
     const uint32_t stages = (G + kGroupsPerB - 1u) / kGroupsPerB, row_bytes = K * BITS / 8u;
     // the wave's quarter of the stages
     const uint32_t st_lo = stages * wave / 4u, st_hi = stages * (wave + 1u) / 4u;
-    const uint32_t g_lo = st_lo * kGroupsPerB, g_hi = min(st_hi * kGroupsPerB, G), groups = g_hi - g_lo, my_stages = st_hi - st_lo;
+    const uint32_t g_lo = st_lo * kGroupsPerB, g_hi = min(st_hi * kGroupsPerB, G), groups = g_hi - g_lo;
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds)) + wave * L::kWave;
     const uint8_t *my_lds = lds + wave * L::kWave;
     // An XCD takes a contiguous eighth of the (tile, column block) pairs, its workgroups one after the other: tiles of an
@@ -841,7 +840,6 @@ __global__ __launch_bounds__(256, 2) void k_ffn_split(FfnArgs a) {
                 for (uint32_t i = 0; i < 4u; ++i) v[nt][i] = *reinterpret_cast<const uint16_t *>(p + min(i, groups - 1u - i0) * 2u);
             }
         };
-        const uint32_t chunks = (groups + 3u) / 4u;
 
         for (uint32_t skip = 0; skip < tile.rows; skip += 32u) {  // (dense: once)
             const uint32_t rows = min(32u, tile.rows - skip), first = tile.pair_start + skip;
