@@ -26,28 +26,28 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// ---- the shape of a workgroup's work and its LDS: places for two groups (of the codes: stages) of the operands, the one in
-// use and the one on its way (kAhead: for three), that asynchronous loads fill (lane l's piece of a load lands 16 l bytes behind the load's
-// address), and after the last product the rows on their way out.
+// ---- the shape of a workgroup's work and its LDS: a ring of places for groups of the rows and one for 64-byte units of the
+// codes, that asynchronous loads fill (lane l's piece of a load lands 16 l bytes behind the load's address).
 enum class FfnShape {
     kSplit,  // up to 32 rows against 64 weight rows, a quarter of k a wave (k_ffn_split)
-    kTile,   // one row tile, up to 64 rows, against 256 weight rows; three workgroups a compute unit
+    kTile,   // one row tile, up to 64 rows, against 256 weight rows, 4-bit codes; three workgroups a compute unit
+    kDeep,   // the same with more groups on their way; two workgroups a compute unit
     kWide,   // two row tiles of one expert, up to 128 rows, against 256 weight rows; two workgroups a compute unit
-    kAhead,  // as kTile, 8-bit codes, with the operands of two groups on their way; two workgroups a compute unit
 };
 constexpr uint32_t kUnitB = 64u * 64u;  // 64 bytes of codes of a wave's 64 weight rows: two groups at 4 bits, one at 8
 constexpr uint32_t kUnitS = 64u * 16u;  // four groups' scales (biases) of those rows, in a 12-byte window each
-template <FfnShape S>
+template <FfnShape S, int BITS>
 struct Lds {
     static constexpr bool kIsWide = S == FfnShape::kWide;
-    static constexpr uint32_t kPlaces = S == FfnShape::kAhead ? 3u : 2u;
+    static constexpr uint32_t kPlacesA = S != FfnShape::kDeep ? 2u : BITS == 4 ? 4u : 3u;  // of groups of rows
+    static constexpr uint32_t kPlacesB = S != FfnShape::kDeep || BITS == 4 ? 2u : 3u;      // of units of codes
     static constexpr uint32_t kRows = kIsWide ? 128u : 64u;
     static constexpr uint32_t kUnitA = kRows * 128u;  // one group (64 k) of the rows
-    static constexpr uint32_t kB = kPlaces * kUnitA, kS = kB + kPlaces * 4u * kUnitB, kBytes = kS + 4u * kUnitS;
-    // a unit (32 groups) of the rows' group sums, two of them, where the rows and the codes of the last place will be
-    static constexpr uint32_t kSums0 = kB - kUnitA, kSums1 = kS - 4u * kUnitB;
+    static constexpr uint32_t kB = kPlacesA * kUnitA, kS = kB + kPlacesB * 4u * kUnitB, kDst = kS + 4u * kUnitS, kBytes = kDst + kRows * 8u;
+    // two units (32 groups each) of the rows' group sums: where the rows and, this one, the codes of the last place will be
+    static constexpr uint32_t kSums1 = kS - 4u * kUnitB;
     static_assert(kUnitA <= 4u * kUnitB, "a unit of sums fits");
-    static constexpr uint32_t kRow = 256u + 8u;  // halves per row on the way out; the pad spreads the banks
+    static constexpr uint32_t kRow = 128u + 8u;  // halves per row of activations on the way out; the pad spreads the banks
     static constexpr uint32_t kResident = S == FfnShape::kTile ? 3u : 2u;  // workgroups a compute unit holds
     static_assert(kRows * kRow * 2u <= kBytes && kBytes * kResident <= 160u * 1024u, "the rows on the way out fit, and the workgroups a compute unit");
 };
@@ -82,6 +82,7 @@ struct FfnArgs {
     uint32_t dense_rows;
     uint32_t round_gate_up;        // gate and up pass through fp16 before the GLU (dequant_int4.metal:206-287)
     const uint16_t *scalar_gate;   // fp16[rows] or null: row m's output * sigmoid(gate[m]) (moe.metal:1195-1207)
+    uint32_t max_tiles;            // records that the tile table has room for
     uint32_t resident_workgroups;  // workgroups of the launched k_grouped_ffn the device holds at once
 };
 
@@ -144,14 +145,20 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // biases (SHRIKE_META_*), both template parameters, so that the main loop is straight-line code.
 //
 // Everything the loop reads comes through LDS by asynchronous loads, a group of 64 k at a time: the rows (shared by the
-// waves), and each wave's own codes and scales. Loaded by the lanes themselves the codes cost the loop most of its time: a
-// lane's sixteen bytes lay a weight row from its neighbour's, 64 lines a load, and the registers that held them left one
-// workgroup a compute unit fewer. What bounds it now: with many rows the two waves of a SIMD, whose matrix and vector work
-// overlap little (the WIDE gate/up launch over 2,048 gpt-oss tokens keeps the matrix pipe busy 38 % of the cycles and vector
-// issue, without the matrix instructions' own, another 37 %, at a clock of 2.1 to 2.2 GHz of 2.4); with few rows the weights'
-// bytes; with few workgroups a wave's own chain of some 1,700 cycles a group (1,200 up to 32 rows). 32 experts of 2,880 x
-// 2,880, 4-bit, 2,048 tokens: 843 -> 576 us (WIDE 541); 256 of 2,048 x 512, 4,096 tokens: 371 -> 337; 256 of 2,304 x 1,024,
-// 8-bit, 4,000 tokens: 926 -> 758.
+// waves), and each wave's own codes and scales. (Loaded by the lanes themselves, a lane's sixteen bytes lie a weight row from
+// its neighbour's, 64 lines a load.)
+//
+// A wave's matrix and vector work run beside each other only where neighbouring instructions do not wait for each other. A
+// chain of four MFMAs from zero and the scaling of its own sums behind it take 173 cycles a chain with two waves a SIMD, the
+// scaling of the chain before between the MFMAs 145, and 131 is the matrix pipe alone; with one wave 238 against 158. So the
+// loop is a pipeline: between the MFMAs of chain c stand the scaling of chain c - 1, a share of the next codes' unpacking and
+// the reads of the rows that the next chain takes, and the wait for the next group's loads stands two chains ahead of their
+// use. What bounds it now: with many rows the power that matrix work, its operands' way through LDS and the loads take
+// together (the kWide gate/up launch over 2,048 gpt-oss tokens runs at 2.0 GHz of 2.4, the matrix pipe busy 42 % of the
+// cycles); with few rows the weights' bytes (kDeep, 8-bit, 1,000 tokens: 4.4 TB/s), and the start and the end of the many
+// short workgroups (30 of 75 us at 256 experts of 2,048 x 512 and 512 tokens). Both products, a chain scaled where it ends ->
+// pipelined: 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens 540 -> 495 us, 300 tokens 179 -> 164; 256 of 2,048 x 512, 4,096
+// tokens 316 -> 302, 37 33.5 -> 31.4; 256 of 2,304 x 1,024, 8-bit, 1,000 tokens 469 -> 439, 4,000 735 -> 710.
 //
 // MODE 0 leaves its activations through LDS: whole 16-byte pieces of a row go out together, and the group sums of the
 // tile's rows that the down product's bias term needs are formed here, in k_row_group_sums' order of additions (eight
@@ -160,7 +167,11 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 template <int BITS, int MODE, bool DENSE, uint32_t MT, int META, FfnShape S>
 __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile &tile, uint32_t act_row, uint32_t col_block,
                                          uint8_t *lds) {
-    typedef Lds<S> L;
+    typedef Lds<S, BITS> L;
+    // (kTile's places for up to 64 rows are twice as many for up to 32)
+    constexpr bool kHalves = S == FfnShape::kTile && MT == 1u;
+    constexpr uint32_t kA = L::kPlacesA * (kHalves ? 2u : 1u), kB = L::kPlacesB, kUnitA = L::kUnitA / (kHalves ? 2u : 1u);
+    constexpr uint32_t kSums0 = L::kB - kUnitA;
     const uint32_t K = MODE == 0 ? a.d : a.f, N = MODE == 0 ? a.f : a.d;
     const uint32_t G = K / kGroup;
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
@@ -173,7 +184,10 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     // ---- A: the tile's rows, a group of them (128 bytes a row) at a time. A load brings eight rows, eight lanes a row, its
     // sixteen-byte pieces xor-ed with the row so that eight rows read at one piece touch every bank once.
     constexpr uint32_t kLoadsA = MT;  // a wave's loads a group
+    constexpr bool kNear = S != FfnShape::kDeep;  // a row is a 32-bit offset from a base (the launch's rule)
     const uint8_t *a_src[kLoadsA];
+    uint32_t a_off[kLoadsA];
+    const uint8_t *a_base = MODE == 0 ? reinterpret_cast<const uint8_t *>(a.hidden) : reinterpret_cast<const uint8_t *>(a.act + size_t(act_row) * a.f);
     const uint32_t *a_sums[kLoadsA];  // the rows' group sums, for the bias term
 #pragma unroll
     for (uint32_t j = 0; j < kLoadsA; ++j) {
@@ -188,10 +202,14 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             a_sums[j] = a.act_sums + (size_t(act_row) + r) * G;
         }
         a_src[j] = reinterpret_cast<const uint8_t *>(row) + (((lane & 7u) ^ (lane >> 3)) * 16u);
+        if (kNear) a_off[j] = uint32_t(a_src[j] - a_base);
     }
     auto load_a = [&](uint32_t slot, uint32_t g) {
 #pragma unroll
-        for (uint32_t j = 0; j < kLoadsA; ++j) lds_load16(lds0 + slot * L::kUnitA + (wave + 4u * j) * 1024u, a_src[j] + size_t(g) * 128u);
+        for (uint32_t j = 0; j < kLoadsA; ++j) {
+            if (kNear) lds_load16(lds0 + slot * kUnitA + (wave + 4u * j) * 1024u, a_base + size_t(g) * 128u, a_off[j]);
+            else lds_load16(lds0 + slot * kUnitA + (wave + 4u * j) * 1024u, a_src[j] + size_t(g) * 128u);
+        }
     };
 
     // ---- B: a wave's own 64 weight rows (two tiles of 32), 64 bytes of each at a time
@@ -199,10 +217,10 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     const uint32_t row_bytes = K * BITS / 8u;
     const uint8_t *w_base[2], *s_base[2];
     const uint16_t *b_base[2];
-    uint32_t n_first[2];  // the tiles' first rows
+    // row c of tile nt: MODE 0 the same of gate and up, MODE 1 every second, so that a lane's two sums of a row are neighbours
+    auto row_of = [&](uint32_t nt, uint32_t c) -> uint32_t { return min(MODE == 0 ? n0 + c : n0 + 2u * c + nt, N - 1u); };
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
-        n_first[nt] = n0 + (MODE == 0 ? 0u : 32u * uint32_t(nt));
         if (DENSE) {
             const int p = MODE == 0 ? nt : 2;
             w_base[nt] = a.dense_w[p];
@@ -222,13 +240,14 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     uint32_t b_off[4];
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-        b_off[j] = min(n_first[j >> 1] + 16u * (j & 1u) + (lane >> 2), N - 1u) * row_bytes + ((lane & 3u) ^ ((lane >> 3) & 3u)) * 16u;
+        b_off[j] = row_of(j >> 1, 16u * (j & 1u) + (lane >> 2)) * row_bytes + ((lane & 3u) ^ ((lane >> 3) & 3u)) * 16u;
     // (at 4 bits a row of an odd number of groups ends halfway through its last stage: the lanes of the missing half take
     // the other half's pieces, so that nothing past a tensor's last row is read)
     const uint32_t half_back = (((lane & 3u) ^ ((lane >> 3) & 3u)) & 2u) * 16u;
+    constexpr uint32_t kGroupsPerB = BITS == 4 ? 2u : 1u;
     const uint32_t lds_b = lds0 + L::kB + wave * kUnitB;
-    auto load_b = [&](uint32_t slot, uint32_t stage) {
-        const uint32_t back = BITS == 4 && 2u * stage + 1u >= G ? half_back : 0u;
+    auto load_b = [&](uint32_t slot, uint32_t stage, bool may_end = true) {
+        const uint32_t back = BITS == 4 && may_end && 2u * stage + 1u >= G ? half_back : 0u;
 #pragma unroll
         for (uint32_t j = 0; j < 4u; ++j) lds_load16(lds_b + slot * (4u * kUnitB) + j * 1024u, w_base[j >> 1] + size_t(stage) * 64u, b_off[j] - back);
     };
@@ -237,7 +256,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     // is loaded is the window of three words that holds it, never past the word of the tensor's last scale. `s_at` is where a
     // row's chunk starts, from the word that holds the tensor's start; the run then starts max(s_at & 3, s_at - last window)
     // bytes into the window.
-    const uint32_t s_row[2] = {min(n_first[0] + col, N - 1u), min(n_first[1] + col, N - 1u)};
+    const uint32_t s_row[2] = {row_of(0, col), row_of(1, col)};
     uint32_t s_at[2], s_last[2];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
@@ -256,16 +275,31 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         const u32x4_by2 v = *reinterpret_cast<const u32x4_by2 *>(row + min(at, G - 8u));
         return make_uint4(v.x, v.y, v.z, v.w);
     };
+    // MODE 1: where the rows go, in bytes from `partials` (all ones: nowhere)
+    uint64_t *s_dst = reinterpret_cast<uint64_t *>(lds + L::kDst);
+    uint64_t dst = ~0ull;
+    if (MODE == 1 && threadIdx.x < MT * 32u && threadIdx.x < tile.rows) {
+        const uint32_t pair = tile.pair_start + threadIdx.x;
+        if (DENSE) {
+            dst = uint64_t(pair) * a.d * 2u;
+        } else if (pair >= a.pair_lo && pair < a.pair_hi) {  // a call over a range of the sorted pairs writes their rows only
+            const shrike_token_expert_pair p = a.pairs[pair];
+            dst = (uint64_t(p.token) * a.top_k + p.rank) * a.d * 2u;
+        }
+    }
     // what the first group needs is on its way before anything else
     load_s(0);
     load_b(0, 0);
     load_a(0, 0);
-    if constexpr (S == FfnShape::kAhead) {
-        if (G > 1u) {
-            load_b(1, 1);
-            load_a(1, 1);
-        }
-    }
+    // (what the first group needs first, then of the rest what fits beside the sums below)
+#pragma unroll
+    for (uint32_t i = 1; i + 1u < kB; ++i)
+        if (i * kGroupsPerB < G) load_b(i, i);
+#pragma unroll
+    for (uint32_t i = 1; i + 1u < kA; ++i)
+        if (i < G) load_a(i, i);
+
+    if (MODE == 1 && threadIdx.x < MT * 32u) s_dst[threadIdx.x] = dst;
 
     f32x16 total[2][MT];
 #pragma unroll
@@ -292,7 +326,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
                 const uint32_t at = min(g0 + 32u * u + 16u * (q >> 2) + 8u * ((q >> 1) & 1u), G - 8u) + 4u * (q & 1u);
 #pragma unroll
                 for (uint32_t j = 0; j < kLoadsA; ++j)
-                    lds_load16(lds0 + (u ? L::kSums1 : L::kSums0) + (wave + 4u * j) * 1024u, a_sums[j] + at);
+                    lds_load16(lds0 + (u ? L::kSums1 : kSums0) + (wave + 4u * j) * 1024u, a_sums[j] + at);
             }
             uint4 b8[2][2][2];  // [unit][load][nt]
             if (active) {
@@ -316,7 +350,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
                     const uint32_t at = g0 + 32u * u + 16u * i + 8u * kb, repeated = at - min(at, G - 8u);
 #pragma unroll
                     for (uint32_t h = 0; h < 2u; ++h) {
-                        const uint8_t *p = lds + (u ? L::kSums1 : L::kSums0) + col * 128u + (((4u * i + 2u * kb + h) ^ (col & 7u)) * 16u);
+                        const uint8_t *p = lds + (u ? L::kSums1 : kSums0) + col * 128u + (((4u * i + 2u * kb + h) ^ (col & 7u)) * 16u);
                         half8 sums[MT];
 #pragma unroll
                         for (uint32_t mt = 0; mt < MT; ++mt) sums[mt] = *reinterpret_cast<const half8 *>(p + mt * 4096u);
@@ -357,99 +391,176 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         }
     }
 
-    // ---- the groups. Step g waits for what its group needs (the first also until nobody reads the sums any more) and asks for
-    // what a later group will, in the place that group g - 1 left.
-    uint32_t run[2][4];  // the scales of a chunk of four groups
-    uint32_t place = 0;  // kAhead: g % 3
-    if constexpr (S == FfnShape::kAhead) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) in the compiler's own count: else it waits for the biases in the loop
-    auto step = [&](uint32_t g, auto par) {
-        constexpr uint32_t P = decltype(par)::value;  // g & 1
-        const uint32_t a_place = S == FfnShape::kAhead ? place : P;
-        const uint32_t b_place = S == FfnShape::kAhead ? place : BITS == 8 ? P : (g >> 1) & 1u;
-        if constexpr (S == FfnShape::kAhead) {
-            if (g + 1u < G) wait_loads_and_sync<kLoadsA + 4>();  // (the next group's may still be on their way)
-            else wait_loads_and_sync<0>();
-            const uint32_t left = place == 0u ? 2u : place - 1u;
-            if (g + 2u < G) {
-                load_b(left, g + 2u);
-                load_a(left, g + 2u);
-            }
-            place = place == 2u ? 0u : place + 1u;
-        } else {
-            if (BITS == 4 && P == 1u && g + 1u < G) wait_loads_and_sync<4>();  // (the next stage's codes may still be on their way)
-            else wait_loads_and_sync<0>();
-            if (g + 1u < G) {
-                load_a(P ^ 1u, g + 1u);
-                if (BITS == 8) load_b(b_place ^ 1u, g + 1u);
-            }
-            if (BITS == 4 && P == 0u && g + 2u < G) load_b(b_place ^ 1u, (g >> 1) + 1u);
-        }
-        if (active) {
-            if ((g & 3u) == 0u) {
+    // ---- the groups: 2 MT chains each, (row tile, weight tile) = (0, 0), (0, 1), (1, 0), ... The fences between the slots
+    // keep the order as it is written.
+    wait_loads_and_sync<0>();  // (nobody reads the sums any more)
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) in the compiler's own count: else it waits for the biases in the loop
+    if (kA != 2u && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
+    if (kA - 1u < G) load_a(kA - 1u, kA - 1u);
+    if (kA == 2u && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
+    uint32_t run[2][2];  // the scales of a chunk of four groups, two a word
+    float sc[2], sc_before = 0.0f;
+    constexpr bool kTwoA = MT <= (S == FfnShape::kTile ? 1u : 2u);  // two sets of a row tile's operands: the next is read a chain earlier
+    half8 af[kTwoA ? 2 : 1][4], bf[2][4];
+    uint4 raw[kTwoA ? 2 : 1][BITS / 4];
+    constexpr bool kBehind = !(S == FfnShape::kTile && MT == 2u);  // (else a chain is scaled where it ends: a third workgroup's waves run beside it)
+    f32x16 p[2];
+    float tot[2][MT][16];  // (single registers: eight tuples of sixteen beside p do not fit round each other, and two were spilled)
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    const int into = max(int(s_at[nt] & 3u), int(s_at[nt] + g * 2u) - int(s_last[nt]));
-                    const uint8_t *p = lds + L::kS + wave * kUnitS + (uint32_t(nt) * 32u + col) * 16u + uint32_t(into);
+    for (int i = 0; i < 16; ++i) {
+        p[1][i] = 0.0f;
 #pragma unroll
-                    for (uint32_t i = 0; i < 4u; ++i) run[nt][i] = *reinterpret_cast<const uint16_t *>(p + min(i, G - 1u - g) * 2u);
-                }
-            }
-        }
-        if ((g & 3u) == 1u && g + 3u < G) load_s((g >> 2) + 1u);  // (a step's wait is for the reads above, too)
-        if (active) {
-            const uint8_t *a_rows = lds + a_place * L::kUnitA + col * 128u;
-            uint4 codes[2][BITS / 4];
-            float sc[2];
+        for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                const uint8_t *rows = lds + L::kB + wave * kUnitB + b_place * (4u * kUnitB) + uint32_t(nt) * 2048u + col * 64u;
+            for (uint32_t mt = 0; mt < MT; ++mt) tot[nt][mt][i] = total[nt][mt][i];
+    }
+    auto read_run = [&](uint32_t g) {  // of the chunk that starts at g
 #pragma unroll
-                for (uint32_t i = 0; i < BITS / 4; ++i) {
-                    const uint32_t piece = BITS == 4 ? P * 2u + kb : kb * 2u + i;
-                    codes[nt][i] = *reinterpret_cast<const uint4 *>(rows + ((piece ^ ((col >> 1) & 3u)) * 16u));
-                }
-                sc[nt] = meta_f32(uint16_t(run[nt][0]), uint32_t(META));
-                run[nt][0] = run[nt][1]; run[nt][1] = run[nt][2]; run[nt][2] = run[nt][3];
-            }
-            auto a_frag = [&](uint32_t mt, uint32_t s) { return *reinterpret_cast<const half8 *>(a_rows + mt * 4096u + (((kb * 4u + s) ^ (col & 7u)) * 16u)); };
-            {
-                half8 bf[2][4];
+        for (int nt = 0; nt < 2; ++nt) {
+            const int into = max(int(s_at[nt] & 3u), int(s_at[nt] + g * 2u) - int(s_last[nt]));
+            const uint8_t *q = lds + L::kS + wave * kUnitS + (uint32_t(nt) * 32u + col) * 16u + uint32_t(into);
+            typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-                for (int nt = 0; nt < 2; ++nt) {
-                    if (BITS == 4) {
-                        const uint4 c = codes[nt][0];
-                        bf[nt][0] = codes4(c.x); bf[nt][1] = codes4(c.y); bf[nt][2] = codes4(c.z); bf[nt][3] = codes4(c.w);
-                    } else {
-                        const uint4 lo = codes[nt][0], hi = codes[nt][BITS / 4 - 1];
-                        bf[nt][0] = codes8(lo.x, lo.y); bf[nt][1] = codes8(lo.z, lo.w);
-                        bf[nt][2] = codes8(hi.x, hi.y); bf[nt][3] = codes8(hi.z, hi.w);
-                    }
-                    sc[nt] *= kTwo24;
-                }
-#pragma unroll
-                for (uint32_t mt = 0; mt < MT; ++mt) {
-                    half8 af[4];
-#pragma unroll
-                    for (uint32_t s = 0; s < 4; ++s) af[s] = a_frag(mt, s);
-#pragma unroll
-                    for (int nt = 0; nt < 2; ++nt) {
-                        f32x16 p = {0};
-#pragma unroll
-                        for (int s = 0; s < 4; ++s) p = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[s], bf[nt][s], p, 0, 0, 0);
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) total[nt][mt][i] = fmaf(sc[nt], p[i], total[nt][mt][i]);
-                    }
-                }
+            for (uint32_t i = 0; i < 2u; ++i) {
+                u16x2 v;
+                v.x = *reinterpret_cast<const uint16_t *>(q + min(2u * i, G - 1u - g) * 2u);
+                v.y = *reinterpret_cast<const uint16_t *>(q + min(2u * i + 1u, G - 1u - g) * 2u);
+                __builtin_memcpy(&run[nt][i], &v, 4);
             }
         }
     };
-    for (uint32_t g = 0; g + 1u < G; g += 2u) {
-        step(g, std::integral_constant<uint32_t, 0>{});
-        step(g + 1u, std::integral_constant<uint32_t, 1>{});
+    auto next_scales = [&](auto odd) {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+            sc[nt] = meta_f32(uint16_t(run[nt][0] >> (decltype(odd)::value ? 16 : 0)), uint32_t(META)) * kTwo24;
+            if (decltype(odd)::value) run[nt][0] = run[nt][1];
+        }
+    };
+    const uint8_t *a_rows = lds + col * 128u, *b_rows = lds + L::kB + wave * kUnitB + col * 64u;
+    auto read_a = [&](uint32_t place, uint32_t mt, uint32_t s) {
+        return *reinterpret_cast<const half8 *>(a_rows + place * kUnitA + mt * 4096u + (((kb * 4u + s) ^ (col & 7u)) * 16u));
+    };
+    auto read_raw = [&](uint32_t nt, uint32_t b_place, uint32_t par) {
+#pragma unroll
+        for (uint32_t i = 0; i < BITS / 4; ++i) {
+            const uint32_t piece = BITS == 4 ? par * 2u + kb : kb * 2u + i;
+            raw[kTwoA ? nt : 0u][i] = *reinterpret_cast<const uint4 *>(b_rows + b_place * (4u * kUnitB) + nt * 2048u + ((piece ^ ((col >> 1) & 3u)) * 16u));
+        }
+    };
+    auto unpack = [&](uint32_t nt, uint32_t s) {
+        const uint4 (&codes)[BITS / 4] = raw[kTwoA ? nt : 0u];
+        if (BITS == 4) {
+            const uint32_t w[4] = {codes[0].x, codes[0].y, codes[0].z, codes[0].w};
+            bf[nt][s] = codes4(w[s]);
+        } else {
+            const uint4 v = codes[s >> 1 & (BITS / 4 - 1)];
+            bf[nt][s] = s & 1u ? codes8(v.z, v.w) : codes8(v.x, v.y);
+        }
+    };
+    // The places of group g's rows and of its codes. Powers of two are known to the compiler four groups at a time.
+    uint32_t place3 = 0;  // g % 3
+    auto next3 = [](uint32_t p) { return p == 2u ? 0u : p + 1u; };
+    auto a_place = [&](uint32_t u) { return kA == 3u ? place3 : u & (kA - 1u); };
+    auto b_place = [&](uint32_t u) { return kB == 3u ? place3 : BITS == 8 ? u & 1u : (u >> 1) & 1u; };
+    // Where group g + 1's operands are all there and the place of group g's rows is free again: what the wave asks for here is
+    // for that place. u = g % 4; far: the groups up to g + 4 exist, and the loads that may still be on their way are counted;
+    // else all are waited for.
+    auto meet = [&](uint32_t g, auto u_, auto far_) {
+        constexpr uint32_t U = decltype(u_)::value;
+        constexpr bool FAR = decltype(far_)::value;
+        constexpr bool kOdd = (U & 1u) != 0u;
+        // what was asked for at the last meeting, or the last two, and is not needed yet
+        constexpr uint32_t kOnTheWay = kA == 2u              ? (BITS == 4 && !kOdd ? 4u : 0u)
+                                       : kA == 3u            ? MT + 4u + (U == 1u ? 1u : 0u)
+                                       : kOdd                ? 2u * MT + (U == 1u ? 1u : 0u)
+                                                             : 2u * MT + 4u + (U == 2u ? 1u : 0u);
+        wait_loads_and_sync<FAR ? int(kOnTheWay) : 0>();
+        if (U == 0u && (FAR || g + 4u < G)) load_s((g >> 2) + 1u);
+        if (kA == 2u && (FAR || g + kA < G)) load_a(a_place(U), g + kA);
+        if (BITS == 8 && (FAR || g + kB < G)) load_b(b_place(U), g + kB);
+        if (BITS == 4 && kOdd && (FAR || g - 1u + 2u * kB < G)) load_b(b_place(U), (g >> 1) + kB, !FAR);
+        if (kA != 2u && (FAR || g + kA < G)) load_a(a_place(U), g + kA);
+    };
+    auto step = [&](uint32_t g, auto u_, auto far_) {
+        constexpr uint32_t U = decltype(u_)::value;
+        if (!active) {
+            meet(g, u_, far_);
+            if (kA == 3u) place3 = next3(place3);
+            return;
+        }
+        const uint32_t a_here = a_place(U), a_next = kA == 3u ? next3(place3) : a_place(U + 1u), b_next = kB == 3u ? a_next : b_place(U + 1u);
+#pragma unroll
+        for (uint32_t c = 0; c < 2u * MT; ++c) {
+            const uint32_t mt = c >> 1, nt = c & 1u;
+            const uint32_t set = kTwoA ? (U * MT + mt) & 1u : 0u;
+            if (c == 2u * MT - 2u) {
+                meet(g, u_, far_);
+                read_raw(0, b_next, (U & 1u) ^ 1u);
+                if (U == 3u && (decltype(far_)::value || g + 1u < G)) read_run(g + 1u);
+            }
+            f32x16 &cur = p[kBehind ? nt : 0u], &old = p[kBehind ? nt ^ 1u : 0u];
+            float (&into)[16] = tot[nt ^ 1u][c ? (c - 1u) >> 1 : MT - 1u];
+            const float scale = c ? sc[nt ^ 1u] : sc_before;
+#pragma unroll
+            for (uint32_t s = 0; s < 4u; ++s) {
+                f32x16 zero = {0};
+                cur = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[set][s], bf[nt][s], s ? cur : zero, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                if (nt == (kTwoA ? 0u : 1u)) af[kTwoA ? set ^ 1u : 0u][s] = mt + 1u < MT ? read_a(a_here, mt + 1u, s) : read_a(a_next, 0u, s);
+                if (c == 0u) unpack(1, s);
+                if (c == 2u * MT - 1u) unpack(0, s);
+                if (c == 2u * MT - 1u && s == (kTwoA ? 0u : 3u)) read_raw(1, b_next, (U & 1u) ^ 1u);
+#pragma unroll
+                for (uint32_t i = 4u * s; kBehind && i < 4u * s + 4u; ++i) into[i] = fmaf(scale, old[i], into[i]);
+                // (named here: else the additions sink past the branches of `meet`, and every chain's sums stay alive until there)
+                if (kBehind) asm volatile("" : "+v"(into[4u * s]), "+v"(into[4u * s + 1u]), "+v"(into[4u * s + 2u]), "+v"(into[4u * s + 3u]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (!kBehind) {
+#pragma unroll
+                for (uint32_t i = 0; i < 16u; ++i) tot[nt][mt][i] = fmaf(sc[nt], cur[i], tot[nt][mt][i]);
+#pragma unroll
+                for (uint32_t i = 0; i < 16u; i += 4u) asm volatile("" : "+v"(tot[nt][mt][i]), "+v"(tot[nt][mt][i + 1u]), "+v"(tot[nt][mt][i + 2u]), "+v"(tot[nt][mt][i + 3u]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (kA == 3u) place3 = a_next;
+        sc_before = sc[1];
+        next_scales(std::integral_constant<bool, (U & 1u) == 0u>{});
+    };
+    if (active) {
+        read_run(0);
+        next_scales(std::false_type{});
+        read_raw(0, 0, 0);
+#pragma unroll
+        for (uint32_t s = 0; s < 4u; ++s) {
+            af[0][s] = read_a(0, 0, s);
+            unpack(0, s);
+        }
+        read_raw(1, 0, 0);
     }
-    if (G & 1u) step(G - 1u, std::integral_constant<uint32_t, 0>{});
-    // nobody reads the rings any more: the LDS takes the rows on their way out
-    wait_loads_and_sync<0>();
+    uint32_t g = 0;
+    for (; g + 8u <= G; g += 4u) {
+        step(g, std::integral_constant<uint32_t, 0>{}, std::true_type{});
+        step(g + 1u, std::integral_constant<uint32_t, 1>{}, std::true_type{});
+        step(g + 2u, std::integral_constant<uint32_t, 2>{}, std::true_type{});
+        step(g + 3u, std::integral_constant<uint32_t, 3>{}, std::true_type{});
+    }
+    for (; g < G; g += 4u) {
+        step(g, std::integral_constant<uint32_t, 0>{}, std::false_type{});
+        if (g + 1u < G) step(g + 1u, std::integral_constant<uint32_t, 1>{}, std::false_type{});
+        if (g + 2u < G) step(g + 2u, std::integral_constant<uint32_t, 2>{}, std::false_type{});
+        if (g + 3u < G) step(g + 3u, std::integral_constant<uint32_t, 3>{}, std::false_type{});
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (kBehind) tot[1][MT - 1u][i] = fmaf(sc_before, p[1][i], tot[1][MT - 1u][i]);
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+            for (uint32_t mt = 0; mt < MT; ++mt) total[nt][mt][i] = tot[nt][mt][i];
+    }
+    if (MODE == 0) wait_loads_and_sync<0>();  // (nobody reads the rings any more: the LDS takes the rows on their way out)
 
     // ---- epilogue: lane holds (m = 32 mt + 8 (i / 4) + 4 kb + i % 4, n = n0 + col)
     const uint32_t n = n0 + col;
@@ -482,80 +593,52 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         }
         __syncthreads();
         const uint32_t c0 = col_block * 128u, columns = min(128u, N - c0);  // N is a multiple of 64
-        for (uint32_t idx = threadIdx.x; idx < tile.rows * 16u; idx += 256u) {
-            const uint32_t m = idx >> 4, pc = idx & 15u;
-            if (pc * 8u < columns)
-                *reinterpret_cast<uint4 *>(a.act + (size_t(act_row) + m) * a.f + c0 + pc * 8u) =
-                    *reinterpret_cast<const uint4 *>(&s_out[m][pc * 8u]);
-        }
+        // a thread takes an eighth of a (row, group): eight neighbouring columns, out as they are and into the group's sum
         uint32_t *sums_out = const_cast<uint32_t *>(a.act_sums);
-        for (uint32_t slot = threadIdx.x; slot < L::kRows * 16u; slot += 256u) {  // (row, group of the block, eighth)
-            const uint32_t m = slot >> 4, gl = (slot >> 3) & 1u, eighth = slot & 7u;
+#pragma unroll
+        for (uint32_t i = 0; i < MT * 2u; ++i) {
+            const uint32_t slot = threadIdx.x + 256u * i, m = slot >> 4, gl = (slot >> 3) & 1u, eighth = slot & 7u;
             const uint4 v = *reinterpret_cast<const uint4 *>(&s_out[m][gl * 64u + eighth * 8u]);
             const uint32_t w[4] = {v.x, v.y, v.z, v.w};
             const float sum = eighth_sum(w);
-            if (eighth == 0u && m < tile.rows && gl * 64u < columns)
-                sums_out[(size_t(act_row) + m) * (a.f / kGroup) + c0 / kGroup + gl] = split_hi_lo(sum);
+            if (m < tile.rows && gl * 64u < columns) {
+                *reinterpret_cast<uint4 *>(a.act + (size_t(act_row) + m) * a.f + c0 + gl * 64u + eighth * 8u) = v;
+                if (eighth == 0u) sums_out[(size_t(act_row) + m) * (a.f / kGroup) + c0 / kGroup + gl] = split_hi_lo(sum);
+            }
         }
     } else {
-        // the down product's rows leave through the LDS too, [row][column of this block of 256], and go
-        // to their (token, rank) rows as whole 16-byte pieces; a call over a range of the sorted pairs writes the rows of
-        // its pairs only
-        const uint32_t row_lo = DENSE ? 0u : max(a.pair_lo, tile.pair_start) - tile.pair_start;
-        const uint32_t row_hi = DENSE ? tile.rows : min(a.pair_hi, tile.pair_start + tile.rows) - tile.pair_start;
+        // a lane's two sums of a row are neighbours: a row's 64 columns of the wave leave as one run of 128 bytes
         if (active) {
+            const uint32_t n2 = n0 + 2u * col;
             float dab[2] = {0.0f, 0.0f};
             if (!DENSE && a.ebias) {
-                dab[0] = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off)[n]);
-                dab[1] = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off)[n + 32u]);
+                dab[0] = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off)[n2]);
+                dab[1] = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off)[n2 + 1u]);
             }
+            uint8_t *out = reinterpret_cast<uint8_t *>(a.partials) + n2 * 2u;
 #pragma unroll
             for (uint32_t mt = 0; mt < MT; ++mt) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const uint32_t m = mt * 32u + 8u * (i / 4) + 4u * kb + (i % 4);
+                    const uint64_t to = s_dst[m];
                     uint16_t y0 = f32_to_f16(total[0][mt][i] + dab[0]), y1 = f32_to_f16(total[1][mt][i] + dab[1]);
                     if (DENSE && a.scalar_gate && m < tile.rows) {  // one gate a token row (moe.metal:1195-1207)
                         const float gate_mul = 1.0f + expf(-f16_to_f32(a.scalar_gate[tile.pair_start + m]));
                         y0 = f32_to_f16(f16_to_f32(y0) / gate_mul);
                         y1 = f32_to_f16(f16_to_f32(y1) / gate_mul);
                     }
-                    s_out[m][wave * 64u + col] = y0;
-                    s_out[m][wave * 64u + col + 32u] = y1;
+                    if (to != ~0ull) *reinterpret_cast<uint32_t *>(out + to) = uint32_t(y0) | uint32_t(y1) << 16;
                 }
-            }
-        }
-        __syncthreads();
-        const uint32_t c0 = col_block * 256u, columns = min(256u, N - c0);  // N is a multiple of 64
-        // 32 pieces a row, eight rows a pass; the pair records of eight passes are fetched together
-        const uint32_t pc = threadIdx.x & 31u;
-        constexpr uint32_t kPasses = MT * 32u / 8u, kBatch = kPasses < 8u ? kPasses : 8u;
-        for (uint32_t pass0 = 0; pass0 < kPasses; pass0 += kBatch) {
-            const uint16_t *dst_row[kBatch];
-#pragma unroll
-            for (uint32_t i = 0; i < kBatch; ++i) {
-                const uint32_t mm = min((pass0 + i) * 8u + (threadIdx.x >> 5), tile.rows - 1u);
-                if (DENSE) {
-                    dst_row[i] = a.partials + size_t(tile.pair_start + mm) * a.d;
-                } else {
-                    const shrike_token_expert_pair p = a.pairs[tile.pair_start + mm];
-                    dst_row[i] = a.partials + (size_t(p.token) * a.top_k + p.rank) * a.d;
-                }
-            }
-#pragma unroll
-            for (uint32_t i = 0; i < kBatch; ++i) {
-                const uint32_t m = (pass0 + i) * 8u + (threadIdx.x >> 5);
-                if (m >= row_lo && m < row_hi && pc * 8u < columns)
-                    *reinterpret_cast<uint4 *>(const_cast<uint16_t *>(dst_row[i]) + c0 + pc * 8u) = *reinterpret_cast<const uint4 *>(&s_out[m][pc * 8u]);
             }
         }
     }
 }
 
 template <int BITS, int MODE, bool DENSE, int META, FfnShape S>
-__global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArgs a) {
+__global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(FfnArgs a) {
     warm_kernel_arguments(a);
-    __shared__ __align__(16) uint8_t lds[Lds<S>::kBytes];
+    __shared__ __align__(16) uint8_t lds[Lds<S, BITS>::kBytes];
     constexpr bool WIDE = S == FfnShape::kWide;
     // Which (row tile, column block) this workgroup takes. Workgroups go to the chip's eight XCDs (each
     // with an L2 of its own) round robin in launch order, so workgroup w runs on XCD w % 8 as that XCD's
@@ -563,6 +646,9 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
     // of tiles with all their column blocks, so that the column blocks of a tile find its gathered rows,
     // and the row tiles of an expert its codes, in the L2 that fetched them first.
     const uint32_t column_blocks = gridDim.y;
+    // (a record a lane, asked for beside the count and not behind it)
+    uint4 short_table = zero4();
+    if (!WIDE && !DENSE) short_table = reinterpret_cast<const uint4 *>(a.tiles)[min(threadIdx.x & 63u, a.max_tiles - 1u)];
     const uint32_t tile_total = DENSE ? (a.dense_rows + kRowTile - 1u) / kRowTile : *a.tile_count;
     const uint32_t w = blockIdx.y * gridDim.x + blockIdx.x;
     const uint32_t xcd = w & 7u, item = w >> 3;
@@ -573,11 +659,8 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
     // read and converted twice for nothing, so the tiles stay whole. A row's result does not depend on its place in a tile.
     uint32_t parts = tile_total;
     uint64_t larger = 0;
-    uint4 short_table = zero4();
     if (!WIDE && !DENSE && tile_total <= 64u) {
-        const uint32_t lane = threadIdx.x & 63u;
-        if (lane < tile_total) short_table = reinterpret_cast<const uint4 *>(a.tiles)[lane];
-        larger = __ballot(short_table.z > 32u);
+        larger = __ballot((threadIdx.x & 63u) < tile_total && short_table.z > 32u);
         parts += uint32_t(__popcll(larger));
         if (parts * column_blocks > a.resident_workgroups || parts + 7u > gridDim.x) {
             parts = tile_total;
@@ -626,7 +709,7 @@ __global__ __launch_bounds__(256, (Lds<S>::kResident)) void k_grouped_ffn(FfnArg
         } else if (!WIDE && tile_total <= 256u && tile_total * gate_up_blocks <= a.resident_workgroups) {
             // (four named records, not an array: the compiler kept an array of them in private memory)
             const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
-            const uint4 rec0 = lane < tile_total ? table[lane] : zero4();
+            const uint4 rec0 = short_table;
             const uint4 rec1 = lane + 64u < tile_total ? table[lane + 64u] : zero4();
             const uint4 rec2 = lane + 128u < tile_total ? table[lane + 128u] : zero4();
             const uint4 rec3 = lane + 192u < tile_total ? table[lane + 192u] : zero4();
@@ -1027,7 +1110,8 @@ static uint32_t compute_units() {
 
 template <int BITS, bool DENSE, int META, FfnShape S>
 static int launch_ffn_shape(FfnArgs a, uint32_t max_tiles, hipStream_t s) {
-    a.resident_workgroups = Lds<S>::kResident * compute_units();
+    a.max_tiles = max_tiles;
+    a.resident_workgroups = Lds<S, BITS>::kResident * compute_units();
     const dim3 block(256);
     const uint32_t grid_tiles = (max_tiles + 7u) & ~7u;  // whole runs for the kernel's XCD mapping
     hipLaunchKernelGGL((k_grouped_ffn<BITS, 0, DENSE, META, S>), dim3(grid_tiles, (a.f + 127u) / 128u), block, 0, s, a);
@@ -1053,9 +1137,9 @@ static int launch_ffn_meta(const FfnArgs &a, uint32_t max_tiles, FfnShape shape,
     if (shape == FfnShape::kSplit) return launch_ffn_split<BITS, DENSE, META>(a, max_tiles, s);
     if constexpr (!DENSE)
         if (shape == FfnShape::kWide) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kWide>(a, max_tiles, s);
-    if constexpr (!DENSE && BITS == 8)
-        if (shape == FfnShape::kAhead) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kAhead>(a, max_tiles, s);
-    return launch_ffn_shape<BITS, DENSE, META, FfnShape::kTile>(a, max_tiles, s);
+    if constexpr (!DENSE && BITS == 4)
+        if (shape == FfnShape::kTile) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kTile>(a, max_tiles, s);
+    return launch_ffn_shape<BITS, DENSE, META, FfnShape::kDeep>(a, max_tiles, s);
 }
 template <int BITS, bool DENSE>
 static int launch_ffn(const FfnArgs &a, uint32_t max_tiles, FfnShape shape, hipStream_t s) {
@@ -1088,29 +1172,30 @@ size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max
 // The shape of the routed products, from what the host knows (and what a call over a range of the pairs shares with the call
 // over all of them: their outputs are the same bytes).
 //  - kSplit up to 1,024 pieces of its gate/up launch, two for each of the 512 workgroups it keeps: with 16 experts of
-//    1,536 x 1,024 it takes 21 us for 16 tokens where kTile takes 30, and 24.6 against 37.9 for 100 (8-bit codes). Past that it
-//    loses: its pieces are short and none of them overlaps the next in its workgroup (256 experts of 2,048 x 512, 128 tokens:
-//    150 against 126 us).
-//  - kWide where the experts' rows fill its tiles: from 48 pairs an expert at 8 bits (256 experts of 2,304 x 1,024, 2,000 tokens: 528 against
-//    645 us), from 64 at 4 bits, there only where the launch still has several workgroups for every compute unit (32 experts
-//    of 2,880 x 2,880, 2,048 tokens: 541 against 576 us; 256 experts of 2,048 x 512: 337 against 339 at 4,096 tokens, but 193
-//    against 169 at 2,000 unevenly spread ones).
-//  - kAhead for 8-bit codes up to 16 pairs an expert: the launch is then the weights coming in, and two groups on their way in
-//    two workgroups draw more of them than one group in three (256 experts of 2,304 x 1,024: 16 tokens 182 -> 156 us, 64 346
-//    -> 316, 200 404 -> 376, that is 4.8 TB/s). With more rows the third workgroup's products count (256 experts of 2,048 x
-//    512, 1,000 uneven tokens: 125 against 136 us), and with 4-bit codes they count from the start.
+//    1,536 x 1,024 it takes 21 us for 16 tokens where one row tile a workgroup takes 30, and 24.6 against 37.9 for 100 (8-bit
+//    codes). Past that it loses: its pieces are short and none of them overlaps the next in its workgroup (256 experts of 2,048
+//    x 512, 128 tokens: 150 against 126 us).
+//  - kWide where the experts' rows fill its tiles: from 48 pairs an expert at 8 bits (256 experts of 2,304 x 1,024, 2,000 tokens:
+//    502 against 613 us with kDeep; 1,400 tokens 447 against 442), from 64 at 4 bits, there only where the launch still has several
+//    workgroups for every compute unit (32 experts of 2,880 x 2,880, 2,048 tokens: 495 us).
+//  - kTile for 4-bit codes and a short k of the down product, kDeep for the others. kTile's third workgroup a compute unit hides
+//    the start and the end of the short ones, kDeep's loads start earlier: 32 experts of 2,880 x 2,880, 300 tokens 186 against
+//    163 us, 64 of 2,048 x 1,536, 600 tokens 116 against 112; 128 of 3,072 x 768, 512 uneven tokens 107 against 113, 256 of 1,536
+//    x 1,280, 2,000 uneven ones 264 against 270, 256 of 2,048 x 512, 512 uneven ones (129 tiles of 64 rows: more workgroups than
+//    kDeep has places for) 71 against 76. Three workgroups with 8-bit codes leave their loads one group ahead: 256 experts of
+//    2,304 x 1,024, 1,000 tokens 469 against 439.
 static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t f, uint32_t bits) {
     const uint64_t most_tiles = min(pairs, uint64_t(experts)) + pairs / kRowTile;
     if (most_tiles * (f / 32u) <= 1024u) return FfnShape::kSplit;
     if (bits == 8 ? pairs >= 48u * uint64_t(experts) : pairs >= 64u * uint64_t(experts) && pairs / kRowTile * ((f + 127u) / 128u) >= 1400u)
         return FfnShape::kWide;
-    return bits == 8 && pairs <= 16u * uint64_t(experts) ? FfnShape::kAhead : FfnShape::kTile;
+    return bits == 4 && f < 1536u ? FfnShape::kTile : FfnShape::kDeep;
 }
 // ... and of a dense expert's, whose rows are its tiles: kSplit up to two pieces a workgroup (2,048 x 512, 4-bit: 13 against
-// 45 us for 37 rows, 16 against 48 for 512, 32 against 47 for 1,500; 2,304 x 1,024, 8-bit: 44 against 54 for 1,000), kTile
-// past that (60 against 79 us for 4,096 rows).
+// 45 us for 37 rows, 16 against 48 for 512, 32 against 47 for 1,500; 2,304 x 1,024, 8-bit: 44 against 54 for 1,000), kDeep
+// past that (57 against 79 us for 4,096 rows).
 static FfnShape dense_shape(uint64_t rows, uint32_t f) {
-    return (rows + 31u) / 32u * (f / 32u) <= 1024u ? FfnShape::kSplit : FfnShape::kTile;
+    return (rows + 31u) / 32u * (f / 32u) <= 1024u ? FfnShape::kSplit : FfnShape::kDeep;
 }
 
 static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_bases *pool, uint64_t pool_slot_stride,
@@ -1155,7 +1240,8 @@ static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_base
     hipStream_t s = as_stream(stream);
     if (!presummed)
         if (int rc = launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, const_cast<uint32_t *>(a.hidden_sums), nullptr, s)) return rc;
-    const FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, f, moe->desc.routed_weight_bits);
+    FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, f, moe->desc.routed_weight_bits);
+    if (shape != FfnShape::kSplit && uint64_t(query_count) * hidden_stride_elements * 2u > 0xffffffffull) shape = FfnShape::kDeep;  // (the others' rows are 32-bit offsets)
     return moe->desc.routed_weight_bits == 8 ? launch_ffn<8, false>(a, max_row_tiles, shape, s) : launch_ffn<4, false>(a, max_row_tiles, shape, s);
 }
 

@@ -367,6 +367,22 @@ def test_grouped_ffn_shapes_of_a_workgroup(gpu, d, f, ne, k, t, bits, meta):
         pc.check_pair(got, int(tok), int(rank), f"token {tok} rank {rank}")
 
 
+@pytest.mark.parametrize("d,f,ne,t,bits", [
+    # groups of 64 in k around the four that the loop takes at once and the places of its rings, of both products; experts of up
+    # to 32 rows, up to 64 and, in the last three, of two row tiles; more than 64 tiles, so that none is cut in two
+    (448, 576, 70, 700, 4), (512, 704, 70, 700, 4), (832, 1408, 70, 700, 4),
+    (576, 1600, 70, 700, 4), (704, 1536, 70, 700, 4), (768, 1664, 70, 700, 4),
+    (448, 576, 70, 700, 8), (512, 704, 70, 700, 8), (832, 768, 70, 700, 8),
+    (448, 576, 70, 1000, 8), (704, 1408, 70, 1000, 8), (512, 4096, 30, 500, 4)])
+def test_grouped_ffn_rings(gpu, d, f, ne, t, bits):
+    L = Layer(0x5EED0700 + d + f, d, f, ne, 4, bits=bits, meta=S.META_F16 if f % 128 else S.META_BF16)
+    pc = PrefillCase(gpu, L, t)
+    got = pc.run()
+    assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
+    for pair in np.random.default_rng(12).choice(t * 4, 40, replace=False):
+        pc.check_pair(got, int(pair) // 4, int(pair) % 4, f"pair {pair}")
+
+
 @pytest.mark.parametrize("d,f,bits,meta", [(320, 640, 4, S.META_BF16), (1088, 704, 8, S.META_F16)])
 def test_grouped_ffn_of_few_larger_tiles(gpu, d, f, bits, meta):
     """Experts of 0, 1, 32, 33, 64 and more rows, few enough for a tile's rows past 32 to be a workgroup's of their own."""
