@@ -301,6 +301,11 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
 
     if (MODE == 1 && threadIdx.x < MT * 32u) s_dst[threadIdx.x] = dst;
 
+    // (4-bit codes: the place of the second unit of sums is free where there is none. 128 experts of 2,048 x 1,024, 300 tokens,
+    // weights from memory: 124 -> 120 us.)
+    const bool last_b_early = BITS == 4 && G <= 32u && (kB - 1u) * kGroupsPerB < G;
+    if (last_b_early) load_b(kB - 1u, kB - 1u);
+
     f32x16 total[2][MT];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt)
@@ -395,9 +400,9 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     // keep the order as it is written.
     wait_loads_and_sync<0>();  // (nobody reads the sums any more)
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) in the compiler's own count: else it waits for the biases in the loop
-    if (kA != 2u && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
+    if (kA != 2u && !last_b_early && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
     if (kA - 1u < G) load_a(kA - 1u, kA - 1u);
-    if (kA == 2u && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
+    if (kA == 2u && !last_b_early && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
     uint32_t run[2][2];  // the scales of a chunk of four groups, two a word
     float sc[2], sc_before = 0.0f;
     constexpr bool kTwoA = MT <= (S == FfnShape::kTile ? 1u : 2u);  // two sets of a row tile's operands: the next is read a chain earlier
@@ -474,7 +479,8 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
                                        : kA == 3u            ? MT + 4u + (U == 1u ? 1u : 0u)
                                        : kOdd                ? 2u * MT + (U == 1u ? 1u : 0u)
                                                              : 2u * MT + 4u + (U == 2u ? 1u : 0u);
-        wait_loads_and_sync<FAR ? int(kOnTheWay) : 0>();
+        if (kA == 2u && BITS == 4 && FAR && U == 0u && g == 0u) wait_loads_and_sync<0>();  // (the codes may have been asked for ahead of the rows)
+        else wait_loads_and_sync<FAR ? int(kOnTheWay) : 0>();
         if (U == 0u && (FAR || g + 4u < G)) load_s((g >> 2) + 1u);
         if (kA == 2u && (FAR || g + kA < G)) load_a(a_place(U), g + kA);
         if (BITS == 8 && (FAR || g + kB < G)) load_b(b_place(U), g + kB);
@@ -1175,19 +1181,28 @@ size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max
 //    1,536 x 1,024 it takes 21 us for 16 tokens where one row tile a workgroup takes 30, and 24.6 against 37.9 for 100 (8-bit
 //    codes). Past that it loses: its pieces are short and none of them overlaps the next in its workgroup (256 experts of 2,048
 //    x 512, 128 tokens: 150 against 126 us).
-//  - kWide where the experts' rows fill its tiles: from 48 pairs an expert at 8 bits (256 experts of 2,304 x 1,024, 2,000 tokens:
-//    502 against 613 us with kDeep; 1,400 tokens 447 against 442), from 64 at 4 bits, there only where the launch still has several
-//    workgroups for every compute unit (32 experts of 2,880 x 2,880, 2,048 tokens: 495 us).
+//  - kWide where the experts' rows fill its tiles and its launch still has several workgroups for every compute unit; its loop
+//    is the most products an unpacked code, its start and end the longest, so k must not be short. kWide against kTile or
+//    kDeep, us (pairs an expert; row tiles by column blocks of the gate/up launch):
+//      8 bits   256 experts of 2,304 x 1,024: 447, 442 (44; 1,368), 502, 613 (62; 2,000); 32 of 2,880 x 2,880: 294, 315 (62; 713);
+//               128 of 1,024 x 512: 73, 81 (70; 560); 100 of 1,024 x 512, uneven: 55, 57 (80; 500); 64 of 2,048 x 512: 92, 92 (87; 348);
+//               32 of 1,024 x 1,024: 55, 48 (75; 296); 64 of 512 x 256: 67, 60 (500; 1,000)
+//      4 bits   32 of 2,880 x 2,880: 183, 175 (50; 575), 212, 222 (62; 713), 224, 259 (87; 989); 256 of 2,048 x 512, even: 190, 207 (62;
+//               1,000), 230, 262 (94; 1,500), uneven: 165, 160 (62; 1,000), 208, 218 (94; 1,500); 128 of 2,048 x 768, even: 162, 187
+//               (75; 900), uneven: 169, 164; 64 of 2,048 x 1,024, uneven: 136, 128 (87; 696); 128 of 1,024 x 512: 67, 64 (70; 560); 64 of
+//               512 x 256: 66, 54 (500; 1,000)
 //  - kTile for 4-bit codes and a short k of the down product, kDeep for the others. kTile's third workgroup a compute unit hides
 //    the start and the end of the short ones, kDeep's loads start earlier: 32 experts of 2,880 x 2,880, 300 tokens 186 against
 //    163 us, 64 of 2,048 x 1,536, 600 tokens 116 against 112; 128 of 3,072 x 768, 512 uneven tokens 107 against 113, 256 of 1,536
 //    x 1,280, 2,000 uneven ones 264 against 270, 256 of 2,048 x 512, 512 uneven ones (129 tiles of 64 rows: more workgroups than
 //    kDeep has places for) 71 against 76. Three workgroups with 8-bit codes leave their loads one group ahead: 256 experts of
 //    2,304 x 1,024, 1,000 tokens 469 against 439.
-static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t f, uint32_t bits) {
+static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits) {
     const uint64_t most_tiles = min(pairs, uint64_t(experts)) + pairs / kRowTile;
     if (most_tiles * (f / 32u) <= 1024u) return FfnShape::kSplit;
-    if (bits == 8 ? pairs >= 48u * uint64_t(experts) : pairs >= 64u * uint64_t(experts) && pairs / kRowTile * ((f + 127u) / 128u) >= 1400u)
+    const uint64_t workgroups = pairs / kRowTile * ((f + 127u) / 128u);
+    if (bits == 8 ? pairs >= 48u * uint64_t(experts) && workgroups >= 450u && d + f >= 1536u
+                  : pairs >= 56u * uint64_t(experts) && workgroups >= 900u && d + f >= 2048u)
         return FfnShape::kWide;
     return bits == 4 && f < 1536u ? FfnShape::kTile : FfnShape::kDeep;
 }
@@ -1240,7 +1255,7 @@ static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_base
     hipStream_t s = as_stream(stream);
     if (!presummed)
         if (int rc = launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, const_cast<uint32_t *>(a.hidden_sums), nullptr, s)) return rc;
-    FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, f, moe->desc.routed_weight_bits);
+    FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, d, f, moe->desc.routed_weight_bits);
     if (shape != FfnShape::kSplit && uint64_t(query_count) * hidden_stride_elements * 2u > 0xffffffffull) shape = FfnShape::kDeep;  // (the others' rows are 32-bit offsets)
     return moe->desc.routed_weight_bits == 8 ? launch_ffn<8, false>(a, max_row_tiles, shape, s) : launch_ffn<4, false>(a, max_row_tiles, shape, s);
 }
