@@ -918,6 +918,12 @@ def test_decode_family_epilogues_against_oracle(gpu, d, f, k, bits, act, additiv
     assert np.array_equal(dl.hidden.download(np.uint16, d), O.residual_add_f16(L.hidden.copy(), y))
 
 
+@pytest.mark.parametrize("d,f,k,bits", [(512, 256, 4, 4), (64, 64, 2, 4), (320, 512, 3, 8), (192, 4096, 8, 8)])
+def test_additive_biases_of_packed_and_of_long_down_rows(gpu, d, f, k, bits):
+    """A wave's biases are loaded a lane each: rows packed eight and fewer a wave load, and rows of several loads."""
+    test_decode_family_epilogues_against_oracle(gpu, d, f, k, bits, capi.ACT_SILU, True)
+
+
 def test_gpt_oss_layer_with_its_epilogue_matches_the_oracle(gpu):
     """The fused layer entry with gpt-oss's family switches at its shape: routes bit for bit, y against the oracle."""
     d, f, ne, k = 2880, 2880, 32, 4
