@@ -658,9 +658,18 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
     // of tiles with all their column blocks, so that the column blocks of a tile find its gathered rows,
     // and the row tiles of an expert its codes, in the L2 that fetched them first.
     const uint32_t column_blocks = gridDim.y;
-    // (a record a lane, asked for beside the count and not behind it)
-    uint4 short_table = zero4();
-    if (!WIDE && !DENSE) short_table = reinterpret_cast<const uint4 *>(a.tiles)[min(threadIdx.x & 63u, a.max_tiles - 1u)];
+    // (The records of a table of up to 256 tiles, asked for beside the count and not behind it. Four named ones, not an array: the
+    // compiler kept an array of them in private memory.)
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
+    uint4 rec0 = zero4(), rec1 = zero4(), rec2 = zero4(), rec3 = zero4();
+    if (!WIDE && !DENSE) {
+        const uint32_t last = a.max_tiles - 1u;
+        rec0 = table[min(lane, last)];
+        rec1 = table[min(lane + 64u, last)];
+        rec2 = table[min(lane + 128u, last)];
+        rec3 = table[min(lane + 192u, last)];
+    }
     const uint32_t tile_total = DENSE ? (a.dense_rows + kRowTile - 1u) / kRowTile : *a.tile_count;
     const uint32_t w = blockIdx.y * gridDim.x + blockIdx.x;
     const uint32_t xcd = w & 7u, item = w >> 3;
@@ -672,7 +681,7 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
     uint32_t parts = tile_total;
     uint64_t larger = 0;
     if (!WIDE && !DENSE && tile_total <= 64u) {
-        larger = __ballot((threadIdx.x & 63u) < tile_total && short_table.z > 32u);
+        larger = __ballot(lane < tile_total && rec0.z > 32u);
         parts += uint32_t(__popcll(larger));
         if (parts * column_blocks > a.resident_workgroups || parts + 7u > gridDim.x) {
             parts = tile_total;
@@ -703,7 +712,6 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
         //  - Otherwise the XCD's eighth is a contiguous run of the table, its larger tiles first: the workgroups that start
         //    late are then the short ones, on the XCDs with the least work.
         // A lane reads one record; the chosen one is read across (no second load).
-        const uint32_t lane = threadIdx.x & 63u;
         const uint32_t gate_up_blocks = (a.f + 127u) / 128u;
         bool chosen = larger != 0u;
         if (chosen) {
@@ -713,18 +721,12 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
                 tile_index = uint32_t(__ffsll((long long)rest)) - 1u;
                 skip = 32u;
             }
-            tile.cell = uint32_t(__builtin_amdgcn_readlane(int(short_table.x), int(tile_index)));
-            tile.pair_start = uint32_t(__builtin_amdgcn_readlane(int(short_table.y), int(tile_index))) + skip;
-            const uint32_t rows = uint32_t(__builtin_amdgcn_readlane(int(short_table.z), int(tile_index)));
+            tile.cell = uint32_t(__builtin_amdgcn_readlane(int(rec0.x), int(tile_index)));
+            tile.pair_start = uint32_t(__builtin_amdgcn_readlane(int(rec0.y), int(tile_index))) + skip;
+            const uint32_t rows = uint32_t(__builtin_amdgcn_readlane(int(rec0.z), int(tile_index)));
             tile.rows = skip ? rows - 32u : min(rows, 32u);
-            tile.expert = uint32_t(__builtin_amdgcn_readlane(int(short_table.w), int(tile_index)));
+            tile.expert = uint32_t(__builtin_amdgcn_readlane(int(rec0.w), int(tile_index)));
         } else if (!WIDE && tile_total <= 256u && tile_total * gate_up_blocks <= a.resident_workgroups) {
-            // (four named records, not an array: the compiler kept an array of them in private memory)
-            const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
-            const uint4 rec0 = short_table;
-            const uint4 rec1 = lane + 64u < tile_total ? table[lane + 64u] : zero4();
-            const uint4 rec2 = lane + 128u < tile_total ? table[lane + 128u] : zero4();
-            const uint4 rec3 = lane + 192u < tile_total ? table[lane + 192u] : zero4();
             const bool in0 = lane < tile_total, in1 = lane + 64u < tile_total, in2 = lane + 128u < tile_total, in3 = lane + 192u < tile_total;
             const uint64_t larger0 = __ballot(in0 && rec0.z > 32u), larger1 = __ballot(in1 && rec1.z > 32u);
             const uint64_t larger2 = __ballot(in2 && rec2.z > 32u), larger3 = __ballot(in3 && rec3.z > 32u);
@@ -770,7 +772,6 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
             // grouping leaves them; a caller's table may leave tiles out): the first of them takes both. A tile is a first one
             // where an even number of tiles ahead of it, each continuing the one before, run into it. Lane l reads record
             // at - l; the one before it is lane l + 1's.
-            const uint4 *table = reinterpret_cast<const uint4 *>(a.tiles);
             uint32_t ahead = 0, second_rows = 0;
             for (uint32_t at = tile_index + 1u, skip_links = 1u;; at -= 63u, skip_links = 0u) {
                 const uint4 rec = lane <= at && at - lane < tile_total ? table[at - lane] : zero4();
@@ -792,7 +793,7 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
             tile.rows += second_rows;
         } else if (chosen) {
         } else if (count <= 64u) {
-            const uint4 rec = lane < count ? reinterpret_cast<const uint4 *>(a.tiles)[first + lane] : zero4();
+            const uint4 rec = lane < count ? table[first + lane] : zero4();
             const uint64_t heavy = __ballot(lane < count && rec.z > 32u), light = __ballot(lane < count && rec.z <= 32u);
             const uint32_t heavies = uint32_t(__popcll(heavy));
             const uint64_t set = place < heavies ? heavy : light;
