@@ -770,27 +770,61 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
         if (WIDE) {
             // Two neighbouring tiles of an expert are one workgroup's work where the second continues the first's pairs (as
             // grouping leaves them; a caller's table may leave tiles out): the first of them takes both. A tile is a first one
-            // where an even number of tiles ahead of it, each continuing the one before, run into it. Lane l reads record
-            // at - l; the one before it is lane l + 1's.
-            uint32_t ahead = 0, second_rows = 0;
-            for (uint32_t at = tile_index + 1u, skip_links = 1u;; at -= 63u, skip_links = 0u) {
-                const uint4 rec = lane <= at && at - lane < tile_total ? table[at - lane] : zero4();
-                const uint4 before = make_uint4(__shfl_down(rec.x, 1), __shfl_down(rec.y, 1), __shfl_down(rec.z, 1), __shfl_down(rec.w, 1));
-                const bool follows = lane < min(at, 63u) && rec.w == before.w && rec.x == before.x && before.z == kRowTile && rec.y == before.y + kRowTile;
-                const uint64_t links = __ballot(follows);
-                if (skip_links) {
-                    tile.cell = uint32_t(__builtin_amdgcn_readlane(int(rec.x), 1));
-                    tile.pair_start = uint32_t(__builtin_amdgcn_readlane(int(rec.y), 1));
-                    tile.rows = uint32_t(__builtin_amdgcn_readlane(int(rec.z), 1));
-                    tile.expert = uint32_t(__builtin_amdgcn_readlane(int(rec.w), 1));
-                    if (links & 1u) second_rows = uint32_t(__builtin_amdgcn_readlane(int(rec.z), 0));
-                }
-                const uint32_t run_in = uint32_t(__ffsll((long long)~(links >> skip_links))) - 1u;
+            // where an even number of tiles ahead of it, each continuing the one before, run into it. The workgroup's place is
+            // among the first ones of its XCD's run, so that the workgroups without a tile are the last ones. Where every tile had
+            // its workgroups and those of the second ones left at once, the compute units did not fill evenly: 32 experts of
+            // 2,880 x 2,880, 2,048 tokens 500 -> 483 us, 700 tokens 224 -> 217 (with the two tiles' workgroups in turn 680 and 318).
+            // Where few tiles fill the XCD's places, those of more than 64 rows go ahead of the others of the same 64 records (497
+            // without that; 256 experts of 2,304 x 1,024, 8 column blocks a tile, 4,000 tokens 716 in the table's order, 758 so).
+            auto continues = [&](const uint4 &rec, const uint4 &before) {
+                return rec.w == before.w && rec.x == before.x && before.z == kRowTile && rec.y == before.y + kRowTile;
+            };
+            auto record = [&](uint32_t at) { return at < tile_total ? table[at] : zero4(); };
+            uint4 rec = record(first + lane), next = record(first + lane + 1u);
+            // the tiles that run into the run's first one: lane l reads record at - l, the one before it is lane l + 1's
+            uint32_t ahead = 0;
+            for (uint32_t at = first;; at -= 63u) {
+                const uint4 back = lane <= at ? record(at - lane) : zero4();
+                const uint4 before = make_uint4(__shfl_down(back.x, 1), __shfl_down(back.y, 1), __shfl_down(back.z, 1), __shfl_down(back.w, 1));
+                const uint64_t links = __ballot(lane < min(at, 63u) && continues(back, before));
+                const uint32_t run_in = uint32_t(__ffsll((long long)~links)) - 1u;
                 ahead += run_in;
-                if (run_in < 63u - skip_links) break;
+                if (run_in < 63u) break;
             }
-            if (ahead & 1u) return;
-            tile.rows += second_rows;
+            bool found = false;
+            uint32_t rank = place;
+            for (uint32_t at = first; at < first + run && !found; at += 64u) {
+                const bool goes_on = next.z != 0u && continues(next, rec);
+                const uint64_t links = __ballot(goes_on) << 1;  // bit l: record at + l continues the one before it
+                const uint64_t breaks = ~links & ((2ull << lane) - 1ull);  // (bit 0 always: `ahead` is what runs into it)
+                const uint32_t from = 63u - uint32_t(__clzll((long long)breaks)), mine_ahead = lane - from + (from == 0u ? ahead : 0u);
+                const bool is_first = at + lane < first + run && (mine_ahead & 1u) == 0u;
+                const uint32_t rows = rec.z + (goes_on ? next.z : 0u);
+                const bool is_heavy = column_blocks < 12u || rows > kRowTile;
+                const uint64_t heavy = __ballot(is_first && is_heavy), light = __ballot(is_first && !is_heavy);
+                const uint32_t heavies = uint32_t(__popcll(heavy)), firsts = heavies + uint32_t(__popcll(light));
+                if (rank < firsts) {
+                    const uint64_t set = rank < heavies ? heavy : light;
+                    const uint32_t want = rank < heavies ? rank : rank - heavies;
+                    const bool me = ((set >> lane) & 1ull) != 0ull && uint32_t(__popcll(set & ((1ull << lane) - 1ull))) == want;
+                    const int src = __builtin_amdgcn_readfirstlane(__ffsll((long long)__ballot(me)) - 1);
+                    tile.cell = uint32_t(__builtin_amdgcn_readlane(int(rec.x), src));
+                    tile.pair_start = uint32_t(__builtin_amdgcn_readlane(int(rec.y), src));
+                    tile.rows = uint32_t(__builtin_amdgcn_readlane(int(rows), src));
+                    tile.expert = uint32_t(__builtin_amdgcn_readlane(int(rec.w), src));
+                    tile_index = at + uint32_t(src);
+                    found = true;
+                }
+                rank -= firsts;
+                // what runs into the next 64's first record
+                const uint32_t last_ahead = uint32_t(__builtin_amdgcn_readlane(int(mine_ahead), 63));
+                ahead = __builtin_amdgcn_readlane(int(goes_on), 63) ? last_ahead + 1u : 0u;
+                if (!found && at + 64u < first + run) {
+                    rec = record(at + 64u + lane);
+                    next = record(at + 65u + lane);
+                }
+            }
+            if (!found) return;
         } else if (chosen) {
         } else if (count <= 64u) {
             const uint4 rec = lane < count ? table[first + lane] : zero4();
