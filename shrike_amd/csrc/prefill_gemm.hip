@@ -182,7 +182,10 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     uint16_t (*s_out)[L::kRow] = reinterpret_cast<uint16_t (*)[L::kRow]>(lds);
 
     // ---- A: the tile's rows, a group of them (128 bytes a row) at a time. A load brings eight rows, eight lanes a row, its
-    // sixteen-byte pieces xor-ed with the row so that eight rows read at one piece touch every bank once.
+    // sixteen-byte pieces xor-ed with half the row's number so that sixteen rows read at one piece touch each of the 64 banks once
+    // (and those of the codes below, four a row, with a quarter of it). Conflicts of the kWide gate/up launch over 2,048 gpt-oss
+    // tokens 25.4 M -> 4.9 M cycles of the compute units (of 170 M), where eight and four rows counted as one read's; both products of 512 tokens of
+    // 256 x 2,048 x 512 76.2 -> 74.3 us, long chunks within 1 %.
     constexpr uint32_t kLoadsA = MT;  // a wave's loads a group
     constexpr bool kNear = S != FfnShape::kDeep;  // a row is a 32-bit offset from a base (the launch's rule)
     const uint8_t *a_src[kLoadsA];
@@ -201,7 +204,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             row = a.act + (size_t(act_row) + r) * a.f;
             a_sums[j] = a.act_sums + (size_t(act_row) + r) * G;
         }
-        a_src[j] = reinterpret_cast<const uint8_t *>(row) + (((lane & 7u) ^ (lane >> 3)) * 16u);
+        a_src[j] = reinterpret_cast<const uint8_t *>(row) + (((lane & 7u) ^ (4u * (wave & 1u) + (lane >> 4))) * 16u);
         if (kNear) a_off[j] = uint32_t(a_src[j] - a_base);
     }
     auto load_a = [&](uint32_t slot, uint32_t g) {
@@ -240,10 +243,10 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     uint32_t b_off[4];
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-        b_off[j] = row_of(j >> 1, 16u * (j & 1u) + (lane >> 2)) * row_bytes + ((lane & 3u) ^ ((lane >> 3) & 3u)) * 16u;
+        b_off[j] = row_of(j >> 1, 16u * (j & 1u) + (lane >> 2)) * row_bytes + ((lane & 3u) ^ (lane >> 4)) * 16u;
     // (at 4 bits a row of an odd number of groups ends halfway through its last stage: the lanes of the missing half take
     // the other half's pieces, so that nothing past a tensor's last row is read)
-    const uint32_t half_back = (((lane & 3u) ^ ((lane >> 3) & 3u)) & 2u) * 16u;
+    const uint32_t half_back = (((lane & 3u) ^ (lane >> 4)) & 2u) * 16u;
     constexpr uint32_t kGroupsPerB = BITS == 4 ? 2u : 1u;
     const uint32_t lds_b = lds0 + L::kB + wave * kUnitB;
     auto load_b = [&](uint32_t slot, uint32_t stage, bool may_end = true) {
@@ -443,13 +446,13 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     };
     const uint8_t *a_rows = lds + col * 128u, *b_rows = lds + L::kB + wave * kUnitB + col * 64u;
     auto read_a = [&](uint32_t place, uint32_t mt, uint32_t s) {
-        return *reinterpret_cast<const half8 *>(a_rows + place * kUnitA + mt * 4096u + (((kb * 4u + s) ^ (col & 7u)) * 16u));
+        return *reinterpret_cast<const half8 *>(a_rows + place * kUnitA + mt * 4096u + (((kb * 4u + s) ^ ((col >> 1) & 7u)) * 16u));
     };
     auto read_raw = [&](uint32_t nt, uint32_t b_place, uint32_t par) {
 #pragma unroll
         for (uint32_t i = 0; i < BITS / 4; ++i) {
             const uint32_t piece = BITS == 4 ? par * 2u + kb : kb * 2u + i;
-            raw[kTwoA ? nt : 0u][i] = *reinterpret_cast<const uint4 *>(b_rows + b_place * (4u * kUnitB) + nt * 2048u + ((piece ^ ((col >> 1) & 3u)) * 16u));
+            raw[kTwoA ? nt : 0u][i] = *reinterpret_cast<const uint4 *>(b_rows + b_place * (4u * kUnitB) + nt * 2048u + ((piece ^ ((col >> 2) & 3u)) * 16u));
         }
     };
     auto unpack = [&](uint32_t nt, uint32_t s) {
