@@ -1231,24 +1231,25 @@ size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max
 //      8 bits   256 experts of 2,304 x 1,024: 447, 442 (44; 1,368), 502, 613 (62; 2,000); 32 of 2,880 x 2,880: 294, 315 (62; 713);
 //               128 of 1,024 x 512: 73, 81 (70; 560); 100 of 1,024 x 512, uneven: 55, 57 (80; 500); 64 of 2,048 x 512: 92, 92 (87; 348);
 //               32 of 1,024 x 1,024: 55, 48 (75; 296); 64 of 512 x 256: 67, 60 (500; 1,000)
-//      4 bits   32 of 2,880 x 2,880: 183, 175 (50; 575), 212, 222 (62; 713), 224, 259 (87; 989); 256 of 2,048 x 512, even: 190, 207 (62;
-//               1,000), 230, 262 (94; 1,500), uneven: 165, 160 (62; 1,000), 208, 218 (94; 1,500); 128 of 2,048 x 768, even: 162, 187
-//               (75; 900), uneven: 169, 164; 64 of 2,048 x 1,024, uneven: 136, 128 (87; 696); 128 of 1,024 x 512: 67, 64 (70; 560); 64 of
-//               512 x 256: 66, 54 (500; 1,000)
-//  - kTile for 4-bit codes and a short k of the down product, kDeep for the others. kTile's third workgroup a compute unit hides
-//    the start and the end of the short ones, kDeep's loads start earlier: 32 experts of 2,880 x 2,880, 300 tokens 186 against
-//    163 us, 64 of 2,048 x 1,536, 600 tokens 116 against 112; 128 of 3,072 x 768, 512 uneven tokens 107 against 113, 256 of 1,536
-//    x 1,280, 2,000 uneven ones 264 against 270, 256 of 2,048 x 512, 512 uneven ones (129 tiles of 64 rows: more workgroups than
-//    kDeep has places for) 71 against 76. Three workgroups with 8-bit codes leave their loads one group ahead: 256 experts of
-//    2,304 x 1,024, 1,000 tokens 469 against 439.
+//      4 bits, kWide against the better of the others, even and uneven experts (pairs an expert; workgroups times groups of both k):
+//               64 of 1,088 x 1,664: 108, 117 and 107, 93 (79; 44 k); 128 of 2,048 x 768: 162, 175 and 167, 155 (75; 40 k); 256 of
+//               2,048 x 512: 189, 199 and 162, 154 (62; 40 k), 232, 258 and 216, 212 (94; 60 k); 48 of 3,072 x 1,536, uneven: 182, 188
+//               (75; 49 k); 256 of 1,536 x 1,280, uneven: 255, 257 (62; 110 k); 32 of 2,880 x 2,880: 183, 173 (50; 52 k), 210, 222 (62;
+//               65 k), 219, 259 (87; 89 k). The line lies where uneven experts stop losing.
+//  - kTile for 4-bit codes but for the longest k, kDeep for the others. kTile's third workgroup a compute unit hides the start and
+//    the end of the short ones, kDeep's loads start earlier: 32 experts of 2,880 x 2,880, 400 tokens 186 against 173 us; 128 of 3,072 x
+//    768, 512 uneven tokens 107 against 113; 48 of 3,072 x 1,536, 900 uneven ones 188 against 199, 64 of 1,280 x 2,048, 700 even ones
+//    106 against 104, uneven 91 against 95; 256 of 2,048 x 512, 512 uneven ones (129 tiles of 64 rows: more workgroups than kDeep
+//    has places for) 71 against 76. Three workgroups with 8-bit codes leave their loads one group ahead: 256 experts of 2,304 x
+//    1,024, 1,000 tokens 469 against 439.
 static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits) {
     const uint64_t most_tiles = min(pairs, uint64_t(experts)) + pairs / kRowTile;
     if (most_tiles * (f / 32u) <= 1024u) return FfnShape::kSplit;
     const uint64_t workgroups = pairs / kRowTile * ((f + 127u) / 128u);
     if (bits == 8 ? pairs >= 48u * uint64_t(experts) && workgroups >= 450u && d + f >= 1536u
-                  : pairs >= 56u * uint64_t(experts) && workgroups >= 900u && d + f >= 2048u)
+                  : pairs >= 56u * uint64_t(experts) && workgroups * ((d + f) / kGroup) >= 46000u && d + f >= 2048u)
         return FfnShape::kWide;
-    return bits == 4 && f < 1536u ? FfnShape::kTile : FfnShape::kDeep;
+    return bits == 4 && d + f < 5120u ? FfnShape::kTile : FfnShape::kDeep;
 }
 // ... and of a dense expert's, whose rows are its tiles: kSplit up to two pieces a workgroup (2,048 x 512, 4-bit: 13 against
 // 45 us for 37 rows, 16 against 48 for 512, 32 against 47 for 1,500; 2,304 x 1,024, 8-bit: 44 against 54 for 1,000), kDeep
