@@ -154,8 +154,8 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // loop is a pipeline: between the MFMAs of chain c stand the scaling of chain c - 1, a share of the next codes' unpacking and
 // the reads of the rows that the next chain takes, and the wait for the next group's loads stands two chains ahead of their
 // use. What bounds it now: with many rows the power that matrix work, its operands' way through LDS and the loads take
-// together (the kWide gate/up launch over 2,048 gpt-oss tokens runs at 2.0 GHz of 2.4, the matrix pipe busy 42 % of the
-// cycles); with few rows the weights' bytes (kDeep, 8-bit, 1,000 tokens: 4.4 TB/s), and the start and the end of the many
+// together (the kWide gate/up launch over 2,048 gpt-oss tokens runs at 1.9 GHz of 2.4, the matrix pipe busy 49 % of the
+// cycles, vector issue 47 %); with few rows the weights' bytes (kDeep, 8-bit, 1,000 tokens: 4.4 TB/s), and the start and the end of the many
 // short workgroups (30 of 75 us at 256 experts of 2,048 x 512 and 512 tokens). Both products, a chain scaled where it ends ->
 // pipelined: 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens 540 -> 495 us, 300 tokens 179 -> 164; 256 of 2,048 x 512, 4,096
 // tokens 316 -> 302, 37 33.5 -> 31.4; 256 of 2,304 x 1,024, 8-bit, 1,000 tokens 469 -> 439, 4,000 735 -> 710.
@@ -183,9 +183,9 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
 
     // ---- A: the tile's rows, a group of them (128 bytes a row) at a time. A load brings eight rows, eight lanes a row, its
     // sixteen-byte pieces xor-ed with half the row's number so that sixteen rows read at one piece touch each of the 64 banks once
-    // (and those of the codes below, four a row, with a quarter of it). Conflicts of the kWide gate/up launch over 2,048 gpt-oss
-    // tokens 25.4 M -> 4.9 M cycles of the compute units (of 170 M), where eight and four rows counted as one read's; both products of 512 tokens of
-    // 256 x 2,048 x 512 76.2 -> 74.3 us, long chunks within 1 %.
+    // (and those of the codes below, four a row, with a quarter of it). With the whole of it and half, right for 32 banks, the
+    // kWide gate/up launch over 2,048 gpt-oss tokens had conflicts of 25.4 M cycles of the compute units' 170 M, now 4.9 M; both
+    // products of 512 tokens, 256 experts of 2,048 x 512, 76.2 -> 74.3 us, long chunks within 1 %.
     constexpr uint32_t kLoadsA = MT;  // a wave's loads a group
     constexpr bool kNear = S != FfnShape::kDeep;  // a row is a 32-bit offset from a base (the launch's rule)
     const uint8_t *a_src[kLoadsA];
