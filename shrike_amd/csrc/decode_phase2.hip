@@ -86,11 +86,13 @@ __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
     const uint16_t *s_all = reinterpret_cast<const uint16_t *>(base + a.off.down_s_off);
     const uint16_t *b_all = reinterpret_cast<const uint16_t *>(base + a.off.down_b_off);
 
-    // (an additive bias a lane, asked for ahead of the rows: fetched where a row's sum is written it was a round trip to memory a
-    // row group, 5 of 23 us for four tokens of 2,880 x 2,880)
+    // The rows' additive biases are asked for behind the first rows, whose arithmetic does not wait for them: fetched where a
+    // row's sum is written they were a round trip to memory a row group, 5 of 23 us for four tokens of 2,880 x 2,880. Where rows
+    // take a wave each, lane l holds row l's; where several share one, each lane loads those of its own rows. (Asked for ahead
+    // of the rows, and added to the sums by way of LDS, packed rows lost: a layer of 2,048 x 512, one token, 12.9 -> 13.3 us,
+    // now 12.8; 1,024 x 256, sixteen tokens, 17.9 -> 18.4, now 17.7.)
+    const uint16_t *biases = reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off);
     uint16_t bias = 0;
-    if (live && a.ebias && lane < kPhase2Rows && d0 + lane < a.d) bias = reinterpret_cast<const uint16_t *>(base + a.off.down_ab_off)[d0 + lane];
-
     if (live) {
         const uint32_t n_groups = kPhase2Rows / rpl;
         typename C::X x[NCH];
@@ -108,15 +110,22 @@ __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
                 load_row<BITS, NCH, STREAM, TAIL>(rows[j], base + a.off.down_w_off + size_t(rr) * row_bytes,
                                     s_all + size_t(rr) * groups, b_all + size_t(rr) * groups, cpr, col, on[j]);
             }
+            uint16_t own[BATCH];
+            if (!kWholeWave && a.ebias) {  // (one branch round all of them: a choice a row was a branch a row, 45 -> 50 us for
+                                           // four tokens of 2,048 x 1,024, 8-bit)
+#pragma unroll
+                for (int j = 0; j < BATCH; ++j) own[j] = biases[on[j] ? row[j] : 0u];
+            }
+            if (kWholeWave && a.ebias && g0 == 0 && lane < kPhase2Rows && d0 + lane < a.d) bias = biases[d0 + lane];
             if (g0 == 0) unpack_slices<BITS, NCH, TAIL>(xr, x, xs, xt);
 #pragma unroll
             for (int j = 0; j < BATCH; ++j) {
                 const float v = seg_sum(row_partial<BITS, NCH, TAIL>(rows[j], x, xs, xt, uint32_t(META)), seg);
                 const bool writer = on[j] && writer_lane;
-                if (writer) partial[k][row[j] - d0] = a.ebias ? v : wk * v;  // moe.metal:1049
+                const uint32_t row_bias = kWholeWave ? uint32_t(__builtin_amdgcn_readlane(int(bias), int(g0) + j)) : own[j];
+                if (writer) partial[k][row[j] - d0] = wk * (a.ebias ? v + bf16_to_f32(uint16_t(row_bias)) : v);  // moe.metal:1049
             }
         }
-        if (a.ebias && lane < kPhase2Rows) partial[k][lane] = wk * (partial[k][lane] + bf16_to_f32(bias));
     } else if (lane < kPhase2Rows) {
         partial[k][lane] = 0.0f;
     }

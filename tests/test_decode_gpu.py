@@ -920,7 +920,8 @@ def test_decode_family_epilogues_against_oracle(gpu, d, f, k, bits, act, additiv
 
 @pytest.mark.parametrize("d,f,k,bits", [(512, 256, 4, 4), (64, 64, 2, 4), (320, 512, 3, 8), (192, 4096, 8, 8)])
 def test_additive_biases_of_packed_and_of_long_down_rows(gpu, d, f, k, bits):
-    """A wave's biases are loaded a lane each: rows packed eight and fewer a wave load, and rows of several loads."""
+    """Rows packed eight and fewer a wave load, whose lanes load their own rows' biases, and rows of several loads, whose biases
+    the wave's first lanes hold."""
     test_decode_family_epilogues_against_oracle(gpu, d, f, k, bits, capi.ACT_SILU, True)
 
 

@@ -1,5 +1,6 @@
-"""The hand-written loads into LDS beside the compiler's own: both take their LDS address from m0, so each must know of the
-other's. Read from the AMD assembly that the library's own header compiles to; no GPU."""
+"""What the library's own sources compile to, read from their AMD assembly; no GPU. The hand-written loads into LDS beside the
+compiler's own: both take their LDS address from m0, so each must know of the other's. And phase 2's partial sums: lanes
+exchange them through LDS behind the workgroup's barrier only."""
 import re
 import subprocess
 
@@ -42,3 +43,18 @@ def test_the_compiler_knows_what_m0_holds_after_a_hand_written_load(tmp_path, lo
             addresses.append(m0)
     assert len(addresses) == 3
     assert addresses[0] == addresses[2] != addresses[1], f"the loads' LDS addresses: {addresses}"
+
+
+@pytest.mark.parametrize("instance", ["4, 1, 2, true, 8, false, SHRIKE_META_F16", "8, 1, 4, false, 8, false, SHRIKE_META_BF16",  # rows that share a wave load
+                                      "8, 3, 4, true, 4, false, SHRIKE_META_BF16", "4, 1, 4, false, 16, true, SHRIKE_META_F16"])
+def test_phase_2_reads_no_partial_sum_ahead_of_its_barrier(tmp_path, instance):
+    """A lane's word of LDS is another lane's only behind the barrier: nothing else orders the two for the compiler."""
+    with open(f"{ROOT}/shrike_amd/csrc/decode_phase2.hip") as f:
+        text = f.read()
+    source = tmp_path / "k.hip"
+    source.write_text(text[:text.index("template <int BITS, int NCH>\n__global__ __launch_bounds__(256) void k_gemv")] +
+                      f"template __global__ void k_phase2<{instance}>(Phase2Args);\n}}\n")
+    subprocess.run(["/opt/rocm/bin/hipcc", *FLAGS, f"-I{ROOT}/shrike_amd/csrc", str(source), "-o", str(tmp_path / "k.s")], check=True)
+    code = (tmp_path / "k.s").read_text().split("s_barrier")
+    assert len(code) == 2 and re.search(r"\bds_write", code[0]) and re.search(r"\bds_read", code[1])
+    assert not re.search(r"\bds_read", code[0]), "a partial sum is read ahead of the barrier"
