@@ -415,7 +415,9 @@ typedef struct {
  * PrefillMoEGrouping.swift:32-50): sorted_pairs are 16-byte PrefillTokenExpertPair
  * records (token, expert, rank, fp16 weight bits); per_expert_offsets is UINT32_MAX
  * where an expert has no pair. row_tiles has room for
- * shrike_hip_group_max_row_tiles() entries; row_tile_count is one word. */
+ * shrike_hip_group_max_row_tiles() entries; row_tile_count is one word. The grouped FFN may read any entry of that room
+ * (for its query_count * top_k pairs and the handle's experts; never more than its max_row_tiles), also those past the
+ * count, which need not have been written. */
 typedef struct {
     void *sorted_pairs;
     uint32_t *per_expert_offsets;
@@ -443,7 +445,8 @@ int shrike_hip_group_pairs(void *stream, const uint32_t *d_indices, const void *
  * row tiles in two MFMA launches: route_partials[(token * top_k + rank) * d ..] =
  * fp16(down . fp16(glu(gate . x, up . x))) for every pair of a resident expert.
  * hidden: fp16[query_count, hidden_stride_elements]. d_workspace: caller-owned, at least
- * shrike_hip_prefill_ffn_workspace_bytes(). Tiles of absent experts are skipped (their
+ * shrike_hip_prefill_ffn_workspace_bytes(). max_row_tiles bounds the table's count; it may exceed what these pairs can
+ * need (one bound for several chunks). Tiles of absent experts are skipped (their
  * partial rows are left untouched).
  * Which bits: a pair's row depends on its token, its expert and on the kernel that query_count * top_k, the handle's
  * experts and widths and f choose, not on the rows beside it, and a call over a range of the pairs

@@ -2,17 +2,10 @@
 // grouping kernels write and the grouped FFN reads.
 #pragma once
 
+#include "ffn_rules.h"
 #include "gemv_common.h"
 
 namespace shrike {
-
-constexpr uint32_t kRowTile = 64;  // rows per row-tile entry (PrefillGroupedRoutedMoE.groupedRowTile)
-
-// Worst case of row tiles for `pairs` pairs over `experts` experts: every expert may end
-// in a partly filled tile.
-inline uint32_t max_row_tiles(uint64_t pairs, uint32_t experts) {
-    return uint32_t(pairs / kRowTile) + experts;
-}
 
 // fp16 halves of an fp32 value: hi + lo reproduces it to about 2^-22 relative
 __device__ __forceinline__ uint32_t split_hi_lo(float v) {

@@ -3,11 +3,16 @@ benchmark definition, and device/oracle runners over the same bytes."""
 from __future__ import annotations
 
 import ctypes as C
+import functools
+import os
+import subprocess
+import tempfile
 
 import numpy as np
 
 from oracle import oracle as O
 from shrike_amd import synth as S
+from tests.conftest import ROOT
 
 ABS_TOL, REL_TOL = 2e-3, 1e-3   # FFN outputs: max-abs 2e-3 / relative 1e-3 (benchmark definition)
 
@@ -79,3 +84,19 @@ class Layer:
         return dict(weights=self.router_w, scales=self.router_s, biases=self.router_b,
                     kind=self.router_bits, eff_scale=self.eff_scale, expert_scale=self.expert_scale,
                     bias=self.logit_bias, meta=self.meta)
+
+
+@functools.lru_cache(maxsize=None)
+def ffn_rules() -> C.CDLL:
+    """csrc/ffn_rules.h, compiled for the host."""
+    with tempfile.TemporaryDirectory() as where:
+        lib = os.path.join(where, "rules.so")
+        source = """
+#include "ffn_rules.h"
+extern "C" uint32_t readable_records(uint32_t bound, uint64_t pairs, uint32_t experts) { return shrike::readable_records(bound, pairs, experts); }
+"""
+        subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/shrike_amd/csrc", "-x", "c++", "-", "-o", lib],
+                       input=source.encode(), check=True)
+        rules = C.CDLL(lib)
+    rules.readable_records.argtypes, rules.readable_records.restype = [C.c_uint32, C.c_uint64, C.c_uint32], C.c_uint32
+    return rules

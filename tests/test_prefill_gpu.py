@@ -419,6 +419,28 @@ def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out):
                 pc.check_pair(got[:, None], int(tok), 0, f"tile {i} token {tok}")
 
 
+@pytest.mark.parametrize("d,f,ne,t,bits", [(192, 2048, 16, 40, 4), (512, 512, 200, 60, 8)])  # up to 64 tiles, and more
+def test_grouped_ffn_of_a_table_shorter_than_the_bound(gpu, d, f, ne, t, bits):
+    """One bound and one workspace for several chunks: this chunk's table has room for its own tiles only, at the end of its memory."""
+    k = 2
+    L = Layer(0x5EED0900 + ne, d, f, ne, k, bits=bits)
+    pc = PrefillCase(gpu, L, t)
+    want = pc.run()
+    records = pc.routes.row_tiles.download(np.uint32, 4 * pc.routes.max_row_tiles)
+    memory = gpu.empty(1 << 21)
+    table_at = memory.ptr + (1 << 21) - records.nbytes
+    memory.upload(records.view(np.uint8), offset=(1 << 21) - records.nbytes)
+    routes = capi.HipGroupedRoutes.from_buffer_copy(pc.routes.c)
+    routes.row_tiles = table_at
+    bound = 4 * pc.routes.max_row_tiles
+    pc.routes.c = routes
+    pc.partials = gpu.dev(np.full(t * k * d, 0xD4D0, np.uint16))
+    pc.ws = gpu.empty(pc.pf.ffn_workspace_bytes(t, bound))
+    pc.pf.encode_grouped_expert_gemms(pc.dl.pool, pc.dl.off, pc.routes, pc.hidden, pc.stride, pc.partials, pc.ws, t, k, max_row_tiles=bound)
+    gpu.synchronize()
+    assert np.array_equal(pc.partials.download(np.uint16, t * k * d).reshape(t, k, d), want)
+
+
 @pytest.mark.parametrize("d,f,ne,bits,chunks,split", [
     (512, 4096, 12, 4, (90, 400, 2900), ()),     # one and two row tiles a workgroup
     (512, 1024, 40, 8, (150, 1000, 2000), ()),   # 8-bit codes: two groups ahead, one, two row tiles
