@@ -778,8 +778,14 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
             // among the first ones of its XCD's run, so that the workgroups without a tile are the last ones. Where every tile had
             // its workgroups and those of the second ones left at once, the compute units did not fill evenly: 32 experts of
             // 2,880 x 2,880, 2,048 tokens 500 -> 483 us, 700 tokens 224 -> 217 (with the two tiles' workgroups in turn 680 and 318).
-            // Where few tiles fill the XCD's places, those of more than 64 rows go ahead of the others of the same 64 records (497
-            // without that; 256 experts of 2,304 x 1,024, 8 column blocks a tile, 4,000 tokens 716 in the table's order, 758 so).
+            // Within each 64 records the experts of one tile go last: the workgroups that start late are then the short ones (uneven
+            // experts, both products, in the table's order against this: 64 of 2,048 x 512, 8-bit, 2,000 tokens 164 -> 160 us, 32 of
+            // 2,880 x 2,880, 8-bit, 1,000 tokens 423 -> 398, 48 of 2,816 x 1,408, 4-bit, 1,500 tokens 277 -> 271).
+            // What is left over of a longer expert stays behind that expert's other tiles, whose codes the L2 then has. Left-overs
+            // last as well, against this: 256 even experts of 2,304 x 1,024, 8-bit, 4,000 tokens 766, 713 us; 256 of 2,048 x 512,
+            // 4-bit, 4,096 tokens, whole pass 491, 475; 128 of 3,072 x 1,024, 8-bit, 2,000 tokens 514, 492; 32 of 3,072 x 2,048, 8-bit,
+            // 700 tokens 369, 351; but 32 of 2,880 x 2,880, 4-bit, 2,048 tokens 478, 490 and 48 of 2,816 x 1,408, 4-bit 263, 279:
+            // the short ones fill the end there. Over 29 shapes the two come to the same; the larger losses are last's.
             auto continues = [&](const uint4 &rec, const uint4 &before) {
                 return rec.w == before.w && rec.x == before.x && before.z == kRowTile && rec.y == before.y + kRowTile;
             };
@@ -804,7 +810,7 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
                 const uint32_t from = 63u - uint32_t(__clzll((long long)breaks)), mine_ahead = lane - from + (from == 0u ? ahead : 0u);
                 const bool is_first = at + lane < first + run && (mine_ahead & 1u) == 0u;
                 const uint32_t rows = rec.z + (goes_on ? next.z : 0u);
-                const bool is_heavy = column_blocks < 12u || rows > kRowTile;
+                const bool is_heavy = rows > kRowTile || mine_ahead != 0u;
                 const uint64_t heavy = __ballot(is_first && is_heavy), light = __ballot(is_first && !is_heavy);
                 const uint32_t heavies = uint32_t(__popcll(heavy)), firsts = heavies + uint32_t(__popcll(light));
                 if (rank < firsts) {
