@@ -12,7 +12,7 @@
 // the group biases.
 //
 // Two kernels: k_grouped_ffn gives a workgroup a row tile (or two) and a block of weight rows, k_ffn_split a smaller piece
-// whose k its waves share; routed_shape and dense_shape choose.
+// whose k its waves share; routed_shape and dense_shape (ffn_rules.h) choose.
 #include "decode_launch.h"
 #include "prefill_common.h"
 
@@ -26,14 +26,8 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// ---- the shape of a workgroup's work and its LDS: a ring of places for groups of the rows and one for 64-byte units of the
+// ---- the LDS of a workgroup of each shape: a ring of places for groups of the rows and one for 64-byte units of the
 // codes, that asynchronous loads fill (lane l's piece of a load lands 16 l bytes behind the load's address).
-enum class FfnShape {
-    kSplit,  // up to 32 rows against 64 weight rows, a quarter of k a wave (k_ffn_split)
-    kTile,   // one row tile, up to 64 rows, against 256 weight rows, 4-bit codes; three workgroups a compute unit
-    kDeep,   // the same with more groups on their way; two workgroups a compute unit
-    kWide,   // two row tiles of one expert, up to 128 rows, against 256 weight rows; two workgroups a compute unit
-};
 constexpr uint32_t kUnitB = 64u * 64u;  // 64 bytes of codes of a wave's 64 weight rows: two groups at 4 bits, one at 8
 constexpr uint32_t kUnitS = 64u * 16u;  // four groups' scales (biases) of those rows, in a 12-byte window each
 template <FfnShape S, int BITS>
@@ -1223,45 +1217,6 @@ using namespace shrike;
 extern "C" {
 size_t shrike_hip_prefill_ffn_workspace_bytes(uint32_t query_count, uint32_t max_row_tiles, uint32_t d, uint32_t f) {
     return workspace_layout(query_count, max_row_tiles, d, f).total;
-}
-
-// The shape of the routed products, from what the host knows (and what a call over a range of the pairs shares with the call
-// over all of them: their outputs are the same bytes).
-//  - kSplit up to 1,024 pieces of its gate/up launch, two for each of the 512 workgroups it keeps: with 16 experts of
-//    1,536 x 1,024 it takes 21 us for 16 tokens where one row tile a workgroup takes 30, and 24.6 against 37.9 for 100 (8-bit
-//    codes). Past that it loses: its pieces are short and none of them overlaps the next in its workgroup (256 experts of 2,048
-//    x 512, 128 tokens: 150 against 126 us).
-//  - kWide where the experts' rows fill its tiles and its launch still has several workgroups for every compute unit; its loop
-//    is the most products an unpacked code, its start and end the longest, so k must not be short. kWide against kTile or
-//    kDeep, us (pairs an expert; row tiles by column blocks of the gate/up launch):
-//      8 bits   256 experts of 2,304 x 1,024: 447, 442 (44; 1,368), 502, 613 (62; 2,000); 32 of 2,880 x 2,880: 294, 315 (62; 713);
-//               128 of 1,024 x 512: 73, 81 (70; 560); 100 of 1,024 x 512, uneven: 55, 57 (80; 500); 64 of 2,048 x 512: 92, 92 (87; 348);
-//               32 of 1,024 x 1,024: 55, 48 (75; 296); 64 of 512 x 256: 67, 60 (500; 1,000)
-//      4 bits, kWide against the better of the others, even and uneven experts (pairs an expert; workgroups times groups of both k):
-//               64 of 1,088 x 1,664: 108, 117 and 107, 93 (79; 44 k); 128 of 2,048 x 768: 162, 175 and 167, 155 (75; 40 k); 256 of
-//               2,048 x 512: 189, 199 and 162, 154 (62; 40 k), 232, 258 and 216, 212 (94; 60 k); 48 of 3,072 x 1,536, uneven: 182, 188
-//               (75; 49 k); 256 of 1,536 x 1,280, uneven: 255, 257 (62; 110 k); 32 of 2,880 x 2,880: 183, 173 (50; 52 k), 210, 222 (62;
-//               65 k), 219, 259 (87; 89 k). The line lies where uneven experts stop losing.
-//  - kTile for 4-bit codes but for the longest k, kDeep for the others. kTile's third workgroup a compute unit hides the start and
-//    the end of the short ones, kDeep's loads start earlier: 32 experts of 2,880 x 2,880, 400 tokens 186 against 173 us; 128 of 3,072 x
-//    768, 512 uneven tokens 107 against 113; 48 of 3,072 x 1,536, 900 uneven ones 188 against 199, 64 of 1,280 x 2,048, 700 even ones
-//    106 against 104, uneven 91 against 95; 256 of 2,048 x 512, 512 uneven ones (129 tiles of 64 rows: more workgroups than kDeep
-//    has places for) 71 against 76. Three workgroups with 8-bit codes leave their loads one group ahead: 256 experts of 2,304 x
-//    1,024, 1,000 tokens 469 against 439.
-static FfnShape routed_shape(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits) {
-    const uint64_t most_tiles = min(pairs, uint64_t(experts)) + pairs / kRowTile;
-    if (most_tiles * (f / 32u) <= 1024u) return FfnShape::kSplit;
-    const uint64_t workgroups = pairs / kRowTile * ((f + 127u) / 128u);
-    if (bits == 8 ? pairs >= 48u * uint64_t(experts) && workgroups >= 450u && d + f >= 1536u
-                  : pairs >= 56u * uint64_t(experts) && workgroups * ((d + f) / kGroup) >= 46000u && d + f >= 2048u)
-        return FfnShape::kWide;
-    return bits == 4 && d + f < 5120u ? FfnShape::kTile : FfnShape::kDeep;
-}
-// ... and of a dense expert's, whose rows are its tiles: kSplit up to two pieces a workgroup (2,048 x 512, 4-bit: 13 against
-// 45 us for 37 rows, 16 against 48 for 512, 32 against 47 for 1,500; 2,304 x 1,024, 8-bit: 44 against 54 for 1,000), kDeep
-// past that (57 against 79 us for 4,096 rows).
-static FfnShape dense_shape(uint64_t rows, uint32_t f) {
-    return (rows + 31u) / 32u * (f / 32u) <= 1024u ? FfnShape::kSplit : FfnShape::kDeep;
 }
 
 static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_bases *pool, uint64_t pool_slot_stride,

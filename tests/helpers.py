@@ -94,9 +94,14 @@ def ffn_rules() -> C.CDLL:
         source = """
 #include "ffn_rules.h"
 extern "C" uint32_t readable_records(uint32_t bound, uint64_t pairs, uint32_t experts) { return shrike::readable_records(bound, pairs, experts); }
+extern "C" const char *routed_shape(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits) {
+    static const char *const names[] = {"split", "tile", "deep", "wide"};
+    return names[int(shrike::routed_shape(pairs, experts, d, f, bits))];
+}
 """
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/shrike_amd/csrc", "-x", "c++", "-", "-o", lib],
                        input=source.encode(), check=True)
         rules = C.CDLL(lib)
     rules.readable_records.argtypes, rules.readable_records.restype = [C.c_uint32, C.c_uint64, C.c_uint32], C.c_uint32
+    rules.routed_shape.argtypes, rules.routed_shape.restype = [C.c_uint64, *[C.c_uint32] * 4], C.c_char_p
     return rules

@@ -2,6 +2,7 @@
 import pytest
 
 from shrike_amd import capi
+from tests import test_prefill_gpu as T
 from tests.helpers import ffn_rules
 
 
@@ -13,3 +14,13 @@ def test_no_record_is_read_past_the_tables_room(tokens, top_k, experts):
     for bound in (1, room - 1, room, room + 1, room + 1000, 0xffffffff):
         if bound:
             assert ffn_rules().readable_records(bound, pairs, experts) == min(bound, room)
+
+
+@pytest.mark.parametrize("pairs,experts,d,f,bits,shape", [
+    *[(k * t, ne, d, f, bits, shape) for d, f, ne, k, t, bits, _, shape in T.SHAPE_CASES],
+    *[(4 * t, ne, d, f, bits, shape) for d, f, ne, t, bits, shape in T.RING_CASES + T.WIDE_EPILOGUE_CASES],
+    *[(2 * t, ne, d, f, bits, shape) for d, f, ne, t, bits, shape in T.TABLE_CASES],
+    *[(sum(counts), len(counts), d, f, bits, shape) for counts, _, d, f, bits, shape in T.HOLE_CASES],
+    *[(t, ne, d, f, bits, shape) for d, f, ne, bits, chunks in T.CHUNK_CASES for t, shape in chunks.items()]])
+def test_the_gpu_tests_reach_the_shapes_they_name(pairs, experts, d, f, bits, shape):
+    assert ffn_rules().routed_shape(pairs, experts, d, f, bits).decode() == shape

@@ -255,11 +255,13 @@ class WorkspaceActs:
 
 
 class PrefillCase:
-    def __init__(self, gpu, L: Layer, t, stride_pad=0, idx=None, moe_kwargs=None, resident=None):
+    def __init__(self, gpu, L: Layer, t, stride_pad=0, idx=None, moe_kwargs=None, resident=None, scale=1.0):
         self.gpu, self.L, self.t = gpu, L, t
         self.dl = DeviceLayer(gpu, L, moe_kwargs=moe_kwargs, resident=resident)
         self.stride = L.d + stride_pad
         self.x = token_rows(L, t, self.stride)
+        if scale != 1.0:
+            self.x = S.f32_to_f16_bits(f16(self.x) * np.float32(scale))
         self.hidden = gpu.dev(self.x)
         self.pf = gpu.Prefill(self.dl.moe)
         if idx is None:
@@ -345,19 +347,32 @@ def test_grouped_ffn_shape_sweep(gpu, case):
     assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
 
 
-@pytest.mark.parametrize("d,f,ne,k,t,bits,meta", [
+def row_scale(d, f):
+    """Of rows so long that N(0, 1) inputs make outputs of 75: a partial row is then a sum of products that come to 4,000 to 5,000
+    in magnitude, of which fp32 keeps 2^-24 = 3e-4 a step, and where it cancels, two orders of addition differ by more than the
+    2e-3 that is stated for outputs of order 1. An eighth of the inputs gives those (gate, up and so their product: a 64th)."""
+    return 0.125 if d >= 2048 and f >= 1152 else 1.0
+
+
+# The cases name the shape that the FFN's products take, which ffn_rules.h chooses (test_ffn_rules.py asks it).
+SHAPE_CASES = [  # d, f, experts, k, tokens, bits, meta, shape
     # k over the waves: one group and one stage in all, a quarter without any, 9 to 16 rows and two pieces of a row tile,
     # groups that no quarter shares evenly
-    (64, 64, 3, 2, 20, 4, S.META_BF16), (128, 192, 2, 1, 45, 8, S.META_F16), (2880, 64, 4, 2, 50, 4, S.META_F16),
+    (64, 64, 3, 2, 20, 4, S.META_BF16, "split"), (128, 192, 2, 1, 45, 8, S.META_F16, "split"), (2880, 64, 4, 2, 50, 4, S.META_F16, "split"),
     # one row tile a workgroup: fewer than eight groups and more than sixty-four, both odd
-    (192, 4160, 6, 2, 70, 4, S.META_BF16), (192, 1088, 24, 4, 120, 8, S.META_F16),
-    # the same two groups ahead: one group, two, and odd many
-    (64, 4096, 9, 2, 12, 8, S.META_BF16), (128, 4096, 9, 2, 70, 8, S.META_F16), (4032, 1088, 40, 3, 33, 8, S.META_F16),
+    (192, 4160, 6, 2, 70, 4, S.META_BF16, "tile"), (192, 1088, 24, 4, 120, 8, S.META_F16, "deep"),
+    # the same with more groups ahead: one group, two, and odd many
+    (64, 4096, 9, 2, 12, 8, S.META_BF16, "deep"), (128, 4096, 9, 2, 70, 8, S.META_F16, "deep"), (4032, 1088, 40, 3, 33, 8, S.META_F16, "deep"),
+    (960, 832, 24, 4, 300, 8, S.META_BF16, "deep"), (4032, 1152, 40, 3, 33, 4, S.META_F16, "deep"), (64, 5184, 9, 2, 70, 4, S.META_BF16, "deep"),
     # two row tiles of an expert a workgroup: 128 rows and what is left over, odd groups, column blocks that end inside it
-    (128, 8192, 6, 4, 360, 4, S.META_BF16), (576, 3008, 8, 4, 960, 4, S.META_F16), (960, 832, 24, 4, 300, 8, S.META_BF16)])
+    (128, 8192, 6, 4, 360, 4, S.META_BF16, "wide"), (576, 3008, 8, 4, 960, 4, S.META_F16, "wide"), (960, 832, 24, 4, 1050, 8, S.META_BF16, "wide"),
+    (192, 1344, 24, 4, 700, 8, S.META_F16, "wide")]
+
+
+@pytest.mark.parametrize("d,f,ne,k,t,bits,meta", [c[:-1] for c in SHAPE_CASES])
 def test_grouped_ffn_shapes_of_a_workgroup(gpu, d, f, ne, k, t, bits, meta):
     L = Layer(0x5EED0400 + d + f, d, f, ne, k, bits=bits, meta=meta)
-    pc = PrefillCase(gpu, L, t, stride_pad=8, resident=[e for e in range(ne) if e != 1])
+    pc = PrefillCase(gpu, L, t, stride_pad=8, resident=[e for e in range(ne) if e != 1], scale=row_scale(d, f))
     got = pc.run()
     here = pc.idx.reshape(t, k) != 1
     assert np.all(got[~here] == 0xD4D0), "an absent expert's row was written"
@@ -367,16 +382,23 @@ def test_grouped_ffn_shapes_of_a_workgroup(gpu, d, f, ne, k, t, bits, meta):
         pc.check_pair(got, int(tok), int(rank), f"token {tok} rank {rank}")
 
 
-@pytest.mark.parametrize("d,f,ne,t,bits", [
-    # groups of 64 in k around the four that the loop takes at once and the places of its rings, of both products; experts of up
-    # to 32 rows, up to 64 and, in the last three, of two row tiles; more than 64 tiles, so that none is cut in two
-    (448, 576, 70, 700, 4), (512, 704, 70, 700, 4), (832, 1408, 70, 700, 4),
-    (576, 1600, 70, 700, 4), (704, 1536, 70, 700, 4), (768, 1664, 70, 700, 4),
-    (448, 576, 70, 700, 8), (512, 704, 70, 700, 8), (832, 768, 70, 700, 8),
-    (448, 576, 70, 1000, 8), (704, 1408, 70, 1000, 8), (512, 4096, 30, 500, 4)])
+# Groups of 64 in k around the four that the loop takes at once and the places of each shape's rings, of both products; experts of
+# up to 32 rows, up to 64 and, where two tiles are one workgroup's, more; more than 64 tiles, or too many workgroups, so that none
+# is cut in two.
+RING_CASES = [  # d, f, experts, tokens, bits, shape
+    (448, 576, 70, 700, 4, "tile"), (512, 704, 70, 700, 4, "tile"), (832, 1408, 70, 700, 4, "tile"),
+    (576, 1600, 70, 700, 4, "tile"), (704, 1536, 70, 700, 4, "tile"), (768, 1664, 70, 700, 4, "tile"),
+    (448, 576, 70, 700, 8, "deep"), (512, 704, 70, 700, 8, "deep"), (832, 768, 70, 700, 8, "deep"), (448, 576, 70, 1000, 8, "deep"),
+    (2816, 2304, 8, 450, 4, "deep"), (2624, 2496, 8, 450, 4, "deep"), (2688, 2432, 8, 450, 4, "deep"),
+    (576, 4672, 8, 160, 4, "deep"), (448, 4800, 8, 160, 4, "deep"),
+    (704, 1408, 70, 1000, 8, "wide"), (512, 1024, 20, 920, 8, "wide"), (832, 704, 20, 1200, 8, "wide"), (576, 960, 20, 920, 8, "wide"),
+    (512, 4096, 30, 500, 4, "wide"), (832, 3136, 16, 480, 4, "wide"), (1472, 1600, 20, 1190, 4, "wide"), (640, 2880, 16, 620, 4, "wide")]
+
+
+@pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in RING_CASES])
 def test_grouped_ffn_rings(gpu, d, f, ne, t, bits):
     L = Layer(0x5EED0700 + d + f, d, f, ne, 4, bits=bits, meta=S.META_F16 if f % 128 else S.META_BF16)
-    pc = PrefillCase(gpu, L, t)
+    pc = PrefillCase(gpu, L, t, scale=row_scale(d, f))
     got = pc.run()
     assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
     for pair in np.random.default_rng(12).choice(t * 4, 40, replace=False):
@@ -397,13 +419,22 @@ def test_grouped_ffn_of_few_larger_tiles(gpu, d, f, bits, meta):
             pc.check_pair(got, int(tokens[r]), 0, f"expert {e} row {r}")
 
 
-@pytest.mark.parametrize("counts,out", [([200, 330] + [30] * 22, [1, 6]), ([4200, 200, 300, 100], [68])])
-def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out):
+HOLE_CASES = [  # pairs of each expert, tiles left out of the table, d, f, bits, shape
+    ([200, 330] + [30] * 22, [1, 6], 192, 896, 8, "deep"), ([4200, 200, 300, 100], [68], 192, 896, 8, "deep"),
+    ([200, 330] + [170] * 22, [1, 6], 640, 896, 8, "wide"), ([4200, 200, 300, 100], [68], 640, 896, 8, "wide"),
+    # an expert's first tile, its last, two neighbours and every second one; 4-bit codes
+    ([700, 130, 260, 70, 500, 1] + [190] * 6, [0, 10, 15, 16, 22, 24, 26], 448, 2944, 4, "wide"),
+    # over 64 tiles an XCD, experts that run from one XCD's into the next and over several 64s of records, in odd and even numbers
+    ([9000, 64, 129, 65, 63] + [128, 1, 193, 33] * 40 + [12345, 100, 20, 6400], [70, 150, 151, 500], 128, 1408, 8, "wide")]
+
+
+@pytest.mark.parametrize("counts,out,d,f,bits", [c[:-1] for c in HOLE_CASES], ids=[f"{c[5]}-{len(c[0])}-{c[4]}" for c in HOLE_CASES])
+def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out, d, f, bits):
     """Two row tiles a workgroup are two that continue each other, not any two neighbours of the table: tiles inside an expert's
     left out; an expert of more tiles than a wave reads at once."""
     ne = len(counts)
     idx = np.random.default_rng(10).permutation(np.repeat(np.arange(ne), counts)).astype(np.uint32)
-    pc = PrefillCase(gpu, Layer(0x5EED0600, 192, 896, ne, 1, bits=8, meta=S.META_BF16), len(idx), idx=idx)
+    pc = PrefillCase(gpu, Layer(0x5EED0600, d, f, ne, 1, bits=bits, meta=S.META_BF16), len(idx), idx=idx)
     table = pc.routes.download()["row_tiles"]
     kept = np.delete(table, out, axis=0)
     pc.routes.row_tiles.upload(np.ascontiguousarray(kept))
@@ -414,12 +445,16 @@ def test_grouped_ffn_takes_a_table_that_leaves_tiles_out(gpu, counts, out):
         tokens = pair_tokens[start:start + rows]
         written = ~np.all(got[tokens] == 0xD4D0, axis=-1)
         assert np.all(written == (i not in out)), f"tile {i} of expert {expert}: {written.sum()} of {rows} rows written"
-        if i not in out and (i < 10 or 60 < i < 70):
+        if i not in out and (i < 10 or 60 < i < 70 or min(abs(i - o) for o in out) <= 2):
             for tok in tokens[[0, -1]]:
                 pc.check_pair(got[:, None], int(tok), 0, f"tile {i} token {tok}")
 
 
-@pytest.mark.parametrize("d,f,ne,t,bits", [(192, 2048, 16, 40, 4), (512, 512, 200, 60, 8)])  # up to 64 tiles, and more
+TABLE_CASES = [  # d, f, experts, tokens, bits, shape; up to 64 tiles, and more
+    (192, 2048, 16, 40, 4, "tile"), (512, 512, 200, 60, 8, "deep")]
+
+
+@pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in TABLE_CASES])
 def test_grouped_ffn_of_a_table_shorter_than_the_bound(gpu, d, f, ne, t, bits):
     """One bound and one workspace for several chunks: this chunk's table has room for its own tiles only, at the end of its memory."""
     k = 2
@@ -441,12 +476,13 @@ def test_grouped_ffn_of_a_table_shorter_than_the_bound(gpu, d, f, ne, t, bits):
     assert np.array_equal(pc.partials.download(np.uint16, t * k * d).reshape(t, k, d), want)
 
 
-@pytest.mark.parametrize("d,f,ne,bits,chunks,split", [
-    (512, 4096, 12, 4, (90, 400, 2900), ()),     # one and two row tiles a workgroup
-    (512, 1024, 40, 8, (150, 1000, 2000), ()),   # 8-bit codes: two groups ahead, one, two row tiles
-    (512, 512, 12, 4, (13, 40), (13, 40)),       # k over the waves
-    (512, 2048, 12, 4, (40, 400), (40,))])       # ... in the shorter chunk
-def test_a_row_of_the_ffn_over_chunks_of_different_lengths(gpu, d, f, ne, bits, chunks, split):
+CHUNK_CASES = [  # d, f, experts, bits, tokens and their shape
+    (512, 4096, 12, 4, {90: "tile", 400: "tile", 2900: "wide"}), (512, 1024, 40, 8, {150: "deep", 1000: "deep", 2000: "deep", 3700: "wide"}),
+    (512, 512, 12, 4, {13: "split", 40: "split"}), (512, 2048, 12, 4, {40: "split", 400: "tile"})]
+
+
+@pytest.mark.parametrize("d,f,ne,bits,chunks", CHUNK_CASES)
+def test_a_row_of_the_ffn_over_chunks_of_different_lengths(gpu, d, f, ne, bits, chunks):
     """The same bytes where in both chunks one wave sums all of k, or four waves a quarter each; else the end-to-end bound (the
     sums' rounding moves fp16 activations by their last place)."""
     first = min(chunks)
@@ -459,7 +495,7 @@ def test_a_row_of_the_ffn_over_chunks_of_different_lengths(gpu, d, f, ne, bits, 
         pc.hidden = gpu.dev(x[:t * d])
         rows[t] = pc.run()[:first, 0]
     for t in chunks:
-        if (t in split) == (first in split):
+        if (chunks[t] == "split") == (chunks[first] == "split"):
             assert np.array_equal(rows[t], rows[first]), f"{t} tokens against {first}"
         else:
             assert_rel_close(rows[t].reshape(-1), rows[first].reshape(-1), f"{t} tokens against {first}")
@@ -496,6 +532,20 @@ def test_grouped_ffn_gpt_oss_epilogues(gpu):
     for tok in range(5):
         for rank in range(2):
             pc.check_pair(got, tok, rank, f"gpt-oss token {tok} rank {rank}", O.ACT_CLAMPED_SWIGLU)
+
+
+WIDE_EPILOGUE_CASES = [  # d, f, experts, tokens, bits, shape
+    (2880, 2880, 8, 370, 4, "wide"), (960, 832, 24, 1050, 8, "wide")]
+
+
+@pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in WIDE_EPILOGUE_CASES])
+def test_grouped_ffn_gpt_oss_epilogues_with_two_tiles_a_workgroup(gpu, d, f, ne, t, bits):
+    L = Layer(0x5EED0A04, d, f, ne, 4, bits=bits, additive_biases=True)
+    pc = PrefillCase(gpu, L, t, moe_kwargs=dict(activation=capi.ACT_CLAMPED_SWIGLU, additive_biases=True), scale=row_scale(d, f))
+    got = pc.run()
+    assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
+    for pair in np.random.default_rng(13).choice(t * 4, 24, replace=False):
+        pc.check_pair(got, int(pair) // 4, int(pair) % 4, f"pair {pair}", O.ACT_CLAMPED_SWIGLU)
 
 
 @pytest.mark.parametrize("d,f,ne,k,t,bits", [(512, 256, 6, 2, 70, 4), (320, 192, 5, 3, 21, 8)])
