@@ -80,7 +80,8 @@ void gemv_rows_scalar(const uint8_t *weights, const uint16_t *scales, const uint
 // for all rows (each the very product the scalar loop forms), and a row's code picks its product by a permute, which
 // reads the low four bits of its index lane alone: per sixteen rows and byte of codes two shifts, two permutes, two
 // additions and 0.8 of a shuffle. One expert of 2048 x 512 (1.77 MB) on one core of an EPYC with 512-bit pipes:
-// 591 us row by row (3.0 GB/s), so 82 us from the caches and 105 to 120 from DRAM (15 to 17 GB/s, by the machine); 2880 x
+// 591 us row by row (3.0 GB/s), so 82 us from the caches and 105 to 120 from DRAM (by the machine; reading the bytes and nothing
+// else takes that core 38 us from DRAM, 11 from the third-level cache: the instructions bound it, not the memory); 2880 x
 // 2880: 4,643 us, and 585 and 815 to 860. (Tables of eight groups, which fit the first-level cache, have every row visited in
 // shorter pieces: 114 and 1,137 us from DRAM where these took 108 and 815; a table over the whole row: 126 and 793.)
 #define SHRIKE_AVX512 __attribute__((target("avx512f,avx512bw,avx512vl")))

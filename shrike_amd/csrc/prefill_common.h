@@ -31,7 +31,9 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_u32(uint32_t v, uint32_t
 }
 
 // Asynchronous loads into LDS. The compiler does not know of them: the waits for them are counted by hand, and nothing
-// between the first and the last of them may make it issue a vector load of its own. The LDS address goes in m0, which the
+// between the first and the last of them should make it issue a vector load of its own. (One more load on its way makes a
+// counted wait last longer, never end sooner, loads landing in order; but the wait for that load is for all of them. So it is
+// where the loop of kWide reloads a spilled register, with 8-bit codes, twice in four groups.) The LDS address goes in m0, which the
 // compiler sets as the operand it is there: a write of m0 inside the assembly would be one that it does not know of either,
 // and its own uses of m0 on both sides would take each other's value for still there.
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {

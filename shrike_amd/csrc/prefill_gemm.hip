@@ -148,9 +148,10 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // loop is a pipeline: between the MFMAs of chain c stand the scaling of chain c - 1, a share of the next codes' unpacking and
 // the reads of the rows that the next chain takes, and the wait for the next group's loads stands two chains ahead of their
 // use. What bounds it now: with many rows the power that matrix work, its operands' way through LDS and the loads take
-// together (the kWide gate/up launch over 2,048 gpt-oss tokens runs at 1.9 GHz of 2.4, the matrix pipe busy 49 % of the
-// cycles, vector issue 47 %); with few rows the weights' bytes (kDeep, 8-bit, 1,000 tokens: 4.4 TB/s), and the start and the end of the many
-// short workgroups (30 of 75 us at 256 experts of 2,048 x 512 and 512 tokens). Both products, a chain scaled where it ends ->
+// together (2,048 gpt-oss tokens back to back: the clock at 1.95 GHz of 2.4; the kWide gate/up launch keeps the matrix pipe
+// busy 44 % of the cycles, vector issue 43 %); with few rows the weights' bytes (kDeep, 8-bit, 1,000 tokens: 4.4 TB/s), and the start and
+// the end of the many short workgroups (256 experts of 2,048 x 512, 512 tokens: 29 % of the workgroups' time in gate/up and 53 % in
+// down lie outside the loop, 27 of 69 us; 37 tokens: 29 and 56 %). Both products, a chain scaled where it ends ->
 // pipelined: 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens 540 -> 495 us, 300 tokens 179 -> 164; 256 of 2,048 x 512, 4,096
 // tokens 316 -> 302, 37 33.5 -> 31.4; 256 of 2,304 x 1,024, 8-bit, 1,000 tokens 469 -> 439, 4,000 735 -> 710.
 //
