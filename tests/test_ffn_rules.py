@@ -18,7 +18,7 @@ def test_no_record_is_read_past_the_tables_room(tokens, top_k, experts):
 
 @pytest.mark.parametrize("pairs,experts,d,f,bits,shape", [
     *[(k * t, ne, d, f, bits, shape) for d, f, ne, k, t, bits, _, shape in T.SHAPE_CASES],
-    *[(4 * t, ne, d, f, bits, shape) for d, f, ne, t, bits, shape in T.RING_CASES + T.WIDE_EPILOGUE_CASES],
+    *[(4 * t, ne, d, f, bits, shape) for d, f, ne, t, bits, shape in T.RING_CASES + T.EPILOGUE_CASES + T.RANGE_CASES],
     *[(2 * t, ne, d, f, bits, shape) for d, f, ne, t, bits, shape in T.TABLE_CASES],
     *[(sum(counts), len(counts), d, f, bits, shape) for counts, _, d, f, bits, shape in T.HOLE_CASES],
     *[(t, ne, d, f, bits, shape) for d, f, ne, bits, chunks in T.CHUNK_CASES for t, shape in chunks.items()]])

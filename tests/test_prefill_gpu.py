@@ -534,12 +534,13 @@ def test_grouped_ffn_gpt_oss_epilogues(gpu):
             pc.check_pair(got, tok, rank, f"gpt-oss token {tok} rank {rank}", O.ACT_CLAMPED_SWIGLU)
 
 
-WIDE_EPILOGUE_CASES = [  # d, f, experts, tokens, bits, shape
-    (2880, 2880, 8, 370, 4, "wide"), (960, 832, 24, 1050, 8, "wide")]
+EPILOGUE_CASES = [  # d, f, experts, tokens, bits, shape; the additive biases stand in each shape's own order of a tile's columns
+    (2880, 2880, 8, 370, 4, "wide"), (960, 832, 24, 1050, 8, "wide"),
+    (832, 1408, 70, 700, 4, "tile"), (2880, 2880, 8, 160, 4, "deep"), (832, 768, 70, 700, 8, "deep")]
 
 
-@pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in WIDE_EPILOGUE_CASES])
-def test_grouped_ffn_gpt_oss_epilogues_with_two_tiles_a_workgroup(gpu, d, f, ne, t, bits):
+@pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in EPILOGUE_CASES])
+def test_grouped_ffn_gpt_oss_epilogues_of_each_shape(gpu, d, f, ne, t, bits):
     L = Layer(0x5EED0A04, d, f, ne, 4, bits=bits, additive_biases=True)
     pc = PrefillCase(gpu, L, t, moe_kwargs=dict(activation=capi.ACT_CLAMPED_SWIGLU, additive_biases=True), scale=row_scale(d, f))
     got = pc.run()
@@ -638,6 +639,32 @@ def test_streamed_batched_over_pair_ranges_equals_the_whole_chunk(gpu, bits, til
     with pytest.raises(capi.ShrikeError):
         cut.pf.encode_streamed_batched(cut.dl.pool, cut.dl.off, cut.routes, cut.hidden, cut.stride, cut.partials, cut.ws,
                                        t, k, t * k - 3, 4)
+
+
+RANGE_CASES = [  # d, f, experts, tokens, bits, shape
+    (448, 576, 70, 700, 4, "tile"), (576, 4672, 8, 160, 4, "deep"), (448, 576, 70, 700, 8, "deep"), (640, 2880, 16, 620, 4, "wide"),
+    (576, 960, 20, 920, 8, "wide")]
+
+
+@pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in RANGE_CASES])
+def test_pair_ranges_of_each_shape_equal_the_whole_chunk(gpu, d, f, ne, t, bits):
+    """Ranges that start and end inside row tiles, one of a single pair and one to the chunk's end: their pairs' rows are the whole
+    call's bytes, and no others are written."""
+    k = 4
+    L = Layer(0x5EED0B00 + d, d, f, ne, k, bits=bits)
+    pc = PrefillCase(gpu, L, t, scale=row_scale(d, f))
+    want = pc.run()
+    order = pc.routes.download()["sorted_pairs"].astype(int)  # token, expert, rank, weight
+    at = order[:, 0] * k + order[:, 2]
+    for lo, count in ((37, 203), (t * k - 90, 90), (130, 1)):
+        pc.partials = gpu.dev(np.full(t * k * d, 0xD4D0, np.uint16))
+        pc.pf.encode_streamed_batched(pc.dl.pool, pc.dl.off, pc.routes, pc.hidden, pc.stride, pc.partials, pc.ws, t, k, lo, count)
+        gpu.synchronize()
+        got = pc.partials.download(np.uint16, t * k * d).reshape(t * k, d)
+        inside = np.zeros(t * k, bool)
+        inside[at[lo:lo + count]] = True
+        assert np.array_equal(got[inside], want.reshape(t * k, d)[inside]), f"pairs {lo} to {lo + count}"
+        assert np.all(got[~inside] == 0xD4D0), f"pairs {lo} to {lo + count}: a row of another pair was written"
 
 
 def test_reduce_and_residual_bit_exact(gpu):
