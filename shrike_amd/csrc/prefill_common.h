@@ -39,8 +39,10 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_u32(uint32_t v, uint32_t
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
+template <bool ONCE = false>  // ONCE: non-temporal, of whole lines that nobody else reads
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
+    if constexpr (ONCE) asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
+    else asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
 // All but the wave's last COUNT loads have landed, and its reads of LDS are done.
 template <int COUNT>

@@ -33,8 +33,9 @@ constexpr uint32_t kUnitS = 64u * 16u;  // four groups' scales (biases) of those
 template <FfnShape S, int BITS>
 struct Lds {
     static constexpr bool kIsWide = S == FfnShape::kWide;
-    static constexpr uint32_t kPlacesA = S != FfnShape::kDeep ? 2u : BITS == 4 ? 4u : 3u;  // of groups of rows
-    static constexpr uint32_t kPlacesB = S != FfnShape::kDeep || BITS == 4 ? 2u : 3u;      // of units of codes
+    static constexpr bool kIsDeep = S == FfnShape::kDeep || S == FfnShape::kLines;
+    static constexpr uint32_t kPlacesA = !kIsDeep ? 2u : BITS == 4 ? 4u : 3u;  // of groups of rows
+    static constexpr uint32_t kPlacesB = !kIsDeep || BITS == 4 ? 2u : 3u;      // of units of codes
     static constexpr uint32_t kRows = kIsWide ? 128u : 64u;
     static constexpr uint32_t kUnitA = kRows * 128u;  // one group (64 k) of the rows
     static constexpr uint32_t kB = kPlacesA * kUnitA, kS = kB + kPlacesB * 4u * kUnitB, kDst = kS + 4u * kUnitS, kBytes = kDst + kRows * 8u;
@@ -78,6 +79,7 @@ struct FfnArgs {
     const uint16_t *scalar_gate;   // fp16[rows] or null: row m's output * sigmoid(gate[m]) (moe.metal:1195-1207)
     uint32_t table_room;           // records that the tile table has room for
     uint32_t resident_workgroups;  // workgroups of the launched k_grouped_ffn the device holds at once
+    uint64_t blob_bytes;           // of an expert
 };
 
 // The sum of a group of 64 fp16 values of which eight neighbouring lanes hold eight each, in every one of them: a lane's
@@ -149,11 +151,21 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // the reads of the rows that the next chain takes, and the wait for the next group's loads stands two chains ahead of their
 // use. What bounds it now: with many rows the power that matrix work, its operands' way through LDS and the loads take
 // together (2,048 gpt-oss tokens back to back: the clock at 1.95 GHz of 2.4; the kWide gate/up launch keeps the matrix pipe
-// busy 44 % of the cycles, vector issue 43 %); with few rows the weights' bytes (kDeep, 8-bit, 1,000 tokens: 4.4 TB/s), and the start and
+// busy 44 % of the cycles, vector issue 43 %); with few rows the weights' bytes (kLines, 8-bit, 1,000 tokens: 4.9 TB/s), and the start and
 // the end of the many short workgroups (256 experts of 2,048 x 512, 512 tokens: 29 % of the workgroups' time in gate/up and 53 % in
 // down lie outside the loop, 27 of 69 us; 37 tokens: 29 and 56 %). Both products, a chain scaled where it ends ->
 // pipelined: 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens 540 -> 495 us, 300 tokens 179 -> 164; 256 of 2,048 x 512, 4,096
 // tokens 316 -> 302, 37 33.5 -> 31.4; 256 of 2,304 x 1,024, 8-bit, 1,000 tokens 469 -> 439, 4,000 735 -> 710.
+//
+// kLines: what a card's memory gives depends on how it is asked. Read once and non-temporally, in whole 128-byte lines, 1.2 GB come
+// at 7.1 TB/s; without the hint at 6.2; in halves of a line, a group of 64 codes a row as the other shapes ask for 8-bit ones, at
+// 5.9, and at 4.4 with the hint, which drops a line between its halves. So a unit of codes is a line (two groups) of the rows of one
+// of a wave's two tiles, three such places take the room of three half-line ones, and the wave takes a unit into registers as soon
+// as it has landed, so that its place is asked for again two groups early. Both products of 1,000 kimi tokens (8-bit): 453 -> 407 us;
+// whole passes 551 -> 505 us, of 60 uneven tokens 108 -> 95, 17 tokens of 256 x 2,048 x 512 100 -> 92. What is left: the loads alone
+// take 214 of the gate/up launch's 257 us. (Four places for tiles of up to 32 rows 263 -> 257 us, the loads dealt over the
+// MFMAs that follow a meeting 260 -> 258, the group sums straight to registers 260 -> 258 and elsewhere slower: taken back. The
+// same for 4-bit codes: 1,000 even kimi tokens 352 -> 334 us, uneven ones 264 -> 271, 100 tokens of 256 x 2,048 x 512 137 -> 139.)
 //
 // MODE 0 leaves its activations through LDS: whole 16-byte pieces of a row go out together, and the group sums of the
 // tile's rows that the down product's bias term needs are formed here, in k_row_group_sums' order of additions (eight
@@ -161,12 +173,14 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // their own between the two products. Every wave of the workgroup stays to the end for the barriers.
 template <int BITS, int MODE, bool DENSE, uint32_t MT, int META, FfnShape S>
 __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile &tile, uint32_t act_row, uint32_t col_block,
-                                         uint8_t *lds) {
+                                         uint8_t *lds, bool once) {
     typedef Lds<S, BITS> L;
     // (kTile's places for up to 64 rows are twice as many for up to 32)
     constexpr bool kHalves = S == FfnShape::kTile && MT == 1u;
     constexpr uint32_t kA = L::kPlacesA * (kHalves ? 2u : 1u), kB = L::kPlacesB, kUnitA = L::kUnitA / (kHalves ? 2u : 1u);
     constexpr uint32_t kSums0 = L::kB - kUnitA;
+    constexpr bool kLines = S == FfnShape::kLines;
+    static_assert(!kLines || (BITS == 8 && !DENSE && MT <= 2u), "kLines is for 8-bit codes of routed experts");
     const uint32_t K = MODE == 0 ? a.d : a.f, N = MODE == 0 ? a.f : a.d;
     const uint32_t G = K / kGroup;
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
@@ -244,6 +258,24 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     const uint32_t half_back = (((lane & 3u) ^ (lane >> 4)) & 2u) * 16u;
     constexpr uint32_t kGroupsPerB = BITS == 4 ? 2u : 1u;
     const uint32_t lds_b = lds0 + L::kB + wave * kUnitB;
+    // kLines: a unit is a line, 128 bytes or two groups, of each row of ONE of the wave's tiles; load j brings eight rows of it,
+    // eight lanes a row.
+    const uint32_t line_row0 = min(n0, N - (MODE == 0 ? 32u : 64u));
+    uint32_t line_off[4];
+    if constexpr (kLines) {
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; ++j)
+            line_off[j] = (line_row0 + (MODE == 0 ? 1u : 2u) * (8u * j + (lane >> 3))) * row_bytes + ((lane & 7u) ^ (4u * (j & 1u) + (lane >> 4))) * 16u;
+    }
+    auto load_line = [&](uint32_t slot, uint32_t nt, uint32_t unit) {
+        const uint8_t *at = w_base[nt] + size_t(unit) * 128u + (MODE == 1 && nt ? row_bytes : 0u);
+        auto load = [&](auto once) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) lds_load16<decltype(once)::value>(lds_b + slot * (4u * kUnitB) + j * 1024u, at, line_off[j]);
+        };
+        if (once) load(std::true_type{});
+        else load(std::false_type{});
+    };
     auto load_b = [&](uint32_t slot, uint32_t stage, bool may_end = true) {
         const uint32_t back = BITS == 4 && may_end && 2u * stage + 1u >= G ? half_back : 0u;
 #pragma unroll
@@ -287,11 +319,16 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     }
     // what the first group needs is on its way before anything else
     load_s(0);
-    load_b(0, 0);
+    if (kLines) {
+        load_line(0, 0, 0);
+        load_line(1, 1, 0);
+    } else {
+        load_b(0, 0);
+    }
     load_a(0, 0);
     // (what the first group needs first, then of the rest what fits beside the sums below)
 #pragma unroll
-    for (uint32_t i = 1; i + 1u < kB; ++i)
+    for (uint32_t i = 1; !kLines && i + 1u < kB; ++i)
         if (i * kGroupsPerB < G) load_b(i, i);
 #pragma unroll
     for (uint32_t i = 1; i + 1u < kA; ++i)
@@ -398,14 +435,15 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     // keep the order as it is written.
     wait_loads_and_sync<0>();  // (nobody reads the sums any more)
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) in the compiler's own count: else it waits for the biases in the loop
-    if (kA != 2u && !last_b_early && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
+    if (kLines && 2u < G) load_line(2, 0, 1);
+    if (!kLines && kA != 2u && !last_b_early && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
     if (kA - 1u < G) load_a(kA - 1u, kA - 1u);
     if (kA == 2u && !last_b_early && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
     uint32_t run[2][2];  // the scales of a chunk of four groups, two a word
     float sc[2], sc_before = 0.0f;
     constexpr bool kTwoA = MT <= (S == FfnShape::kTile ? 1u : 2u);  // two sets of a row tile's operands: the next is read a chain earlier
     half8 af[kTwoA ? 2 : 1][4], bf[2][4];
-    uint4 raw[kTwoA ? 2 : 1][BITS / 4];
+    uint4 raw[kTwoA ? 2 : 1][kLines ? 4 : BITS / 4];
     constexpr bool kBehind = !(S == FfnShape::kTile && MT == 2u);  // (else a chain is scaled where it ends: a third workgroup's waves run beside it)
     f32x16 p[2];
     float tot[2][MT][16];  // (single registers: eight tuples of sixteen beside p do not fit round each other, and two were spilled)
@@ -450,9 +488,17 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             raw[kTwoA ? nt : 0u][i] = *reinterpret_cast<const uint4 *>(b_rows + b_place * (4u * kUnitB) + nt * 2048u + ((piece ^ ((col >> 2) & 3u)) * 16u));
         }
     };
-    auto unpack = [&](uint32_t nt, uint32_t s) {
-        const uint4 (&codes)[BITS / 4] = raw[kTwoA ? nt : 0u];
-        if (BITS == 4) {
+    auto read_line = [&](uint32_t slot, uint32_t nt) {
+        const uint8_t *p = lds + L::kB + wave * kUnitB + slot * (4u * kUnitB) + col * 128u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) raw[kTwoA ? nt : 0u][i] = *reinterpret_cast<const uint4 *>(p + (((4u * (i >> 1) + 2u * kb + (i & 1u)) ^ ((col >> 1) & 7u)) * 16u));
+    };
+    auto unpack = [&](uint32_t nt, uint32_t s, uint32_t par) {
+        const uint4 (&codes)[kLines ? 4 : BITS / 4] = raw[kTwoA ? nt : 0u];
+        if (kLines) {
+            const uint4 v = codes[2u * par + (s >> 1)];
+            bf[nt][s] = s & 1u ? codes8(v.z, v.w) : codes8(v.x, v.y);
+        } else if (BITS == 4) {
             const uint32_t w[4] = {codes[0].x, codes[0].y, codes[0].z, codes[0].w};
             bf[nt][s] = codes4(w[s]);
         } else {
@@ -462,6 +508,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     };
     // The places of group g's rows and of its codes. Powers of two are known to the compiler four groups at a time.
     uint32_t place3 = 0;  // g % 3
+    uint32_t line_at = 0;  // kLines: the place that held the first tile's codes of this unit
     auto next3 = [](uint32_t p) { return p == 2u ? 0u : p + 1u; };
     auto a_place = [&](uint32_t u) { return kA == 3u ? place3 : u & (kA - 1u); };
     auto b_place = [&](uint32_t u) { return kB == 3u ? place3 : BITS == 8 ? u & 1u : (u >> 1) & 1u; };
@@ -473,6 +520,18 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         constexpr uint32_t U = decltype(u_)::value;
         constexpr bool FAR = decltype(far_)::value;
         constexpr bool kOdd = (U & 1u) != 0u;
+        if constexpr (kLines) {
+            constexpr int kLeft = kOdd ? 4 : 8 + int(MT);
+            if (FAR || g + (kOdd ? 3u : 2u) < G) wait_loads_and_sync<kLeft>();
+            else wait_loads_and_sync<0>();
+            if (U == 0u && (FAR || g + 4u < G)) load_s((g >> 2) + 1u);
+            if (FAR || g + kA < G) load_a(a_place(U), g + kA);
+            if (!kOdd) {
+                if (FAR || g + 2u < G) load_line(line_at, 1, (g >> 1) + 1u);
+                if (FAR || g + 4u < G) load_line(next3(line_at), 0, (g >> 1) + 2u);
+            }
+            return;
+        }
         // what was asked for at the last meeting, or the last two, and is not needed yet
         constexpr uint32_t kOnTheWay = kA == 2u              ? (BITS == 4 && !kOdd ? 4u : 0u)
                                        : kA == 3u            ? MT + 4u + (U == 1u ? 1u : 0u)
@@ -496,6 +555,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         if (!active) {
             meet(g, u_, far_);
             if (kA == 3u) place3 = next3(place3);
+            if (kLines && (U & 1u)) line_at = next3(next3(line_at));
             return;
         }
         const uint32_t a_here = a_place(U), a_next = kA == 3u ? next3(place3) : a_place(U + 1u), b_next = kB == 3u ? a_next : b_place(U + 1u);
@@ -505,7 +565,8 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             const uint32_t set = kTwoA ? (U * MT + mt) & 1u : 0u;
             if (c == 2u * MT - 2u) {
                 meet(g, u_, far_);
-                read_raw(0, b_next, (U & 1u) ^ 1u);
+                if (kLines && (U & 1u)) read_line(next3(next3(line_at)), 0);
+                if (!kLines) read_raw(0, b_next, (U & 1u) ^ 1u);
                 if (U == 3u && (decltype(far_)::value || g + 1u < G)) read_run(g + 1u);
             }
             f32x16 &cur = p[kBehind ? nt : 0u], &old = p[kBehind ? nt ^ 1u : 0u];
@@ -517,9 +578,12 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
                 cur = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[set][s], bf[nt][s], s ? cur : zero, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (nt == (kTwoA ? 0u : 1u)) af[kTwoA ? set ^ 1u : 0u][s] = mt + 1u < MT ? read_a(a_here, mt + 1u, s) : read_a(a_next, 0u, s);
-                if (c == 0u) unpack(1, s);
-                if (c == 2u * MT - 1u) unpack(0, s);
-                if (c == 2u * MT - 1u && s == (kTwoA ? 0u : 3u)) read_raw(1, b_next, (U & 1u) ^ 1u);
+                if (c == 0u) unpack(1, s, U & 1u);
+                if (c == 2u * MT - 1u) unpack(0, s, (U & 1u) ^ 1u);
+                if (c == 2u * MT - 1u && s == (kTwoA ? 0u : 3u)) {
+                    if (kLines && (U & 1u)) read_line(line_at, 1);
+                    if (!kLines) read_raw(1, b_next, (U & 1u) ^ 1u);
+                }
 #pragma unroll
                 for (uint32_t i = 4u * s; kBehind && i < 4u * s + 4u; ++i) into[i] = fmaf(scale, old[i], into[i]);
                 // (named here: else the additions sink past the branches of `meet`, and every chain's sums stay alive until there)
@@ -535,19 +599,22 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
             }
         }
         if (kA == 3u) place3 = a_next;
+        if (kLines && (U & 1u)) line_at = next3(next3(line_at));
         sc_before = sc[1];
         next_scales(std::integral_constant<bool, (U & 1u) == 0u>{});
     };
     if (active) {
         read_run(0);
         next_scales(std::false_type{});
-        read_raw(0, 0, 0);
+        if (kLines) read_line(0, 0);
+        else read_raw(0, 0, 0);
 #pragma unroll
         for (uint32_t s = 0; s < 4u; ++s) {
             af[0][s] = read_a(0, 0, s);
-            unpack(0, s);
+            unpack(0, s, 0);
         }
-        read_raw(1, 0, 0);
+        if (kLines) read_line(1, 1);
+        else read_raw(1, 0, 0);
     }
     uint32_t g = 0;
     for (; g + 8u <= G; g += 4u) {
@@ -856,10 +923,19 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
     }
 
     const uint32_t act_row = tile_index * kRowTile + skip;
-    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, S>(a, tile, act_row, col_block, lds);
-    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, S>(a, tile, act_row, col_block, lds);
-    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, S>(a, tile, act_row, col_block, lds);
-    else ffn_tile<BITS, MODE, DENSE, 1, META, S>(a, tile, act_row, col_block, lds);
+    // Whether nobody else reads the tile's codes, in this launch or, as far as the memory-side cache goes, in the next: the
+    // experts in use are counted by their last tiles, which are not full (but for a multiple of 64 pairs), in the first 256 records.
+    bool once = false;
+    if constexpr (S == FfnShape::kLines) {
+        auto last_tiles = [&](const uint4 &rec, uint32_t at) { return uint32_t(__popcll(__ballot(lane + at < tile_total && rec.z < kRowTile))); };
+        const uint32_t in_use = last_tiles(rec0, 0) + last_tiles(rec1, 64) + last_tiles(rec2, 128) + last_tiles(rec3, 192);
+        const bool in_two = larger != 0u && ((larger >> tile_index) & 1u) != 0u;
+        once = tile.rows < kRowTile && !in_two && past_the_cache(in_use, a.blob_bytes);
+    }
+    if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, S>(a, tile, act_row, col_block, lds, once);
+    else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, S>(a, tile, act_row, col_block, lds, once);
+    else if (tile.rows > 32u) ffn_tile<BITS, MODE, DENSE, 2, META, S>(a, tile, act_row, col_block, lds, once);
+    else ffn_tile<BITS, MODE, DENSE, 1, META, S>(a, tile, act_row, col_block, lds, once);
 }
 
 // ---- few rows: the same products with k split over the waves.
@@ -1188,6 +1264,8 @@ static int launch_ffn_meta(const FfnArgs &a, uint32_t max_tiles, FfnShape shape,
     if (shape == FfnShape::kSplit) return launch_ffn_split<BITS, DENSE, META>(a, max_tiles, s);
     if constexpr (!DENSE)
         if (shape == FfnShape::kWide) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kWide>(a, max_tiles, s);
+    if constexpr (!DENSE && BITS == 8)
+        if (shape == FfnShape::kLines) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kLines>(a, max_tiles, s);
     if constexpr (!DENSE && BITS == 4)
         if (shape == FfnShape::kTile) return launch_ffn_shape<BITS, DENSE, META, FfnShape::kTile>(a, max_tiles, s);
     return launch_ffn_shape<BITS, DENSE, META, FfnShape::kDeep>(a, max_tiles, s);
@@ -1264,6 +1342,10 @@ static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_base
     if (!presummed)
         if (int rc = launch_row_group_sums(a.hidden, hidden_stride_elements, query_count, d, const_cast<uint32_t *>(a.hidden_sums), nullptr, s)) return rc;
     FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, d, f, moe->desc.routed_weight_bits);
+    uint64_t align = pool_slot_stride | offsets->gate_w_off | offsets->up_w_off | offsets->down_w_off | d | f;  // (a row of 8-bit codes is d or f bytes)
+    for (const void *base : pool->base) align |= reinterpret_cast<uintptr_t>(base);
+    a.blob_bytes = pool_slot_stride;
+    shape = lines_shape(shape, uint64_t(query_count) * top_k, moe->desc.num_experts, moe->desc.routed_weight_bits, a.blob_bytes, align);
     if (shape != FfnShape::kSplit && uint64_t(query_count) * hidden_stride_elements * 2u > 0xffffffffull) shape = FfnShape::kDeep;  // (the others' rows are 32-bit offsets)
     return moe->desc.routed_weight_bits == 8 ? launch_ffn<8, false>(a, max_row_tiles, shape, s) : launch_ffn<4, false>(a, max_row_tiles, shape, s);
 }

@@ -98,10 +98,15 @@ extern "C" const char *routed_shape(uint64_t pairs, uint32_t experts, uint32_t d
     static const char *const names[] = {"split", "tile", "deep", "wide"};
     return names[int(shrike::routed_shape(pairs, experts, d, f, bits))];
 }
+extern "C" bool takes_lines(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits, uint64_t blob_bytes, uint64_t align) {
+    const shrike::FfnShape shape = shrike::routed_shape(pairs, experts, d, f, bits);
+    return shrike::lines_shape(shape, pairs, experts, bits, blob_bytes, align) == shrike::FfnShape::kLines;
+}
 """
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/shrike_amd/csrc", "-x", "c++", "-", "-o", lib],
                        input=source.encode(), check=True)
         rules = C.CDLL(lib)
     rules.readable_records.argtypes, rules.readable_records.restype = [C.c_uint32, C.c_uint64, C.c_uint32], C.c_uint32
     rules.routed_shape.argtypes, rules.routed_shape.restype = [C.c_uint64, *[C.c_uint32] * 4], C.c_char_p
+    rules.takes_lines.argtypes, rules.takes_lines.restype = [C.c_uint64, *[C.c_uint32] * 4, C.c_uint64, C.c_uint64], C.c_bool
     return rules

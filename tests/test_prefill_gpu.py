@@ -11,7 +11,7 @@ from shrike_amd import capi
 from shrike_amd import host as HL
 from shrike_amd import synth as S
 from harness import runners
-from tests.helpers import Layer, assert_ffn_close, assert_rel_close, f16
+from tests.helpers import Layer, assert_ffn_close, assert_rel_close, f16, ffn_rules
 from tests.test_decode_gpu import DeviceLayer
 
 pytestmark = pytest.mark.gpu
@@ -403,6 +403,37 @@ def test_grouped_ffn_rings(gpu, d, f, ne, t, bits):
     assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
     for pair in np.random.default_rng(12).choice(t * 4, 40, replace=False):
         pc.check_pair(got, int(pair) // 4, int(pair) % 4, f"pair {pair}")
+
+
+# Units of two groups, one in all and around the ring of three places; experts of up to 32 rows, up to 64 and more; enough workgroups
+# for whole tiles, few enough tiles for their second halves to be workgroups of their own (the 8 experts), and fewer experts in use
+# than the pool has (the last: the hint is then left out).
+LINE_CASES = [  # d, f, experts, tokens, meta, experts in use
+    (128, 4096, 9, 40, S.META_F16, 9), (256, 2176, 70, 300, S.META_BF16, 70), (384, 1152, 70, 500, S.META_F16, 70), (512, 1024, 70, 700, S.META_BF16, 70),
+    (640, 768, 70, 900, S.META_F16, 70), (768, 640, 70, 700, S.META_BF16, 70), (1152, 896, 24, 300, S.META_F16, 24), (2304, 1024, 24, 150, S.META_BF16, 24),
+    (256, 4096, 8, 60, S.META_BF16, 8), (512, 1024, 70, 300, S.META_BF16, 9)]
+
+
+@pytest.mark.parametrize("d,f,ne,t,meta,in_use", LINE_CASES)
+def test_grouped_ffn_of_codes_past_the_caches(gpu, d, f, ne, t, meta, in_use):
+    """The same experts in cells so far apart that they count as more than the memory-side cache holds: the codes then come in
+    whole lines, and every row has the bytes that it has from a small pool."""
+    L = Layer(0x5EED0C00 + d + f, d, f, ne, 4, bits=8, meta=meta)
+    idx = random_routes(t + ne, t, 4, in_use)[0]
+    pc = PrefillCase(gpu, L, t, stride_pad=8, idx=idx, scale=row_scale(d, f))
+    near = pc.run()
+    for pair in np.random.default_rng(13).choice(t * 4, 12, replace=False):
+        pc.check_pair(near, int(pair) // 4, int(pair) % 4, f"pair {pair}")
+    far = gpu.ExpertPool(ne, (320 << 20) // ne, ne)
+    assert ffn_rules().takes_lines(4 * t, ne, d, f, 8, far.stride, far.stride | d | f)
+    assert not ffn_rules().takes_lines(4 * t, ne, d, f, 8, pc.dl.pool.stride, 0)
+    for e, cell in pc.dl.cell_of.items():
+        far.upload(cell, L.blobs[e])
+        far.publish(e, cell, capi.RESIDENT)
+    pc.dl.pool = far
+    pc.pf.group_pairs(pc.d_idx, pc.d_w, t, 4, ne, pc.routes, residency=far.table)
+    pc.partials = gpu.dev(np.full(t * 4 * d, 0xD4D0, np.uint16))
+    assert np.array_equal(pc.run(), near)
 
 
 @pytest.mark.parametrize("d,f,bits,meta", [(320, 640, 4, S.META_BF16), (1088, 704, 8, S.META_F16)])
