@@ -39,10 +39,15 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan_u32(uint32_t v, uint32_t
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(p) : "memory");
 }
+// The base is moved on the scalar unit first: where the compiler has just brought it back from a vector register's lane
+// (v_readlane of a spilled one), a memory instruction that reads it needs five wait states, which the compiler keeps for
+// instructions that it knows and this one is not; the scalar unit waits by itself, and so does what reads its result. (The move
+// stands where the wait state behind the write of m0 would.)
 template <bool ONCE = false>  // ONCE: non-temporal, of whole lines that nobody else reads
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
-    if constexpr (ONCE) asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
-    else asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"{m0}"(lds), "v"(offset), "s"(base) : "memory");
+    const void *moved;
+    if constexpr (ONCE) asm volatile("s_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0 nt" : "=&s"(moved) : "{m0}"(lds), "v"(offset), "s"(base) : "memory");
+    else asm volatile("s_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(moved) : "{m0}"(lds), "v"(offset), "s"(base) : "memory");
 }
 // All but the wave's last COUNT loads have landed, and its reads of LDS are done.
 template <int COUNT>
