@@ -252,17 +252,31 @@ __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t q
 // waves in LDS. An affine row's chunk sums its codes' products from zero, in 8 or 16 chains of their own, and takes scale
 // (a multiply-add an output) and bias (one more MFMA) as router_row does.
 //
-// A workgroup takes 16 tokens and 16 experts and brings both sides' chunks of a j in through LDS, four workgroups a compute
-// unit so that one's loads run beside the others' products (two with the next j's loads beside its own were slower: 82
-// against 69 us in all). The matrix cores do twice the plain vector unit's fp32 multiply-adds, and the vector unit keeps the
-// widening only: 31 us of them for 4,096 tokens of 2,048 against 256 rows, where the vector kernel below has 55. With the
-// selection's 11: 91 -> 67 us; 1,000 tokens of 2,304, 8-bit rows, 51 -> 36; 4-bit rows, 512 of 2,048, 25 -> 18.
+// A workgroup takes 16 tokens and 16 experts, four workgroups a compute unit. Both sides' chunks come through a ring in LDS, a walk
+// (four chunks of each wave's) a unit, asked for one or two units ahead. The effective scales come that way too and are widened
+// in LDS once. What bounds it: a SIMD does not run a fp32 matrix instruction beside a vector one (a chain of them fed by two
+// vector instructions each, two waves a SIMD: 44 cycles a step, 32 without), so 4,096 tokens of 2,048 against 256 rows, 28 us
+// of matrix instructions alone, take 45 with the two conversions a product that nothing shares, and more with the loads' addresses.
+// A step's chunks all asked for, waited for and multiplied by turns -> the ring, us: fp16 rows, 256 of 2,048: 512 tokens 13.2 ->
+// 12.4, 1,000 21.0 -> 19.7, 4,096 69.5 -> 67.0, 128 of 3,072, 2,048 tokens 33.8 -> 26.9; 8-bit rows, 256 of 2,304: 300 tokens 18.4 ->
+// 17.8, 1,000 34.1 -> 30.7, 2,000 60.0 -> 55.9; 4-bit rows the same. A place more each: 3 to 8 % slower past 1,000 tokens (a workgroup
+// fewer a compute unit). Two tiles of tokens, or of experts, a workgroup: 512 tokens 13.5, 4,096 71 (half the workgroups); two of both spill.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+template <int RK>
+struct LogitsLds {
+    static constexpr uint32_t kPieces = kRouterChunk<RK> / 8;                       // 16-byte pieces of x a chunk
+    static constexpr uint32_t kUnit = 4u * (kPieces + 1u) * 1024u;                  // a walk's chunks of sixteen tokens and sixteen experts
+    static constexpr uint32_t kPlaces = RK == 0 ? 3u : 2u, kEff = kPlaces * kUnit;
+    static_assert(SHRIKE_MAX_HIDDEN * 2u <= kUnit, "the effective scales fit a unit's place");
+    static uint32_t bytes(uint32_t d) { return kEff + 4u * d + (RK ? 2u * 16u * (d / kGroup) * 2u : 0u); }
+};
 
 template <int RK>
 __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, uint32_t query_count, uint32_t stride, float *logits) {
     warm_kernel_arguments(a);
-    constexpr uint32_t E = kRouterChunk<RK>, Q = E / 8;  // a chunk's elements, 16-byte pieces of x
+    typedef LogitsLds<RK> L;
+    constexpr uint32_t E = kRouterChunk<RK>, Q = L::kPieces;  // a chunk's elements, 16-byte pieces of x
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
     const uint32_t num_experts = a.sel.num_experts, d = a.d, chunks = d / E, walks = (chunks + 63u) / 64u, groups = d / kGroup;
@@ -270,28 +284,36 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     const uint32_t expert_tiles = (num_experts + 15u) / 16u;
     const uint32_t t0 = ((blockIdx.x >> 3) / expert_tiles * 8u + (blockIdx.x & 7u)) * 16u, e0 = (blockIdx.x >> 3) % expert_tiles * 16u;
     if (t0 >= query_count) return;
-    const uint32_t w_at = 4u * walks * Q * 1024u;  // behind x
-    float *l_eff = reinterpret_cast<float *>(lds + 4u * walks * (Q + 1u) * 1024u);
+    float *l_eff = reinterpret_cast<float *>(lds + L::kEff);
     uint16_t *l_scale = reinterpret_cast<uint16_t *>(l_eff + d), *l_bias = l_scale + 16u * groups;
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds));
+    // the effective scales as they are, into the last place, for now
+    constexpr uint32_t kEffAt = (L::kPlaces - 1u) * L::kUnit;
+    for (uint32_t i = wave * 1024u; i < 2u * d; i += 4096u)
+        lds_load16(lds0 + kEffAt + i, reinterpret_cast<const uint8_t *>(a.effective_scale) + min(i + lane * 16u, 2u * d - 16u));
     // A load brings a 16-byte piece of four chunks of sixteen rows, the chunks xor-ed with the row so that sixteen rows read
     // at one chunk touch every bank once. Wave w brings block w's.
     const uint32_t l_row = lane >> 2, l_chunk = ((lane & 3u) ^ ((l_row >> 2) & 3u)) + 16u * wave;
     const uint8_t *w_row = static_cast<const uint8_t *>(a.weights) + size_t(min(e0 + l_row, num_experts - 1u)) * chunks * 16u;
     const uint16_t *x_row = a.hidden + size_t(min(t0 + l_row, query_count - 1u)) * stride;
-    auto load = [&](uint32_t j) {
-        for (uint32_t i = 0; i < walks; ++i) {
-            const uint32_t c = min(4u * j + l_chunk + 64u * i, chunks - 1u);  // past the row: a copy, taken as zero
+    constexpr uint32_t kOrder[4] = {0, 2, 1, 3};  // of j: the butterfly's
+    const uint32_t units = 4u * walks;
+    uint32_t ask_j = 0, ask_i = 0, ask_place = 0;  // the unit to ask for next: its step, its walk, its place
+    auto ask = [&]() {
+        const uint32_t j = ask_j == 1u ? 2u : ask_j == 2u ? 1u : ask_j;
+        const uint32_t c = min(4u * j + l_chunk + 64u * ask_i, chunks - 1u), at = lds0 + ask_place * L::kUnit;  // past the row: a copy, taken as zero
 #pragma unroll
-            for (uint32_t q = 0; q < Q; ++q) lds_load16(lds0 + ((wave * walks + i) * Q + q) * 1024u, x_row + c * E + q * 8u);
-            lds_load16(lds0 + w_at + (wave * walks + i) * 1024u, w_row + c * 16u);
+        for (uint32_t q = 0; q < Q; ++q) lds_load16(at + (wave * Q + q) * 1024u, x_row + c * E + q * 8u);
+        lds_load16(at + (4u * Q + wave) * 1024u, w_row + c * 16u);
+        if (++ask_i == walks) {
+            ask_i = 0;
+            ++ask_j;
         }
+        ask_place = ask_place + 1u == L::kPlaces ? 0u : ask_place + 1u;
     };
-    load(0);
-    for (uint32_t i = threadIdx.x; i < d / 2u; i += 256u) {
-        const uint32_t pair = reinterpret_cast<const uint32_t *>(a.effective_scale)[i];
-        reinterpret_cast<float2 *>(l_eff)[i] = make_float2(bf16_to_f32(uint16_t(pair)), bf16_to_f32(uint16_t(pair >> 16)));
-    }
+#pragma unroll
+    for (uint32_t u = 0; u + 1u < L::kPlaces; ++u)
+        if (u < units) ask();
     if (RK != 0) {
         for (uint32_t i = threadIdx.x; i < 16u * groups; i += 256u) {
             const uint32_t e = min(e0 + i / groups, num_experts - 1u);
@@ -299,16 +321,25 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
             l_bias[i] = a.biases[size_t(e) * groups + i % groups];
         }
     }
+    if (L::kPlaces - 2u < units) wait_loads_and_sync<int((L::kPlaces - 2u) * (Q + 1u))>();
+    else wait_loads_and_sync<0>();
+    for (uint32_t i = threadIdx.x; i < d / 8u; i += 256u) {
+        const uint4 v = *reinterpret_cast<const uint4 *>(lds + kEffAt + i * 16u);
+        float4 *to = reinterpret_cast<float4 *>(l_eff + 8u * i);
+        to[0] = make_float4(bf16_to_f32(uint16_t(v.x)), bf16_to_f32(uint16_t(v.x >> 16)), bf16_to_f32(uint16_t(v.y)), bf16_to_f32(uint16_t(v.y >> 16)));
+        to[1] = make_float4(bf16_to_f32(uint16_t(v.z)), bf16_to_f32(uint16_t(v.z >> 16)), bf16_to_f32(uint16_t(v.w)), bf16_to_f32(uint16_t(v.w >> 16)));
+    }
     const uint32_t m = lane & 15u, block = lane >> 4;
     const uint32_t read_at = m * 64u + ((wave ^ ((m >> 2) & 3u)) * 16u);
     f32x16_t acc;
     // chunk 64 i + 4 j + wave of each block; CHECK: it may lie past the row
-    auto chunk = [&](uint32_t j, uint32_t i, auto check) {
+    auto chunk = [&](uint32_t place, uint32_t j, uint32_t i, auto check) {
         constexpr bool CHECK = decltype(check)::value;
         const uint32_t c0 = 4u * j + wave + 64u * i, c = c0 + 16u * block;
         const bool inside = !CHECK || c < chunks;
         const uint32_t cc = inside ? c : 0u;
-        const uint4 wv = *reinterpret_cast<const uint4 *>(lds + w_at + (block * walks + i) * 1024u + read_at);
+        const uint8_t *unit = lds + place * L::kUnit + read_at;
+        const uint4 wv = *reinterpret_cast<const uint4 *>(unit + (4u * Q + block) * 1024u);
         uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
         if (CHECK) {
 #pragma unroll
@@ -318,7 +349,7 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
         float sum = 0.0f;
 #pragma unroll
         for (uint32_t q = 0; q < Q; ++q) {
-            const uint4 xv = *reinterpret_cast<const uint4 *>(lds + ((block * walks + i) * Q + q) * 1024u + read_at);
+            const uint4 xv = *reinterpret_cast<const uint4 *>(unit + (block * Q + q) * 1024u);
             const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
             const float4 e0v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u), e1v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u + 4u);
             const float ew[8] = {e0v.x, e0v.y, e0v.z, e0v.w, e1v.x, e1v.y, e1v.z, e1v.w};
@@ -351,16 +382,25 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
         }
     };
     float even[4], odd[4];
+    uint32_t unit = 0, place = L::kPlaces - 1u;
+    // The place of the next unit: it has landed for every wave, and every wave is done with the one before it, whose place is asked
+    // for again.
+    auto take = [&]() {
+        if (unit + L::kPlaces - 2u < units) wait_loads_and_sync<int((L::kPlaces - 2u) * (Q + 1u))>();
+        else wait_loads_and_sync<0>();
+        if (unit + L::kPlaces - 1u < units) ask();
+        ++unit;
+        place = place + 1u == L::kPlaces ? 0u : place + 1u;
+        return place;
+    };
 #pragma unroll
     for (uint32_t step = 0; step < 4u; ++step) {
-        constexpr uint32_t kOrder[4] = {0, 2, 1, 3};  // of j: the butterfly's
-        wait_loads_and_sync<0>();
         acc = f32x16_t{0};
-        for (uint32_t i = 0; i + 1u < walks; ++i) chunk(kOrder[step], i, std::false_type{});
-        if (64u * walks == chunks) chunk(kOrder[step], walks - 1u, std::false_type{});
-        else chunk(kOrder[step], walks - 1u, std::true_type{});
-        __syncthreads();
-        if (step < 3u) load(kOrder[(step + 1u) & 3u]);
+        // (the walk that may end past the row is on its own: in one loop with the others the sums went from register to register)
+        for (uint32_t i = 0; i + 1u < walks; ++i) chunk(take(), kOrder[step], i, std::false_type{});
+        const uint32_t last = take();
+        if (64u * walks == chunks) chunk(last, kOrder[step], walks - 1u, std::false_type{});
+        else chunk(last, kOrder[step], walks - 1u, std::true_type{});
 #pragma unroll
         for (uint32_t r = 0; r < 4u; ++r) {
             const float v = __fadd_rn(__fadd_rn(acc[r], acc[8u + r]), __fadd_rn(acc[4u + r], acc[12u + r]));
@@ -370,9 +410,9 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
             else even[r] = __fadd_rn(even[r], __fadd_rn(odd[r], v));
         }
     }
-    // (the loop's last barrier: nobody reads the operands any more)
+    __syncthreads();  // (nobody reads the operands any more)
     float (*meet)[16][17] = reinterpret_cast<float (*)[16][17]>(lds);
-    static_assert(sizeof(float[4][16][17]) <= 4u * 2u * 1024u, "the waves' sums fit where one walk's chunks were");
+    static_assert(sizeof(float[4][16][17]) <= L::kUnit, "the waves' sums fit where a unit was");
 #pragma unroll
     for (uint32_t r = 0; r < 4u; ++r) meet[wave][4u * block + r][m] = even[r];
     __syncthreads();
@@ -381,18 +421,16 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     if (t0 + row < query_count && e0 + col < num_experts) logits[size_t(t0 + row) * num_experts + e0 + col] = v;
 }
 
-// True if it launched: where 16 tokens by 16 experts make more than one workgroup for most compute units. With fewer the four
-// waits of a workgroup are what it takes, some 8 us, and the vector kernel's many small workgroups are done before (fp16 rows,
+// True if it launched: where 16 tokens by 16 experts make more than one workgroup for most compute units. With fewer a workgroup's
+// chain of units is what it takes, some 8 us, and the vector kernel's many small workgroups are done before (fp16 rows,
 // 256 of 2,048: 300 tokens 16.3 against 15.4 us with the selection, 512 17.3 against 20.2; 8-bit, 2,304: 100 tokens 17.1
 // against 16.2, 300 22.3 against 24.2).
 template <int RK>
 static bool launch_prefill_logits_mfma(const RouterArgs &a, uint32_t query_count, uint32_t stride, float *logits, hipStream_t s) {
-    constexpr uint32_t E = kRouterChunk<RK>, Q = E / 8;
     const uint32_t expert_tiles = (a.sel.num_experts + 15u) / 16u, token_tiles = (query_count + 15u) / 16u;
     if (uint64_t(expert_tiles) * token_tiles <= (RK == 0 ? 384u : 256u)) return false;
-    const uint32_t walks = (a.d / E + 63u) / 64u;
-    const uint32_t bytes = 4u * walks * (Q + 1u) * 1024u + a.d * 4u + (RK ? 2u * 16u * (a.d / kGroup) * 2u : 0u);
-    hipLaunchKernelGGL(k_prefill_logits_mfma<RK>, dim3(((token_tiles + 7u) & ~7u) * expert_tiles), dim3(256), bytes, s, a, query_count, stride, logits);
+    if (reinterpret_cast<uintptr_t>(a.effective_scale) % 4u != 0) return false;  // (whole words of them are loaded)
+    hipLaunchKernelGGL(k_prefill_logits_mfma<RK>, dim3(((token_tiles + 7u) & ~7u) * expert_tiles), dim3(256), LogitsLds<RK>::bytes(a.d), s, a, query_count, stride, logits);
     return true;
 }
 
