@@ -305,13 +305,16 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
         const u32x4_by2 v = *reinterpret_cast<const u32x4_by2 *>(row + min(at, G - 8u));
         return make_uint4(v.x, v.y, v.z, v.w);
     };
-    // MODE 1: where the rows go, in bytes from `partials` (all ones: nowhere)
+    // MODE 1: where the rows go, in bytes from `partials` (all ones: nowhere); a dense expert's rows lie where their tokens do, and
+    // have the divisors of their scalar gates there instead, if any
     uint64_t *s_dst = reinterpret_cast<uint64_t *>(lds + L::kDst);
+    float *s_gate = reinterpret_cast<float *>(lds + L::kDst);
     uint64_t dst = ~0ull;
+    uint16_t gate_bits = 0;
     if (MODE == 1 && threadIdx.x < MT * 32u && threadIdx.x < tile.rows) {
         const uint32_t pair = tile.pair_start + threadIdx.x;
         if (DENSE) {
-            dst = uint64_t(pair) * a.d * 2u;
+            if (a.scalar_gate) gate_bits = a.scalar_gate[pair];
         } else if (pair >= a.pair_lo && pair < a.pair_hi) {  // a call over a range of the sorted pairs writes their rows only
             const shrike_token_expert_pair p = a.pairs[pair];
             dst = (uint64_t(p.token) * a.top_k + p.rank) * a.d * 2u;
@@ -334,7 +337,7 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     for (uint32_t i = 1; i + 1u < kA; ++i)
         if (i < G) load_a(i, i);
 
-    if (MODE == 1 && threadIdx.x < MT * 32u) s_dst[threadIdx.x] = dst;
+    if (MODE == 1 && !DENSE && threadIdx.x < MT * 32u) s_dst[threadIdx.x] = dst;
 
     // (4-bit codes: the place of the second unit of sums is free where there is none. 128 experts of 2,048 x 1,024, 300 tokens,
     // weights from memory: 124 -> 120 us.)
@@ -435,6 +438,8 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
     // keep the order as it is written.
     wait_loads_and_sync<0>();  // (nobody reads the sums any more)
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0) in the compiler's own count: else it waits for the biases in the loop
+    // (formed where a sum is written it was a load, expf and a wait a row: 4,096 rows of 2,048 x 512, the down launch 28.8 -> 22.8 us)
+    if (MODE == 1 && DENSE && threadIdx.x < MT * 32u) s_gate[threadIdx.x] = 1.0f + expf(-f16_to_f32(gate_bits));
     if (kLines && 2u < G) load_line(2, 0, 1);
     if (!kLines && kA != 2u && !last_b_early && (kB - 1u) * kGroupsPerB < G) load_b(kB - 1u, kB - 1u);
     if (kA - 1u < G) load_a(kA - 1u, kA - 1u);
@@ -698,10 +703,10 @@ __device__ __forceinline__ void ffn_tile(const FfnArgs &a, const shrike_row_tile
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const uint32_t m = mt * 32u + 8u * (i / 4) + 4u * kb + (i % 4);
-                    const uint64_t to = s_dst[m];
+                    const uint64_t to = !DENSE ? s_dst[m] : m < tile.rows ? uint64_t(tile.pair_start + m) * a.d * 2u : ~0ull;
                     uint16_t y0 = f32_to_f16(total[0][mt][i] + dab[0]), y1 = f32_to_f16(total[1][mt][i] + dab[1]);
-                    if (DENSE && a.scalar_gate && m < tile.rows) {  // one gate a token row (moe.metal:1195-1207)
-                        const float gate_mul = 1.0f + expf(-f16_to_f32(a.scalar_gate[tile.pair_start + m]));
+                    if (DENSE && a.scalar_gate) {  // one gate a token row (moe.metal:1195-1207)
+                        const float gate_mul = s_gate[m];
                         y0 = f32_to_f16(f16_to_f32(y0) / gate_mul);
                         y1 = f32_to_f16(f16_to_f32(y1) / gate_mul);
                     }
