@@ -43,6 +43,7 @@ struct Phase1Args {
     const RouteEntry *route_table;
     uint32_t lists_block;  // set by launch_phase1: the workgroup that writes the route lists
     uint32_t routed_blocks;
+    uint32_t row_steps;  // set by launch_phase1: steps of row pairs that a wave walks
     GemvArgs shared_down;
 };
 

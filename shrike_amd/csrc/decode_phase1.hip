@@ -22,7 +22,11 @@ constexpr int kPhase1RowPairsNarrow = 2;
 // reads an expert's rows once per token routed to it, and there the caches are what makes the second read cheap).
 // TAIL: the rows end in a step of half chunks (load_slice_regs); NCH then counts the whole steps ahead of it.
 // META: the type of the routed experts' scales and biases (SHRIKE_META_*), known to the instance so that a row converts them one way.
-template <int BITS, int NCH, int RP, bool ROUTE, int SBITS, bool STREAM, bool TAIL, int META>
+// LOOP: a wave walks a.row_steps steps of RP row pairs (phase1_steps), with the activations unpacked once. A large batch is bound by
+// the vector units: 16 tokens of 2,304 x 1,024, 8-bit, 8 of 256 experts, keep them busy for 65 of 118 us, and of a wave's 600
+// operations the selection, which every wave makes for itself, is 100 and the activations' unpacking 50. With two steps the launch
+// takes 98 us.
+template <int BITS, int NCH, int RP, bool ROUTE, int SBITS, bool STREAM, bool TAIL, int META, bool LOOP>
 __global__ __launch_bounds__(256) void k_phase1(Phase1Args a) {
     warm_kernel_arguments(a);
     typedef Chunk<BITS> C;
@@ -58,10 +62,12 @@ __global__ __launch_bounds__(256) void k_phase1(Phase1Args a) {
     uint16_t *acts_tok = a.acts + tok * a.top_k * a.f;
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
     const uint32_t cpr = a.d * BITS / 128u, groups = a.d / kGroup, row_bytes = cpr * 16u;
-    const uint32_t pair0 = (blockIdx.x * 4u + wave) * RP;
+    const uint32_t per_wave = LOOP ? RP * a.row_steps : uint32_t(RP);
+    const uint32_t pair0 = (blockIdx.x * 4u + wave) * per_wave;
     bool in_range = pair0 < (a.active ? a.active_count : a.top_k) * a.f;
     uint32_t k = in_range ? pair0 / a.f : 0u;
-    const uint32_t f0 = pair0 - k * a.f;
+    uint32_t f0 = pair0 - k * a.f;
+    const uint32_t f_end = f0 + per_wave;
     if (!ROUTE && a.active) {  // moe.metal:873-876: the wave's position comes from the list; one past top_k is skipped
         k = in_range ? a.active[k] : 0u;
         in_range = in_range && k < a.top_k;
@@ -91,40 +97,48 @@ __global__ __launch_bounds__(256) void k_phase1(Phase1Args a) {
     }
 
     RowRegs<BITS, NCH, TAIL> rows[2 * RP];
-#pragma unroll
-    for (int r = 0; r < 2 * RP; ++r) {
-        const bool up = r >= RP;
-        const uint32_t f = f0 + uint32_t(r % RP);
-        const uint8_t *w = base + (up ? a.off.up_w_off : a.off.gate_w_off) + size_t(f) * row_bytes;
-        const uint16_t *s = reinterpret_cast<const uint16_t *>(base + (up ? a.off.up_s_off : a.off.gate_s_off)) + size_t(f) * groups;
-        const uint16_t *b = reinterpret_cast<const uint16_t *>(base + (up ? a.off.up_b_off : a.off.gate_b_off)) + size_t(f) * groups;
-        load_row<BITS, NCH, STREAM, TAIL>(rows[r], w, s, b, cpr, lane, true);
-    }
     float gab = 0.0f, uab = 0.0f;
-    if (a.ebias && lane < uint32_t(RP)) {  // moe.metal:261-269
-        gab = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.gate_ab_off)[f0 + lane]);
-        uab = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.up_ab_off)[f0 + lane]);
-    }
-
+    auto load_rows = [&] {
+#pragma unroll
+        for (int r = 0; r < 2 * RP; ++r) {
+            const bool up = r >= RP;
+            const uint32_t f = f0 + uint32_t(r % RP);
+            const uint8_t *w = base + (up ? a.off.up_w_off : a.off.gate_w_off) + size_t(f) * row_bytes;
+            const uint16_t *s = reinterpret_cast<const uint16_t *>(base + (up ? a.off.up_s_off : a.off.gate_s_off)) + size_t(f) * groups;
+            const uint16_t *b = reinterpret_cast<const uint16_t *>(base + (up ? a.off.up_b_off : a.off.gate_b_off)) + size_t(f) * groups;
+            load_row<BITS, NCH, STREAM, TAIL>(rows[r], w, s, b, cpr, lane, true);
+        }
+        if (a.ebias && lane < uint32_t(RP)) {  // moe.metal:261-269
+            gab = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.gate_ab_off)[f0 + lane]);
+            uab = bf16_to_f32(reinterpret_cast<const uint16_t *>(base + a.off.up_ab_off)[f0 + lane]);
+        }
+    };
+    load_rows();
     typename C::X x[NCH];
     float xs[NCH];
     TailX xt;
     unpack_slices<BITS, NCH, TAIL>(xr, x, xs, xt);
-    float res[2 * RP];
+    while (true) {
+        float res[2 * RP];
 #pragma unroll
-    for (int r = 0; r < 2 * RP; ++r) res[r] = wave_sum(row_partial<BITS, NCH, TAIL>(rows[r], x, xs, xt, uint32_t(META)));
-    // lane p < RP finishes row pair p
-    float g = res[0], u = res[RP];
+        for (int r = 0; r < 2 * RP; ++r) res[r] = wave_sum(row_partial<BITS, NCH, TAIL>(rows[r], x, xs, xt, uint32_t(META)));
+        // lane p < RP finishes row pair p
+        float g = res[0], u = res[RP];
 #pragma unroll
-    for (int p = 1; p < RP; ++p) {
-        g = lane == uint32_t(p) ? res[p] : g;
-        u = lane == uint32_t(p) ? res[RP + p] : u;
+        for (int p = 1; p < RP; ++p) {
+            g = lane == uint32_t(p) ? res[p] : g;
+            u = lane == uint32_t(p) ? res[RP + p] : u;
+        }
+        const uint16_t act = f32_to_f16(glu_rt(g + gab, u + uab, a.act));
+        if (lane < uint32_t(RP)) acts_tok[size_t(k) * a.f + f0 + lane] = act;
+        if (!LOOP) return;
+        f0 += RP;
+        if (f0 >= f_end) return;
+        load_rows();
     }
-    const uint16_t act = f32_to_f16(glu_rt(g + gab, u + uab, a.act));
-    if (lane < uint32_t(RP)) acts_tok[size_t(k) * a.f + f0 + lane] = act;
 }
 
-// positions: top_k, or the length of the active list
+// positions: top_k, or the length of the active list; row_pairs: those of a wave
 static uint32_t phase1_blocks_of(uint32_t positions, uint32_t f, uint32_t row_pairs) {
     const uint32_t waves = (positions * f + row_pairs - 1) / row_pairs;
     return (waves + 3) / 4;
@@ -136,21 +150,42 @@ static bool phase1_narrow(bool routing, bool one_token, uint32_t d, uint32_t bit
     return (one_token && !routing) || nch_for(d, bits) >= 3;
 }
 
+// Two steps where a routing launch of one-step waves has 4,096 workgroups, 16 a compute unit, or more, else one: with fewer the
+// last waves' second steps cost more than the selections saved. A layer with one step and with two, us: 16,384 workgroups (16 tokens of
+// 2,304 x 1,024, 8-bit) 172 and 161; 8,192 (8 of them) 95 and 89; 6,144 (16 of 1,536 x 768) 67 and 65; 4,096 (16 of 2,048 x 512)
+// 57.5 and 55.5; 2,048 (8 of them) 32.8 and 33.1; 1,024 (16 of 1,024 x 256) 17.2 and 18.6. Rows of four steps a lane keep one
+// (12 tokens of 4,096 x 1,024, 8-bit: 190.5 and 192), as do rows with half chunks, where the loop's registers cost the launch a wave a
+// SIMD (16 tokens of 2,880 x 2,880: 141 and 144). Two steps' row pairs divide f, a multiple of 64.
+static uint32_t phase1_steps(const Phase1Args &a, bool routing, uint32_t bits) {
+    const bool looped = routing && nch_for(a.d, bits) < 4u && !(bits == 4u && half_chunk_tail(a.d * bits / 128u, bits));
+    return looped && uint64_t(a.tokens) * a.routed_blocks >= 4096u ? 2u : 1u;
+}
+
+template <int BITS, int NCH, int RP, bool ROUTE, int SBITS, bool STREAM, int META>
+static void launch_phase1_steps(const Phase1Args &a, dim3 grid, hipStream_t s) {
+    if constexpr (ROUTE && !STREAM && NCH < 4) {
+        if (a.row_steps > 1u) {
+            hipLaunchKernelGGL((k_phase1<BITS, NCH, RP, ROUTE, SBITS, STREAM, false, META, true>), grid, dim3(256), 0, s, a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_phase1<BITS, NCH, RP, ROUTE, SBITS, STREAM, false, META, false>), grid, dim3(256), 0, s, a);
+}
+
 template <int BITS, bool ROUTE, int SBITS, bool STREAM, int META>
 static void launch_phase1_meta(const Phase1Args &a, dim3 grid, hipStream_t s) {
     // (shorter rows: the one-token routing launch keeps four pairs)
     constexpr int RP = kPhase1RowPairs, RN = (ROUTE && STREAM) ? kPhase1RowPairs : kPhase1RowPairsNarrow;
-    const dim3 block(256);
     if (BITS == 4 && half_chunk_tail(a.d * BITS / 128u, BITS)) {
         // d <= SHRIKE_MAX_HIDDEN: one whole step and the half chunks (65...96 chunks a row)
-        hipLaunchKernelGGL((k_phase1<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, BITS == 4, META>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((k_phase1<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, BITS == 4, META, false>), grid, dim3(256), 0, s, a);
         return;
     }
     switch (nch_for(a.d, BITS)) {
-        case 1: hipLaunchKernelGGL((k_phase1<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_phase1<BITS, 2, STREAM ? RN : RP, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
-        case 3: hipLaunchKernelGGL((k_phase1<BITS, 3, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((k_phase1<BITS, 4, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, false, META>), grid, block, 0, s, a); break;
+        case 1: launch_phase1_steps<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
+        case 2: launch_phase1_steps<BITS, 2, STREAM ? RN : RP, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
+        case 3: launch_phase1_steps<BITS, 3, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
+        default: launch_phase1_steps<BITS, 4, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
     }
 }
 
@@ -173,6 +208,9 @@ int launch_phase1(const Phase1Args &a, uint32_t bits, bool routing, uint32_t sha
     const bool one_token = a.tokens <= 1u;
     if (phase1_narrow(routing, one_token, a.d, bits))
         b.routed_blocks = phase1_blocks_of(a.active ? a.active_count : a.top_k, a.f, kPhase1RowPairsNarrow);
+    b.row_steps = one_token ? 1u : phase1_steps(b, routing, bits);
+    if (b.row_steps > 1u)
+        b.routed_blocks = phase1_blocks_of(a.top_k, a.f, b.row_steps * (phase1_narrow(routing, one_token, a.d, bits) ? kPhase1RowPairsNarrow : kPhase1RowPairs));
     b.lists_block = routing ? b.routed_blocks + extra : 0xffffffffu;
     const dim3 grid(b.routed_blocks + extra + (routing ? 1u : 0u), a.tokens ? a.tokens : 1u);
     if (bits == 4) {

@@ -720,6 +720,14 @@ def test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne,
     assert "shared expert" in capi.last_error()
 
 
+@pytest.mark.parametrize("d,f,ne,k,t,bits,router_bits", [(64, 1024, 24, 8, 8, 4, 0), (3136, 576, 70, 8, 16, 4, 0), (1088, 768, 16, 8, 16, 8, 8),
+                                                          (2112, 1088, 72, 4, 8, 8, 0), (3136, 512, 16, 8, 16, 8, 0)])
+def test_decode_layer_for_a_large_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, router_bits):
+    # phase 1 of 4,096 workgroups (the first) and more, whose waves walk two steps of rows: rows of one, two and three chunks a lane
+    # with a remainder, 4 or 2 row pairs a step; rows of four chunks, which keep one step
+    test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, router_bits)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_config4_stack_of_24_layers_for_four_tokens(gpu, bits):
     """Config 4 as it is stated: 4 independent tokens through 24 stacked gpt-oss-shape layers (hidden = intermediate =
