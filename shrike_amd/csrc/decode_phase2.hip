@@ -20,13 +20,18 @@ __device__ __forceinline__ void phase2_finish(uint16_t *y, uint16_t *hidden, uin
 // rows. When a down row is shorter than a wave's 1 KiB load, the wave covers 64/cpr rows per
 // load and reduces over lane segments. BATCH row groups are in flight per wave.
 // STREAM: one token, every down row is read once: non-temporal row loads (see k_phase1).
-// ROWS: output rows a workgroup owns. Packed rows take 8. Rows of a wave load or more take as many as still leave the launch
-// 640 workgroups, two and a half a compute unit (more rows serve a wave's slice of the activations, fetched once, more often;
+// ROWS: output rows a workgroup owns. Packed rows take 8. Rows that take the wave, with more than a step a lane, take as many as still leave the
+// launch 640 workgroups, two and a half a compute unit (more rows serve a wave's slice of the activations, fetched once, more often;
 // with fewer workgroups too few loads are in flight): one token at hidden 2,880, 4 rows for 8: 10.5 -> 7.9 us with 4-bit
 // codes, 12.9 -> 9.8 with 8-bit ones; two tokens, 8 for 16: 13.4 -> 10.8; four tokens keep 16 (17.6 against 18.7 with 8).
 // TAIL: the rows end in a step of half chunks (load_slice_regs); NCH then counts the whole steps ahead of it.
 // META: the type of the scales and biases (SHRIKE_META_*), known to the instance so that a row converts them one way.
-template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META>
+// WHOLE: a row takes the wave (rows of more than one step a lane, and those whose chunks do not divide 64): rows, their addresses and
+// the sums' steps are then scalar, where an instance for both kinds formed them a lane, and 47 registers leave the launch all its
+// waves, where it had 74. Short rows are bound by the vector units, not by memory (a wave's 8 rows of 1,024, 8-bit: 536 operations). A
+// layer of 16 tokens of 1,536 x 768, 67 -> 57 us; 12 of 2,816 x 1,408, 110 -> 98.5; 16 of 2,304 x 1,024, 8-bit, 161 -> 157 (the launch
+// reads 6.1 TB/s there); one token of 2,048 x 768, 15.4 -> 15.1.
+template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META, bool WHOLE>
 __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
     warm_kernel_arguments(a);
     typedef Chunk<BITS> C;
@@ -59,10 +64,7 @@ __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
         return;
     }
     const uint32_t cpr = a.f * BITS / 128u, groups = a.f / kGroup, row_bytes = cpr * 16u;
-    // (an instance for rows of more than one step a lane never packs rows: its segment is the wave, and the segment sums'
-    // selects fold away)
-    constexpr bool kWholeWave = NCH >= 2 || TAIL;
-    const bool packed = !kWholeWave && cpr < 64u && (64u % cpr) == 0u;
+    constexpr bool packed = !WHOLE;
     const uint32_t rpl = packed ? min(64u / cpr, kPhase2Rows) : 1u;  // rows per wave load
     const uint32_t seg = packed ? cpr : 64u;
     const uint32_t sub = packed ? lane / cpr : 0u, col = packed ? lane % cpr : lane;
@@ -111,18 +113,18 @@ __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
                                     s_all + size_t(rr) * groups, b_all + size_t(rr) * groups, cpr, col, on[j]);
             }
             uint16_t own[BATCH];
-            if (!kWholeWave && a.ebias) {  // (one branch round all of them: a choice a row was a branch a row, 45 -> 50 us for
+            if (!WHOLE && a.ebias) {  // (one branch round all of them: a choice a row was a branch a row, 45 -> 50 us for
                                            // four tokens of 2,048 x 1,024, 8-bit)
 #pragma unroll
                 for (int j = 0; j < BATCH; ++j) own[j] = biases[on[j] ? row[j] : 0u];
             }
-            if (kWholeWave && a.ebias && g0 == 0 && lane < kPhase2Rows && d0 + lane < a.d) bias = biases[d0 + lane];
+            if (WHOLE && a.ebias && g0 == 0 && lane < kPhase2Rows && d0 + lane < a.d) bias = biases[d0 + lane];
             if (g0 == 0) unpack_slices<BITS, NCH, TAIL>(xr, x, xs, xt);
 #pragma unroll
             for (int j = 0; j < BATCH; ++j) {
                 const float v = seg_sum(row_partial<BITS, NCH, TAIL>(rows[j], x, xs, xt, uint32_t(META)), seg);
                 const bool writer = on[j] && writer_lane;
-                const uint32_t row_bias = kWholeWave ? uint32_t(__builtin_amdgcn_readlane(int(bias), int(g0) + j)) : own[j];
+                const uint32_t row_bias = WHOLE ? uint32_t(__builtin_amdgcn_readlane(int(bias), int(g0) + j)) : own[j];
                 if (writer) partial[k][row[j] - d0] = wk * (a.ebias ? v + bf16_to_f32(uint16_t(row_bias)) : v);  // moe.metal:1049
             }
         }
@@ -143,37 +145,52 @@ __global__ __launch_bounds__(256) void k_gemv(GemvArgs a) {
     gemv_job<BITS, NCH>(a, blockIdx.x);
 }
 
-template <int BITS, int NCH, uint32_t ROWS, bool TAIL, int META>
+inline bool packed_rows(uint32_t cpr) { return cpr < 64u && 64u % cpr == 0u; }
+
+template <int BITS, int NCH, uint32_t ROWS, bool TAIL, int META, bool WHOLE>
 static void launch_phase2_meta(const Phase2Args &a, dim3 block, hipStream_t s) {
     const dim3 grid((a.d + ROWS - 1) / ROWS, a.tokens ? a.tokens : 1u);
     const uint32_t cpr = a.f * BITS / 128u;
-    const uint32_t rpl = (cpr < 64u && 64u % cpr == 0u) ? (64u / cpr < ROWS ? 64u / cpr : ROWS) : 1u;
+    const uint32_t rpl = WHOLE ? 1u : (64u / cpr < ROWS ? 64u / cpr : ROWS);
     const uint32_t n_groups = ROWS / rpl;  // row groups per wave; up to 4 in flight
     if (a.tokens <= 1u) {
-        if (n_groups >= 4) hipLaunchKernelGGL((k_phase2<BITS, NCH, 4, true, ROWS, TAIL, META>), grid, block, 0, s, a);
-        else if (n_groups == 2) hipLaunchKernelGGL((k_phase2<BITS, NCH, 2, true, ROWS, TAIL, META>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_phase2<BITS, NCH, 1, true, ROWS, TAIL, META>), grid, block, 0, s, a);
+        if (n_groups >= 4) hipLaunchKernelGGL((k_phase2<BITS, NCH, 4, true, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
+        else if constexpr (!WHOLE) {
+            if (n_groups == 2) hipLaunchKernelGGL((k_phase2<BITS, NCH, 2, true, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
+            else hipLaunchKernelGGL((k_phase2<BITS, NCH, 1, true, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
+        }
     } else {
-        if (n_groups >= 4) hipLaunchKernelGGL((k_phase2<BITS, NCH, 4, false, ROWS, TAIL, META>), grid, block, 0, s, a);
-        else if (n_groups == 2) hipLaunchKernelGGL((k_phase2<BITS, NCH, 2, false, ROWS, TAIL, META>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((k_phase2<BITS, NCH, 1, false, ROWS, TAIL, META>), grid, block, 0, s, a);
+        if (n_groups >= 4) hipLaunchKernelGGL((k_phase2<BITS, NCH, 4, false, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
+        else if constexpr (!WHOLE) {
+            if (n_groups == 2) hipLaunchKernelGGL((k_phase2<BITS, NCH, 2, false, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
+            else hipLaunchKernelGGL((k_phase2<BITS, NCH, 1, false, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
+        }
     }
 }
 
-template <int BITS, int NCH, uint32_t ROWS, bool TAIL>
+template <int BITS, int NCH, uint32_t ROWS, bool TAIL, bool WHOLE>
 static void launch_phase2_rows(const Phase2Args &a, dim3 block, hipStream_t s) {
-    if (a.meta == SHRIKE_META_F16) launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_F16>(a, block, s);
-    else launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_BF16>(a, block, s);
+    if (a.meta == SHRIKE_META_F16) launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_F16, WHOLE>(a, block, s);
+    else launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_BF16, WHOLE>(a, block, s);
 }
 
 template <int BITS, int NCH, bool TAIL>
 static void launch_phase2_batch(const Phase2Args &a, dim3 block, hipStream_t s) {
     constexpr bool kLong = NCH >= 2 || TAIL;  // rows of more than one step a lane, whole or half
-    const uint32_t tokens = a.tokens ? a.tokens : 1u, cpr = a.f * BITS / 128u;
-    auto enough = [&](uint32_t rows) { return uint64_t(tokens) * ((a.d + rows - 1u) / rows) >= 640u; };
-    if (kLong && enough(16u)) launch_phase2_rows<BITS, NCH, 16u, TAIL>(a, block, s);
-    else if (enough(8u) || (cpr < 64u && 64u % cpr == 0u)) launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL>(a, block, s);
-    else launch_phase2_rows<BITS, NCH, 4u, TAIL>(a, block, s);
+    const uint32_t tokens = a.tokens ? a.tokens : 1u;
+    // (rows of one step a lane: 16 from 1,536 workgroups on. A layer with 8 and with 16, us: 1,536, 16 tokens of 1,536 x 768, 59 and
+    // 57; 12 of 2,048 x 768, 64 and 61.5; 2,304, 16 of 2,304 x 1,024, 8-bit, 159 and 157; 1,152, 8 of them, 88 and 90)
+    constexpr uint32_t kEnough16 = kLong ? 640u : 1536u;
+    auto groups = [&](uint32_t rows) { return uint64_t(tokens) * ((a.d + rows - 1u) / rows); };
+    if constexpr (!kLong) {
+        if (packed_rows(a.f * BITS / 128u)) {
+            launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, false>(a, block, s);
+            return;
+        }
+    }
+    if (groups(16u) >= kEnough16) launch_phase2_rows<BITS, NCH, 16u, TAIL, true>(a, block, s);
+    else if (groups(8u) >= 640u) launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, true>(a, block, s);
+    else launch_phase2_rows<BITS, NCH, 4u, TAIL, true>(a, block, s);
 }
 
 template <int BITS>

@@ -671,6 +671,12 @@ def test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, 
     assert_ffn_close(all_y[:d], ref_y, "token 0 y from the device's activations")
 
 
+@pytest.mark.parametrize("d,f,ne,k,t,bits", [(1024, 768, 16, 4, 24, 4), (1088, 960, 16, 8, 7, 8), (1024, 960, 16, 3, 23, 4), (256, 2048, 8, 2, 3, 4)])
+def test_batched_decode_operators_with_down_rows_of_a_wave(gpu, d, f, ne, k, t, bits):
+    # down rows that take a wave with one step a lane: 24, 60, 30 and 64 chunks; 4, 8 and 16 rows a workgroup (from 1,536 of them, just below)
+    test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, t, bits)
+
+
 @pytest.mark.parametrize("d,f,ne,k,t,bits,router_bits", [(2880, 2880, 32, 4, 4, 4, 0), (2880, 2880, 32, 4, 4, 8, 0), (512, 256, 40, 8, 16, 4, 8),
                                                           (2304, 1024, 256, 8, 5, 8, 0), (256, 128, 8, 3, 1, 4, 4)])
 def test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, router_bits):
