@@ -26,12 +26,13 @@ __device__ __forceinline__ void phase2_finish(uint16_t *y, uint16_t *hidden, uin
 // codes, 12.9 -> 9.8 with 8-bit ones; two tokens, 8 for 16: 13.4 -> 10.8; four tokens keep 16 (17.6 against 18.7 with 8).
 // TAIL: the rows end in a step of half chunks (load_slice_regs); NCH then counts the whole steps ahead of it.
 // META: the type of the scales and biases (SHRIKE_META_*), known to the instance so that a row converts them one way.
-// WHOLE: a row takes the wave (rows of more than one step a lane, and those whose chunks do not divide 64): rows, their addresses and
-// the sums' steps are then scalar, where an instance for both kinds formed them a lane, and 47 registers leave the launch all its
-// waves, where it had 74. Short rows are bound by the vector units, not by memory (a wave's 8 rows of 1,024, 8-bit: 536 operations). A
-// layer of 16 tokens of 1,536 x 768, 67 -> 57 us; 12 of 2,816 x 1,408, 110 -> 98.5; 16 of 2,304 x 1,024, 8-bit, 161 -> 157 (the launch
-// reads 6.1 TB/s there); one token of 2,048 x 768, 15.4 -> 15.1.
-template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META, bool WHOLE>
+// SEG: the lanes of a row, 64 (rows of more than one step a lane, and those whose chunks do not divide 64) or the chunks of a packed
+// row. Known to the instance, the rows, their addresses and the sums' steps are scalar or shifts: found at run time they were two
+// divisions ahead of the first load and a select behind every step (one token of 2,048 x 512, three launches and a shared expert: 13.7 ->
+// 13.2 us), and 74 registers where 47 leave a launch all its waves. Short rows in a large batch are bound by the vector units (536
+// operations for a wave's 8 rows of 1,024, 8-bit): a layer of 16 tokens of 1,536 x 768, 67 -> 57 us; 12 of 2,816 x 1,408, 110 -> 98.5; 16
+// of 2,304 x 1,024, 8-bit, 161 -> 157 (the launch reads 6.1 TB/s there); 8 of 2,048 x 1,024, 52.4 -> 50.7.
+template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META, int SEG>
 __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
     warm_kernel_arguments(a);
     typedef Chunk<BITS> C;
@@ -64,10 +65,9 @@ __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
         return;
     }
     const uint32_t cpr = a.f * BITS / 128u, groups = a.f / kGroup, row_bytes = cpr * 16u;
-    constexpr bool packed = !WHOLE;
-    const uint32_t rpl = packed ? min(64u / cpr, kPhase2Rows) : 1u;  // rows per wave load
-    const uint32_t seg = packed ? cpr : 64u;
-    const uint32_t sub = packed ? lane / cpr : 0u, col = packed ? lane % cpr : lane;
+    constexpr bool kWholeWave = SEG == 64;
+    constexpr uint32_t seg = SEG, rpl = 64u / seg < ROWS ? 64u / seg : ROWS;  // rows per wave load
+    const uint32_t sub = lane / seg, col = lane % seg;
     const bool lane_on = sub < rpl;
     const bool writer_lane = (lane & (seg - 1u)) == seg - 1u;  // a segment is a power of two lanes: 64, or a divisor of it
 
@@ -113,18 +113,18 @@ __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
                                     s_all + size_t(rr) * groups, b_all + size_t(rr) * groups, cpr, col, on[j]);
             }
             uint16_t own[BATCH];
-            if (!WHOLE && a.ebias) {  // (one branch round all of them: a choice a row was a branch a row, 45 -> 50 us for
+            if (!kWholeWave && a.ebias) {  // (one branch round all of them: a choice a row was a branch a row, 45 -> 50 us for
                                            // four tokens of 2,048 x 1,024, 8-bit)
 #pragma unroll
                 for (int j = 0; j < BATCH; ++j) own[j] = biases[on[j] ? row[j] : 0u];
             }
-            if (WHOLE && a.ebias && g0 == 0 && lane < kPhase2Rows && d0 + lane < a.d) bias = biases[d0 + lane];
+            if (kWholeWave && a.ebias && g0 == 0 && lane < kPhase2Rows && d0 + lane < a.d) bias = biases[d0 + lane];
             if (g0 == 0) unpack_slices<BITS, NCH, TAIL>(xr, x, xs, xt);
 #pragma unroll
             for (int j = 0; j < BATCH; ++j) {
                 const float v = seg_sum(row_partial<BITS, NCH, TAIL>(rows[j], x, xs, xt, uint32_t(META)), seg);
                 const bool writer = on[j] && writer_lane;
-                const uint32_t row_bias = WHOLE ? uint32_t(__builtin_amdgcn_readlane(int(bias), int(g0) + j)) : own[j];
+                const uint32_t row_bias = kWholeWave ? uint32_t(__builtin_amdgcn_readlane(int(bias), int(g0) + j)) : own[j];
                 if (writer) partial[k][row[j] - d0] = wk * (a.ebias ? v + bf16_to_f32(uint16_t(row_bias)) : v);  // moe.metal:1049
             }
         }
@@ -145,33 +145,19 @@ __global__ __launch_bounds__(256) void k_gemv(GemvArgs a) {
     gemv_job<BITS, NCH>(a, blockIdx.x);
 }
 
-inline bool packed_rows(uint32_t cpr) { return cpr < 64u && 64u % cpr == 0u; }
-
-template <int BITS, int NCH, uint32_t ROWS, bool TAIL, int META, bool WHOLE>
+template <int BITS, int NCH, uint32_t ROWS, bool TAIL, int META, int SEG>
 static void launch_phase2_meta(const Phase2Args &a, dim3 block, hipStream_t s) {
     const dim3 grid((a.d + ROWS - 1) / ROWS, a.tokens ? a.tokens : 1u);
-    const uint32_t cpr = a.f * BITS / 128u;
-    const uint32_t rpl = WHOLE ? 1u : (64u / cpr < ROWS ? 64u / cpr : ROWS);
-    const uint32_t n_groups = ROWS / rpl;  // row groups per wave; up to 4 in flight
-    if (a.tokens <= 1u) {
-        if (n_groups >= 4) hipLaunchKernelGGL((k_phase2<BITS, NCH, 4, true, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
-        else if constexpr (!WHOLE) {
-            if (n_groups == 2) hipLaunchKernelGGL((k_phase2<BITS, NCH, 2, true, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_phase2<BITS, NCH, 1, true, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
-        }
-    } else {
-        if (n_groups >= 4) hipLaunchKernelGGL((k_phase2<BITS, NCH, 4, false, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
-        else if constexpr (!WHOLE) {
-            if (n_groups == 2) hipLaunchKernelGGL((k_phase2<BITS, NCH, 2, false, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
-            else hipLaunchKernelGGL((k_phase2<BITS, NCH, 1, false, ROWS, TAIL, META, WHOLE>), grid, block, 0, s, a);
-        }
-    }
+    constexpr uint32_t rpl = 64u / SEG < ROWS ? 64u / SEG : ROWS;
+    constexpr int kBatch = ROWS / rpl < 4u ? int(ROWS / rpl) : 4;  // row groups per wave; up to 4 in flight
+    if (a.tokens <= 1u) hipLaunchKernelGGL((k_phase2<BITS, NCH, kBatch, true, ROWS, TAIL, META, SEG>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((k_phase2<BITS, NCH, kBatch, false, ROWS, TAIL, META, SEG>), grid, block, 0, s, a);
 }
 
-template <int BITS, int NCH, uint32_t ROWS, bool TAIL, bool WHOLE>
+template <int BITS, int NCH, uint32_t ROWS, bool TAIL, int SEG>
 static void launch_phase2_rows(const Phase2Args &a, dim3 block, hipStream_t s) {
-    if (a.meta == SHRIKE_META_F16) launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_F16, WHOLE>(a, block, s);
-    else launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_BF16, WHOLE>(a, block, s);
+    if (a.meta == SHRIKE_META_F16) launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_F16, SEG>(a, block, s);
+    else launch_phase2_meta<BITS, NCH, ROWS, TAIL, SHRIKE_META_BF16, SEG>(a, block, s);
 }
 
 template <int BITS, int NCH, bool TAIL>
@@ -183,14 +169,18 @@ static void launch_phase2_batch(const Phase2Args &a, dim3 block, hipStream_t s) 
     constexpr uint32_t kEnough16 = kLong ? 640u : 1536u;
     auto groups = [&](uint32_t rows) { return uint64_t(tokens) * ((a.d + rows - 1u) / rows); };
     if constexpr (!kLong) {
-        if (packed_rows(a.f * BITS / 128u)) {
-            launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, false>(a, block, s);
-            return;
+        switch (a.f * BITS / 128u) {  // packed rows (f is a multiple of 64: two chunks or more)
+            case 2: launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, 2>(a, block, s); return;
+            case 4: launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, 4>(a, block, s); return;
+            case 8: launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, 8>(a, block, s); return;
+            case 16: launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, 16>(a, block, s); return;
+            case 32: launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, 32>(a, block, s); return;
+            default: break;
         }
     }
-    if (groups(16u) >= kEnough16) launch_phase2_rows<BITS, NCH, 16u, TAIL, true>(a, block, s);
-    else if (groups(8u) >= 640u) launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, true>(a, block, s);
-    else launch_phase2_rows<BITS, NCH, 4u, TAIL, true>(a, block, s);
+    if (groups(16u) >= kEnough16) launch_phase2_rows<BITS, NCH, 16u, TAIL, 64>(a, block, s);
+    else if (groups(8u) >= 640u) launch_phase2_rows<BITS, NCH, kPhase2Rows, TAIL, 64>(a, block, s);
+    else launch_phase2_rows<BITS, NCH, 4u, TAIL, 64>(a, block, s);
 }
 
 template <int BITS>

@@ -277,10 +277,12 @@ __device__ __forceinline__ void gemv_job(const GemvArgs &a, uint32_t block, XSou
     typedef Chunk<BITS> C;
     const uint32_t lane = threadIdx.x & 63u, wave = wave_index();
     const uint32_t cpr = a.n * BITS / 128u, groups = a.n / kGroup, row_bytes = cpr * 16u;
-    const bool packed = NCH == 1 && cpr < 64u && (64u % cpr) == 0u;  // (NCH >= 2: more than 64 chunks a row, known to the instance)
-    const uint32_t rpl = packed ? 64u / cpr : 1u;
+    // (NCH >= 2: more than 64 chunks a row, known to the instance; below 64, what divides it is a power of two: no division here)
+    const bool packed = NCH == 1 && cpr < 64u && (cpr & (cpr - 1u)) == 0u;
+    const uint32_t shift = uint32_t(__builtin_ctz(cpr));
+    const uint32_t rpl = packed ? 64u >> shift : 1u;
     const uint32_t seg = packed ? cpr : 64u;
-    const uint32_t sub = packed ? lane / cpr : 0u, col = packed ? lane % cpr : lane;
+    const uint32_t sub = packed ? lane >> shift : 0u, col = packed ? lane & (cpr - 1u) : lane;
     const uint32_t total = a.rows + a.rows_b;
     const uint32_t first = (block * 4u + wave) * kGemvRowsPerWave * rpl;
     const bool active = first < total;

@@ -671,9 +671,10 @@ def test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, 
     assert_ffn_close(all_y[:d], ref_y, "token 0 y from the device's activations")
 
 
-@pytest.mark.parametrize("d,f,ne,k,t,bits", [(1024, 768, 16, 4, 24, 4), (1088, 960, 16, 8, 7, 8), (1024, 960, 16, 3, 23, 4), (256, 2048, 8, 2, 3, 4)])
-def test_batched_decode_operators_with_down_rows_of_a_wave(gpu, d, f, ne, k, t, bits):
-    # down rows that take a wave with one step a lane: 24, 60, 30 and 64 chunks; 4, 8 and 16 rows a workgroup (from 1,536 of them, just below)
+@pytest.mark.parametrize("d,f,ne,k,t,bits", [(1024, 768, 16, 4, 24, 4), (1088, 960, 16, 8, 7, 8), (1024, 960, 16, 3, 23, 4), (256, 2048, 8, 2, 3, 4),
+                                              (192, 64, 8, 2, 3, 4), (192, 64, 8, 2, 3, 8), (320, 512, 8, 2, 3, 8)])
+def test_batched_decode_operators_over_down_rows_of_one_step(gpu, d, f, ne, k, t, bits):
+    # down rows that take a wave: 24, 60, 30 and 64 chunks; 4, 8 and 16 rows a workgroup (from 1,536 of them, just below). Packed rows: 2, 4, 32 chunks
     test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, t, bits)
 
 
