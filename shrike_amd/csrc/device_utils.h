@@ -64,6 +64,39 @@ __device__ __forceinline__ float wave_sum(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// The butterfly sums of reproducible orders, v + (v of lane ^ o) step by step, in every lane; all lanes of the wave must be
+// active. Each step is one vector operation or a swap and an addition, where an exchange by lane index goes through the LDS
+// unit, 100 cycles and more a step (k_prefill_select with its group sums, 37 tokens, 6.8 -> 5.6 us; k_scalar_gate_rows, 37 rows 3.8 -> 3.2;
+// the decode router's launch, 32 rows of 512, 3.8 -> 3.6). Two summands in either order are one sum, and after the steps 32, 16 and 8 lanes that differ in those bits only hold the same value, so a rotation
+// by 4 within 16 lanes serves for ^ 4; so do, in rising order, the mirrors of 8 and of 16 lanes for ^ 4 and ^ 8.
+__device__ __forceinline__ float add_xor32(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float add_xor16(float v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// o = 32, 16, 8, 4, 2, 1
+__device__ __forceinline__ float butterfly_from_32(float v) {
+    v = add_xor16(add_xor32(v));
+    v = __fadd_rn(v, dpp_f32<0x128>(v));  // row_ror 8
+    v = __fadd_rn(v, dpp_f32<0x124>(v));  // row_ror 4
+    v = __fadd_rn(v, dpp_f32<0x4E>(v));   // quad_perm [2,3,0,1]
+    return __fadd_rn(v, dpp_f32<0xB1>(v));  // quad_perm [1,0,3,2]
+}
+// o = 1, 2, 4: sums of eight neighbouring lanes
+__device__ __forceinline__ float butterfly_of_8(float v) {
+    v = __fadd_rn(v, dpp_f32<0xB1>(v));
+    v = __fadd_rn(v, dpp_f32<0x4E>(v));
+    return __fadd_rn(v, dpp_f32<0x141>(v));  // row_half_mirror
+}
+// o = 1, 2, 4, 8, 16: sums of half a wave
+__device__ __forceinline__ float butterfly_of_32(float v) {
+    v = butterfly_of_8(v);
+    return add_xor16(__fadd_rn(v, dpp_f32<0x140>(v)));  // row_mirror
+}
+
 // The wave's index in its workgroup, as a scalar: what is derived from it (rows, routed
 // position, the cell and its base) then lives in scalar registers and scalar loads.
 __device__ __forceinline__ uint32_t wave_index() { return uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))); }

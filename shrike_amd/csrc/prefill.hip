@@ -488,9 +488,7 @@ __global__ __launch_bounds__(256) void k_prefill_select(SelectArgs sel, const fl
                 sum = __fadd_rn(sum, f16_to_f32(uint16_t(xw[q])));
                 sum = __fadd_rn(sum, f16_to_f32(uint16_t(xw[q] >> 16)));
             }
-            sum = __fadd_rn(sum, __shfl_xor(sum, 1));
-            sum = __fadd_rn(sum, __shfl_xor(sum, 2));
-            sum = __fadd_rn(sum, __shfl_xor(sum, 4));
+            sum = butterfly_of_8(sum);
             if (c < chunks && (c & 7u) == 0u) group_sums[size_t(t) * (d / 64u) + (c >> 3)] = split_hi_lo(sum);  // d % 64 == 0: whole groups
         }
     }
@@ -638,7 +636,7 @@ __global__ __launch_bounds__(256 * PARTS) void k_group(GroupArgs a) {
                 if (valid < 16u) match &= (1u << valid) - 1u;
             }
             const uint32_t mine = __popc(match);
-            const uint32_t upto = wave_inclusive_scan_u32(mine, lane);
+            const uint32_t upto = wave_inclusive_scan_u32(mine);
             uint32_t at = offset + running + upto - mine;
             while (match) {
                 const uint32_t i = i0 + uint32_t(__ffs(int(match)) - 1);
@@ -699,9 +697,7 @@ __global__ __launch_bounds__(256) void k_row_group_sums(const uint16_t *src, siz
             s = __fadd_rn(s, f16_to_f32(uint16_t(w[t] >> 16)));
         }
     }
-    s = __fadd_rn(s, __shfl_xor(s, 1));
-    s = __fadd_rn(s, __shfl_xor(s, 2));
-    s = __fadd_rn(s, __shfl_xor(s, 4));
+    s = butterfly_of_8(s);
     if (on && (rest & 7u) == 0u) out[size_t(row) * groups + rest / 8u] = split_hi_lo(s);
 }
 
@@ -775,8 +771,7 @@ __global__ __launch_bounds__(256) void k_scalar_gate_rows(const uint8_t *w, cons
         acc = fmaf(meta_f32(scales[g], meta), dot, acc);
         acc = fmaf(meta_f32(biases[g], meta), __fadd_rn(x0, x1), acc);
     }
-#pragma unroll
-    for (int o = 1; o <= 16; o <<= 1) acc = __fadd_rn(acc, __shfl_xor(acc, o));
+    acc = butterfly_of_32(acc);
     if (l == 0) s_partial[p] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {

@@ -47,8 +47,7 @@ __device__ __forceinline__ void rmsnorm_row(uint16_t *hidden_row, const uint16_t
             acc = fmaf(hi, hi, acc);
         }
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) acc = __fadd_rn(acc, __shfl_xor(acc, o));
+    acc = butterfly_from_32(acc);
     if ((threadIdx.x & 63u) == 0) s_partial[threadIdx.x >> 6] = acc;
     __syncthreads();
     const float total = __fadd_rn(__fadd_rn(__fadd_rn(s_partial[0], s_partial[1]), s_partial[2]), s_partial[3]);

@@ -85,8 +85,7 @@ __device__ __forceinline__ float router_row_n(const RouterArgs &a, XSource &&x_s
             }
         }
     }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) acc = __fadd_rn(acc, __shfl_xor(acc, o));
+    acc = butterfly_from_32(acc);
     // publish: the logit is for another workgroup of the same launch and is written through to
     // device-coherent memory
     if (lane == 0) {
