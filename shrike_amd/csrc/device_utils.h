@@ -66,9 +66,10 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 // The butterfly sums of reproducible orders, v + (v of lane ^ o) step by step, in every lane; all lanes of the wave must be
 // active. Each step is one vector operation or a swap and an addition, where an exchange by lane index goes through the LDS
-// unit, 100 cycles and more a step (k_prefill_select with its group sums, 37 tokens, 6.8 -> 5.6 us; k_scalar_gate_rows, 37 rows 3.8 -> 3.2;
-// the decode router's launch, 32 rows of 512, 3.8 -> 3.6). Two summands in either order are one sum, and after the steps 32, 16 and 8 lanes that differ in those bits only hold the same value, so a rotation
-// by 4 within 16 lanes serves for ^ 4; so do, in rising order, the mirrors of 8 and of 16 lanes for ^ 4 and ^ 8.
+// unit, 100 cycles and more a step (k_prefill_select with its group sums, 37 tokens, 6.8 -> 5.6 us; k_scalar_gate_rows, 37
+// rows, 3.8 -> 3.2; the decode router's launch, 32 rows of 512, 3.8 -> 3.6). Two summands in either order are one sum, and
+// after the steps 32, 16 and 8 lanes that differ in those bits only hold the same value, so a rotation by 4 within 16 lanes
+// serves for ^ 4; so do, in rising order, the mirrors of 8 and of 16 lanes for ^ 4 and ^ 8.
 __device__ __forceinline__ float add_xor32(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
