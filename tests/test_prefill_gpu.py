@@ -804,6 +804,21 @@ def test_prefill_layer_at_full_size_agrees_with_the_decode_kernels(gpu):
         assert_rel_close(out[tok], dl.y.download(np.uint16, d), f"token {tok}: prefill h2 vs decode y", tol=2e-3)
 
 
+@pytest.mark.parametrize("rows", [2047, 2048, 2049, 2051])
+def test_scalar_gate_of_many_rows(gpu, rows):
+    # four rows a workgroup from 2,048 on, the last ones short of four; rows of nine groups, one more than the half-waves
+    d, stride = 576, 584
+    L = Layer(0x5EED0009, d, 64, 4, 2)
+    x = token_rows(L, rows, stride)
+    row = S.affine_matrix(L.tree.key("shared.scalar_gate"), 1, d, 8, L.meta)
+    gates = gpu.dev(np.full(rows + 1, 0xD4D0, np.uint16))
+    pf = gpu.Prefill(DeviceLayer(gpu, L, resident=[]).moe)
+    pf.encode_scalar_gate_rows(tuple(gpu.dev(a) for a in row), gpu.dev(x), stride, gates, rows, d)
+    gpu.synchronize()
+    got = gates.download(np.uint16, rows + 1)
+    assert np.array_equal(got[:rows], O.shared_scalar_gate_rows(row, x, rows, d, x_stride=stride, meta=L.meta)) and got[rows] == 0xD4D0
+
+
 @pytest.mark.parametrize("d,fs,bits,t,gated", [(2048, 512, 4, 20, False), (2048, 512, 4, 70, True), (2304, 1024, 8, 16, True),
                                               (192, 320, 4, 70, False), (128, 64, 8, 1, True)])
 def test_shared_expert_for_a_token_block(gpu, d, fs, bits, t, gated):
