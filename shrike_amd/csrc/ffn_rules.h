@@ -74,18 +74,21 @@ inline FfnShape dense_shape(uint64_t rows, uint32_t f) {
     return (rows + 31u) / 32u * (f / 32u) <= 1024u ? FfnShape::kSplit : FfnShape::kDeep;
 }
 
-// Whether the codes of that many experts are more than the memory-side cache (256 MB) holds, with an eighth to spare: what passes
+// The bytes of an expert's codes, scales and biases, wherever its cell lies.
+constexpr uint64_t expert_bytes(uint32_t d, uint32_t f, uint32_t bits) { return 3ull * d * f * bits / 8u + 3ull * d * f / 64u * 4u; }
+
+// Whether that many experts are more than the memory-side cache (256 MB) holds, with an eighth to spare: what passes
 // by the caches is then nothing that the next pass would have found there. Whole passes over one pool again and again, 8-bit, kDeep
 // against non-temporal lines, us: in use 108 MB 85, 91 (128 experts of 832 x 1,408, uneven); 214 MB 72, 77 (128 of 1,024 x 512);
 // 267 MB 115, 116 (256 of 2,048 x 512, uneven); 321 MB 93, 86 (48 of 2,048 x 1,024); 369 MB 142, 127 (64 of 1,088 x 1,664); 428 MB
 // 113, 106 (128 of 1,024 x 1,024); 820 MB 341, 310 (256 of 2,304 x 1,024, uneven); 1.9 GB 467, 415 (even).
-constexpr bool past_the_cache(uint64_t experts, uint64_t blob_bytes) { return experts * blob_bytes >= 288ull << 20; }
+constexpr bool past_the_cache(uint64_t experts, uint32_t d, uint32_t f, uint32_t bits) { return experts * expert_bytes(d, f, bits) >= 288ull << 20; }
 
 // kLines in kDeep's place, where the rows are whole lines from their first byte (`align`: all that a row's address is made of, or-ed)
 // and the experts that may be in use are more than the memory-side cache holds. Where they turn out to be fewer, its loads go
 // without the hint, and are as fast as kDeep's. (Rows that lines run across: 128 experts of 1,088 x 576, 500 tokens 85 -> 90 us.)
-inline FfnShape lines_shape(FfnShape shape, uint64_t pairs, uint32_t experts, uint32_t bits, uint64_t blob_bytes, uint64_t align) {
-    return shape == FfnShape::kDeep && bits == 8 && align % 128u == 0 && past_the_cache(std::min(pairs, uint64_t(experts)), blob_bytes)
+inline FfnShape lines_shape(FfnShape shape, uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits, uint64_t align) {
+    return shape == FfnShape::kDeep && bits == 8 && align % 128u == 0 && past_the_cache(std::min(pairs, uint64_t(experts)), d, f, bits)
                ? FfnShape::kLines
                : shape;
 }

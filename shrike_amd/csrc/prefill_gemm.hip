@@ -79,7 +79,6 @@ struct FfnArgs {
     const uint16_t *scalar_gate;   // fp16[rows] or null: row m's output * sigmoid(gate[m]) (moe.metal:1195-1207)
     uint32_t table_room;           // records that the tile table has room for
     uint32_t resident_workgroups;  // workgroups of the launched k_grouped_ffn the device holds at once
-    uint64_t blob_bytes;           // of an expert
 };
 
 // The sum of a group of 64 fp16 values of which eight neighbouring lanes hold eight each, in every one of them: a lane's
@@ -935,7 +934,7 @@ __global__ __launch_bounds__(256, (Lds<S, BITS>::kResident)) void k_grouped_ffn(
         auto last_tiles = [&](const uint4 &rec, uint32_t at) { return uint32_t(__popcll(__ballot(lane + at < tile_total && rec.z < kRowTile))); };
         const uint32_t in_use = last_tiles(rec0, 0) + last_tiles(rec1, 64) + last_tiles(rec2, 128) + last_tiles(rec3, 192);
         const bool in_two = larger != 0u && ((larger >> tile_index) & 1u) != 0u;
-        once = tile.rows < kRowTile && !in_two && past_the_cache(in_use, a.blob_bytes);
+        once = tile.rows < kRowTile && !in_two && past_the_cache(in_use, a.d, a.f, BITS);
     }
     if (WIDE && tile.rows > 96u) ffn_tile<BITS, MODE, DENSE, WIDE ? 4 : 2, META, S>(a, tile, act_row, col_block, lds, once);
     else if (WIDE && tile.rows > 64u) ffn_tile<BITS, MODE, DENSE, WIDE ? 3 : 2, META, S>(a, tile, act_row, col_block, lds, once);
@@ -1349,8 +1348,7 @@ static int grouped_ffn(shrike_hip_moe *moe, void *stream, const shrike_pool_base
     FfnShape shape = routed_shape(uint64_t(query_count) * top_k, moe->desc.num_experts, d, f, moe->desc.routed_weight_bits);
     uint64_t align = pool_slot_stride | offsets->gate_w_off | offsets->up_w_off | offsets->down_w_off | d | f;  // (a row of 8-bit codes is d or f bytes)
     for (const void *base : pool->base) align |= reinterpret_cast<uintptr_t>(base);
-    a.blob_bytes = pool_slot_stride;
-    shape = lines_shape(shape, uint64_t(query_count) * top_k, moe->desc.num_experts, moe->desc.routed_weight_bits, a.blob_bytes, align);
+    shape = lines_shape(shape, uint64_t(query_count) * top_k, moe->desc.num_experts, d, f, moe->desc.routed_weight_bits, align);
     if (shape != FfnShape::kSplit && uint64_t(query_count) * hidden_stride_elements * 2u > 0xffffffffull) shape = FfnShape::kDeep;  // (the others' rows are 32-bit offsets)
     return moe->desc.routed_weight_bits == 8 ? launch_ffn<8, false>(a, max_row_tiles, shape, s) : launch_ffn<4, false>(a, max_row_tiles, shape, s);
 }

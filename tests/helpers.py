@@ -46,15 +46,16 @@ class Layer:
     """One synthetic MoE layer: E routed expert blobs, router, optional shared expert."""
 
     def __init__(self, seed, d, f, num_experts, top_k, bits=4, meta=S.META_BF16, router_bits=0,
-                 shared_f=0, shared_bits=None, additive_biases=False, label="layer.0"):
+                 shared_f=0, shared_bits=None, additive_biases=False, label="layer.0", distinct=None):
+        """distinct: of the experts' blobs, where making them all would take long; expert e has number e % distinct."""
         self.d, self.f, self.ne, self.k = d, f, num_experts, top_k
         self.bits, self.meta, self.router_bits = bits, meta, router_bits
         self.additive = additive_biases
         tree = S.SeedTree(seed)
         self.tree = tree
         self.off, self.stride = S.expert_offsets(d, f, bits, additive_biases)
-        self.blobs = [S.expert_blob(tree, f"{label}.expert.{e}", d, f, bits, meta, additive_biases)
-                      for e in range(num_experts)]
+        made = [S.expert_blob(tree, f"{label}.expert.{e}", d, f, bits, meta, additive_biases) for e in range(distinct or num_experts)]
+        self.blobs = [made[e % len(made)] for e in range(num_experts)]
         # router
         if router_bits == 0:
             self.router_w = S.router_f16(tree, f"{label}.router.w", num_experts, d)
@@ -98,15 +99,17 @@ extern "C" const char *routed_shape(uint64_t pairs, uint32_t experts, uint32_t d
     static const char *const names[] = {"split", "tile", "deep", "wide"};
     return names[int(shrike::routed_shape(pairs, experts, d, f, bits))];
 }
-extern "C" bool takes_lines(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits, uint64_t blob_bytes, uint64_t align) {
+extern "C" bool takes_lines(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits, uint64_t align) {
     const shrike::FfnShape shape = shrike::routed_shape(pairs, experts, d, f, bits);
-    return shrike::lines_shape(shape, pairs, experts, bits, blob_bytes, align) == shrike::FfnShape::kLines;
+    return shrike::lines_shape(shape, pairs, experts, d, f, bits, align) == shrike::FfnShape::kLines;
 }
+extern "C" bool past_the_cache(uint64_t experts, uint32_t d, uint32_t f, uint32_t bits) { return shrike::past_the_cache(experts, d, f, bits); }
 """
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/shrike_amd/csrc", "-x", "c++", "-", "-o", lib],
                        input=source.encode(), check=True)
         rules = C.CDLL(lib)
     rules.readable_records.argtypes, rules.readable_records.restype = [C.c_uint32, C.c_uint64, C.c_uint32], C.c_uint32
     rules.routed_shape.argtypes, rules.routed_shape.restype = [C.c_uint64, *[C.c_uint32] * 4], C.c_char_p
-    rules.takes_lines.argtypes, rules.takes_lines.restype = [C.c_uint64, *[C.c_uint32] * 4, C.c_uint64, C.c_uint64], C.c_bool
+    rules.takes_lines.argtypes, rules.takes_lines.restype = [C.c_uint64, *[C.c_uint32] * 4, C.c_uint64], C.c_bool
+    rules.past_the_cache.argtypes, rules.past_the_cache.restype = [C.c_uint64, *[C.c_uint32] * 3], C.c_bool
     return rules

@@ -24,3 +24,11 @@ def test_no_record_is_read_past_the_tables_room(tokens, top_k, experts):
     *[(t, ne, d, f, bits, shape) for d, f, ne, bits, chunks in T.CHUNK_CASES for t, shape in chunks.items()]])
 def test_the_gpu_tests_reach_the_shapes_they_name(pairs, experts, d, f, bits, shape):
     assert ffn_rules().routed_shape(pairs, experts, d, f, bits).decode() == shape
+
+
+@pytest.mark.parametrize("experts,d,f,lines", [(128, 1024, 512, False), (128, 1024, 1024, True), (48, 2048, 1024, True), (32, 2048, 1024, False)])
+def test_what_counts_against_the_cache_is_the_experts_bytes(experts, d, f, lines):
+    """Cells as far apart as a caller likes are no more bytes to read: the rule is asked with what the rows' addresses are made of, and
+    no spacing of whole lines changes its answer."""
+    for stride in (1 << 14, 1 << 21, 1 << 25):
+        assert ffn_rules().takes_lines(16 * experts, experts, d, f, 8, stride | d | f) == lines

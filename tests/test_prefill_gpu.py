@@ -421,34 +421,60 @@ def test_grouped_ffn_rings(gpu, d, f, ne, t, bits):
 
 
 # Units of two groups, one in all and around the ring of three places; experts of up to 32 rows, up to 64 and more; enough workgroups
-# for whole tiles, few enough tiles for their second halves to be workgroups of their own (the 8 experts), and fewer experts in use
-# than the pool has (the last: the hint is then left out).
-LINE_CASES = [  # d, f, experts, tokens, meta, experts in use
-    (128, 4096, 9, 40, S.META_F16, 9), (256, 2176, 70, 300, S.META_BF16, 70), (384, 1152, 70, 500, S.META_F16, 70), (512, 1024, 70, 700, S.META_BF16, 70),
-    (640, 768, 70, 900, S.META_F16, 70), (768, 640, 70, 700, S.META_BF16, 70), (1152, 896, 24, 300, S.META_F16, 24), (2304, 1024, 24, 150, S.META_BF16, 24),
-    (256, 4096, 8, 60, S.META_BF16, 8), (512, 1024, 70, 300, S.META_BF16, 9)]
+# for whole tiles, few enough tiles for their second halves to be workgroups of their own (the 12 experts). The experts in use are more
+# than the memory-side cache holds, but for the last: the hint is then left out.
+LINE_CASES = [  # d, f, experts, tokens, meta, experts that may be in use, whether the lines carry the hint
+    (128, 4096, 220, 800, S.META_F16, 220, True), (256, 2176, 210, 900, S.META_BF16, 210, True), (384, 1152, 250, 1000, S.META_F16, 250, True),
+    (512, 1024, 220, 1200, S.META_BF16, 220, True), (640, 768, 230, 1100, S.META_F16, 230, True), (768, 640, 230, 1100, S.META_BF16, 230, True),
+    (1152, 896, 110, 600, S.META_F16, 110, True), (2304, 1024, 50, 250, S.META_BF16, 50, True), (2048, 4096, 12, 60, S.META_BF16, 12, True),
+    (512, 1024, 190, 300, S.META_BF16, 9, False)]
 
 
-@pytest.mark.parametrize("d,f,ne,t,meta,in_use", LINE_CASES)
-def test_grouped_ffn_of_codes_past_the_caches(gpu, d, f, ne, t, meta, in_use):
-    """The same experts in cells so far apart that they count as more than the memory-side cache holds: the codes then come in
-    whole lines, and every row has the bytes that it has from a small pool."""
-    L = Layer(0x5EED0C00 + d + f, d, f, ne, 4, bits=8, meta=meta)
-    idx = random_routes(t + ne, t, 4, in_use)[0]
-    pc = PrefillCase(gpu, L, t, stride_pad=8, idx=idx, scale=row_scale(d, f))
-    near = pc.run()
-    for pair in np.random.default_rng(13).choice(t * 4, 12, replace=False):
-        pc.check_pair(near, int(pair) // 4, int(pair) % 4, f"pair {pair}")
-    far = gpu.ExpertPool(ne, (320 << 20) // ne, ne)
-    assert ffn_rules().takes_lines(4 * t, ne, d, f, 8, far.stride, far.stride | d | f)
-    assert not ffn_rules().takes_lines(4 * t, ne, d, f, 8, pc.dl.pool.stride, 0)
-    for e, cell in pc.dl.cell_of.items():
-        far.upload(cell, L.blobs[e])
-        far.publish(e, cell, capi.RESIDENT)
-    pc.dl.pool = far
-    pc.pf.group_pairs(pc.d_idx, pc.d_w, t, 4, ne, pc.routes, residency=far.table)
+class LineCase(PrefillCase):
+    """Experts that together are more than the memory-side cache holds, sixteen of them made. `beside` is the pool whose cells hold
+    the same blobs 16 bytes further on, where no row starts with a line: its codes come as half lines."""
+
+    def __init__(self, gpu, d, f, ne, t, meta, in_use, hint, **layer_and_case):
+        layer = {n: layer_and_case.pop(n) for n in ("additive_biases",) if n in layer_and_case}
+        L = Layer(0x5EED0C00 + d + f, d, f, ne, 4, bits=8, meta=meta, distinct=min(ne, 16, max(3, (48 << 20) // (3 * d * f))), **layer)
+        idx = random_routes(t + ne, t, 4, in_use, skew=0.7)[0]
+        super().__init__(gpu, L, t, idx=idx, scale=row_scale(d, f), **layer_and_case)
+        o = self.dl.off
+        align = self.dl.pool.stride | o.gate_w_off | o.up_w_off | o.down_w_off
+        for base in self.dl.pool.bases.contents.base:
+            align |= base or 0
+        assert ffn_rules().takes_lines(4 * t, ne, d, f, 8, align | d | f)
+        rows = np.bincount(idx, minlength=ne)
+        tiles = [min(64, n - at) for n in rows for at in range(0, n, 64)]  # the table's, in its order
+        last = sum(n < 64 for n in tiles[:256])
+        assert ffn_rules().past_the_cache(last, d, f, 8) == hint and max(rows) > 32
+
+    def beside(self):
+        L = self.L
+        pool, off = self.gpu.ExpertPool(L.ne, L.stride + 16, L.ne), capi.ExpertOffsets()
+        for name, _ in off._fields_:
+            setattr(off, name, getattr(self.dl.off, name) + 16)
+        for e, cell in self.dl.cell_of.items():
+            pool.upload(cell, np.concatenate([np.zeros(16, np.uint8), L.blobs[e]]))
+            pool.publish(e, cell, capi.RESIDENT)
+        assert not ffn_rules().takes_lines(4 * self.t, L.ne, L.d, L.f, 8, off.gate_w_off)
+        return pool, off
+
+    def check(self, got, act=O.ACT_SILU):
+        for pair in np.random.default_rng(13).choice(self.t * 4, 12, replace=False):
+            self.check_pair(got, int(pair) // 4, int(pair) % 4, f"pair {pair}", act)
+
+
+@pytest.mark.parametrize("d,f,ne,t,meta,in_use,hint", LINE_CASES)
+def test_grouped_ffn_of_codes_past_the_caches(gpu, d, f, ne, t, meta, in_use, hint):
+    """Codes as whole lines: the oracle's rows, and the bytes that the same experts give where their codes come as half lines."""
+    pc = LineCase(gpu, d, f, ne, t, meta, in_use, hint, stride_pad=8)
+    got = pc.run()
+    pc.check(got)
+    pc.dl.pool, pc.dl.off = pc.beside()
+    pc.pf.group_pairs(pc.d_idx, pc.d_w, t, 4, ne, pc.routes, residency=pc.dl.pool.table)
     pc.partials = gpu.dev(np.full(t * 4 * d, 0xD4D0, np.uint16))
-    assert np.array_equal(pc.run(), near)
+    assert np.array_equal(pc.run(), got)
 
 
 @pytest.mark.parametrize("d,f,bits,meta", [(320, 640, 4, S.META_BF16), (1088, 704, 8, S.META_F16)])
