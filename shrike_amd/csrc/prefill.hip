@@ -5,6 +5,7 @@
 #include "prefill_common.h"
 #include <type_traits>
 #include "router_row.h"
+#include "router_rules.h"
 
 #include "../../include/shrike_host.h"
 
@@ -26,9 +27,6 @@ namespace shrike {
 // Router launches (logits and select), before and after the affine rows went this way and the butterfly left LDS: 8-bit
 // rows, 1,000 tokens of 2,304 against 256: 195 -> 50 us; 4-bit rows, 512 of 2,048: 176 -> 24; fp16 rows, 1,000 of 2,304:
 // 63 -> 36 (four rows a wave instead of two), 4,096 of 2,048: 94 -> 87.
-template <int RK>
-constexpr int kRouterChunk = RK == 0 ? 8 : RK == 8 ? 16 : 32;  // elements of a 16-byte chunk of a row
-
 // One stage of the split butterfly over LIVE sums (a power of two above 1) at lane distance 32 >> STAGE: the partner with
 // the distance's bit set keeps the upper half of the sums and sends the lower, the other the reverse; each adds the
 // partner's copy of what it keeps. LIVE / 2 sums are left in v[0 .. LIVE / 2). At distances 32 and 16 the exchange is one
@@ -252,25 +250,18 @@ __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t q
 // waves in LDS. An affine row's chunk sums its codes' products from zero, in 8 or 16 chains of their own, and takes scale
 // (a multiply-add an output) and bias (one more MFMA) as router_row does.
 //
-// A workgroup takes 16 tokens and 16 experts, four workgroups a compute unit. Both sides' chunks come through a ring in LDS, a walk
+// A workgroup takes 16 tokens and 16 experts, up to four workgroups a compute unit (three of 8-bit rows past 3,072 and of 4-bit ones
+// past 1,536, two of 4-bit ones past 2,560: LogitsLds). Both sides' chunks come through a ring in LDS, a walk
 // (four chunks of each wave's) a unit, asked for one or two units ahead. The effective scales come that way too and are widened
 // in LDS once. What bounds it: a SIMD does not run a fp32 matrix instruction beside a vector one (a chain of them fed by two
 // vector instructions each, two waves a SIMD: 44 cycles a step, 32 without), so 4,096 tokens of 2,048 against 256 rows, 28 us
 // of matrix instructions alone, take 45 with the two conversions a product that nothing shares, and more with the loads' addresses.
 // A step's chunks all asked for, waited for and multiplied by turns -> the ring, us: fp16 rows, 256 of 2,048: 512 tokens 13.2 ->
 // 12.4, 1,000 21.0 -> 19.7, 4,096 69.5 -> 67.0, 128 of 3,072, 2,048 tokens 33.8 -> 26.9; 8-bit rows, 256 of 2,304: 300 tokens 18.4 ->
-// 17.8, 1,000 34.1 -> 30.7, 2,000 60.0 -> 55.9; 4-bit rows the same. A place more each: 3 to 8 % slower past 1,000 tokens (a workgroup
+// 17.8, 1,000 34.1 -> 30.7, 2,000 60.0 -> 55.9; 4-bit rows, 1,000 tokens: 256 of 1,024 21.9 -> 20.7, of 1,600 22.2 -> 22.6, of 2,048 22.4 -> 21.7,
+// 128 of 4,096, 2,000 tokens 47.1 -> 43.5. A place more each: 3 to 8 % slower past 1,000 tokens (a workgroup
 // fewer a compute unit). Two tiles of tokens, or of experts, a workgroup: 512 tokens 13.5, 4,096 71 (half the workgroups); two of both spill.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-template <int RK>
-struct LogitsLds {
-    static constexpr uint32_t kPieces = kRouterChunk<RK> / 8;                       // 16-byte pieces of x a chunk
-    static constexpr uint32_t kUnit = 4u * (kPieces + 1u) * 1024u;                  // a walk's chunks of sixteen tokens and sixteen experts
-    static constexpr uint32_t kPlaces = RK == 0 ? 3u : 2u, kEff = kPlaces * kUnit;
-    static_assert(SHRIKE_MAX_HIDDEN * 2u <= kUnit, "the effective scales fit a unit's place");
-    static uint32_t bytes(uint32_t d) { return kEff + 4u * d + (RK ? 2u * 16u * (d / kGroup) * 2u : 0u); }
-};
 
 template <int RK>
 __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, uint32_t query_count, uint32_t stride, float *logits) {
@@ -284,13 +275,14 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     const uint32_t expert_tiles = (num_experts + 15u) / 16u;
     const uint32_t t0 = ((blockIdx.x >> 3) / expert_tiles * 8u + (blockIdx.x & 7u)) * 16u, e0 = (blockIdx.x >> 3) % expert_tiles * 16u;
     if (t0 >= query_count) return;
-    float *l_eff = reinterpret_cast<float *>(lds + L::kEff);
+    const uint32_t blocks = L::blocks(d), unit_bytes = L::unit(d);
+    float *l_eff = reinterpret_cast<float *>(lds + L::eff(d));
     uint16_t *l_scale = reinterpret_cast<uint16_t *>(l_eff + d), *l_bias = l_scale + 16u * groups;
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds));
     // the effective scales as they are, into the last place, for now
-    constexpr uint32_t kEffAt = (L::kPlaces - 1u) * L::kUnit;
+    const uint32_t eff_at = (L::kPlaces - 1u) * unit_bytes;  // (2 d bytes: at most what the chunks of x take there)
     for (uint32_t i = wave * 1024u; i < 2u * d; i += 4096u)
-        lds_load16(lds0 + kEffAt + i, reinterpret_cast<const uint8_t *>(a.effective_scale) + min(i + lane * 16u, 2u * d - 16u));
+        lds_load16(lds0 + eff_at + i, reinterpret_cast<const uint8_t *>(a.effective_scale) + min(i + lane * 16u, 2u * d - 16u));
     // A load brings a 16-byte piece of four chunks of sixteen rows, the chunks xor-ed with the row so that sixteen rows read
     // at one chunk touch every bank once. Wave w brings block w's.
     const uint32_t l_row = lane >> 2, l_chunk = ((lane & 3u) ^ ((l_row >> 2) & 3u)) + 16u * wave;
@@ -301,10 +293,12 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     uint32_t ask_j = 0, ask_i = 0, ask_place = 0;  // the unit to ask for next: its step, its walk, its place
     auto ask = [&]() {
         const uint32_t j = ask_j == 1u ? 2u : ask_j == 2u ? 1u : ask_j;
-        const uint32_t c = min(4u * j + l_chunk + 64u * ask_i, chunks - 1u), at = lds0 + ask_place * L::kUnit;  // past the row: a copy, taken as zero
+        const uint32_t c = min(4u * j + l_chunk + 64u * ask_i, chunks - 1u), at = lds0 + ask_place * unit_bytes;  // past the row: a copy, taken as zero
+        if (wave < blocks) {
 #pragma unroll
-        for (uint32_t q = 0; q < Q; ++q) lds_load16(at + (wave * Q + q) * 1024u, x_row + c * E + q * 8u);
-        lds_load16(at + (4u * Q + wave) * 1024u, w_row + c * 16u);
+            for (uint32_t q = 0; q < Q; ++q) lds_load16(at + (wave * Q + q) * 1024u, x_row + c * E + q * 8u);
+            lds_load16(at + (blocks * Q + wave) * 1024u, w_row + c * 16u);
+        }
         if (++ask_i == walks) {
             ask_i = 0;
             ++ask_j;
@@ -324,13 +318,13 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     if (L::kPlaces - 2u < units) wait_loads_and_sync<int((L::kPlaces - 2u) * (Q + 1u))>();
     else wait_loads_and_sync<0>();
     for (uint32_t i = threadIdx.x; i < d / 8u; i += 256u) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(lds + kEffAt + i * 16u);
+        const uint4 v = *reinterpret_cast<const uint4 *>(lds + eff_at + i * 16u);
         float4 *to = reinterpret_cast<float4 *>(l_eff + 8u * i);
         to[0] = make_float4(bf16_to_f32(uint16_t(v.x)), bf16_to_f32(uint16_t(v.x >> 16)), bf16_to_f32(uint16_t(v.y)), bf16_to_f32(uint16_t(v.y >> 16)));
         to[1] = make_float4(bf16_to_f32(uint16_t(v.z)), bf16_to_f32(uint16_t(v.z >> 16)), bf16_to_f32(uint16_t(v.w)), bf16_to_f32(uint16_t(v.w >> 16)));
     }
     const uint32_t m = lane & 15u, block = lane >> 4;
-    const uint32_t read_at = m * 64u + ((wave ^ ((m >> 2) & 3u)) * 16u);
+    const uint32_t read_at = m * 64u + ((wave ^ ((m >> 2) & 3u)) * 16u), held = min(block, blocks - 1u);  // (a block without chunks reads another's: zero)
     f32x16_t acc;
     // chunk 64 i + 4 j + wave of each block; CHECK: it may lie past the row
     auto chunk = [&](uint32_t place, uint32_t j, uint32_t i, auto check) {
@@ -338,8 +332,8 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
         const uint32_t c0 = 4u * j + wave + 64u * i, c = c0 + 16u * block;
         const bool inside = !CHECK || c < chunks;
         const uint32_t cc = inside ? c : 0u;
-        const uint8_t *unit = lds + place * L::kUnit + read_at;
-        const uint4 wv = *reinterpret_cast<const uint4 *>(unit + (4u * Q + block) * 1024u);
+        const uint8_t *unit = lds + place * unit_bytes + read_at;
+        const uint4 wv = *reinterpret_cast<const uint4 *>(unit + (blocks * Q + held) * 1024u);
         uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
         if (CHECK) {
 #pragma unroll
@@ -349,7 +343,7 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
         float sum = 0.0f;
 #pragma unroll
         for (uint32_t q = 0; q < Q; ++q) {
-            const uint4 xv = *reinterpret_cast<const uint4 *>(unit + (block * Q + q) * 1024u);
+            const uint4 xv = *reinterpret_cast<const uint4 *>(unit + (held * Q + q) * 1024u);
             const uint32_t xw[4] = {xv.x, xv.y, xv.z, xv.w};
             const float4 e0v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u), e1v = *reinterpret_cast<const float4 *>(l_eff + cc * E + q * 8u + 4u);
             const float ew[8] = {e0v.x, e0v.y, e0v.z, e0v.w, e1v.x, e1v.y, e1v.z, e1v.w};
@@ -412,7 +406,7 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     }
     __syncthreads();  // (nobody reads the operands any more)
     float (*meet)[16][17] = reinterpret_cast<float (*)[16][17]>(lds);
-    static_assert(sizeof(float[4][16][17]) <= L::kUnit, "the waves' sums fit where a unit was");
+    static_assert(sizeof(float[4][16][17]) <= L::kPlaces * L::kBlock, "the waves' sums fit where the smallest units were");
 #pragma unroll
     for (uint32_t r = 0; r < 4u; ++r) meet[wave][4u * block + r][m] = even[r];
     __syncthreads();

@@ -89,11 +89,12 @@ class Layer:
 
 @functools.lru_cache(maxsize=None)
 def ffn_rules() -> C.CDLL:
-    """csrc/ffn_rules.h, compiled for the host."""
+    """csrc/ffn_rules.h and router_rules.h, compiled for the host."""
     with tempfile.TemporaryDirectory() as where:
         lib = os.path.join(where, "rules.so")
         source = """
 #include "ffn_rules.h"
+#include "router_rules.h"
 extern "C" uint32_t readable_records(uint32_t bound, uint64_t pairs, uint32_t experts) { return shrike::readable_records(bound, pairs, experts); }
 extern "C" const char *routed_shape(uint64_t pairs, uint32_t experts, uint32_t d, uint32_t f, uint32_t bits) {
     static const char *const names[] = {"split", "tile", "deep", "wide"};
@@ -103,6 +104,9 @@ extern "C" bool takes_lines(uint64_t pairs, uint32_t experts, uint32_t d, uint32
     const shrike::FfnShape shape = shrike::routed_shape(pairs, experts, d, f, bits);
     return shrike::lines_shape(shape, pairs, experts, d, f, bits, align) == shrike::FfnShape::kLines;
 }
+extern "C" uint32_t logits_lds(uint32_t router_bits, uint32_t d) {
+    return router_bits == 0 ? shrike::LogitsLds<0>::bytes(d) : router_bits == 8 ? shrike::LogitsLds<8>::bytes(d) : shrike::LogitsLds<4>::bytes(d);
+}
 extern "C" bool past_the_cache(uint64_t experts, uint32_t d, uint32_t f, uint32_t bits) { return shrike::past_the_cache(experts, d, f, bits); }
 """
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/shrike_amd/csrc", "-x", "c++", "-", "-o", lib],
@@ -111,5 +115,6 @@ extern "C" bool past_the_cache(uint64_t experts, uint32_t d, uint32_t f, uint32_
     rules.readable_records.argtypes, rules.readable_records.restype = [C.c_uint32, C.c_uint64, C.c_uint32], C.c_uint32
     rules.routed_shape.argtypes, rules.routed_shape.restype = [C.c_uint64, *[C.c_uint32] * 4], C.c_char_p
     rules.takes_lines.argtypes, rules.takes_lines.restype = [C.c_uint64, *[C.c_uint32] * 4, C.c_uint64], C.c_bool
+    rules.logits_lds.argtypes, rules.logits_lds.restype = [C.c_uint32] * 2, C.c_uint32
     rules.past_the_cache.argtypes, rules.past_the_cache.restype = [C.c_uint64, *[C.c_uint32] * 3], C.c_bool
     return rules

@@ -32,3 +32,11 @@ def test_what_counts_against_the_cache_is_the_experts_bytes(experts, d, f, lines
     no spacing of whole lines changes its answer."""
     for stride in (1 << 14, 1 << 21, 1 << 25):
         assert ffn_rules().takes_lines(16 * experts, experts, d, f, 8, stride | d | f) == lines
+
+
+@pytest.mark.parametrize("router_bits,widths,workgroups", [(0, (64, 2048, 4096), 4), (8, (64, 2048, 3072), 4), (4, (64, 512, 1024, 1536), 4),
+                                                            (4, (1600, 2048), 3), (4, (4096,), 2)])
+def test_workgroups_of_the_router_that_fit_a_compute_unit(router_bits, widths, workgroups):
+    """160 KB a unit; the kernels' registers allow four."""
+    for d in widths:
+        assert 160 * 1024 // ffn_rules().logits_lds(router_bits, d) >= workgroups

@@ -68,7 +68,8 @@ def test_prefill_router_bit_exact_and_equal_to_decode(gpu, router_bits, ne, d, k
     (8, 256, 512, 3), (0, 64, 320, 8), (0, 64, 320, 9), (0, 256, 128, 700), (8, 100, 192, 1300),   # tokens a launch, a workgroup
     # on the matrix cores: part of a lane's chunks, whole ones only, ragged tokens and experts
     (0, 200, 64, 481), (0, 250, 512, 400), (0, 241, 2112, 390), (0, 250, 4096, 391), (8, 250, 64, 300), (8, 241, 1024, 273),
-    (8, 256, 2304, 258), (8, 241, 4096, 272), (4, 249, 128, 270), (4, 256, 2048, 257), (4, 241, 2176, 273), (4, 241, 4096, 258)])
+    (8, 256, 2304, 258), (8, 241, 4096, 272), (4, 249, 128, 270), (4, 256, 2048, 257), (4, 241, 2176, 273), (4, 241, 4096, 258),
+    (4, 250, 512, 260), (4, 241, 576, 273), (4, 256, 1088, 257), (4, 249, 1600, 270)])  # (rows without chunks for the last blocks)
 def test_prefill_router_instances_bit_exact(gpu, router_bits, ne, d, t):
     k = 4
     L = Layer(0x5EED0A00 + router_bits + d, d, 64, ne, k, router_bits=router_bits)
