@@ -250,8 +250,8 @@ __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t q
 // waves in LDS. An affine row's chunk sums its codes' products from zero, in 8 or 16 chains of their own, and takes scale
 // (a multiply-add an output) and bias (one more MFMA) as router_row does.
 //
-// A workgroup takes 16 tokens and 16 experts, up to four workgroups a compute unit (three of 8-bit rows past 3,072 and of 4-bit ones
-// past 1,536, two of 4-bit ones past 2,560: LogitsLds). Both sides' chunks come through a ring in LDS, a walk
+// A workgroup takes 16 tokens and 16 experts, up to four workgroups a compute unit (three of 8-bit rows past 3,264 and of 4-bit ones
+// past 1,536, two of 4-bit ones past 2,688: LogitsLds). Both sides' chunks come through a ring in LDS, a walk
 // (four chunks of each wave's) a unit, asked for one or two units ahead. The effective scales come that way too and are widened
 // in LDS once. What bounds it: a SIMD does not run a fp32 matrix instruction beside a vector one (a chain of them fed by two
 // vector instructions each, two waves a SIMD: 44 cycles a step, 32 without), so 4,096 tokens of 2,048 against 256 rows, 28 us
@@ -263,7 +263,9 @@ __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t q
 // fewer a compute unit). Two tiles of tokens, or of experts, a workgroup: 512 tokens 13.5, 4,096 71 (half the workgroups); two of both spill.
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-template <int RK>
+// PIECES: the effective scales start at a whole piece of 16 bytes; else they are loaded one by one (an instance of its own: the
+// question alone cost the fp16 kernel 1 to 3 %).
+template <int RK, bool PIECES>
 __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, uint32_t query_count, uint32_t stride, float *logits) {
     warm_kernel_arguments(a);
     typedef LogitsLds<RK> L;
@@ -281,7 +283,7 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     const uint32_t lds0 = uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)lds));
     // the effective scales as they are, into the last place, for now
     const uint32_t eff_at = (L::kPlaces - 1u) * unit_bytes;  // (2 d bytes: at most what the chunks of x take there)
-    for (uint32_t i = wave * 1024u; i < 2u * d; i += 4096u)
+    for (uint32_t i = wave * 1024u; PIECES && i < 2u * d; i += 4096u)
         lds_load16(lds0 + eff_at + i, reinterpret_cast<const uint8_t *>(a.effective_scale) + min(i + lane * 16u, 2u * d - 16u));
     // A load brings a 16-byte piece of four chunks of sixteen rows, the chunks xor-ed with the row so that sixteen rows read
     // at one chunk touch every bank once. Wave w brings block w's.
@@ -318,10 +320,16 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     if (L::kPlaces - 2u < units) wait_loads_and_sync<int((L::kPlaces - 2u) * (Q + 1u))>();
     else wait_loads_and_sync<0>();
     for (uint32_t i = threadIdx.x; i < d / 8u; i += 256u) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(lds + eff_at + i * 16u);
+        alignas(16) uint16_t v[8];
+        if (PIECES) {
+            *reinterpret_cast<uint4 *>(v) = *reinterpret_cast<const uint4 *>(lds + eff_at + i * 16u);
+        } else {
+#pragma unroll
+            for (uint32_t n = 0; n < 8u; ++n) v[n] = a.effective_scale[8u * i + n];
+        }
         float4 *to = reinterpret_cast<float4 *>(l_eff + 8u * i);
-        to[0] = make_float4(bf16_to_f32(uint16_t(v.x)), bf16_to_f32(uint16_t(v.x >> 16)), bf16_to_f32(uint16_t(v.y)), bf16_to_f32(uint16_t(v.y >> 16)));
-        to[1] = make_float4(bf16_to_f32(uint16_t(v.z)), bf16_to_f32(uint16_t(v.z >> 16)), bf16_to_f32(uint16_t(v.w)), bf16_to_f32(uint16_t(v.w >> 16)));
+        to[0] = make_float4(bf16_to_f32(v[0]), bf16_to_f32(v[1]), bf16_to_f32(v[2]), bf16_to_f32(v[3]));
+        to[1] = make_float4(bf16_to_f32(v[4]), bf16_to_f32(v[5]), bf16_to_f32(v[6]), bf16_to_f32(v[7]));
     }
     const uint32_t m = lane & 15u, block = lane >> 4;
     const uint32_t read_at = m * 64u + ((wave ^ ((m >> 2) & 3u)) * 16u), held = min(block, blocks - 1u);  // (a block without chunks reads another's: zero)
@@ -423,8 +431,13 @@ template <int RK>
 static bool launch_prefill_logits_mfma(const RouterArgs &a, uint32_t query_count, uint32_t stride, float *logits, hipStream_t s) {
     const uint32_t expert_tiles = (a.sel.num_experts + 15u) / 16u, token_tiles = (query_count + 15u) / 16u;
     if (uint64_t(expert_tiles) * token_tiles <= (RK == 0 ? 384u : 256u)) return false;
-    if (reinterpret_cast<uintptr_t>(a.effective_scale) % 4u != 0) return false;  // (whole words of them are loaded)
-    hipLaunchKernelGGL(k_prefill_logits_mfma<RK>, dim3(((token_tiles + 7u) & ~7u) * expert_tiles), dim3(256), LogitsLds<RK>::bytes(a.d), s, a, query_count, stride, logits);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(((token_tiles + 7u) & ~7u) * expert_tiles), dim3(256), LogitsLds<RK>::bytes(a.d), s, a, query_count, stride, logits);
+    };
+    // (scales at an odd element, us with the selection, on the vector kernel and here: 4,096 tokens of 2,048 against 256 rows 85, 65;
+    // 8-bit rows, 1,000 of 2,304, 48, 32)
+    if (reinterpret_cast<uintptr_t>(a.effective_scale) % 16u == 0) launch(k_prefill_logits_mfma<RK, true>);
+    else launch(k_prefill_logits_mfma<RK, false>);
     return true;
 }
 

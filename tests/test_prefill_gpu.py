@@ -85,17 +85,19 @@ def test_prefill_router_instances_bit_exact(gpu, router_bits, ne, d, t):
 
 @pytest.mark.parametrize("router_bits,ne,d,t", [(0, 241, 2112, 390), (8, 241, 1088, 273), (4, 241, 2176, 273)])
 def test_prefill_router_takes_effective_scales_at_any_element(gpu, router_bits, ne, d, t):
-    """Enough tokens for the matrix cores, which load whole words of the scales: from an odd element on the logits are the same."""
+    """Enough tokens for the matrix cores, whose kernel loads the scales in pieces of 16 bytes where they start at one: from the first,
+    the second and the fourth element on the logits are the same."""
     L = Layer(0x5EED0D00 + router_bits, d, 64, ne, 4, router_bits=router_bits)
     L.eff_scale = S.f32_to_bf16_bits(L.tree.key("eff").uniform(0.5, 1.5, d))
     dl = DeviceLayer(gpu, L, resident=[])
     x = gpu.dev(token_rows(L, t, d))
     _, _, _, ws = run_router(gpu, dl, L, x, t, d)
     want = ws.download(np.uint32, t * ne)
-    odd = gpu.dev(np.concatenate([np.zeros(1, np.uint16), L.eff_scale]))
-    dl.eff_scale = odd.ptr + 2
-    _, _, _, ws = run_router(gpu, dl, L, x, t, d)
-    assert np.array_equal(ws.download(np.uint32, t * ne), want)
+    for ahead in (1, 2, 4):
+        moved = gpu.dev(np.concatenate([np.zeros(ahead, np.uint16), L.eff_scale]))
+        dl.eff_scale = moved.ptr + 2 * ahead
+        _, _, _, ws = run_router(gpu, dl, L, x, t, d)
+        assert np.array_equal(ws.download(np.uint32, t * ne), want), f"{ahead} elements on"
 
 
 @pytest.mark.parametrize("values", ["infinite", "subnormal", "cancelling"])
