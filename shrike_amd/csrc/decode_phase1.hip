@@ -22,7 +22,7 @@ constexpr int kPhase1RowPairsNarrow = 2;
 // reads an expert's rows once per token routed to it, and there the caches are what makes the second read cheap).
 // TAIL: the rows end in a step of half chunks (load_slice_regs); NCH then counts the whole steps ahead of it.
 // META: the type of the routed experts' scales and biases (SHRIKE_META_*), known to the instance so that a row converts them one way.
-// LOOP: a wave walks a.row_steps steps of RP row pairs (phase1_steps), with the activations unpacked once. A large batch is bound by
+// LOOP: a wave walks a.row_steps steps of RP row pairs (phase1_row_steps), with the activations unpacked once. A large batch is bound by
 // the vector units: 16 tokens of 2,304 x 1,024, 8-bit, 8 of 256 experts, keep them busy for 65 of 118 us, and of a wave's 600
 // operations the selection, which every wave makes for itself, is 100 and the activations' unpacking 50. With two steps the launch
 // takes 98 us.
@@ -150,17 +150,6 @@ static bool phase1_narrow(bool routing, bool one_token, uint32_t d, uint32_t bit
     return (one_token && !routing) || nch_for(d, bits) >= 3;
 }
 
-// Two steps where a routing launch of one-step waves has 4,096 workgroups, 16 a compute unit, or more, else one: with fewer the
-// last waves' second steps cost more than the selections saved. A layer with one step and with two, us: 16,384 workgroups (16 tokens of
-// 2,304 x 1,024, 8-bit) 172 and 161; 8,192 (8 of them) 95 and 89; 6,144 (16 of 1,536 x 768) 67 and 65; 4,096 (16 of 2,048 x 512)
-// 57.5 and 55.5; 2,048 (8 of them) 32.8 and 33.1; 1,024 (16 of 1,024 x 256) 17.2 and 18.6. Rows of four steps a lane keep one
-// (12 tokens of 4,096 x 1,024, 8-bit: 190.5 and 192), as do rows with half chunks, where the loop's registers cost the launch a wave a
-// SIMD (16 tokens of 2,880 x 2,880: 141 and 144). Two steps' row pairs divide f, a multiple of 64.
-static uint32_t phase1_steps(const Phase1Args &a, bool routing, uint32_t bits) {
-    const bool looped = routing && nch_for(a.d, bits) < 4u && !(bits == 4u && half_chunk_tail(a.d * bits / 128u, bits));
-    return looped && uint64_t(a.tokens) * a.routed_blocks >= 4096u ? 2u : 1u;
-}
-
 template <int BITS, int NCH, int RP, bool ROUTE, int SBITS, bool STREAM, int META>
 static void launch_phase1_steps(const Phase1Args &a, dim3 grid, hipStream_t s) {
     if constexpr (ROUTE && !STREAM && NCH < 4) {
@@ -208,7 +197,7 @@ int launch_phase1(const Phase1Args &a, uint32_t bits, bool routing, uint32_t sha
     const bool one_token = a.tokens <= 1u;
     if (phase1_narrow(routing, one_token, a.d, bits))
         b.routed_blocks = phase1_blocks_of(a.active ? a.active_count : a.top_k, a.f, kPhase1RowPairsNarrow);
-    b.row_steps = one_token ? 1u : phase1_steps(b, routing, bits);
+    b.row_steps = one_token || !routing ? 1u : phase1_row_steps(uint64_t(a.tokens) * b.routed_blocks, a.d, bits);
     if (b.row_steps > 1u)
         b.routed_blocks = phase1_blocks_of(a.top_k, a.f, b.row_steps * (phase1_narrow(routing, one_token, a.d, bits) ? kPhase1RowPairsNarrow : kPhase1RowPairs));
     b.lists_block = routing ? b.routed_blocks + extra : 0xffffffffu;

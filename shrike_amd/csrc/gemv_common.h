@@ -11,6 +11,7 @@
 
 #include <type_traits>
 
+#include "decode_rules.h"
 #include "device_utils.h"
 #include "host_common.h"
 
@@ -91,9 +92,6 @@ struct SliceRegs {
     uint4 t[2];
     uint32_t off;
 };
-
-// whether a row of `cpr` 16-byte chunks is walked as cpr / 64 whole steps and a step of half chunks
-inline bool half_chunk_tail(uint32_t cpr, uint32_t bits) { return bits == 4u && cpr > 64u && (cpr % 64u) >= 1u && (cpr % 64u) <= 32u; }
 
 template <int BITS, int NCH, bool TAIL = false>
 __device__ __forceinline__ void load_slice_regs(SliceRegs<BITS, NCH, TAIL> &r, const uint4 *vec, uint32_t cpr,
@@ -364,8 +362,6 @@ template <int BITS, int NCH>
 __device__ __forceinline__ void gemv_job(const GemvArgs &a, uint32_t block) {
     gemv_job<BITS, NCH>(a, block, NoXSource{});
 }
-
-inline uint32_t nch_for(uint32_t n, uint32_t bits) { return (n * bits / 128u + 63u) / 64u; }
 
 inline uint32_t gemv_blocks(uint32_t total_rows, uint32_t n, uint32_t bits) {
     const uint32_t cpr = n * bits / 128u;

@@ -89,10 +89,11 @@ class Layer:
 
 @functools.lru_cache(maxsize=None)
 def ffn_rules() -> C.CDLL:
-    """csrc/ffn_rules.h and router_rules.h, compiled for the host."""
+    """csrc/decode_rules.h, ffn_rules.h and router_rules.h, compiled for the host."""
     with tempfile.TemporaryDirectory() as where:
         lib = os.path.join(where, "rules.so")
         source = """
+#include "decode_rules.h"
 #include "ffn_rules.h"
 #include "router_rules.h"
 extern "C" uint32_t readable_records(uint32_t bound, uint64_t pairs, uint32_t experts) { return shrike::readable_records(bound, pairs, experts); }
@@ -107,6 +108,7 @@ extern "C" bool takes_lines(uint64_t pairs, uint32_t experts, uint32_t d, uint32
 extern "C" uint32_t logits_lds(uint32_t router_bits, uint32_t d) {
     return router_bits == 0 ? shrike::LogitsLds<0>::bytes(d) : router_bits == 8 ? shrike::LogitsLds<8>::bytes(d) : shrike::LogitsLds<4>::bytes(d);
 }
+extern "C" uint32_t phase1_row_steps(uint64_t workgroups, uint32_t d, uint32_t bits) { return shrike::phase1_row_steps(workgroups, d, bits); }
 extern "C" bool past_the_cache(uint64_t experts, uint32_t d, uint32_t f, uint32_t bits) { return shrike::past_the_cache(experts, d, f, bits); }
 """
         subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", f"-I{ROOT}/shrike_amd/csrc", "-x", "c++", "-", "-o", lib],
@@ -116,5 +118,6 @@ extern "C" bool past_the_cache(uint64_t experts, uint32_t d, uint32_t f, uint32_
     rules.routed_shape.argtypes, rules.routed_shape.restype = [C.c_uint64, *[C.c_uint32] * 4], C.c_char_p
     rules.takes_lines.argtypes, rules.takes_lines.restype = [C.c_uint64, *[C.c_uint32] * 4, C.c_uint64], C.c_bool
     rules.logits_lds.argtypes, rules.logits_lds.restype = [C.c_uint32] * 2, C.c_uint32
+    rules.phase1_row_steps.argtypes, rules.phase1_row_steps.restype = [C.c_uint64, C.c_uint32, C.c_uint32], C.c_uint32
     rules.past_the_cache.argtypes, rules.past_the_cache.restype = [C.c_uint64, *[C.c_uint32] * 3], C.c_bool
     return rules

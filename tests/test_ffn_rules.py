@@ -1,4 +1,4 @@
-"""The sizes the grouped FFN's host code works out for a launch, asked from the header that it takes them from. No GPU."""
+"""The sizes that the host code works out for a launch, asked from the headers that it takes them from. No GPU."""
 import pytest
 
 from shrike_amd import capi
@@ -40,3 +40,11 @@ def test_workgroups_of_the_router_that_fit_a_compute_unit(router_bits, widths, w
     """160 KB a unit; the kernels' registers allow four."""
     for d in widths:
         assert 160 * 1024 // ffn_rules().logits_lds(router_bits, d) >= workgroups
+
+
+@pytest.mark.parametrize("bits,widths,steps", [(8, (64, 512, 1024, 1088, 1280, 1536, 2112, 2304, 2560), 2), (8, (1600, 1792, 1984, 2048, 2624, 2944, 3072, 3136, 4096), 1),
+                                                (4, (64, 1536, 2048, 3136, 4096), 2), (4, (2112, 2880, 3072), 1)])
+def test_phase_1_walks_two_steps_where_that_was_faster(bits, widths, steps):
+    for d in widths:
+        assert ffn_rules().phase1_row_steps(4096, d, bits) == steps
+        assert ffn_rules().phase1_row_steps(4095, d, bits) == 1
