@@ -166,15 +166,18 @@ static void launch_phase1_meta(const Phase1Args &a, dim3 grid, hipStream_t s) {
     // (shorter rows: the one-token routing launch keeps four pairs)
     constexpr int RP = kPhase1RowPairs, RN = (ROUTE && STREAM) ? kPhase1RowPairs : kPhase1RowPairsNarrow;
     if (BITS == 4 && half_chunk_tail(a.d * BITS / 128u, BITS)) {
-        // d <= SHRIKE_MAX_HIDDEN: one whole step and the half chunks (65...96 chunks a row)
+        // (d <= SHRIKE_MAX_HIDDEN: one whole step and the half chunks, 65...96 chunks a row)
         hipLaunchKernelGGL((k_phase1<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, BITS == 4, META, false>), grid, dim3(256), 0, s, a);
         return;
     }
-    switch (nch_for(a.d, BITS)) {
-        case 1: launch_phase1_steps<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
-        case 2: launch_phase1_steps<BITS, 2, STREAM ? RN : RP, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
-        case 3: launch_phase1_steps<BITS, 3, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
-        default: launch_phase1_steps<BITS, 4, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, META>(a, grid, s); break;
+    const uint32_t steps = nch_for(a.d, BITS);
+    if (steps == 1u) {
+        launch_phase1_steps<BITS, 1, STREAM ? RN : RP, ROUTE, SBITS, STREAM, META>(a, grid, s);
+    } else if (BITS == 4 || steps == 2u) {  // d <= SHRIKE_MAX_HIDDEN: 4-bit rows take two steps at most
+        launch_phase1_steps<BITS, 2, STREAM ? RN : RP, ROUTE, SBITS, STREAM, META>(a, grid, s);
+    } else if constexpr (BITS == 8) {
+        if (steps == 3u) launch_phase1_steps<BITS, 3, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, META>(a, grid, s);
+        else launch_phase1_steps<BITS, 4, kPhase1RowPairsNarrow, ROUTE, SBITS, STREAM, META>(a, grid, s);
     }
 }
 
