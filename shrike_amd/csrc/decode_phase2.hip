@@ -32,8 +32,7 @@ __device__ __forceinline__ void phase2_finish(uint16_t *y, uint16_t *hidden, uin
 // 13.2 us), and 74 registers where 47 leave a launch all its waves. Short rows in a large batch are bound by the vector units (536
 // operations for a wave's 8 rows of 1,024, 8-bit): a layer of 16 tokens of 1,536 x 768, 67 -> 57 us; 12 of 2,816 x 1,408, 110 -> 98.5; 16
 // of 2,304 x 1,024, 8-bit, 161 -> 157 (the launch reads 6.1 TB/s there); 8 of 2,048 x 1,024, 52.4 -> 50.7.
-// (Not named: that of rows whose BATCH loads a wave are the workgroup's ROWS, the wave for rows of more than one step.)
-template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META, int SEG = NCH >= 2 || TAIL ? 64 : 64 * BATCH / int(ROWS)>
+template <int BITS, int NCH, int BATCH, bool STREAM, uint32_t ROWS, bool TAIL, int META, int SEG>
 __global__ __launch_bounds__(512) void k_phase2(Phase2Args a) {
     warm_kernel_arguments(a);
     typedef Chunk<BITS> C;

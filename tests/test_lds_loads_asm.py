@@ -45,8 +45,9 @@ def test_the_compiler_knows_what_m0_holds_after_a_hand_written_load(tmp_path, lo
     assert addresses[0] == addresses[2] != addresses[1], f"the loads' LDS addresses: {addresses}"
 
 
-@pytest.mark.parametrize("instance", ["4, 1, 2, true, 8, false, SHRIKE_META_F16", "8, 1, 4, false, 8, false, SHRIKE_META_BF16",  # rows that share a wave load
-                                      "8, 3, 4, true, 4, false, SHRIKE_META_BF16", "4, 1, 4, false, 16, true, SHRIKE_META_F16"])
+@pytest.mark.parametrize("instance", ["4, 1, 2, true, 8, false, SHRIKE_META_F16, 16", "8, 1, 4, false, 8, false, SHRIKE_META_BF16, 32",  # rows that share a wave load
+                                      "4, 1, 1, true, 8, false, SHRIKE_META_F16, 2", "8, 1, 4, false, 16, false, SHRIKE_META_BF16, 64",
+                                      "8, 3, 4, true, 4, false, SHRIKE_META_BF16, 64", "4, 1, 4, false, 16, true, SHRIKE_META_F16, 64"])
 def test_phase_2_reads_no_partial_sum_ahead_of_its_barrier(tmp_path, instance):
     """A lane's word of LDS is another lane's only behind the barrier: nothing else orders the two for the compiler."""
     with open(f"{ROOT}/shrike_amd/csrc/decode_phase2.hip") as f:
