@@ -2,10 +2,12 @@
 compiler's own: both take their LDS address from m0, so each must know of the other's. And phase 2's partial sums: lanes
 exchange them through LDS behind the workgroup's barrier only."""
 import re
+import shutil
 import subprocess
 
 import pytest
 
+from shrike_amd import capi
 from tests.conftest import ROOT
 
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -59,3 +61,21 @@ def test_phase_2_reads_no_partial_sum_ahead_of_its_barrier(tmp_path, instance):
     code = (tmp_path / "k.s").read_text().split("s_barrier")
     assert len(code) == 2 and re.search(r"\bds_write", code[0]) and re.search(r"\bds_read", code[1])
     assert not re.search(r"\bds_read", code[0]), "a partial sum is read ahead of the barrier"
+
+
+def test_no_load_into_lds_reads_a_base_that_a_vector_instruction_has_just_written(tmp_path):
+    """The library's own device code. A memory instruction that reads a scalar register needs five wait states behind a vector
+    instruction that writes it (v_readlane of a spilled base), and the compiler keeps none ahead of assembly by hand. So the base of every
+    such load is the scalar unit's own move, right ahead of it, and what stands between a write of m0 and the load is that or a wait state."""
+    library = shutil.copy(capi.LIB_PATH, tmp_path)
+    subprocess.run(["/opt/rocm/llvm/bin/llvm-objdump", "--offloading", library], cwd=tmp_path, check=True, stdout=subprocess.DEVNULL)
+    loads = {"base": 0, "off": 0}
+    for image in tmp_path.glob("*gfx950"):
+        before = ""
+        for line in subprocess.run(["/opt/rocm/llvm/bin/llvm-objdump", "-d", "--no-show-raw-insn", image], check=True, capture_output=True, text=True).stdout.splitlines():
+            if "global_load_lds_dwordx" in line:
+                base = re.search(r"(s\[\d+:\d+\])(?: nt)?\s", line)
+                loads["base" if base else "off"] += 1
+                assert f"s_mov_b64 {base[1]}, s[" in before if base else "s_nop" in before, f"{before.strip()} / {line.strip()}"
+            before = line
+    assert min(loads.values()) > 0
