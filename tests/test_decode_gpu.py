@@ -616,14 +616,14 @@ def test_argument_errors_are_reported_not_trapped(gpu):
 
 @pytest.mark.parametrize("d,f,ne,k,t,bits", [(2880, 2880, 6, 4, 4, 4), (2880, 2880, 5, 4, 3, 8), (2304, 1024, 24, 8, 16, 8), (512, 256, 16, 4, 7, 4),
                                             (2880, 2880, 32, 4, 4, 4), (2880, 2880, 32, 4, 4, 8)])  # the last two: config 4 as it is stated
-def test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, t, bits):
+def test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, t, bits, additive=False):
     """A batch of independent decode tokens (config 4: 4 tokens; config 5: 16 sequences): resolve,
     phase 1 and phase 2 with the token dimension on the grid give, per token, the bytes of the
     single-token operators, which the tests above hold to the oracle; routes come from the
     block router and are checked against the oracle bit for bit."""
-    L = Layer(0x5EED0004, d, f, ne, k, bits=bits)
+    L = Layer(0x5EED0004, d, f, ne, k, bits=bits, additive_biases=additive)
     resident = [e for e in range(ne) if e % 5 != 3]  # some experts miss
-    dl = DeviceLayer(gpu, L, resident=resident)
+    dl = DeviceLayer(gpu, L, resident=resident, moe_kwargs=dict(additive_biases=additive))
     stride = d + 16
     x = S.activations_f16(L.tree, "batch.x", t * stride)
     hidden0 = S.activations_f16(L.tree, "batch.hidden", t * d)
@@ -664,10 +664,10 @@ def test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, 
     # and against the oracle for the first token
     blobs = [None if c == SENT else dl.pool_blobs()[c] for c in want[:k]]
     off = L.oracle_offsets()
-    ref_acts = O.moe_phase1(blobs, off, np.ascontiguousarray(x[:d]), d, f, bits, L.meta)
+    ref_acts = O.moe_phase1(blobs, off, np.ascontiguousarray(x[:d]), d, f, bits, L.meta, additive_biases=additive)
     live0 = np.repeat(np.array(want[:k]) != SENT, f)
     assert_ffn_close(all_acts[:k * f][live0], ref_acts[live0], "token 0 activations")
-    ref_y = O.moe_phase2(blobs, off, np.ascontiguousarray(all_acts[:k * f]), h_w[:k].copy(), res_host[:d].copy(), d, f, bits, L.meta)
+    ref_y = O.moe_phase2(blobs, off, np.ascontiguousarray(all_acts[:k * f]), h_w[:k].copy(), res_host[:d].copy(), d, f, bits, L.meta, additive)
     assert_ffn_close(all_y[:d], ref_y, "token 0 y from the device's activations")
 
 
@@ -678,16 +678,22 @@ def test_batched_decode_operators_over_down_rows_of_one_step(gpu, d, f, ne, k, t
     test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, t, bits)
 
 
+@pytest.mark.parametrize("d,f,ne,k,t,bits", [(1024, 768, 16, 4, 24, 4), (1088, 960, 16, 8, 7, 8), (256, 2048, 8, 2, 3, 4), (192, 64, 8, 2, 3, 8)])
+def test_batched_decode_operators_with_additive_biases_over_down_rows_of_one_step(gpu, d, f, ne, k, t, bits):
+    # 16, 8 and 4 rows a workgroup, packed ones
+    test_batched_decode_operators_equal_the_single_token_ones(gpu, d, f, ne, k, t, bits, additive=True)
+
+
 @pytest.mark.parametrize("d,f,ne,k,t,bits,router_bits", [(2880, 2880, 32, 4, 4, 4, 0), (2880, 2880, 32, 4, 4, 8, 0), (512, 256, 40, 8, 16, 4, 8),
                                                           (2304, 1024, 256, 8, 5, 8, 0), (256, 128, 8, 3, 1, 4, 4)])
-def test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, router_bits):
+def test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, router_bits, additive=False):
     """shrike_hip_moe_decode_layer_batch: the three launches with the token on the grid give, for every token, the
     routes, cells, y and hidden bytes of shrike_hip_moe_decode_layer on that token alone (which the tests above hold
     to the oracle); routes also against the oracle bit for bit. Some experts are missing from the pool."""
-    L = Layer(0x5EED0044 + bits, d, f, ne, k, bits=bits, router_bits=router_bits)
+    L = Layer(0x5EED0044 + bits, d, f, ne, k, bits=bits, router_bits=router_bits, additive_biases=additive)
     L.logit_bias = S.f32_to_bf16_bits(L.tree.key("bias").normal(ne, std=0.01))
     resident = [e for e in range(ne) if e % 7 != 2]
-    dl = DeviceLayer(gpu, L, resident=resident)
+    dl = DeviceLayer(gpu, L, resident=resident, moe_kwargs=dict(additive_biases=additive))
     stride = d + 24
     x = S.activations_f16(L.tree, "batch.x", t * stride)
     hidden0 = S.activations_f16(L.tree, "batch.hidden", t * d)
@@ -733,6 +739,12 @@ def test_decode_layer_for_a_large_batch_equals_the_layer_token_by_token(gpu, d, 
     # phase 1 of 4,096 workgroups (the first) and more, whose waves walk two steps of rows: rows of one, two and three chunks a lane
     # with a remainder, 4 or 2 row pairs a step; rows of four chunks, which keep one step
     test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, router_bits)
+
+
+@pytest.mark.parametrize("d,f,ne,k,t,bits", [(64, 1024, 24, 8, 8, 4), (2112, 1088, 24, 4, 8, 8)])
+def test_decode_layer_for_a_large_batch_with_additive_biases_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits):
+    # both steps' biases, of 4 and of 2 row pairs a step
+    test_decode_layer_for_a_batch_equals_the_layer_token_by_token(gpu, d, f, ne, k, t, bits, 0, additive=True)
 
 
 @pytest.mark.parametrize("bits", [4, 8])

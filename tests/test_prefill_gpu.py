@@ -365,6 +365,24 @@ def test_grouped_ffn_shape_sweep(gpu, case):
     assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
 
 
+def check_pair_ranges(gpu, pc):
+    """Ranges that start and end inside row tiles, one of a single pair and one to the chunk's end: their pairs' rows are the whole
+    call's bytes, and no others are written."""
+    t, d, k = pc.t, pc.L.d, pc.L.k
+    want = pc.run()
+    order = pc.routes.download()["sorted_pairs"].astype(int)  # token, expert, rank, weight
+    at = order[:, 0] * k + order[:, 2]
+    for lo, count in ((37, 203), (t * k - 90, 90), (130, 1)):
+        pc.partials = gpu.dev(np.full(t * k * d, 0xD4D0, np.uint16))
+        pc.pf.encode_streamed_batched(pc.dl.pool, pc.dl.off, pc.routes, pc.hidden, pc.stride, pc.partials, pc.ws, t, k, lo, count)
+        gpu.synchronize()
+        got = pc.partials.download(np.uint16, t * k * d).reshape(t * k, d)
+        inside = np.zeros(t * k, bool)
+        inside[at[lo:lo + count]] = True
+        assert np.array_equal(got[inside], want.reshape(t * k, d)[inside]), f"pairs {lo} to {lo + count}"
+        assert np.all(got[~inside] == 0xD4D0), f"pairs {lo} to {lo + count}: a row of another pair was written"
+
+
 def row_scale(d, f):
     """Of rows so long that N(0, 1) inputs make outputs of 75: a partial row is then a sum of products that come to 4,000 to 5,000
     in magnitude, of which fp32 keeps 2^-24 = 3e-4 a step, and where it cancels, two orders of addition differ by more than the
@@ -478,6 +496,30 @@ def test_grouped_ffn_of_codes_past_the_caches(gpu, d, f, ne, t, meta, in_use, hi
     pc.pf.group_pairs(pc.d_idx, pc.d_w, t, 4, ne, pc.routes, residency=pc.dl.pool.table)
     pc.partials = gpu.dev(np.full(t * 4 * d, 0xD4D0, np.uint16))
     assert np.array_equal(pc.run(), got)
+
+
+@pytest.mark.parametrize("d,f,ne,t", [(1152, 896, 110, 600), (2048, 4096, 12, 60)])
+def test_gpt_oss_epilogues_of_codes_past_the_caches(gpu, d, f, ne, t):
+    pc = LineCase(gpu, d, f, ne, t, S.META_BF16, ne, True, additive_biases=True, moe_kwargs=dict(activation=capi.ACT_CLAMPED_SWIGLU, additive_biases=True))
+    got = pc.run()
+    assert not np.any(np.all(got == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
+    pc.check(got, O.ACT_CLAMPED_SWIGLU)
+
+
+def test_codes_past_the_caches_of_absent_experts(gpu):
+    absent = [0, 1, 17, 63, 108]
+    pc = LineCase(gpu, 1152, 896, 110, 600, S.META_F16, 110, True, resident=[e for e in range(110) if e not in absent])
+    got = pc.run()
+    there = ~np.isin(pc.idx, absent).reshape(pc.t, 4)
+    assert np.all(got[~there] == 0xD4D0), "an absent expert's row was written"
+    assert not np.any(np.all(got[there] == 0xD4D0, axis=-1)), "a pair's partial row was left unwritten"
+    for tok, rank in np.argwhere(there)[::131]:
+        pc.check_pair(got, int(tok), int(rank), f"token {tok} rank {rank}")
+
+
+@pytest.mark.parametrize("d,f,ne,t", [(384, 1152, 250, 1000), (2048, 4096, 12, 60)])
+def test_pair_ranges_of_codes_past_the_caches_equal_the_whole_chunk(gpu, d, f, ne, t):
+    check_pair_ranges(gpu, LineCase(gpu, d, f, ne, t, S.META_BF16, ne, True))
 
 
 @pytest.mark.parametrize("d,f,bits,meta", [(320, 640, 4, S.META_BF16), (1088, 704, 8, S.META_F16)])
@@ -723,23 +765,7 @@ RANGE_CASES = [  # d, f, experts, tokens, bits, shape
 
 @pytest.mark.parametrize("d,f,ne,t,bits", [c[:-1] for c in RANGE_CASES])
 def test_pair_ranges_of_each_shape_equal_the_whole_chunk(gpu, d, f, ne, t, bits):
-    """Ranges that start and end inside row tiles, one of a single pair and one to the chunk's end: their pairs' rows are the whole
-    call's bytes, and no others are written."""
-    k = 4
-    L = Layer(0x5EED0B00 + d, d, f, ne, k, bits=bits)
-    pc = PrefillCase(gpu, L, t, scale=row_scale(d, f))
-    want = pc.run()
-    order = pc.routes.download()["sorted_pairs"].astype(int)  # token, expert, rank, weight
-    at = order[:, 0] * k + order[:, 2]
-    for lo, count in ((37, 203), (t * k - 90, 90), (130, 1)):
-        pc.partials = gpu.dev(np.full(t * k * d, 0xD4D0, np.uint16))
-        pc.pf.encode_streamed_batched(pc.dl.pool, pc.dl.off, pc.routes, pc.hidden, pc.stride, pc.partials, pc.ws, t, k, lo, count)
-        gpu.synchronize()
-        got = pc.partials.download(np.uint16, t * k * d).reshape(t * k, d)
-        inside = np.zeros(t * k, bool)
-        inside[at[lo:lo + count]] = True
-        assert np.array_equal(got[inside], want.reshape(t * k, d)[inside]), f"pairs {lo} to {lo + count}"
-        assert np.all(got[~inside] == 0xD4D0), f"pairs {lo} to {lo + count}: a row of another pair was written"
+    check_pair_ranges(gpu, PrefillCase(gpu, Layer(0x5EED0B00 + d, d, f, ne, 4, bits=bits), t, scale=row_scale(d, f)))
 
 
 def test_reduce_and_residual_bit_exact(gpu):
