@@ -86,6 +86,12 @@ __device__ __forceinline__ float butterfly_from_32(float v) {
     v = __fadd_rn(v, dpp_f32<0x4E>(v));   // quad_perm [2,3,0,1]
     return __fadd_rn(v, dpp_f32<0xB1>(v));  // quad_perm [1,0,3,2]
 }
+// o = 4, 2, 1, whatever the other eight lanes of sixteen hold
+__device__ __forceinline__ float butterfly_from_4(float v) {
+    v = __fadd_rn(v, dpp_f32<0x141>(dpp_f32<0x1B>(v)));  // the quad reversed, then the half row mirrored: lane ^ 3 ^ 7
+    v = __fadd_rn(v, dpp_f32<0x4E>(v));
+    return __fadd_rn(v, dpp_f32<0xB1>(v));
+}
 // o = 1, 2, 4: sums of eight neighbouring lanes
 __device__ __forceinline__ float butterfly_of_8(float v) {
     v = __fadd_rn(v, dpp_f32<0xB1>(v));

@@ -51,25 +51,6 @@ __device__ __forceinline__ void split_stage(float *v, uint32_t lane) {
         }
     }
 }
-// A whole stage on one sum: every lane adds the lane at the distance.
-template <uint32_t DISTANCE>
-__device__ __forceinline__ float xor_add(float v) {
-    if constexpr (DISTANCE == 32u) {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    } else if constexpr (DISTANCE == 16u) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        return __fadd_rn(__uint_as_float(r[0]), __uint_as_float(r[1]));
-    } else if constexpr (DISTANCE == 8u) {
-        return __fadd_rn(v, dpp_f32<0x128>(v));                // row_ror:8
-    } else if constexpr (DISTANCE == 4u) {
-        return __fadd_rn(v, dpp_f32<0x141>(dpp_f32<0x1B>(v)));  // quad reversed, then the half row mirrored: lane ^ 3 ^ 7
-    } else if constexpr (DISTANCE == 2u) {
-        return __fadd_rn(v, dpp_f32<0x4E>(v));                 // quad_perm [2,3,0,1]
-    } else {
-        return __fadd_rn(v, dpp_f32<0xB1>(v));                 // quad_perm [1,0,3,2]
-    }
-}
 
 template <int RK, int MAXC, int ROWS, uint32_t TPS>
 __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t query_count, uint32_t stride, float *logits,
@@ -216,8 +197,8 @@ __global__ __launch_bounds__(256) void k_prefill_logits(RouterArgs a, uint32_t q
         split_stage<kSums, 0>(v, lane);
         split_stage<kSums / 2u, 1>(v, lane);
         if constexpr (kSums == 8u) split_stage<2u, 2>(v, lane);
-        else v[0] = xor_add<8>(v[0]);
-        v[0] = xor_add<1>(xor_add<2>(xor_add<4>(v[0])));
+        else v[0] = __fadd_rn(v[0], dpp_f32<0x128>(v[0]));  // row_ror:8
+        v[0] = butterfly_from_4(v[0]);
         // which sum this lane holds: one bit a split, from the first split (xor 32) down
         constexpr uint32_t kSplits = kSums == 8u ? 3u : 2u;
         const uint32_t mine = lane >> (6u - kSplits);
@@ -290,12 +271,11 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     const uint32_t l_row = lane >> 2, l_chunk = ((lane & 3u) ^ ((l_row >> 2) & 3u)) + 16u * wave;
     const uint8_t *w_row = static_cast<const uint8_t *>(a.weights) + size_t(min(e0 + l_row, num_experts - 1u)) * chunks * 16u;
     const uint16_t *x_row = a.hidden + size_t(min(t0 + l_row, query_count - 1u)) * stride;
-    constexpr uint32_t kOrder[4] = {0, 2, 1, 3};  // of j: the butterfly's
+    auto order = [](uint32_t step) { return step == 1u ? 2u : step == 2u ? 1u : step; };  // of j: the butterfly's
     const uint32_t units = 4u * walks;
     uint32_t ask_j = 0, ask_i = 0, ask_place = 0;  // the unit to ask for next: its step, its walk, its place
     auto ask = [&]() {
-        const uint32_t j = ask_j == 1u ? 2u : ask_j == 2u ? 1u : ask_j;
-        const uint32_t c = min(4u * j + l_chunk + 64u * ask_i, chunks - 1u), at = lds0 + ask_place * unit_bytes;  // past the row: a copy, taken as zero
+        const uint32_t c = min(4u * order(ask_j) + l_chunk + 64u * ask_i, chunks - 1u), at = lds0 + ask_place * unit_bytes;  // past the row: a copy, taken as zero
         if (RK != 4 || wave < blocks) {  // (a wave of the others always has chunks, and the branch is not free: 4,096 fp16 tokens 67.5, 69.1 us)
 #pragma unroll
             for (uint32_t q = 0; q < Q; ++q) lds_load16(at + (wave * Q + q) * 1024u, x_row + c * E + q * 8u);
@@ -399,10 +379,10 @@ __global__ __launch_bounds__(256, 4) void k_prefill_logits_mfma(RouterArgs a, ui
     for (uint32_t step = 0; step < 4u; ++step) {
         acc = f32x16_t{0};
         // (the walk that may end past the row is on its own: in one loop with the others the sums went from register to register)
-        for (uint32_t i = 0; i + 1u < walks; ++i) chunk(take(), kOrder[step], i, std::false_type{});
+        for (uint32_t i = 0; i + 1u < walks; ++i) chunk(take(), order(step), i, std::false_type{});
         const uint32_t last = take();
-        if (64u * walks == chunks) chunk(last, kOrder[step], walks - 1u, std::false_type{});
-        else chunk(last, kOrder[step], walks - 1u, std::true_type{});
+        if (64u * walks == chunks) chunk(last, order(step), walks - 1u, std::false_type{});
+        else chunk(last, order(step), walks - 1u, std::true_type{});
 #pragma unroll
         for (uint32_t r = 0; r < 4u; ++r) {
             const float v = __fadd_rn(__fadd_rn(acc[r], acc[8u + r]), __fadd_rn(acc[4u + r], acc[12u + r]));

@@ -90,9 +90,7 @@ __device__ __forceinline__ float eighth_sum(const uint32_t (&w)[4]) {
         sum = __fadd_rn(sum, f16_to_f32(uint16_t(w[t])));
         sum = __fadd_rn(sum, f16_to_f32(uint16_t(w[t] >> 16)));
     }
-    sum = __fadd_rn(sum, dpp_f32<0xB1>(sum));  // the lane at distance 1, 2, and (its quad being equal) 4
-    sum = __fadd_rn(sum, dpp_f32<0x4E>(sum));
-    return __fadd_rn(sum, dpp_f32<0x141>(sum));
+    return butterfly_of_8(sum);
 }
 
 // The two fp16 values of a word, added to c in fp32.
