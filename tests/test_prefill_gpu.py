@@ -101,7 +101,7 @@ def test_prefill_router_takes_effective_scales_at_any_element(gpu, router_bits, 
 
 
 @pytest.mark.parametrize("values", ["infinite", "subnormal", "cancelling"])
-@pytest.mark.parametrize("router_bits,ne,d,t", [(0, 241, 2112, 390), (8, 241, 1088, 273), (4, 241, 2176, 273)])
+@pytest.mark.parametrize("router_bits,ne,d,t", [(0, 241, 2112, 390), (8, 241, 1088, 273), (4, 241, 2176, 273), (4, 241, 576, 273)])
 def test_prefill_router_on_the_matrix_cores_takes_any_values(gpu, router_bits, ne, d, t, values):
     """Rows that end inside a walk of chunks, on the matrix cores: an infinite effective scale, products and sums down to
     fp32's smallest subnormals, neighbours that cancel to their last bit."""
