@@ -42,7 +42,7 @@ __device__ __forceinline__ void lds_load16(uint32_t lds, const void *p) {
 // (v_readlane of a spilled one), a memory instruction that reads it needs five wait states, which the compiler keeps for
 // instructions that it knows and this one is not; the scalar unit waits by itself, and so does what reads its result. (The move
 // stands where the wait state behind the write of m0 would.)
-template <bool ONCE = false>  // ONCE: non-temporal, of whole lines that nobody else reads
+template <bool ONCE = false>  // ONCE: non-temporal, for whole lines only: the hint drops a line between its halves
 __device__ __forceinline__ void lds_load16(uint32_t lds, const void *base, uint32_t offset) {
     const void *moved;
     if constexpr (ONCE) asm volatile("s_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0 nt" : "=&s"(moved) : "{m0}"(lds), "v"(offset), "s"(base) : "memory");

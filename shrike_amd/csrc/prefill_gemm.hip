@@ -148,7 +148,7 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 // the reads of the rows that the next chain takes, and the wait for the next group's loads stands two chains ahead of their
 // use. What bounds it now: with many rows the power that matrix work, its operands' way through LDS and the loads take
 // together (2,048 gpt-oss tokens back to back: the clock at 1.95 GHz of 2.4; the kWide gate/up launch keeps the matrix pipe
-// busy 44 % of the cycles, vector issue 43 %); with few rows the weights' bytes (kLines, 8-bit, 1,000 tokens: 4.9 TB/s), and the start and
+// busy 47 % of the cycles, vector issue 45 %); with few rows the weights' bytes (kLines, 8-bit, 1,000 tokens: 4.9 TB/s), and the start and
 // the end of the many short workgroups (256 experts of 2,048 x 512, 512 tokens: 29 % of the workgroups' time in gate/up and 53 % in
 // down lie outside the loop, 27 of 69 us; 37 tokens: 29 and 56 %). Both products, a chain scaled where it ends ->
 // pipelined: 32 experts of 2,880 x 2,880, 4-bit, 2,048 tokens 540 -> 495 us, 300 tokens 179 -> 164; 256 of 2,048 x 512, 4,096
@@ -156,11 +156,11 @@ typedef uint32_t u32x4_by2 __attribute__((ext_vector_type(4), aligned(2)));  // 
 //
 // kLines: what a card's memory gives depends on how it is asked. Read once and non-temporally, in whole 128-byte lines, 1.2 GB come
 // at 7.1 TB/s; without the hint at 6.2; in halves of a line, a group of 64 codes a row as the other shapes ask for 8-bit ones, at
-// 5.9, and at 4.4 with the hint, which drops a line between its halves. So a unit of codes is a line (two groups) of the rows of one
+// 5.7, and at 4.7 with the hint, which drops a line between its halves. So a unit of codes is a line (two groups) of the rows of one
 // of a wave's two tiles, three such places take the room of three half-line ones, and the wave takes a unit into registers as soon
 // as it has landed, so that its place is asked for again two groups early. Both products of 1,000 kimi tokens (8-bit): 453 -> 407 us;
 // whole passes 551 -> 505 us, of 60 uneven tokens 108 -> 95, 17 tokens of 256 x 2,048 x 512 100 -> 92. What is left: the loads alone
-// take 214 of the gate/up launch's 257 us. (Four places for tiles of up to 32 rows 263 -> 257 us, the loads dealt over the
+// take 221 of the gate/up launch's 240 us and 97 of down's 137. (Four places for tiles of up to 32 rows 263 -> 257 us, the loads dealt over the
 // MFMAs that follow a meeting 260 -> 258, the group sums straight to registers 260 -> 258 and elsewhere slower: taken back. The
 // same for 4-bit codes: 1,000 even kimi tokens 352 -> 334 us, uneven ones 264 -> 271, 100 tokens of 256 x 2,048 x 512 137 -> 139.)
 //
